@@ -1,6 +1,7 @@
-"""ctypes binding of libmortar_hip.so (the C-ABI declared in include/mortar_hip.h).
+"""ctypes binding of libmortar_hip.so (the C-ABI declared in include/mortar_hip.h) and the native call layer above it
+(_mortar_native.so, csrc/mortar_torch.cpp).
 
-There is no fallback: if the library is missing or a call fails, a RuntimeError is raised.
+There is no fallback: if a library is missing or a call fails, a RuntimeError is raised.
 """
 from __future__ import annotations
 
@@ -9,6 +10,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmortar_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "_mortar_native.so")
 
 c_i32, c_i64, c_vp, c_f32 = C.c_int32, C.c_int64, C.c_void_p, C.c_float
 
@@ -84,8 +86,14 @@ _SIGS = {
                                            c_vp, c_i32, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp]),
 }
 
+class PackHandle(C.Structure):
+    """One packed matrix for the native call layer: its mortar_bcsr_t and the schedules built so far."""
+    _fields_ = [("w", c_vp), ("sched1", c_vp), ("sched2", c_vp)]
+
+
 EXPORTS = tuple(_SIGS)
 _lib = None
+_native = None
 
 
 def lib():
@@ -102,6 +110,23 @@ def lib():
             fn.restype, fn.argtypes = res, args
         _lib = l
     return _lib
+
+
+def native():
+    """The native call layer.  Raises if it has not been built."""
+    global _native
+    if _native is None:
+        lib()                                   # one copy of the library for both bindings
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(f"{NATIVE_PATH} is missing: the native call layer has not been built "
+                               "(run __graft_entry__.build() or `python build.py` in the package directory)")
+        import importlib.machinery
+        import importlib.util
+        loader = importlib.machinery.ExtensionFileLoader("_mortar_native", NATIVE_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mortar_native", loader))
+        loader.exec_module(mod)
+        _native = mod
+    return _native
 
 
 def check(rc: int, what: str) -> int:

@@ -6,8 +6,11 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from . import ops
+from . import _lib, ops
 from .pack import MortarPack
+from .routing import TileRouter
+
+_module = torch.nn.modules.module
 
 
 def mortar_pack_strips(cms) -> MortarPack:
@@ -47,8 +50,30 @@ class MortarDecodeMLP:
         self.norm_weight, self.eps, self.iter_idx = norm_weight, eps, iter_idx
         self.d_ff = mlp.d_ff
 
-    @torch.no_grad()
     def __call__(self, x: Tensor, gates: Tensor | None = None) -> Tensor:
+        mlp = self.mlp
+        if gates is None and not (mlp._forward_hooks or mlp._forward_pre_hooks or _module._global_forward_hooks or _module._global_forward_pre_hooks):
+            y = self._native(mlp, x)
+            if y is not None:
+                return y
+        return self._general(x, gates)
+
+    def _native(self, mlp, x: Tensor):
+        """The whole step as one native call; None when the layers are not deployed packs or the call is not covered."""
+        pair = mlp.native_pair()
+        if pair is None:
+            return None
+        rt = mlp._modules.get("router")
+        if rt is None:
+            return _lib.native().mlp(x, *pair, True, True, self.norm_weight, self.eps)
+        if type(rt) is not TileRouter or mlp.gate_up._cms._pack is not self.Mgu or mlp.down._cms._pack is not self.Mdown:
+            return None
+        proj, norm = rt._modules["query_proj"], rt._modules["query_norm"]
+        return _lib.native().routed_decode(x, *pair, self.norm_weight, self.eps, rt._parameters, proj._parameters, norm._parameters,
+                                           (rt.n_iters, rt.n_sub_keys, rt.n_tile_groups, rt.activation_k), norm.eps, self.iter_idx)
+
+    @torch.no_grad()
+    def _general(self, x: Tensor, gates: Tensor | None = None) -> Tensor:
         B = x.shape[0]
         rt = getattr(self.mlp, "router", None)
         if (gates is not None or rt is None) and ops.norm_fusable(self.Mgu):

@@ -10,7 +10,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from . import ops
+from . import _lib, ops
 from .sparsity import MortarLinear
 
 
@@ -123,11 +123,32 @@ class _SwiGLUMortar(nn.Module):
         return any(isinstance(getattr(m._cms, "mortar_data", None), torch.nn.Parameter) and m._cms.mortar_data.requires_grad
                    and "mortar_packed" not in m._cms._buffers for m in (self.gate_up, self.down))
 
+    def native_pair(self) -> tuple | None:
+        """Handles (gate_up, down) for the native call layer when both layers hold a deployed pack (mortar_packed) in the
+        runtime's blocking, else None.  A pack that was dropped (moved, loaded again) or a layer that was replaced is
+        noticed by identity."""
+        gu, dn = self._modules["gate_up"]._modules["_cms"], self._modules["down"]._modules["_cms"]
+        c = self.__dict__.get("_native_cache")
+        if c is None or c[0] is not gu._pack or c[1] is not dn._pack or c[2] is not gu or c[3] is not dn:
+            if not all(m._mortar and m._mortar_blocking == 16 and "mortar_packed" in m._buffers and m._pack is not None for m in (gu, dn)):
+                return None
+            if gu._pack.Rb % 2 or gu._pack.Rb != 2 * dn._pack.Cb or not gu._pack.codes.is_cuda:
+                return None
+            c = self.__dict__["_native_cache"] = (gu._pack, dn._pack, gu, dn, (gu._pack.handle(2), dn._pack.handle(1)))
+        return c[4]
+
     def forward(self, x: Tensor, iter_idx: int = 0, gates: Tensor | None = None, norm: tuple | None = None) -> Tensor:
         """x [..., d_model] -> [..., d_model].  ``gates`` overrides the router output (fp32 [N, n_clusters]);
         it exists so that a caller which already evaluated the router (or holds seeded logits) can feed it.
         ``norm`` = (weight or None, eps): x is the activation BEFORE the block's RMSNorm (norm_mlp) and the norm is
         applied here, inside the gate_up launch when the matrix allows it; same result as mlp(rmsnorm(x))."""
+        if gates is None and "router" not in self._modules:
+            pair = self.native_pair()
+            if pair is not None:
+                nw, eps = norm if norm is not None else (None, 0.0)
+                y = _lib.native().mlp(x, *pair, False, norm is not None, nw, eps)
+                if y is not None:
+                    return y
         train = self._carved() and self._wants_grad(x)
         if norm is not None:
             fused = (self._carved() and x.is_cuda and not train and (self.router is None or gates is not None)

@@ -290,8 +290,20 @@ class MortarPack:
         self._pos = self._ws = self._status = self.src_block = self._sdd = None
         self._status_host = self._status_event = None
         self._transposed: "MortarPack | None" = None
+        self._bind_struct()
+
+    def _bind_struct(self) -> None:
+        """(Re)builds what the entry points take this matrix by: the C struct, its reference, the native call layer's handle."""
         self.struct = self._make_struct()
         self.ref = C.byref(self.struct)
+        self._handle = _lib.PackHandle(C.addressof(self.struct), None, None)
+        for rpu, t in self._scheds.items():
+            setattr(self._handle, f"sched{rpu}", t.data_ptr())
+
+    def handle(self, rows_per_unit: int) -> int:
+        """Address of the native call layer's handle, with the schedule for plain (1) or gate/up (2) units in place."""
+        self.sched(rows_per_unit)
+        return C.addressof(self._handle)
 
     def _make_struct(self):
         return _lib.BcsrStruct(self.codes.data_ptr(), self.sdup.data_ptr(), self.col.data_ptr(),
@@ -325,8 +337,7 @@ class MortarPack:
             v.codes4_o = None
             v._scheds, v._worklists, v._transposed, v._dview = {}, {}, None, {}
             v._h_codes = v._h_sdup = None
-            v.struct = v._make_struct()
-            v.ref = C.byref(v.struct)
+            v._bind_struct()
             self._dview[tile] = v
         return self._dview[tile]
 
@@ -483,7 +494,8 @@ class MortarPack:
             if self.nseg > 1:
                 o = unit_order_segments(self.h_row_desc, self.Rb, self.nseg, rows_per_unit, o)
             sc = schedule(self.h_row_desc, self.Rb, self.nseg, rows_per_unit, o)
-            self._scheds[rows_per_unit] = torch.from_numpy(sc).to(self.device)
+            self._scheds[rows_per_unit] = t = torch.from_numpy(sc).to(self.device)
+            setattr(self._handle, f"sched{rows_per_unit}", t.data_ptr())
         return self._scheds[rows_per_unit]
 
     def worklist(self, rows_per_unit: int, kseg: int, max_blocks: int):
@@ -508,6 +520,5 @@ class MortarPack:
         c._scheds = {k: v.clone() for k, v in self._scheds.items()}
         c._worklists = {k: (v[0].clone(), v[1], v[2].clone(), v[3]) for k, v in self._worklists.items()}
         c._transposed, c._dview = None, {}      # the clone builds its own views
-        c.struct = c._make_struct()
-        c.ref = C.byref(c.struct)
+        c._bind_struct()
         return c
