@@ -270,10 +270,24 @@ int mortar_router_bf16(const void *x, int32_t x_is_f32, int64_t B, int32_t d, in
                        const float *kb, int32_t nsk, const float *bias, int32_t n, int32_t k, float *qv,
                        float *logits_out, float *gates, uint8_t *active, void *stream);
 
-/* The router behind a library GEMM, for prefill-sized calls: TileRouter.forward steps 2-8 (morph/model/routing.py:188-284)
- * on the projected query qv = x Wq^T (fp32 [N, d], row stride ldq; the dense projection of step 1, routing.py:181-186,
- * is a plain GEMM and stays with the caller's BLAS).  q = LayerNorm(qv + iter_vec), sub-key scores, product-key logits
- * (direct, wrapped or ranked exactly as in mortar_router_bf16), gating tail as mortar_remoe_gates: one launch instead
+/* The router's dense query projection for prefill-sized calls (routing.py:181-186): qv[m, o] = sum_i x[m, i] wq[o, i] for
+ * bf16 x [M, d_in] (row stride ldx, a multiple of 8) and fp32 wq [d_out, d_in], qv fp32 [M, d_out] (row stride ldq, a
+ * multiple of 4); d_in a multiple of 8, d_out of 4, everything 16-byte aligned.  Exact products (the weights enter the
+ * matrix cores as three bf16 terms that add up to them), fp32 sums. */
+int mortar_router_project_bf16(const uint16_t *x, int64_t M, int32_t d_in, int64_t ldx, const float *wq, int32_t d_out,
+                               float *qv, int64_t ldq, void *stream);
+
+/* The load statistics behind the gates (routing.py:262-284), n <= 1024 groups: ema[g] = alpha ema[g] + one_minus_alpha *
+ * (share of the M tokens with gates[m, g] > 0), in place, and *aux = coeff * var over the groups (unbiased) of the mean gate.
+ * workspace: mortar_router_stats_workspace_bytes(M, n) bytes. */
+int64_t mortar_router_stats_workspace_bytes(int64_t M, int32_t n);
+int mortar_router_stats(const float *gates, int64_t M, int32_t n, float alpha, float one_minus_alpha, float coeff, float *ema,
+                        float *aux, void *workspace, void *stream);
+
+/* The router behind the projection, for prefill-sized calls: TileRouter.forward steps 2-8 (morph/model/routing.py:188-284)
+ * on the projected query qv = x Wq^T (fp32 [N, d], row stride ldq; the dense projection of step 1, routing.py:181-186:
+ * mortar_router_project_bf16, or the caller's BLAS for fp32 activations).  q = LayerNorm(qv + iter_vec), sub-key scores, product-key logits
+ * (direct, wrapped or ranked exactly as in mortar_router_bf16), gating tail as mortar_remoe_gates: one or two launches instead
  * of the reference's layer_norm, two matmuls, broadcast add, topk, bias add, topk, relu, sum, divide.
  * iter_vec fp32 [d] or NULL; ln_w, ln_b fp32 [d]; ka, kb fp32 [nsk, d/2]; bias fp32 [n]; all 16-byte aligned.
  * logits_out fp32 [N, n] or NULL; gates fp32 [N, n]; active uint8 [N, n] or NULL.  d a multiple of 8 up to 8192,

@@ -8,6 +8,8 @@
 #include "mortar_device.h"
 #include "mortar_internal.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int MAXPL_LIMIT = 16;   // logits per lane -> n <= 1024
@@ -192,52 +194,78 @@ __device__ __forceinline__ float block_sum256(float v, float *red) {      // red
     return red[0] + red[1] + red[2] + red[3];
 }
 
+// The value of lane (lane ^ X), X a power of two: DPP within quads and 16-lane rows, the LDS crossbar for 4, half-wave and
+// row swaps of gfx950 for 16 and 32.
+template <int X>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+    if constexpr (X == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true);          // quad_perm [1,0,3,2]
+    else if constexpr (X == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true);     // quad_perm [2,3,0,1]
+    else if constexpr (X == 4) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x101F);                // xor 4
+    else if constexpr (X == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true);    // row_ror:8
+    else return (uint32_t)__shfl_xor((int)v, X, 64);
+}
+
 // Descending bitonic sort of 64 * KPL keys held KPL per lane (element lane * KPL + r in register r): steps between
-// elements of one lane are register compare-exchanges, steps between lanes one shuffle per register.  No LDS, no barrier.
-template <int KPL>
-__device__ __forceinline__ void wave_sort_desc(uint32_t (&key)[KPL], int lane) {
-    for (int k2 = 2; k2 <= 64 * KPL; k2 <<= 1) {
-        const bool lane_desc = ((lane * KPL) & k2) == 0;       // direction of this lane's elements once k2 >= KPL
-        for (int lj = k2 / (2 * KPL); lj >= 1; lj >>= 1) {       // partners in other lanes (distance j = lj * KPL)
-            const bool keep_max = ((lane & lj) == 0) == lane_desc;
+// elements of one lane are register compare-exchanges, steps between lanes one exchange per register.  No LDS memory, no
+// barrier.  Fully unrolled: every exchange distance is a constant (lane_xor), which a loop over shuffles cannot have.
+template <int KPL, int LJ>
+__device__ __forceinline__ void sort_lane_step(uint32_t (&key)[KPL], bool keep_max) {
+#pragma unroll
+    for (int r = 0; r < KPL; ++r) {
+        const uint32_t a = key[r], o = lane_xor<LJ>(a);
+        const uint32_t hi = a > o ? a : o, lo = a > o ? o : a;
+        key[r] = keep_max ? hi : lo;
+    }
+}
+template <int KPL, int K2>
+__device__ __forceinline__ void sort_stage(uint32_t (&key)[KPL], int lane) {
+    const bool lane_desc = ((lane * KPL) & K2) == 0;           // direction of this lane's elements once K2 >= KPL
+    auto step = [&](auto lj) {
+        constexpr int LJ = decltype(lj)::value;
+        if constexpr (LJ * KPL * 2 <= K2) sort_lane_step<KPL, LJ>(key, ((lane & LJ) == 0) == lane_desc);
+    };
+    step(std::integral_constant<int, 32>{});
+    step(std::integral_constant<int, 16>{});
+    step(std::integral_constant<int, 8>{});
+    step(std::integral_constant<int, 4>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int j = KPL / 2; j > 0; j >>= 1) {                      // partners in this lane's registers (distance j < K2)
+        if (j < K2) {
 #pragma unroll
             for (int r = 0; r < KPL; ++r) {
-                const uint32_t a = key[r], o = (uint32_t)__shfl_xor((int)a, lj, 64);
-                key[r] = keep_max ? (a > o ? a : o) : (a > o ? o : a);
-            }
-        }
-#pragma unroll
-        for (int j = KPL / 2; j > 0; j >>= 1) {                  // partners in this lane's registers (distance j < k2)
-            if (j < k2) {
-#pragma unroll
-                for (int r = 0; r < KPL; ++r) {
-                    if ((r & j) == 0) {
-                        const bool desc = k2 < KPL ? (r & k2) == 0 : lane_desc;
-                        const uint32_t a = key[r], c = key[r | j];
-                        const uint32_t hi = a > c ? a : c, lo = a > c ? c : a;
-                        key[r] = desc ? hi : lo;
-                        key[r | j] = desc ? lo : hi;
-                    }
+                if ((r & j) == 0) {
+                    const bool desc = K2 < KPL ? (r & K2) == 0 : lane_desc;
+                    const uint32_t a = key[r], c = key[r | j];
+                    const uint32_t hi = a > c ? a : c, lo = a > c ? c : a;
+                    key[r] = desc ? hi : lo;
+                    key[r | j] = desc ? lo : hi;
                 }
             }
         }
     }
+    if constexpr (K2 < 64 * KPL) sort_stage<KPL, K2 * 2>(key, lane);
 }
+template <int KPL>
+__device__ __forceinline__ void wave_sort_desc(uint32_t (&key)[KPL], int lane) { sort_stage<KPL, 2>(key, lane); }
 
 // The n largest of the P = nsk * nsk product scores of one token in descending order (+ bias) -> lgt[0 .. n), on one wave.
 template <int KPL>
 __device__ __attribute__((noinline)) void ranked_logits(const float *sct, int nsk, int P, const float *bias, int n, float *lgt,
                                               float *logits_row, int lane) {
     uint32_t key[KPL];
+    int ia = lane * KPL / nsk, ib = lane * KPL - ia * nsk;      // product i = ia * nsk + ib
 #pragma unroll
     for (int r = 0; r < KPL; ++r) {
         const int i = lane * KPL + r;
         uint32_t kk = 0u;                                    // padding: the smallest key
         if (i < P) {
-            const uint32_t u = __float_as_uint(sct[i / nsk] + sct[nsk + i % nsk]);
+            const uint32_t u = __float_as_uint(sct[ia] + sct[nsk + ib]);
             kk = (u & 0x80000000u) ? ~u : (u | 0x80000000u);   // NaN ranks above +inf, as torch.topk has it
         }
         key[r] = kk;
+        if (++ib == nsk) { ib = 0; ++ia; }
     }
     wave_sort_desc<KPL>(key, lane);
 #pragma unroll
@@ -578,6 +606,156 @@ __global__ void __launch_bounds__(256, J == 8 ? 2 : 3) router_tail_group_kernel(
     }
 }
 
+// ---- the same tail in two launches (rows of up to 4096 values, up to 32 sub-keys) --------------------------------------
+// The group kernel above is one chain of latencies per 4 tokens (loads, LayerNorm, key rows one after another, then a sort
+// per wave with the other phases waiting): 62 us for 4096 tokens x 352 groups, 20 us of it bandwidth or arithmetic.  Cut in
+// two, each half fills the chip on its own terms:
+//   router_scores_kernel   16 tokens per workgroup; the 2 nsk dot products per token run on the fp32 matrix instructions
+//                          (16 keys x 16 tokens), so the key rows are read once per 16 tokens and no product needs a wave
+//                          reduction.  Wave w takes every fourth 16-value chunk of query half w / 4; a lane holds 4 values
+//                          of one token per chunk in registers from the one read of the row to the products.
+//   router_rank_kernel     one wave per token: logits (ranked when there are more products than groups), gating tail.
+// The scores travel in the token's own row of `gates` (2 nsk <= n), which the second kernel reads before it writes it.
+template <int KT, int CH>     // key tiles of 16 per half, chunks of 16 values per wave
+__global__ void __launch_bounds__(512) router_scores_kernel(const float *qv, int64_t N, int d, int64_t ldq, const float *iter_vec,
+                                                             const float *ln_w, const float *ln_b, float ln_eps, const float *ka,
+                                                             const float *kb, int nsk, int n, float *scores) {
+    __shared__ float red[2][8][16];
+    __shared__ __attribute__((aligned(16))) f32x4_t part[8][KT][64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tok = lane & 15, g = lane >> 4, half = wave >> 2, sub = wave & 3;
+    const int d2 = d / 2;
+    const int64_t t0 = (int64_t)blockIdx.x * 16;
+    const int64_t row = t0 + tok < N ? t0 + tok : N - 1;
+    const float4 zero4 = float4{0.f, 0.f, 0.f, 0.f};
+    const float *q = qv + row * ldq + half * d2, *iv = iter_vec ? iter_vec + half * d2 : nullptr;
+    // chunk j of this wave: values 16 (sub + 4 j) + 4 g .. + 3 of the half (d2 % 4 == 0: in or out as a whole)
+    auto at = [&](int j) { return 16 * (sub + 4 * j) + 4 * g; };
+    float4 v[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        const int i = at(j) < d2 ? at(j) : 0;
+        v[j] = *reinterpret_cast<const float4 *>(q + i);
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        if (iv) {
+            const float4 c = *reinterpret_cast<const float4 *>(iv + (at(j) < d2 ? at(j) : 0));
+            v[j].x += c.x; v[j].y += c.y; v[j].z += c.z; v[j].w += c.w;
+        }
+        if (at(j) >= d2) v[j] = zero4;
+        s += (v[j].x + v[j].y) + (v[j].z + v[j].w);
+    }
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if (g == 0) red[0][wave][tok] = s;
+    __syncthreads();
+    float mean = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) mean += red[0][w][tok];
+    mean /= (float)d;
+    s = 0.f;
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        if (at(j) < d2) {
+            const float a = v[j].x - mean, b = v[j].y - mean, c = v[j].z - mean, e = v[j].w - mean;
+            s = __builtin_fmaf(e, e, __builtin_fmaf(c, c, __builtin_fmaf(b, b, __builtin_fmaf(a, a, s))));
+        }
+    }
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if (g == 0) red[1][wave][tok] = s;
+    __syncthreads();
+    float var = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) var += red[1][w][tok];
+    const float rstd = 1.0f / sqrtf(var / (float)d + ln_eps);
+    const float *lw = ln_w + half * d2, *lb = ln_b + half * d2;
+    const float *kr[KT];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) kr[t] = (half ? kb : ka) + (int64_t)(t * 16 + tok < nsk ? t * 16 + tok : nsk - 1) * d2;
+    f32x4_t acc[KT];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // LayerNorm parameters and key pieces are fetched PF chunks ahead of their products
+    constexpr int PF = 4;
+    float4 pw[PF], pb[PF], pk[PF][KT];
+    auto fetch = [&](int j) {
+        const int i = at(j) < d2 ? at(j) : 0;
+        pw[j % PF] = *reinterpret_cast<const float4 *>(lw + i);
+        pb[j % PF] = *reinterpret_cast<const float4 *>(lb + i);
+#pragma unroll
+        for (int t = 0; t < KT; ++t) pk[j % PF][t] = *reinterpret_cast<const float4 *>(kr[t] + i);
+    };
+#pragma unroll
+    for (int j = 0; j < PF; ++j) fetch(j);
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        const bool in = at(j) < d2;
+        const float4 w = pw[j % PF], b = pb[j % PF];
+        float4 kk[KT];
+#pragma unroll
+        for (int t = 0; t < KT; ++t) kk[t] = pk[j % PF][t];
+        if (j + PF < CH) fetch(j + PF);
+        float4 x = v[j];
+        x = float4{(x.x - mean) * rstd * w.x + b.x, (x.y - mean) * rstd * w.y + b.y, (x.z - mean) * rstd * w.z + b.z, (x.w - mean) * rstd * w.w + b.w};
+        if (!in) x = zero4;
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+            const float4 k = kk[t];
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.x, x.x, acc[t], 0, 0, 0);
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.y, x.y, acc[t], 0, 0, 0);
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.z, x.z, acc[t], 0, 0, 0);
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k.w, x.w, acc[t], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < KT; ++t) part[wave][t][lane] = acc[t];
+    __syncthreads();
+    // the four waves of a half meet; wave 4 half + t (t < KT) finishes key tile t: lane (token, g) holds keys 16 t + 4 g + e
+    if (sub < KT && t0 + tok < N) {
+        const f32x4_t a = (part[half * 4][sub][lane] + part[half * 4 + 1][sub][lane]) + (part[half * 4 + 2][sub][lane] + part[half * 4 + 3][sub][lane]);
+        float *o = scores + (t0 + tok) * n + half * nsk;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (sub * 16 + 4 * g + e < nsk) o[sub * 16 + 4 * g + e] = a[e];
+    }
+}
+
+template <int MAXPL>
+__global__ void __launch_bounds__(256) router_rank_kernel(int64_t N, int nsk, const float *bias, int n, int k, float *logits_out, float *gates,
+                                                           uint8_t *active) {
+    extern __shared__ __attribute__((aligned(16))) float sm[];       // per wave: sc[2 nsk] | lg[n]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t tok = (int64_t)blockIdx.x * 4 + wave;
+    if (tok >= N) return;
+    float *sct = sm + wave * (2 * nsk + n), *lgt = sct + 2 * nsk, *lrow = logits_out ? logits_out + tok * n : nullptr;
+    float *grow = gates + tok * n;
+    const int P = nsk * nsk;
+    if (lane < 2 * nsk) sct[lane] = grow[lane];
+    auto wave_fence = [] {                   // LDS serves a wave's accesses in order; this keeps the compiler from moving them
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    wave_fence();
+    if (P > n) {
+        if (P <= 512) ranked_logits<8>(sct, nsk, P, bias, n, lgt, lrow, lane);
+        else ranked_logits<16>(sct, nsk, P, bias, n, lgt, lrow, lane);
+    } else {
+        for (int g = lane; g < n; g += 64) {
+            const int pr = g % P;
+            const float l = (sct[pr / nsk] + sct[nsk + pr % nsk]) + bias[g];
+            lgt[g] = l;
+            if (lrow) lrow[g] = l;
+        }
+    }
+    wave_fence();
+    remoe_gates_wave<MAXPL>(lgt, n, k, grow, active ? active + tok * n : nullptr, lane);
+}
+
 // Workgroup = (token tile, chunk of 64 clusters).  The tile's active bytes for the chunk are staged in LDS
 // with coalesced reads; then every wave compacts whole clusters: lanes = tokens, ballot -> prefix popcount.
 __global__ void __launch_bounds__(256) remoe_route_kernel(const uint8_t *active, int64_t M, int n, int tile,
@@ -751,6 +929,25 @@ extern "C" int mortar_router_tail_f32(const float *qv, int64_t N, int32_t d, int
     if ((int64_t)nsk * nsk > n && (int64_t)nsk * nsk > 1024)
         return mortar_fail(MORTAR_ERR_LIMIT, "router tail: %d x %d product keys for %d groups exceed the 1024 the kernel ranks", nsk, nsk, n);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (d <= 4096 && nsk <= 32 && 2 * nsk <= n) {      // two launches; wider rows, more keys or fewer groups than scores: one
+        const dim3 sg((unsigned)((N + 15) / 16)), rg((unsigned)((N + 3) / 4));
+        const int ch = (d / 2 + 63) / 64;
+#define MORTAR_SCORES(KT, CH) hipLaunchKernelGGL((router_scores_kernel<KT, CH>), sg, dim3(512), 0, st, qv, N, d, ldq, iter_vec, ln_w, ln_b, ln_eps, \
+                                                 ka, kb, nsk, n, gates)
+#define MORTAR_SCORESK(KT) do { if (ch <= 8) MORTAR_SCORES(KT, 8); else if (ch <= 16) MORTAR_SCORES(KT, 16); else MORTAR_SCORES(KT, 32); } while (0)
+        if (nsk <= 16) MORTAR_SCORESK(1);
+        else MORTAR_SCORESK(2);
+#undef MORTAR_SCORESK
+#undef MORTAR_SCORES
+        const size_t rs = (size_t)4 * (2 * nsk + n) * sizeof(float);
+        const int pl = (n + 63) / 64;
+#define MORTAR_RANK(PL) hipLaunchKernelGGL((router_rank_kernel<PL>), rg, dim3(256), rs, st, N, nsk, bias, n, k, logits_out, gates, active)
+        if (pl <= 2) MORTAR_RANK(2);
+        else if (pl <= 6) MORTAR_RANK(6);
+        else MORTAR_RANK(16);
+#undef MORTAR_RANK
+        return check_launch("router tail");
+    }
     // a thread holds J float4 pieces of every row of its group (J = 1, 2, 4 or 8 for d <= 1024 J) and tt = min(4, 8 / J)
     // tokens share a group, so the normalised rows take at most 32 KB of LDS
     const int J = d <= 1024 ? 1 : d <= 2048 ? 2 : d <= 4096 ? 4 : 8;

@@ -8,6 +8,8 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <algorithm>
+
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
@@ -97,12 +99,12 @@ int run_mlp(const PackHandle *gu, const PackHandle *dn, const at::Tensor &x, int
     return rc;
 }
 
-// mlp(x, gate_up handle, down handle, decode, norm, norm_w, eps) -> y: the carved MLP on the rows of x.
-// decode: x [B, ...] is one row per stream and y is [B, 1, d] whatever autograd records (MortarDecodeMLP); otherwise y
+// mlp(x, gate_up handle, down handle, decode, norm, norm_w, eps, gates) -> y: the carved MLP on the rows of x.
+// gates: None or fp32 [..., n_clusters], one row per row of x.  decode: x [B, ...] is one row per stream and y is [B, 1, d] whatever autograd records (MortarDecodeMLP); otherwise y
 // has the shape of x and a call that autograd would record is declined.
 PyObject *py_mlp(PyObject *, PyObject *const *a, Py_ssize_t na) {
-    if (na != 7) {
-        PyErr_SetString(PyExc_TypeError, "mlp: 7 arguments");
+    if (na != 8) {
+        PyErr_SetString(PyExc_TypeError, "mlp: 8 arguments");
         return nullptr;
     }
     const at::Tensor *xt = tensor_of(a[0]);
@@ -118,6 +120,16 @@ PyObject *py_mlp(PyObject *, PyObject *const *a, Py_ssize_t na) {
     Norm n;
     if (norm && !read_norm(a[5], PyFloat_AsDouble(a[6]), d, x, n)) Py_RETURN_NONE;
     if (PyErr_Occurred()) return nullptr;
+    const float *gates = nullptr;
+    int64_t ncl = 0;
+    if (a[7] != Py_None) {
+        const at::Tensor *gt = tensor_of(a[7]);
+        const int64_t f = (int64_t)gu->w->Rb * 8;
+        if (!gt || gt->scalar_type() != at::kFloat || gt->device() != x.device() || gt->dim() < 1 || !gt->is_contiguous()) Py_RETURN_NONE;
+        ncl = gt->size(-1);
+        if (ncl <= 0 || gt->numel() != M * ncl || f % ncl || (f / ncl) % 4) Py_RETURN_NONE;
+        gates = static_cast<const float *>(gt->const_data_ptr());
+    }
     const int64_t dy = (int64_t)dn->w->Rb * 16;
     const c10::DeviceGuard guard(x.device());
     at::Tensor y;
@@ -128,7 +140,7 @@ PyObject *py_mlp(PyObject *, PyObject *const *a, Py_ssize_t na) {
         shape.back() = dy;
         y = new_bf16(x, shape);
     }
-    const int rc = run_mlp(gu, dn, x, M, n, nullptr, 0, u16m(y), stream_of(x));
+    const int rc = run_mlp(gu, dn, x, M, n, gates, (int)ncl, u16m(y), stream_of(x));
     if (rc) return raise_rc(rc, "mortar_mlp");
     return THPVariable_Wrap(std::move(y));
 }
@@ -212,6 +224,65 @@ PyObject *py_routed_decode(PyObject *, PyObject *const *a, Py_ssize_t na) {
     return THPVariable_Wrap(std::move(y));
 }
 
+// route(x, own, proj, norm, shape, ln_eps, iter_idx, ema, alpha, coeff) -> (gates [M, n], active [M, n], aux): the router of
+// the M rows of x, without autograd.  With ema (the load statistics buffer, fp32 [n]) the statistics are updated in place
+// and aux is the load-balance loss; with ema = None aux is None.
+PyObject *py_route(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 10 || !PyTuple_Check(a[4]) || PyTuple_GET_SIZE(a[4]) != 4) {
+        PyErr_SetString(PyExc_TypeError, "route: 10 arguments");
+        return nullptr;
+    }
+    int64_t sh[4];
+    for (int i = 0; i < 4; ++i) sh[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(a[4], i));
+    const double ln_eps = PyFloat_AsDouble(a[5]), alpha = PyFloat_AsDouble(a[8]), coeff = PyFloat_AsDouble(a[9]);
+    const int64_t it = PyLong_AsLongLong(a[6]), nsk = sh[1], n = sh[2];
+    if (PyErr_Occurred()) return nullptr;
+    const at::Tensor *xt = tensor_of(a[0]);
+    if (!xt || c10::GradMode::is_enabled() || xt->dim() < 1) Py_RETURN_NONE;
+    const at::Tensor &x = *xt;
+    const int64_t d = x.size(-1);
+    if (d % 8 || d > 8192 || nsk <= 0 || n <= 0 || n > 1024 || !is_rows(x, d)) Py_RETURN_NONE;
+    const int64_t M = x.numel() / d;
+    const bool small = M <= DECODE_MAX_ROWS;
+    if (nsk * nsk > (small ? 2048 : std::max<int64_t>(1024, n))) Py_RETURN_NONE;
+    RouterParams r;
+    if (!read_router(a[1], a[2], a[3], it, sh[0], nsk, n, d, x, r)) Py_RETURN_NONE;
+    const at::Tensor *ema = a[7] == Py_None ? nullptr : tensor_of(a[7]);
+    if (a[7] != Py_None && (!ema || ema->scalar_type() != at::kFloat || ema->device() != x.device() || ema->dim() != 1 || ema->size(0) != n ||
+                            !ema->is_contiguous()))
+        Py_RETURN_NONE;
+    const c10::DeviceGuard guard(x.device());
+    void *st = stream_of(x);
+    const auto f32 = x.options().dtype(at::kFloat).requires_grad(false);
+    at::Tensor gates = at::empty({M, n}, f32), active = at::empty({M, n}, f32.dtype(at::kByte)), aux;
+    float *gp = static_cast<float *>(gates.data_ptr());
+    uint8_t *ap = static_cast<uint8_t *>(active.data_ptr());
+    const at::Tensor qvt = at::empty({M, d}, f32);
+    float *qv = static_cast<float *>(qvt.data_ptr());
+    int rc;
+    if (small) {
+        rc = mortar_router_bf16(u16(x), 0, M, (int32_t)d, d, r.wq, r.iter_vec, r.ln_w, r.ln_b, (float)ln_eps, r.ka, r.kb, r.nsk, r.bias, r.n,
+                                (int32_t)sh[3], qv, nullptr, gp, ap, st);
+    } else {
+        rc = mortar_router_project_bf16(u16(x), M, (int32_t)d, d, r.wq, (int32_t)d, qv, d, st);
+        if (rc == MORTAR_OK)
+            rc = mortar_router_tail_f32(qv, M, (int32_t)d, d, r.iter_vec, r.ln_w, r.ln_b, (float)ln_eps, r.ka, r.kb, r.nsk, r.bias, r.n,
+                                        (int32_t)sh[3], nullptr, gp, ap, st);
+    }
+    if (rc == MORTAR_OK && ema) {
+        aux = at::empty({}, f32);
+        const at::Tensor ws = at::empty({mortar_router_stats_workspace_bytes(M, r.n)}, f32.dtype(at::kByte));
+        rc = mortar_router_stats(gp, M, r.n, (float)alpha, (float)(1.0 - alpha), (float)coeff, static_cast<float *>(ema->data_ptr()),
+                                 static_cast<float *>(aux.data_ptr()), ws.data_ptr(), st);
+    }
+    if (rc) return raise_rc(rc, "mortar_route");
+    PyObject *g = THPVariable_Wrap(std::move(gates)), *ac = THPVariable_Wrap(std::move(active));
+    PyObject *au = Py_None;
+    if (aux.defined()) au = THPVariable_Wrap(std::move(aux));
+    else Py_INCREF(Py_None);
+    return Py_BuildValue("(NNN)", g, ac, au);
+}
+
 template <PyObject *(*F)(PyObject *, PyObject *const *, Py_ssize_t)>
 PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t na) {      // torch's C++ exceptions (out of memory) as Python ones
     HANDLE_TH_ERRORS
@@ -223,6 +294,7 @@ PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t na) {      // t
 PyMethodDef methods[] = {
     MORTAR_METHOD("mlp", py_mlp, "The carved MLP on the rows of x, or None when the call is not covered."),
     MORTAR_METHOD("routed_decode", py_routed_decode, "RMSNorm, router and gated MLP for decode rows, or None."),
+    MORTAR_METHOD("route", py_route, "The router of the rows of x and its load statistics, or None."),
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_mortar_native", "Native call layer of the MORTAR runtime.", -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -65,7 +65,7 @@ class MortarDecodeMLP:
             return None
         rt = mlp._modules.get("router")
         if rt is None:
-            return _lib.native().mlp(x, *pair, True, True, self.norm_weight, self.eps)
+            return _lib.native().mlp(x, *pair, True, True, self.norm_weight, self.eps, None)
         if type(rt) is not TileRouter or mlp.gate_up._cms._pack is not self.Mgu or mlp.down._cms._pack is not self.Mdown:
             return None
         proj, norm = rt._modules["query_proj"], rt._modules["query_norm"]

@@ -11,6 +11,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from . import _lib, ops
+from .routing import TileRouter
 from .sparsity import MortarLinear
 
 
@@ -98,7 +99,6 @@ class _SwiGLUMortar(nn.Module):
                        n_iters: int = 1, n_sub_keys: int = 0, detach_input: bool = True) -> None:
         """Attach an iteration-aware TileRouter over the d_ff hidden neuron bank (transformer.py:344-400)."""
         self._aux_detach_input = bool(detach_input)
-        from .routing import TileRouter
         try:
             dev = next(self.down.parameters()).device
         except StopIteration:
@@ -146,7 +146,7 @@ class _SwiGLUMortar(nn.Module):
             pair = self.native_pair()
             if pair is not None:
                 nw, eps = norm if norm is not None else (None, 0.0)
-                y = _lib.native().mlp(x, *pair, False, norm is not None, nw, eps)
+                y = _lib.native().mlp(x, *pair, False, norm is not None, nw, eps, None)
                 if y is not None:
                     return y
         train = self._carved() and self._wants_grad(x)
@@ -163,6 +163,15 @@ class _SwiGLUMortar(nn.Module):
                 norm = None
             elif norm[0] is not None and norm[0].dtype != torch.bfloat16:
                 norm = (norm[0].to(torch.bfloat16), norm[1])
+        if self._carved() and not train and x.is_cuda and norm is None and not self.route_skip and (pair := self.native_pair()) is not None:
+            if gates is None and self.router is not None:
+                rx, rt = (x.detach() if self._aux_detach_input else x), self.router
+                r = rt.forward_native(rx, iter_idx) if type(rt) is TileRouter and not (rt._forward_hooks or rt._forward_pre_hooks) else None
+                gates, self._last_aux_loss = r if r is not None else rt(rx, iter_idx=iter_idx)
+                gates = gates.detach()
+            y = _lib.native().mlp(x, *pair, False, False, None, 0.0, gates)
+            if y is not None:
+                return y
         if (train and x.is_cuda and self.router is None and gates is None and norm is None
                 and all(m._cms._values_ternary_mode and "mortar_packed" not in m._cms._buffers and m._cms.bias is None
                         for m in (self.gate_up, self.down))):

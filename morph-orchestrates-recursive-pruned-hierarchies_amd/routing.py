@@ -2,9 +2,9 @@
 
 Interface mirror of the reference's morph/model/routing.py (same parameters, forward signature, outputs).
 The gating tail (steps 5-8: k-th largest threshold, ReLU, normalise to sum k, active mask) runs in the HIP
-kernel for inference.  For decode-sized calls (up to 64 rows) the front end (query projection, LayerNorm, sub-key
-scores, product-key logits) runs in HIP as well, two launches in all; larger calls run the dense query projection as
-a library GEMM through torch and everything behind it (LayerNorm to gates) in one HIP launch.
+kernel for inference.  The front end (query projection, LayerNorm, sub-key scores, product-key logits) and the
+load statistics run in HIP as well for bf16 activations: two launches for decode-sized calls (up to 64 rows), projection,
+scores and ranking for larger ones; fp32 activations beyond 64 rows take a library GEMM for the projection.
 With autograd enabled the tail stays in differentiable torch ops.
 """
 from __future__ import annotations
@@ -16,7 +16,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from . import ops
+from . import _lib, ops
 
 
 def gates_from_logits(group_logits: Tensor, k: int) -> tuple[Tensor, Tensor]:
@@ -65,6 +65,26 @@ class TileRouter(nn.Module):
         idx = torch.arange(self.n_tile_groups, device=x_flat.device) % n_products
         return ps[:, idx] + self.group_bias.unsqueeze(0)
 
+    def _native_route(self, x: Tensor, iter_idx: int, stats: bool):
+        """(gates, active, aux or None) of the rows of a bf16 x in one native call, the load statistics updated when
+        ``stats``; None when the call is not covered (autograd, another dtype or layout)."""
+        if not x.is_cuda:
+            return None
+        return _lib.native().route(x, self._parameters, self._modules["query_proj"]._parameters, self._modules["query_norm"]._parameters,
+                                   (self.n_iters, self.n_sub_keys, self.n_tile_groups, self.activation_k), self.query_norm.eps, int(iter_idx),
+                                   self._buffers["group_load_ema"] if stats else None, self._load_ema_alpha, self.aux_loss_coeff)
+
+    def forward_native(self, x: Tensor, iter_idx: int = 0):
+        """forward() with the projection on the matrix cores: (gates [rows, n], aux_loss) and the same updates, or None when
+        the native call does not cover x.  The MLP module routes through this; above 64 rows the router's own entry points
+        keep the library's fp32 GEMM, so that their gates are bit for bit those of ops.router_tail on F.linear(x, Wq) (here
+        the same products are added in another order)."""
+        r = self._native_route(x, iter_idx, True)
+        if r is None:
+            return None
+        self.last_active = r[1]
+        return r[0], r[2]
+
     def _fused_ok(self, x_flat: Tensor) -> bool:
         """Decode-sized inference calls on the GPU with fp32 router parameters go through the two-launch HIP router."""
         return (x_flat.is_cuda and 0 < x_flat.shape[0] <= ops.ROUTER_MAX_TOKENS and not torch.is_grad_enabled()
@@ -74,7 +94,7 @@ class TileRouter(nn.Module):
 
     def _tail_ok(self, x_flat: Tensor) -> bool:
         """Inference calls of any size on the GPU with fp32 router parameters: library GEMM for the projection, then the
-        one-launch tail."""
+        tail launches."""
         return (x_flat.is_cuda and x_flat.shape[0] > 0 and not torch.is_grad_enabled()
                 and x_flat.dtype in (torch.bfloat16, torch.float32) and self.query_proj.weight.dtype == torch.float32
                 and self.n_sub_keys * self.n_sub_keys <= max(1024, self.n_tile_groups) and self.d_model % 8 == 0
@@ -85,7 +105,11 @@ class TileRouter(nn.Module):
         """Inference-only routing of [N, d_model] rows: (gates fp32 [N, n], active uint8 [N, n]) and nothing else (no
         load statistics, no auxiliary loss), as the reference's decode engine calls its fused router
         (morph/kernels/triton/fused_router.py:100-140).  Two launches for decode-sized N; a library GEMM for the query
-        projection plus one launch for everything behind it otherwise."""
+        projection and the tail launches otherwise."""
+        if x_flat.shape[0] <= ops.ROUTER_MAX_TOKENS:
+            r = self._native_route(x_flat, iter_idx, False)
+            if r is not None:
+                return r[0], r[1]
         if self._fused_ok(x_flat):
             it = max(0, min(int(iter_idx), self.n_iters - 1))
             return ops.router_fused(x_flat, self.query_proj.weight, self.iter_embed[it], self.query_norm.weight,
@@ -100,6 +124,10 @@ class TileRouter(nn.Module):
 
     def forward(self, x: Tensor, iter_idx: int = 0) -> Tuple[Tensor, Tensor]:
         orig_shape = x.shape
+        if x.numel() <= ops.ROUTER_MAX_TOKENS * orig_shape[-1]:
+            r = self.forward_native(x, iter_idx)
+            if r is not None:
+                return (r[0].view(orig_shape[0], orig_shape[1], -1) if len(orig_shape) == 3 else r[0]), r[1]
         x_flat = x.reshape(-1, orig_shape[-1])
         k = self.activation_k
         if self._fused_ok(x_flat) or self._tail_ok(x_flat):

@@ -1,0 +1,84 @@
+"""The prefill router's own kernels: projection on the matrix cores, score and rank launches, load statistics."""
+import pytest
+import torch
+
+from mortar_amd import _lib, ops
+from mortar_amd.routing import TileRouter
+
+pytestmark = pytest.mark.gpu
+
+
+def _project(x, w):
+    qv = torch.full((x.shape[0], w.shape[0]), float("nan"), device=x.device)
+    _lib.check(_lib.lib().mortar_router_project_bf16(x.data_ptr(), x.shape[0], x.shape[1], x.stride(0), w.data_ptr(), w.shape[0], qv.data_ptr(),
+                                                     qv.stride(0), torch.cuda.current_stream().cuda_stream), "project")
+    return qv
+
+
+@pytest.mark.parametrize("M", [1, 63, 65, 129, 257, 1000, 4097])          # each token tile of the dispatch, whole and ragged
+@pytest.mark.parametrize("d_in,d_out", [(8, 4), (72, 136), (256, 260), (2048, 2048)])
+def test_projection_has_fp32_accuracy(dev, M, d_in, d_out):
+    g = torch.Generator(device=dev).manual_seed(M + d_in)
+    x = torch.randn(M, d_in, device=dev, generator=g).to(torch.bfloat16)
+    w = torch.randn(d_out, d_in, device=dev, generator=g) * 0.05
+    qv = _project(x, w).double()
+    ref = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * 2.0 ** -22           # fp32 sums of exact products
+    assert ((qv - ref).abs() <= bound).all(), (qv - ref).abs().max().item()
+
+
+def test_projection_is_exact_on_small_integers(dev):
+    x = torch.randint(-8, 9, (300, 128), device=dev).to(torch.bfloat16)
+    w = torch.randint(-2 ** 15, 2 ** 15, (96, 128), device=dev).float()       # needs two of the three terms; every sum fits 24 bits
+    assert torch.equal(_project(x, w).double(), x.double() @ w.double().t())
+
+
+@pytest.mark.parametrize("M,n", [(1, 2), (31, 16), (65, 352), (4097, 1024)])
+def test_load_statistics(dev, M, n):
+    gates = torch.relu(torch.randn(M, n, device=dev))
+    ema = torch.rand(n, device=dev)
+    want = ema * 0.99 + (gates > 0).float().mean(0) * 0.01
+    aux = torch.empty((), device=dev)
+    L = _lib.lib()
+    ws = torch.empty(L.mortar_router_stats_workspace_bytes(M, n), dtype=torch.uint8, device=dev)
+    _lib.check(L.mortar_router_stats(gates.data_ptr(), M, n, 0.99, 0.01, 0.5, ema.data_ptr(), aux.data_ptr(), ws.data_ptr(),
+                                     torch.cuda.current_stream().cuda_stream), "stats")
+    assert torch.allclose(ema, want, rtol=1e-6, atol=1e-7)
+    assert torch.allclose(aux.double(), 0.5 * gates.double().mean(0).var(), rtol=1e-4, atol=1e-9)
+
+
+@pytest.mark.parametrize("N,d,nsk,n", [(65, 8, 4, 16), (66, 136, 4, 13), (100, 1032, 16, 256), (130, 2048, 17, 300), (77, 4096, 32, 1024),
+                                       (70, 256, 4, 8), (70, 256, 4, 7)])       # (last: fewer groups than scores, the one-launch form)
+@pytest.mark.parametrize("iter_vec", [False, True])
+def test_tail_against_float64(dev, N, d, nsk, n, iter_vec):
+    g = torch.Generator(device=dev).manual_seed(N + d)
+    qv = torch.randn(N, d, device=dev, generator=g)
+    iv = torch.randn(d, device=dev, generator=g) if iter_vec else None
+    lw, lb = torch.rand(d, device=dev, generator=g) + 0.5, torch.randn(d, device=dev, generator=g) * 0.1
+    ka, kb = (torch.randn(nsk, d // 2, device=dev, generator=g) * (d // 2) ** -0.5 for _ in range(2))
+    bias, k = torch.randn(n, device=dev, generator=g) * 0.1, max(1, n // 3)
+    gates, active, logits = ops.router_tail(qv, iv, lw, lb, 1e-5, ka, kb, bias, k, want_logits=True)
+    q = torch.nn.functional.layer_norm((qv + iv if iter_vec else qv).double(), (d,), lw.double(), lb.double(), 1e-5)
+    ps = ((q[:, :d // 2] @ ka.double().t()).unsqueeze(2) + (q[:, d // 2:] @ kb.double().t()).unsqueeze(1)).reshape(N, -1)
+    ref = (ps.topk(n, dim=-1).values if nsk * nsk > n else ps[:, torch.arange(n, device=dev) % (nsk * nsk)]) + bias.double()
+    assert torch.allclose(logits.double(), ref, rtol=0, atol=2e-5)
+    want = torch.relu(logits - logits.topk(k, dim=-1).values[:, -1:])
+    want = want * (k / want.sum(-1, keepdim=True).clamp(min=1e-6))
+    assert torch.allclose(gates, want, rtol=1e-4, atol=1e-5)
+    assert torch.equal(active.bool(), gates > 0)
+
+
+@pytest.mark.parametrize("M", [64, 65, 600])
+def test_router_module_call_equals_the_torch_ops(dev, M):
+    torch.manual_seed(2)
+    rt = TileRouter(44, 256, activation_ratio=0.25, n_iters=2).to(dev)
+    with torch.no_grad():
+        rt.iter_embed.normal_()
+        x = torch.randn(2, M // 2, 256, device=dev).to(torch.bfloat16) if M % 2 == 0 else torch.randn(M, 256, device=dev).to(torch.bfloat16)
+        flat = x.reshape(-1, 256)
+        want, act = ops.remoe_gates(rt.group_logits(flat, 1), rt.activation_k)
+        ema = rt.group_load_ema * 0.99 + act.float().mean(0) * (1 - 0.99)
+        gates, aux = rt.forward_native(x, iter_idx=1)
+    assert gates.shape == (flat.shape[0], 44) and torch.allclose(gates.reshape(-1, 44), want, rtol=1e-3, atol=1e-4)
+    assert torch.allclose(rt.group_load_ema, ema, rtol=1e-3, atol=1e-4) and rt.last_active.shape == (flat.shape[0], 44)
+    assert torch.allclose(aux, rt.aux_loss_coeff * want.mean(0).var(), rtol=1e-2)
