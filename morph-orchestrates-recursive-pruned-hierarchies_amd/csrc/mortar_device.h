@@ -66,6 +66,18 @@ __device__ __forceinline__ float bf16_to_f32(uint32_t b) { return __builtin_bit_
 // f rounded to bf16, as a float: the conversion of (0, f) leaves the bf16 of f in the high half and zeros below it.
 __device__ __forceinline__ float bf16r(float f) { return __builtin_bit_cast(float, bf16_pack2(0.f, f)); }
 
+#define MORTAR_GLOBAL __attribute__((address_space(1)))
+
+// Asynchronous 16-byte-per-lane copy global -> LDS (lane l's bytes land at lds_base + 16 * l): no registers, no
+// address arithmetic beyond the source pointer.  The caller waits with s_waitcnt vmcnt(0) and a barrier before the
+// destination is read.  (One wait state separates the write of M0 from its use as the LDS base.)
+__device__ __forceinline__ void mortar_load_to_lds(const MORTAR_GLOBAL char *gsrc, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gsrc) : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t mortar_lds_addr(const void *p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char *)p;
+}
+
 // ---- RMSNorm pieces shared by the stand-alone kernel and the fused staging of gate_up, so that both round alike.
 // A row is handled by one wavefront in 16-byte units (8 bf16): a lane adds the squares of its units in ascending
 // unit order (fused multiply-adds, low half-word first), the lanes meet in a xor butterfly.

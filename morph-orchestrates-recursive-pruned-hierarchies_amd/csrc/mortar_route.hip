@@ -638,6 +638,22 @@ __global__ void __launch_bounds__(512) router_scores_kernel(const float *qv, int
         const int i = at(j) < d2 ? at(j) : 0;
         v[j] = *reinterpret_cast<const float4 *>(q + i);
     }
+    const float *lw = ln_w + half * d2, *lb = ln_b + half * d2;
+    const float *kr[KT];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) kr[t] = (half ? kb : ka) + (int64_t)(t * 16 + tok < nsk ? t * 16 + tok : nsk - 1) * d2;
+    // LayerNorm parameters and key pieces are fetched PF chunks ahead of their products, the first before the statistics
+    constexpr int PF = 4;
+    float4 pw[PF], pb[PF], pk[PF][KT];
+    auto fetch = [&](int j) {
+        const int i = at(j) < d2 ? at(j) : 0;
+        pw[j % PF] = *reinterpret_cast<const float4 *>(lw + i);
+        pb[j % PF] = *reinterpret_cast<const float4 *>(lb + i);
+#pragma unroll
+        for (int t = 0; t < KT; ++t) pk[j % PF][t] = *reinterpret_cast<const float4 *>(kr[t] + i);
+    };
+#pragma unroll
+    for (int j = 0; j < PF; ++j) fetch(j);
     float s = 0.f;
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
@@ -672,25 +688,9 @@ __global__ void __launch_bounds__(512) router_scores_kernel(const float *qv, int
 #pragma unroll
     for (int w = 0; w < 8; ++w) var += red[1][w][tok];
     const float rstd = 1.0f / sqrtf(var / (float)d + ln_eps);
-    const float *lw = ln_w + half * d2, *lb = ln_b + half * d2;
-    const float *kr[KT];
-#pragma unroll
-    for (int t = 0; t < KT; ++t) kr[t] = (half ? kb : ka) + (int64_t)(t * 16 + tok < nsk ? t * 16 + tok : nsk - 1) * d2;
     f32x4_t acc[KT];
 #pragma unroll
     for (int t = 0; t < KT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    // LayerNorm parameters and key pieces are fetched PF chunks ahead of their products
-    constexpr int PF = 4;
-    float4 pw[PF], pb[PF], pk[PF][KT];
-    auto fetch = [&](int j) {
-        const int i = at(j) < d2 ? at(j) : 0;
-        pw[j % PF] = *reinterpret_cast<const float4 *>(lw + i);
-        pb[j % PF] = *reinterpret_cast<const float4 *>(lb + i);
-#pragma unroll
-        for (int t = 0; t < KT; ++t) pk[j % PF][t] = *reinterpret_cast<const float4 *>(kr[t] + i);
-    };
-#pragma unroll
-    for (int j = 0; j < PF; ++j) fetch(j);
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
         const bool in = at(j) < d2;

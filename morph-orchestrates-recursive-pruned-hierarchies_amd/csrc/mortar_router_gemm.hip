@@ -11,15 +11,16 @@ namespace {
 //
 // An fp32 weight is exactly the sum of three bf16 values (its top 8, next 8 and last 8 significant bits), so three bf16
 // MFMAs on the same activation operand give exact products in fp32 accumulators: the arithmetic of an fp32 GEMM at three
-// times the cost of a bf16 one instead of the sixteen times of the fp32 matrix instructions (4096 x 2048 x 2048: 257 us
-// through the library's fp32 GEMM with its conversion of x).
+// times the cost of a bf16 one instead of the sixteen times of the fp32 matrix instructions (4096 x 2048 x 2048: 81 us,
+// 1270 TFLOP/s of the three terms, against 257 us through the library's fp32 GEMM with its conversion of x; the MFMAs
+// alone take 60 us at the clocks the part holds under them).
 //
 // A workgroup of NW waves owns MT tokens x 16 NW outputs; a wave owns 16 outputs for all MT tokens, so that a weight is
-// loaded (straight from global memory in the MFMA operand order: 16 rows x 128 bytes per instruction) and split once per
-// workgroup: 44 vector instructions per 3 MT / 16 MFMAs, hidden behind the matrix pipe from 128 tokens up.  The
-// activations go through LDS in steps of 64 values, two buffers, one barrier per step; a fragment of 16 tokens x 32
-// values is 1 KB in operand order, its 16-byte units swizzled (token ^ 4 * group) so that both the staging writes (4
-// tokens x 4 units per 16 lanes) and the operand reads touch every bank once.
+// split once per workgroup: 44 vector instructions per 3 MT / 16 MFMAs, hidden behind the matrix pipe from 128 tokens up.
+// Both operands travel in steps of 64 values through D buffers in LDS, copied asynchronously (global_load_lds, no registers)
+// D - 1 steps ahead; storing the activations from registers instead cost 1000 of 5300 cycles per step.  One barrier per
+// step.  Four consecutive lanes copy 64 contiguous bytes (in another order per lane group: `n`-dependent swizzles), so that
+// the copies stay coalesced and the operand reads touch every bank once.
 constexpr int RG_KS = 64;
 
 __device__ __forceinline__ void split3(const float (&w)[8], u32x4_t (&p)[3]) {
@@ -41,11 +42,12 @@ __device__ __forceinline__ void split3(const float (&w)[8], u32x4_t (&p)[3]) {
     }
 }
 
-template <int MT, int NW>
+template <int MT, int NW, int D>
 __global__ void __launch_bounds__(NW * 64) router_gemm_kernel(const uint16_t *x, int M, int K, int64_t ldx, const float *W, int N, float *qv,
                                                               int64_t ldq, int n_ntiles) {
-    constexpr int MI = MT / 16, FR = MI * 2, U = FR / NW, MG = MI < 8 ? MI : 8;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[2][MT * RG_KS * 2];
+    constexpr int MI = MT / 16, FR = MI * 2, U = FR / NW, MG = MI < 4 ? MI : 4;
+    constexpr int XB = MT * RG_KS * 2, WB = 16 * RG_KS * 4, BUF = XB + NW * WB;       // activations, then one block of weights per wave
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
@@ -56,79 +58,86 @@ __global__ void __launch_bounds__(NW * 64) router_gemm_kernel(const uint16_t *x,
     if (id >= n_mtiles * n_ntiles) return;
     const int m0 = (id / n_ntiles) * MT, o0 = (id % n_ntiles) * (16 * NW) + wave * 16;
 
-    // staging role: fragment wave + NW * i, token lane >> 2, 16-byte unit lane & 3
+    // Activations: fragments (16 tokens x 32 values, 1 KB) wave + NW * i; slot l of a fragment holds 16-byte unit
+    // (l & 3) ^ (token >> 2) of token l / 4.  Weights: row 4 i + l / 16, slot l & 15 of its 256 bytes holds unit (l & 15) ^ row.
     const uint16_t *xs[U];
-    uint32_t dst[U];
-    int ks[U];
+    const float *ws[4];
+    int kx[U], kw[4];
 #pragma unroll
     for (int i = 0; i < U; ++i) {
-        const int f = wave + NW * i, row = m0 + (f >> 1) * 16 + (lane >> 2), u = lane & 3;
-        ks[i] = (f & 1) * 32 + u * 8;
-        xs[i] = x + (int64_t)(row < M ? row : M - 1) * ldx + ks[i];
-        dst[i] = (uint32_t)(f * 1024 + u * 256 + (((lane >> 2) ^ (4 * u)) * 16));
+        const int f = wave + NW * i, t = lane >> 2, row = m0 + (f >> 1) * 16 + t;
+        kx[i] = (f & 1) * 32 + ((lane & 3) ^ (t >> 2)) * 8;
+        xs[i] = x + (int64_t)(row < M ? row : M - 1) * ldx + kx[i];
     }
-    const int orow = o0 + n < N ? o0 + n : N - 1;
-    const float *ws = W + (int64_t)orow * K + g * 8;
-    const uint32_t rd = (uint32_t)(g * 256 + ((n ^ (4 * g)) * 16));
-
-    u32x4_t xr[U];
-    float4 wr[2][2];
-    auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 4 * i + g;
+        kw[i] = (n ^ r) * 4;
+        ws[i] = W + (int64_t)(o0 + r < N ? o0 + r : N - 1) * K + kw[i];
+    }
+    const uint32_t rd = (uint32_t)(n * 64 + (g ^ (n >> 2)) * 16);
+    // K % 8 == 0: a unit is in the row or past its end as a whole; the ones past the end are cleared (last step only)
+    auto stage = [&](int k0, int buf) {
+        const bool part = k0 + RG_KS > K;
+        unsigned char *xd = lds + buf * BUF + wave * 1024, *wd = lds + buf * BUF + XB + wave * WB;
 #pragma unroll
         for (int i = 0; i < U; ++i) {
-            const bool in = k0 + ks[i] < K;                                   // K % 8 == 0: a unit is in or out as a whole
-            xr[i] = *reinterpret_cast<const u32x4_t *>(xs[i] + (in ? k0 : -ks[i]));
-            if (!in) xr[i] = u32x4_t{0u, 0u, 0u, 0u};
+            if (part && k0 + kx[i] >= K) *reinterpret_cast<u32x4_t *>(xd + i * NW * 1024 + lane * 16) = u32x4_t{0u, 0u, 0u, 0u};
+            else mortar_load_to_lds((const MORTAR_GLOBAL char *)(xs[i] + k0), __builtin_amdgcn_readfirstlane(mortar_lds_addr(xd + i * NW * 1024)));
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const bool in = k0 + h * 32 + g * 8 < K;
-            const float4 *p = reinterpret_cast<const float4 *>(ws + (in ? k0 + h * 32 : -g * 8));
-            wr[h][0] = p[0];
-            wr[h][1] = p[1];
-            if (!in) wr[h][0] = wr[h][1] = float4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < 4; ++i) {
+            if (part && k0 + kw[i] >= K) *reinterpret_cast<u32x4_t *>(wd + i * 1024 + lane * 16) = u32x4_t{0u, 0u, 0u, 0u};
+            else mortar_load_to_lds((const MORTAR_GLOBAL char *)(ws[i] + k0), __builtin_amdgcn_readfirstlane(mortar_lds_addr(wd + i * 1024)));
         }
-    };
-    auto put = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < U; ++i) *reinterpret_cast<u32x4_t *>(&lds[buf][dst[i]]) = xr[i];
     };
     f32x4_t acc[MI];
 #pragma unroll
     for (int i = 0; i < MI; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    fetch(0);
-    put(0);
+#pragma unroll
+    for (int b = 0; b < D - 1; ++b)
+        if (b * RG_KS < K) stage(b * RG_KS, b);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     int buf = 0;
     for (int k0 = 0; k0 < K; k0 += RG_KS) {
+        const int kn = k0 + (D - 1) * RG_KS;
+        if (kn < K) stage(kn, buf == 0 ? D - 1 : buf - 1);
+        const unsigned char *cur = lds + buf * BUF;
         float w[2][8];
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                w[h][4 * j] = wr[h][j].x; w[h][4 * j + 1] = wr[h][j].y; w[h][4 * j + 2] = wr[h][j].z; w[h][4 * j + 3] = wr[h][j].w;
+                const float4 v = *reinterpret_cast<const float4 *>(cur + XB + wave * WB + n * 256 + ((8 * h + 2 * g + j) ^ n) * 16);
+                w[h][4 * j] = v.x; w[h][4 * j + 1] = v.y; w[h][4 * j + 2] = v.z; w[h][4 * j + 3] = v.w;
             }
-        const bool more = k0 + RG_KS < K;
-        if (more) fetch(k0 + RG_KS);
+        // groups of MG token fragments; the operands of the next group are read while the current one multiplies
+        constexpr int NG = 2 * MI / MG;
+        u32x4_t b[2][MG];
+        auto operands = [&](int q) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            u32x4_t p[3];
-            split3(w[h], p);
+            for (int i = 0; i < MG; ++i)
+                b[q & 1][i] = *reinterpret_cast<const u32x4_t *>(cur + ((q * MG % MI + i) * 2 + q * MG / MI) * 1024 + rd);
+        };
+        operands(0);
+        u32x4_t p[3];
 #pragma unroll
-            for (int i0 = 0; i0 < MI; i0 += MG) {
-                u32x4_t b[MG];
+        for (int q = 0; q < NG; ++q) {
+            if (q * MG % MI == 0) split3(w[q * MG / MI], p);
+            if (q + 1 < NG) operands(q + 1);
 #pragma unroll
-                for (int i = 0; i < MG; ++i) b[i] = *reinterpret_cast<const u32x4_t *>(&lds[buf][((i0 + i) * 2 + h) * 1024 + rd]);
+            for (int t = 2; t >= 0; --t)                                      // small terms first
 #pragma unroll
-                for (int t = 2; t >= 0; --t)                                  // small terms first
-#pragma unroll
-                    for (int i = 0; i < MG; ++i) acc[i0 + i] = mortar_mfma(p[t], b[i], acc[i0 + i]);
-            }
+                for (int i = 0; i < MG; ++i) acc[q * MG % MI + i] = mortar_mfma(p[t], b[q & 1][i], acc[q * MG % MI + i]);
         }
-        if (more) put(buf ^ 1);
+        // The next step has landed: at most the copies of the D - 2 steps after it are still in flight.  (Every whole step
+        // issues U + 4 copies per wave; a partial or missing one issues fewer, so the last steps wait for everything.)
+        if (D > 2 && kn + RG_KS <= K) asm volatile("s_waitcnt vmcnt(%0)" ::"i"((D - 2) * (U + 4)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        buf ^= 1;
+        buf = buf + 1 == D ? 0 : buf + 1;
     }
     const int o = o0 + 4 * g;
     if (o < N) {
@@ -140,11 +149,20 @@ __global__ void __launch_bounds__(NW * 64) router_gemm_kernel(const uint16_t *x,
     }
 }
 
-template <int MT, int NW>
-void launch_gemm(const uint16_t *x, int M, int K, int64_t ldx, const float *W, int N, float *qv, int64_t ldq, hipStream_t st) {
+template <int MT, int NW, int D>
+int launch_gemm(const uint16_t *x, int M, int K, int64_t ldx, const float *W, int N, float *qv, int64_t ldq, hipStream_t st) {
+    constexpr int smem = D * (MT * RG_KS * 2 + NW * 16 * RG_KS * 4);
+    static_assert(smem <= 160 * 1024, "LDS of a CU");
+    static bool done = false;
+    if (!done) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(router_gemm_kernel<MT, NW, D>), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "router projection: %s", hipGetErrorString(e));
+        done = true;
+    }
     const int nt = (N + 16 * NW - 1) / (16 * NW), mt = (M + MT - 1) / MT;
     const unsigned grid = (unsigned)(((int64_t)mt * nt + 7) / 8 * 8);
-    hipLaunchKernelGGL((router_gemm_kernel<MT, NW>), dim3(grid), dim3(NW * 64), 0, st, x, M, K, ldx, W, N, qv, ldq, nt);
+    hipLaunchKernelGGL((router_gemm_kernel<MT, NW, D>), dim3(grid), dim3(NW * 64), smem, st, x, M, K, ldx, W, N, qv, ldq, nt);
+    return MORTAR_OK;
 }
 
 // ---- load statistics -----------------------------------------------------------------------------------------------
@@ -234,15 +252,17 @@ extern "C" int mortar_router_project_bf16(const uint16_t *x, int64_t M, int32_t 
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wq) | reinterpret_cast<uintptr_t>(qv)) & 15)
         return mortar_fail(MORTAR_ERR_ARG, "router projection: x, wq and qv must be 16-byte aligned");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // Tokens per workgroup: the choice with the least rounds of 256 workgroups (one per CU) x work of a workgroup; a
-    // workgroup costs its tokens plus the split of its weights, which weighs about 40 tokens.
-    const int64_t nt8 = (d_out + 127) / 128;
-    auto cost = [&](int mt) { return (((M + mt - 1) / mt * nt8 + 255) / 256) * (mt + 40); };
-    const int64_t c256 = cost(256), c128 = cost(128), c64 = cost(64);
-    if (c256 <= c128 && c256 <= c64) launch_gemm<256, 8>(x, (int)M, d_in, ldx, wq, d_out, qv, ldq, st);
-    else if (c128 <= c64) launch_gemm<128, 8>(x, (int)M, d_in, ldx, wq, d_out, qv, ldq, st);
-    else if ((M + 63) / 64 * nt8 > 128) launch_gemm<64, 8>(x, (int)M, d_in, ldx, wq, d_out, qv, ldq, st);
-    else launch_gemm<64, 4>(x, (int)M, d_in, ldx, wq, d_out, qv, ldq, st);      // few tiles: half the outputs per workgroup, twice the workgroups
+    // Tokens per workgroup: the choice with the least rounds of workgroups x time of a round.  A round of 256 workgroups (one
+    // per CU) of 128 outputs takes mt + 100 units (49 us at 128 tokens and 2048 inputs, 72 us at 256); the 64-token tile of 64
+    // outputs fits a CU twice and takes 131 units alone, 164 with a neighbour.
+    const int64_t nt8 = (d_out + 127) / 128, w64 = (M + 63) / 64 * ((d_out + 63) / 64);
+    const int64_t c256 = ((M + 255) / 256 * nt8 + 255) / 256 * 356, c128 = ((M + 127) / 128 * nt8 + 255) / 256 * 228;
+    const int64_t c64 = w64 <= 256 ? 131 : (w64 + 511) / 512 * 164;
+    int rc;
+    if (c256 <= c128 && c256 <= c64) rc = launch_gemm<256, 8, 2>(x, (int)M, d_in, ldx, wq, d_out, qv, ldq, st);
+    else if (c128 <= c64) rc = launch_gemm<128, 8, 2>(x, (int)M, d_in, ldx, wq, d_out, qv, ldq, st);
+    else rc = launch_gemm<64, 4, 3>(x, (int)M, d_in, ldx, wq, d_out, qv, ldq, st);
+    if (rc) return rc;
     return check_launch("router projection");
 }
 

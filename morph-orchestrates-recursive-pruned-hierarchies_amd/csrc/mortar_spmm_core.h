@@ -58,7 +58,6 @@ struct SpmmParams {
 // Device-side view of the launch parameters: the pointers carry the global address space in their type, so
 // that every access compiles to global_load / global_store (a pointer read from a parameter table in memory
 // would otherwise be generic and cost flat instructions).
-#define MORTAR_GLOBAL __attribute__((address_space(1)))
 struct SpmmView {
     const MORTAR_GLOBAL u32x4_t *row_desc, *codes_o, *sched;
     const MORTAR_GLOBAL uint32_t *sd_dw, *cc_dw;      // scale patterns / block-columns of the octet stream as dwords
@@ -294,13 +293,6 @@ __device__ __forceinline__ void mortar_stage_quads(const SpmmView &p, unsigned c
             }
         }
     }
-}
-
-// Asynchronous 16-byte-per-lane copy global -> LDS (lane l's bytes land at lds_base + 16 * l): no registers, no
-// address arithmetic beyond the source pointer.  The caller waits with s_waitcnt vmcnt(0) and a barrier before the
-// destination is read.  (One wait state separates the write of M0 from its use as the LDS base.)
-__device__ __forceinline__ void mortar_load_to_lds(const MORTAR_GLOBAL char *gsrc, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gsrc) : "memory", "m0");
 }
 
 // Stages block-columns [c0, c0 + ncb) of token tile `mt` from activations stored in tile order (SpmmParams::x_tiled):
