@@ -355,14 +355,17 @@ int mortar_gemv_bf16(const mortar_bcsr_t *W, const int32_t *entries, int64_t n_e
  *   part       device workspace of part_bytes >= mortar_gemv_f32_workspace_bytes(W, B, nslots) bytes, 16-byte aligned
  *              (may be NULL when nslots == 1; then only the work-list kernel runs)
  *   other arguments as mortar_gemv_bf16.  Agreement with a float64 evaluation: fp32 rounding of the sums only.
- * With one scale (scale_count = 1, the reference's format), a schedule and the workspace, the product runs on
- * the bandwidth-bound SpMM kernels instead of the work list: the three bf16 terms of the B rows become 3 * B bf16 rows,
- * the one-scale SpMM kernels contract them with the +-2 / 0 blocks and keep the fp32 sums unrounded, and a last pass
- * adds the three sums of a row and applies the scale and the epilogue - the same exact products and fp32 sums, in
- * another order of addition (2 to 3 times faster at the headline shapes).  Flags keep their per-stream meaning there: a chunk of x
- * whose column is off for its stream enters as zeros, and the sum of a row that is off for a stream is written as
- * zero; no weight is skipped, which is still faster than the work list with skipping (17 against 25 us per MLP at
- * one row, 21 against 49 us at 16 rows). */
+ * With one scale (scale_count = 1, the reference's format) and a schedule, the product runs as mortar_gemv_f32_one instead
+ * of the work list: the same exact products and fp32 sums in another order of addition.  Flags keep their per-stream
+ * meaning there: a chunk of x whose column is off for its stream enters as zeros, and the sum of a row that is off for a
+ * stream is written as zero. */
+/* The one-scale form of that product in one launch, without schedule, work list or workspace: scale fp32 [1], other
+ * arguments as mortar_gemv_f32 with x rows 16-byte aligned.  Returns MORTAR_NO_KERNEL (-100, nothing launched) for rows too wide for
+ * any tile of all K (in_features > 27000); mortar_gemv_f32 uses it by itself where it is the faster form. */
+#define MORTAR_NO_KERNEL (-100)
+int mortar_gemv_f32_one(const mortar_bcsr_t *W, const float *scale, int32_t mode, int32_t swiglu_x, const float *x, int32_t B,
+                        int64_t ldx, float *y, int64_t ldy, const float *gates, int32_t n_clusters, int64_t ldg,
+                        const int32_t *row_act, int64_t ldr, const int32_t *col_act, int64_t ldc, void *stream);
 int64_t mortar_gemv_f32_workspace_bytes(const mortar_bcsr_t *W, int32_t B, int32_t nslots);
 int mortar_gemv_f32(const mortar_bcsr_t *W, const float *scale, int64_t scale_count, const int32_t *sched,
                     const int32_t *entries,

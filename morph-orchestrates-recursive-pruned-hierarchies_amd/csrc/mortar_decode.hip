@@ -547,6 +547,7 @@ int64_t gemv_f32_fast_bytes(const mortar_bcsr_t *W, int B) {
     return (int64_t)3 * B * ((int64_t)W->Rb * 16 * 4 + (int64_t)W->Cb * 16 * 2);
 }
 
+// Rows too wide for a tile of all K of even one token (mortar_gemv_f32_one): split, SpMM on the 3 B term rows, combine.
 // Returns MORTAR_NO_KERNEL when the SpMM kernels cannot serve the shape (the caller then runs the work-list kernel).
 int gemv_f32_fast(const mortar_bcsr_t *W, const int32_t *sched, const GemvF32Params &p, void *ws, hipStream_t st) {
     const int K = W->Cb * 16, N = W->Rb * 16;
@@ -608,6 +609,10 @@ extern "C" int mortar_gemv_f32(const mortar_bcsr_t *W, const float *scale, int64
     if (nslots > 1 && part_bytes < (int64_t)nslots * B * W->Rb * 16 * 4)
         return mortar_fail(MORTAR_ERR_ARG, "gemv_f32: the partial workspace holds %lld bytes, need %lld", (long long)part_bytes,
                            (long long)nslots * B * W->Rb * 16 * 4);
+    if (scale_count == 1 && sched && W->row_desc && W->codes_o && W->col_o && (B == 1 || ldx % 4 == 0) && !(reinterpret_cast<uintptr_t>(x) & 15)) {
+        const int rc = mortar_gemv_f32_one(W, scale, mode, swiglu_x, x, B, ldx, y, ldy, gates, n_clusters, ldg, row_act, ldr, col_act, ldc, stream);
+        if (rc != MORTAR_NO_KERNEL) return rc;
+    }
     if (scale_count == 1 && sched && W->codes_o && part && !(reinterpret_cast<uintptr_t>(part) & 15) &&
         part_bytes >= gemv_f32_fast_bytes(W, B) && ldx % 4 == 0 && !(reinterpret_cast<uintptr_t>(x) & 15)) {
         const int rc = gemv_f32_fast(W, sched, p, part, st);

@@ -1,0 +1,229 @@
+// Decode GEMV in the reference engine's arithmetic on a matrix with one scale, in ONE launch.
+//
+// mortar_gemv (morph/kernels/triton/fused_decode_step.py:1341-1459, 1502-1547): fp32 activations, exact +-x / 0 products, fp32
+// sums, the fp32 scale after the sum, SwiGLU and gates in fp32.  The part-split decode kernel of mortar_spmm_core.h with
+// another prologue and epilogue: an fp32 activation is split exactly into three bf16 terms while the tile is staged (row
+// term * T + t of the tile is a term of token t), the blocks are contracted as +-2 / 0, and the epilogue adds the three sums
+// of a token (columns of the accumulator, two lane exchanges), scales, and applies SwiGLU and gates.
+// Three launches per product (split, SpMM on 3 B rows, combine) took 11.9 us of GPU time and 16 us of host time at 8 rows of
+// the 2048 -> 11264 matrix; what they moved through memory between them is now in LDS and registers.
+#include "mortar_spmm_core.h"
+
+namespace {
+
+struct GemvOneArgs {
+    const float *x, *scale, *gates;
+    float *y;
+    const int32_t *row_act, *col_act;
+    int64_t ldx, ldy, ldg, ldr, ldc;
+    int swiglu_x;
+};
+
+__device__ __forceinline__ float sigmoid_f32(float g) { return 1.0f / (1.0f + __expf(-g)); }
+
+// T tokens per tile (3 T rows of 16 MFMA columns), PW waves share the parts of a unit, 4 units per workgroup.
+template <int T, int NACC, int PW>
+__global__ void __launch_bounds__(PW * 4 * 64) gemv_f32_one_kernel(const SpmmParams p0, const GemvOneArgs a) {
+    constexpr int MT = 3 * T, UW = 4, WAVES = PW * UW, THREADS = WAVES * 64;
+    const SpmmView p = mortar_view(p0);
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    uint4 *lx = reinterpret_cast<uint4 *>(smem);
+    f32x4_t *red = reinterpret_cast<f32x4_t *>(smem + tile_bytes(MT, p.Cb));          // [WAVES][NACC][64]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4, bsel = g >> 1, hsel = g & 1;
+    const int mt = blockIdx.x / p.n_split, sp = blockIdx.x % p.n_split;
+    const int t0 = mt * T, nt = p.M - t0 < T ? p.M - t0 : T;                           // p.M counts tokens here
+    const int ug = wave / PW, wq = wave % PW, pos = sp * UW + ug;
+    const bool valid = pos < p.n_units;
+    const int nparts = p.nseg * NACC;
+    MortarBatch first;
+    u32x4_t d = u32x4_t{0u, 0u, 0u, 0u};
+    if (valid && wq < nparts) {          // the first weights are on their way before the tile is staged
+        d = mortar_part_desc<NACC>(p, pos, wq / NACC, wq % NACC);
+        const int g0 = __builtin_amdgcn_readfirstlane((int)d[0]), g1 = __builtin_amdgcn_readfirstlane((int)d[1]);
+        if (g0 < g1) mortar_load_batch<CODE_UNIFORM>(p, first, g0, g1, n, bsel, hsel);
+    }
+    // what the epilogue reads besides the sums, requested early: the lane's gate and row flags (token n)
+    const int tok = t0 + n;
+    const bool mine = valid && n < nt;
+    float gate = 1.f;
+    int on_a = 1, on_b = 1;
+    if (mine) {
+        if (NACC == 2 && a.gates) gate = a.gates[(int64_t)tok * a.ldg + (pos * 16 + 4 * g) / p.cluster_size];
+        if (a.row_act) {
+            on_a = a.row_act[(int64_t)tok * a.ldr + pos];
+            if (NACC == 2) on_b = a.row_act[(int64_t)tok * a.ldr + p.n_units + pos];
+        }
+    }
+    const float scale = a.scale[0];
+
+    // stage: item = (token, 8 consecutive inputs)
+    const int K = p.Cb * 16, nch = K / 8;
+    for (int i0 = tid; i0 < nt * nch; i0 += 4 * THREADS) {
+        float4 q[4][2];
+        int off[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = i0 + u * THREADS;
+            if (i >= nt * nch) break;
+            const int t = i / nch, c = i - t * nch;
+            const float4 *src = reinterpret_cast<const float4 *>(a.x + (int64_t)(t0 + t) * a.ldx + c * 8);
+            q[u][0] = src[0];
+            q[u][1] = src[1];
+            if (a.swiglu_x) {
+                const float4 u0 = src[K / 4], u1 = src[K / 4 + 1];
+                float4 &f = q[u][0], &h = q[u][1];
+                f = float4{f.x * sigmoid_f32(f.x) * u0.x, f.y * sigmoid_f32(f.y) * u0.y, f.z * sigmoid_f32(f.z) * u0.z, f.w * sigmoid_f32(f.w) * u0.w};
+                h = float4{h.x * sigmoid_f32(h.x) * u1.x, h.y * sigmoid_f32(h.y) * u1.y, h.z * sigmoid_f32(h.z) * u1.z, h.w * sigmoid_f32(h.w) * u1.w};
+            }
+            if (a.col_act && a.col_act[(int64_t)(t0 + t) * a.ldc + (c >> 1)] == 0) q[u][0] = q[u][1] = float4{0.f, 0.f, 0.f, 0.f};
+            off[u] = (c >> 1) * (MT * 32) + t * 32 + (c & 1) * 16;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (i0 + u * THREADS >= nt * nch) break;
+            const float v[8] = {q[u][0].x, q[u][0].y, q[u][0].z, q[u][0].w, q[u][1].x, q[u][1].y, q[u][1].z, q[u][1].w};
+            u32x4_t hi, mid, lo;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                hi[k] = bf16_pack2(v[2 * k], v[2 * k + 1]);
+                const float r0 = v[2 * k] - bf16_to_f32(hi[k] & 0xffffu), r1 = v[2 * k + 1] - bf16_to_f32(hi[k] >> 16);
+                mid[k] = bf16_pack2(r0, r1);
+                lo[k] = bf16_pack2(r0 - bf16_to_f32(mid[k] & 0xffffu), r1 - bf16_to_f32(mid[k] >> 16));
+            }
+            *reinterpret_cast<u32x4_t *>(smem + off[u]) = hi;
+            *reinterpret_cast<u32x4_t *>(smem + off[u] + T * 32) = mid;
+            *reinterpret_cast<u32x4_t *>(smem + off[u] + 2 * T * 32) = lo;
+        }
+    }
+    __syncthreads();
+    // a unit whose rows are off, or whose gate is zero, for every token of the tile multiplies nothing
+    const bool work = valid && __ballot(mine && gate != 0.f && (on_a != 0 || (NACC == 2 && on_b != 0))) != 0ull;
+
+    f32x4_t acc[NACC][1];
+#pragma unroll
+    for (int b = 0; b < NACC; ++b) acc[b][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const uint32_t tk[1] = {(uint32_t)n};
+    if (work) {
+        for (int sg = 0; sg < p.nseg; ++sg) {
+            const uint32_t xo = (uint32_t)(hsel * 16 + n * 32) + (uint32_t)(sg * p.seg_cb) * (uint32_t)(MT * 32);
+#pragma unroll
+            for (int b = 0; b < NACC; ++b) {
+                const int q = sg * NACC + b;
+                if (q % PW != wq) continue;
+                const u32x4_t dq = q == wq ? d : mortar_part_desc<NACC>(p, pos, sg, b);
+                const int g0 = __builtin_amdgcn_readfirstlane((int)dq[0]), g1 = __builtin_amdgcn_readfirstlane((int)dq[1]);
+                if (g0 >= g1) continue;
+                if (q != wq) mortar_load_batch<CODE_UNIFORM>(p, first, g0, g1, n, bsel, hsel);
+                mortar_row_part<1, MT, false, CODE_UNIFORM>(p, lx, first, g0, g1, __builtin_amdgcn_readfirstlane((int)dq[2]), xo, tk, 1, n, bsel,
+                                                            hsel, acc[b]);
+            }
+        }
+    }
+    if (PW > 1) {
+#pragma unroll
+        for (int b = 0; b < NACC; ++b) red[(wave * NACC + b) * 64 + lane] = acc[b][0];
+        __syncthreads();
+        if (wq != 0) return;
+#pragma unroll
+        for (int w = 1; w < PW; ++w)
+#pragma unroll
+            for (int b = 0; b < NACC; ++b) acc[b][0] += red[((wave + w) * NACC + b) * 64 + lane];
+    }
+    if (!valid) return;
+    // columns n, n + T and n + 2 T of the accumulator are the three terms of token n
+    f32x4_t r[NACC];
+#pragma unroll
+    for (int b = 0; b < NACC; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float m = __shfl(acc[b][0][v], lane + T, 64), l = __shfl(acc[b][0][v], lane + 2 * T, 64);
+            r[b][v] = scale * (0.5f * ((acc[b][0][v] + m) + l));
+        }
+    if (!mine) return;
+    if (!on_a) r[0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (NACC == 2) {
+        if (!on_b) r[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            r[0][v] = r[0][v] * sigmoid_f32(r[0][v]) * r[1][v];
+            if (a.gates) r[0][v] *= gate;
+        }
+    }
+    *reinterpret_cast<f32x4_t *>(a.y + (int64_t)tok * a.ldy + pos * 16 + 4 * g) = r[0];
+}
+
+template <int T, int NACC, int PW>
+int launch_one(SpmmParams &p, const GemvOneArgs &a, hipStream_t st) {
+    const int smem = tile_bytes(3 * T, p.Cb) + (PW > 1 ? PW * 4 * NACC * 1024 : 0);
+    static bool done = false;
+    int rc = mortar_allow_big_lds(gemv_f32_one_kernel<T, NACC, PW>, done);
+    if (rc) return rc;
+    p.n_mtiles = (p.M + T - 1) / T;
+    p.n_split = (p.n_units + 3) / 4;
+    if ((rc = mortar_launch_check((int64_t)p.n_mtiles * p.n_split, 1))) return rc;
+    hipLaunchKernelGGL((gemv_f32_one_kernel<T, NACC, PW>), dim3((unsigned)(p.n_mtiles * p.n_split)), dim3(PW * 256), smem, st, p, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "gemv_f32 launch: %s", hipGetErrorString(e));
+    return MORTAR_OK;
+}
+
+template <int T, int NACC>
+int launch_pw(int pw, SpmmParams &p, const GemvOneArgs &a, hipStream_t st) {
+    switch (pw) {
+        case 1: return launch_one<T, NACC, 1>(p, a, st);
+        case 2: return launch_one<T, NACC, 2>(p, a, st);
+        case 3: return launch_one<T, NACC, 3>(p, a, st);
+    }
+    return launch_one<T, NACC, 4>(p, a, st);
+}
+
+template <int NACC>
+int launch_t(int t, int pw, SpmmParams &p, const GemvOneArgs &a, hipStream_t st) {
+    switch (t) {
+        case 1: return launch_pw<1, NACC>(pw, p, a, st);
+        case 2: return launch_pw<2, NACC>(pw, p, a, st);
+        case 4: return launch_pw<4, NACC>(pw, p, a, st);
+    }
+    return launch_pw<5, NACC>(pw, p, a, st);
+}
+
+}  // namespace
+
+extern "C" int mortar_gemv_f32_one(const mortar_bcsr_t *W, const float *scale, int32_t mode, int32_t swiglu_x, const float *x, int32_t B,
+                                   int64_t ldx, float *y, int64_t ldy, const float *gates, int32_t n_clusters, int64_t ldg,
+                                   const int32_t *row_act, int64_t ldr, const int32_t *col_act, int64_t ldc, void *stream) {
+    if (!W || !W->row_desc || !W->codes_o || !W->col_o || !scale || !x || !y) return mortar_fail(MORTAR_ERR_ARG, "gemv_f32_one: null pointer");
+    if (B <= 0 || B > 64) return mortar_fail(MORTAR_ERR_LIMIT, "gemv_f32_one: B=%d outside 1..64", B);
+    if (mode != 0 && mode != 1) return mortar_fail(MORTAR_ERR_ARG, "gemv_f32_one: mode must be 0 or 1");
+    if (W->Rb <= 0 || W->Cb <= 0 || W->nnz <= 0 || W->seg_cb <= 0 || (mode == 1 && (W->Rb & 1)))
+        return mortar_fail(MORTAR_ERR_ARG, "gemv_f32_one: bad matrix");
+    const int64_t nout = mode == 0 ? (int64_t)W->Rb * 16 : (int64_t)W->Rb * 8, need = (int64_t)W->Cb * 16 * (swiglu_x ? 2 : 1);
+    if (ldx < need || (B > 1 && ldx % 4) || ldy < nout || ldy % 4 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15))
+        return mortar_fail(MORTAR_ERR_ARG, "gemv_f32_one: bad leading dimension or alignment (rows 16-byte aligned)");
+    if (gates && (mode != 1 || n_clusters <= 0 || nout % n_clusters || (nout / n_clusters) % 4))
+        return mortar_fail(MORTAR_ERR_ARG, "gemv_f32_one: gates need mode 1 and d_ff / n_clusters a whole multiple of 4");
+    SpmmParams p{};
+    p.row_desc = reinterpret_cast<const u32x4_t *>(W->row_desc);
+    p.codes_o = reinterpret_cast<const u32x4_t *>(W->codes_o);
+    p.sd_o = reinterpret_cast<const u32x4_t *>(W->sd_o);
+    p.col_o = reinterpret_cast<const u32x4_t *>(W->col_o);
+    p.seg_cb = W->seg_cb < W->Cb ? W->seg_cb : W->Cb;
+    p.nseg = (W->Cb + p.seg_cb - 1) / p.seg_cb;
+    p.Rb = W->Rb; p.Cb = W->Cb; p.M = B;
+    p.n_units = mode == 0 ? W->Rb : W->Rb / 2;
+    p.n_clusters = 1; p.cluster_size = gates ? (int)(nout / n_clusters) : 1 << 30;
+    const int nacc = mode + 1, nparts = p.nseg * nacc;
+    // waves per unit: a divisor of the part count where there is one (as the bf16 part-split launches)
+    const int pw = nparts == 1 ? 1 : nparts % 4 == 0 ? 4 : nparts % 3 == 0 ? 3 : nparts % 2 == 0 ? 2 : (nparts + 3) / 4 < (nparts + 2) / 3 ? 4 : 3;
+    // tokens per tile: all of them where they fit (at most five: 15 of the MFMA's 16 columns), else the most that LDS takes
+    auto fits = [&](int t) { return tile_bytes(3 * t, p.Cb) + (pw > 1 ? pw * 4 * nacc * 1024 : 0) <= 160 * 1024; };
+    int t = 0;
+    for (int c : {1, 2, 4, 5})
+        if (fits(c)) { t = c; if (c >= B) break; }
+    if (t == 0) return MORTAR_NO_KERNEL;
+    const GemvOneArgs a{x, scale, gates, y, row_act, col_act, ldx, ldy, ldg, ldr, ldc, swiglu_x != 0};
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return mode == 0 ? launch_t<1>(t, pw, p, a, st) : launch_t<2>(t, pw, p, a, st);
+}

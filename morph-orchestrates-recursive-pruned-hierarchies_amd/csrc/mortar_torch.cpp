@@ -283,6 +283,62 @@ PyObject *py_route(PyObject *, PyObject *const *a, Py_ssize_t na) {
     return Py_BuildValue("(NNN)", g, ac, au);
 }
 
+// Optional integer flags [B, >= n] of a decode product.  False: not flags this layer takes.
+bool read_flags(PyObject *o, const at::Tensor &x, int64_t B, int64_t n, const int32_t *&p, int64_t &ld) {
+    p = nullptr;
+    ld = 0;
+    if (o == Py_None) return true;
+    const at::Tensor *t = tensor_of(o);
+    if (!t || t->scalar_type() != at::kInt || t->device() != x.device() || t->dim() != 2 || t->size(0) != B || t->size(1) < n || t->stride(1) != 1)
+        return false;
+    p = static_cast<const int32_t *>(t->const_data_ptr());
+    ld = t->stride(0);
+    return true;
+}
+
+// gemv_f32(x, handle, scale, swiglu_x, swiglu_out, gates, row_act, col_act) -> y fp32 [B, out]: the decode product in the
+// reference engine's arithmetic for a matrix with one scale.
+PyObject *py_gemv_f32(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 8) {
+        PyErr_SetString(PyExc_TypeError, "gemv_f32: 8 arguments");
+        return nullptr;
+    }
+    const at::Tensor *xt = tensor_of(a[0]), *sc = tensor_of(a[2]);
+    const PackHandle *h = handle_of(a[1]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!xt || !sc || !h || sc->numel() != 1 || sc->scalar_type() != at::kFloat) Py_RETURN_NONE;
+    const at::Tensor &x = *xt;
+    const bool swx = a[3] == Py_True, swo = a[4] == Py_True;
+    const int64_t K = (int64_t)h->w->Cb * 16, nout = (int64_t)h->w->Rb * (swo ? 8 : 16);
+    if (!x.is_cuda() || sc->device() != x.device() || x.scalar_type() != at::kFloat || x.dim() != 2 || x.size(1) != K * (swx ? 2 : 1) ||
+        !x.is_contiguous() || !aligned16(x.const_data_ptr()) || (swo && (h->w->Rb & 1)))
+        Py_RETURN_NONE;
+    const int64_t B = x.size(0);
+    if (B < 1 || B > DECODE_MAX_ROWS) Py_RETURN_NONE;
+    const float *gates = nullptr;
+    int64_t ncl = 0, ldg = 0;
+    if (a[5] != Py_None) {
+        const at::Tensor *gt = tensor_of(a[5]);
+        if (!gt || !swo || gt->scalar_type() != at::kFloat || gt->device() != x.device() || gt->dim() != 2 || gt->size(0) != B || gt->stride(1) != 1)
+            Py_RETURN_NONE;
+        ncl = gt->size(1);
+        ldg = gt->stride(0);
+        if (ncl <= 0 || nout % ncl || (nout / ncl) % 4) Py_RETURN_NONE;
+        gates = static_cast<const float *>(gt->const_data_ptr());
+    }
+    const int32_t *ra, *ca;
+    int64_t ldr, ldc;
+    if (!read_flags(a[6], x, B, h->w->Rb, ra, ldr) || !read_flags(a[7], x, B, h->w->Cb, ca, ldc)) Py_RETURN_NONE;
+    const c10::DeviceGuard guard(x.device());
+    at::Tensor y = at::empty({B, nout}, x.options().requires_grad(false));
+    const int rc = mortar_gemv_f32_one(h->w, static_cast<const float *>(sc->const_data_ptr()), swo, swx, static_cast<const float *>(x.const_data_ptr()),
+                                       (int32_t)B, x.size(1), static_cast<float *>(y.data_ptr()), nout, gates, (int32_t)ncl, ldg, ra, ldr, ca, ldc,
+                                       stream_of(x));
+    if (rc == MORTAR_NO_KERNEL) Py_RETURN_NONE;
+    if (rc) return raise_rc(rc, "mortar_gemv_f32");
+    return THPVariable_Wrap(std::move(y));
+}
+
 template <PyObject *(*F)(PyObject *, PyObject *const *, Py_ssize_t)>
 PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t na) {      // torch's C++ exceptions (out of memory) as Python ones
     HANDLE_TH_ERRORS
@@ -295,6 +351,7 @@ PyMethodDef methods[] = {
     MORTAR_METHOD("mlp", py_mlp, "The carved MLP on the rows of x, or None when the call is not covered."),
     MORTAR_METHOD("routed_decode", py_routed_decode, "RMSNorm, router and gated MLP for decode rows, or None."),
     MORTAR_METHOD("route", py_route, "The router of the rows of x and its load statistics, or None."),
+    MORTAR_METHOD("gemv_f32", py_gemv_f32, "The fp32 decode product of a one-scale matrix, or None."),
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_mortar_native", "Native call layer of the MORTAR runtime.", -1, methods, nullptr, nullptr, nullptr, nullptr};

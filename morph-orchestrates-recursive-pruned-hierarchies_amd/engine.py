@@ -33,6 +33,10 @@ def mortar_gemv(x: Tensor, pack: MortarPack, swiglu_x: bool = False, swiglu_out:
     route_flags of the same step's gates, which is how the reference engine calls (engine.py:984-994)."""
     if gates is not None and cluster_size and (pack.out_features // 2) // gates.shape[-1] != cluster_size:
         raise ValueError("cluster_size does not match d_ff / n_clusters")
+    if x.dtype is torch.float32 and pack.codes.is_cuda and pack.scales_f32 is not None:
+        y = _lib.native().gemv_f32(x, pack.address, pack.scales_f32, swiglu_x, swiglu_out, gates, row_act, col_act)
+        if y is not None:
+            return y
     if x.dtype == torch.float32 or swiglu_x:
         y = ops.gemv_f32(x.float(), pack, swiglu_x=swiglu_x, swiglu_out=swiglu_out, gates=gates, row_act=row_act, col_act=col_act)
         return y if x.dtype == torch.float32 else y.to(x.dtype)

@@ -297,13 +297,14 @@ class MortarPack:
         self.struct = self._make_struct()
         self.ref = C.byref(self.struct)
         self._handle = _lib.PackHandle(C.addressof(self.struct), None, None)
+        self.address = C.addressof(self._handle)
         for rpu, t in self._scheds.items():
             setattr(self._handle, f"sched{rpu}", t.data_ptr())
 
     def handle(self, rows_per_unit: int) -> int:
         """Address of the native call layer's handle, with the schedule for plain (1) or gate/up (2) units in place."""
         self.sched(rows_per_unit)
-        return C.addressof(self._handle)
+        return self.address
 
     def _make_struct(self):
         return _lib.BcsrStruct(self.codes.data_ptr(), self.sdup.data_ptr(), self.col.data_ptr(),

@@ -53,3 +53,38 @@ def test_routed_decode_call_equals_the_general_path(dev, B, n_clusters):
         mlp.router.query_proj.weight = torch.nn.Parameter(mlp.router.query_proj.weight.flip(0).contiguous())      # a replaced parameter is seen
     y2, ref2 = dec(x), dec._general(x)
     assert torch.allclose(y2.float(), ref2.float(), rtol=1e-2, atol=1e-2 * ref2.float().abs().max().item())
+
+
+@pytest.mark.parametrize("K_blocks,seg", [(3, None), (48, None), (352, None), (352, 40), (704, None), (1376, None)])   # every token tile, 1 .. 9 parts
+@pytest.mark.parametrize("B", [1, 2, 4, 5, 6, 11])
+def test_one_launch_fp32_decode_product(dev, K_blocks, seg, B):
+    """mortar_gemv on a one-scale matrix against float64: plain and SwiGLU-on-load products with per-stream flags, and the
+    gated gate_up form."""
+    m = synth.synth_matrix(16 * 10, 16 * K_blocks, 0.25, seed=K_blocks, per_tensor_scale=True)
+    W = mortar_amd.MortarPack(synth.flat_pack(m["codes"]), m["scales"], m["col_idx"], m["offsets"], *m["shape"], dev, seg_cb=seg)
+    dense = torch.zeros(10, K_blocks, 16, 16, dtype=torch.float64, device=dev)
+    dense[torch.from_numpy(m["row_idx"]).long(), torch.from_numpy(m["col_idx"]).long()] = torch.from_numpy(m["codes"]).to(dev).double()
+    dense = dense.permute(0, 2, 1, 3).reshape(160, -1) * float(m["scales"][0])
+    g = torch.Generator(device=dev).manual_seed(B)
+    K = 16 * K_blocks
+    x2 = torch.randn(B, 2 * K, device=dev, generator=g)
+    x = x2[:, :K].contiguous()
+    ca = (torch.rand(B, K_blocks, device=dev, generator=g) < 0.6).int()
+    ra = (torch.rand(B, 10, device=dev, generator=g) < 0.6).int()
+    ra[:, 3] = 0                                                             # off for every stream
+
+    def close(got, want):
+        assert (got.double() - want).abs().max() <= 3e-6 * want.abs().max().clamp(min=1e-30) + 1e-12
+
+    close(mortar_amd.mortar_gemv(x, W), x.double() @ dense.t())
+    on = ca.repeat_interleave(16, 1).double()
+    want = (x.double() * on) @ dense.t() * ra.repeat_interleave(16, 1)
+    close(mortar_amd.mortar_gemv(x, W, row_act=ra, col_act=ca), want)
+    h = torch.nn.functional.silu(x2[:, :K].double()) * x2[:, K:].double()
+    close(mortar_amd.mortar_gemv(x2, W, swiglu_x=True), h @ dense.t())
+    gates = torch.relu(torch.randn(B, 5, device=dev, generator=g))
+    gates[:, 2] = 0
+    gu = x.double() @ dense.t()
+    want = torch.nn.functional.silu(gu[:, :80]) * gu[:, 80:] * gates.double().repeat_interleave(16, 1)
+    got = mortar_amd.mortar_gemv(x, W, swiglu_out=True, gates=gates)
+    assert torch.allclose(got.double(), want, rtol=1e-4, atol=1e-5 * want.abs().max().item() + 1e-12)
