@@ -413,6 +413,11 @@ int mortar_dds_values_bf16(const int32_t *row_ptr, const int16_t *col, const int
                            int32_t Rb, int32_t Cb, int64_t nnz, const uint16_t *x, int64_t M, int64_t ldx, uint16_t *y,
                            int64_t ldy, void *stream);
 
+/* out[j] = data[src_block[j]]^T for bf16 blocks [nnz, 16, 16]: the values of W in the block order of W^T
+ * (mortar_transpose_topology_host), so that the dX product is mortar_dds_values_bf16 on the transposed topology. */
+int mortar_transpose_blocks_bf16(const uint16_t *data, const int32_t *src_block, int64_t nnz, uint16_t *out, void *stream);
+
+
 /* ---- RMSNorm ---------------------------------------------------------------------------------- */
 
 /* mortar_gateup_swiglu_bf16 with the RMSNorm in front of the MLP (attention.RMSNorm, morph/model/attention.py:133-141,

@@ -59,14 +59,14 @@ __global__ void __launch_bounds__(NW * 64) router_gemm_kernel(const uint16_t *x,
     const int m0 = (id / n_ntiles) * MT, o0 = (id % n_ntiles) * (16 * NW) + wave * 16;
 
     // Activations: fragments (16 tokens x 32 values, 1 KB) wave + NW * i; slot l of a fragment holds 16-byte unit
-    // (l & 3) ^ (token >> 2) of token l / 4.  Weights: row 4 i + l / 16, slot l & 15 of its 256 bytes holds unit (l & 15) ^ row.
+    // (l & 3) ^ s(token) of token l / 4 (mortar_unit_swz).  Weights: row 4 i + l / 16, slot l & 15 of its 256 bytes holds unit (l & 15) ^ row.
     const uint16_t *xs[U];
     const float *ws[4];
     int kx[U], kw[4];
 #pragma unroll
     for (int i = 0; i < U; ++i) {
         const int f = wave + NW * i, t = lane >> 2, row = m0 + (f >> 1) * 16 + t;
-        kx[i] = (f & 1) * 32 + ((lane & 3) ^ (t >> 2)) * 8;
+        kx[i] = (f & 1) * 32 + ((lane & 3) ^ mortar_unit_swz(t)) * 8;
         xs[i] = x + (int64_t)(row < M ? row : M - 1) * ldx + kx[i];
     }
 #pragma unroll
@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(NW * 64) router_gemm_kernel(const uint16_t *x,
         kw[i] = (n ^ r) * 4;
         ws[i] = W + (int64_t)(o0 + r < N ? o0 + r : N - 1) * K + kw[i];
     }
-    const uint32_t rd = (uint32_t)(n * 64 + (g ^ (n >> 2)) * 16);
+    const uint32_t rd = (uint32_t)(n * 64 + (g ^ mortar_unit_swz(n)) * 16);
     // K % 8 == 0: a unit is in the row or past its end as a whole; the ones past the end are cleared (last step only)
     auto stage = [&](int k0, int buf) {
         const bool part = k0 + RG_KS > K;

@@ -88,6 +88,14 @@ def dds_values(x: Tensor, data: Tensor, T: BcsrTopology, out: Tensor | None = No
     return y
 
 
+def transpose_blocks(data: Tensor, src: Tensor) -> Tensor:
+    """out[j] = data[src[j]]^T: stored block values in the order of the transposed topology (BcsrTopology.transposed)."""
+    _need_gpu(data, "transpose_blocks")
+    out = torch.empty_like(data)
+    _lib.check(_lib.lib().mortar_transpose_blocks_bf16(_p(data), _p(src), data.shape[0], _p(out), _stream(data)), "mortar_transpose_blocks_bf16")
+    return out
+
+
 def spmm_hc_post(x: Tensor, W: MortarPack, carrier: Tensor, hres: Tensor, hpost: Tensor, term: Tensor | None = None,
                  active: Tensor | None = None, out: Tensor | None = None) -> Tensor:
     """`down` with the hyper-connection POST write in its epilogue (decode batches, M <= 64): returns

@@ -203,11 +203,11 @@ class BcsrTopology:
         self._t = None
 
     def transposed(self):
-        """(topology of W^T, src): block j of W^T is block src[j] of W, transposed (int64 device index)."""
+        """(topology of W^T, src): block j of W^T is block src[j] of W, transposed (int32 device index)."""
         if self._t is None:
             off_t, col_t, src = transpose_topology(self.h_offsets, self.h_col, self.Rb, self.Cb)
             self._t = (BcsrTopology(off_t, col_t, self.in_features, self.out_features, self.device),
-                       torch.from_numpy(src.astype(np.int64)).to(self.device))
+                       torch.from_numpy(src).to(self.device))
         return self._t
 
 

@@ -127,7 +127,7 @@ def stk_dds(lhs: Tensor, data: Tensor, offsets: Tensor, row_indices: Tensor, col
         T = _bcsr(offsets, column_indices, int(d.shape[0]), shape1, shape0, d.device)
     else:
         T, src = _bcsr(offsets, column_indices, int(d.shape[0]), shape0, shape1, d.device).transposed()
-        db = db[src].transpose(1, 2).contiguous()
+        db = ops.transpose_blocks(db, src)
     y = ops.dds_values(x, db, T)
     return y if y.dtype == lhs.dtype else y.to(lhs.dtype)
 

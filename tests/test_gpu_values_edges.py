@@ -1,0 +1,38 @@
+"""Product over stored block values at the edges of its tiles and segments, and the block transpose that feeds dX."""
+import numpy as np
+import pytest
+import torch
+
+from mortar_amd import ops
+from mortar_amd.pack import BcsrTopology
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("Rb,Cb,M", [(1, 1, 1), (33, 5, 63), (97, 79, 65), (160, 3, 15), (257, 48, 1030), (70, 155, 31),   # all of K in one tile
+                                     (49, 156, 65), (5, 390, 130), (12, 191, 4097), (200, 228, 16)])                     # K segments, whole and ragged
+@pytest.mark.parametrize("density", [0.0, 0.04, 0.5])
+def test_values_product_edges(dev, Rb, Cb, M, density):
+    rng = np.random.default_rng(Rb * 1000 + Cb)
+    mask = rng.random((Rb, Cb)) < density
+    mask[::3] = False                                     # whole rows without blocks
+    if density == 0.5:
+        mask[Rb // 2] = True                              # and one full row
+    offsets = np.concatenate([[0], np.cumsum(mask.sum(1))]).astype(np.int32)
+    col = np.nonzero(mask)[1].astype(np.int16)
+    T = BcsrTopology(offsets, col, Rb * 16, Cb * 16, dev)
+    g = torch.Generator(device=dev).manual_seed(M)
+    data = (torch.randn(T.nnz, 16, 16, device=dev, generator=g) * 0.5).bfloat16()
+    x = torch.randn(M, Cb * 16, device=dev, generator=g).bfloat16()
+    dense = torch.zeros(Rb, Cb, 16, 16, device=dev, dtype=torch.float64)
+    rows = np.repeat(np.arange(Rb), mask.sum(1))
+    dense[torch.from_numpy(rows).to(dev), torch.from_numpy(col.astype(np.int64)).to(dev)] = data.double()
+    dense = dense.permute(0, 2, 1, 3).reshape(Rb * 16, Cb * 16)
+    out = torch.full((M + 1, Rb * 16), 7.0, device=dev, dtype=torch.bfloat16)
+    y = ops.dds_values(x, data, T, out=out[:M])
+    ref, bound = x.double() @ dense.t(), x.double().abs() @ dense.abs().t()
+    assert ((y.double() - ref).abs() <= ref.abs() * 2.0 ** -8 + bound * 2.0 ** -20).all()
+    assert (out[M] == 7.0).all()                          # nothing past the last token
+    if T.nnz:
+        _, src = T.transposed()
+        assert torch.equal(ops.transpose_blocks(data, src), data[src.long()].transpose(1, 2))
