@@ -16,13 +16,23 @@
 // slice of a is fetched from HBM once and a slice of b only by the XCDs that hold its token range.  Every token range
 // writes its fp32 sums to its own slab of the workspace; a last pass adds the slabs in a fixed order and rounds to
 // bf16, so results are reproducible.
+//
+// What bounds it: a kept block needs its own b tile per MFMA (no other block of the row shares it), 1 KB of LDS reads for 16
+// cycles of the matrix core, and the two overlap only in part: three tile reads and two MFMAs per wavefront measured 298
+// cycles beside 217 and 144 alone, two reads 231.  So a is read again only where the block-row changes, nothing but reads and
+// MFMAs stands in the inner loop (a pair of slots never straddles two rows, addresses and copies are fixed over the steps),
+// and the rest is the slabs.  dW of 11264 x 2048 at 25 %, 4096 tokens: 103 -> 84 us; 4096 x 768, 16384 tokens: 68 -> 54 us;
+// 2048 x 5632, 4096 tokens: 65 -> 54 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <climits>
 #include <cstdint>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
+#include "mortar_device.h"
 #include "mortar_internal.h"
 
 namespace {
@@ -38,15 +48,10 @@ constexpr int SDD_CS = 1024 + 32;                // LDS bytes per chunk = 8 toke
 constexpr int SDD_QS = 4 * SDD_CS;               // LDS bytes per quad: 32 tokens
 constexpr int SDD_BUF = (SDD_NQ + SDD_RMAX / 4) * SDD_QS;    // one buffer: the slice of b, then the slice of a
 constexpr int SDD_STEP = 32;                     // tokens per step = K of one MFMA
-constexpr int SDD_SLAB_BLOCKS = 272;             // blocks of one fp32 slab (written, read back) that cost one unit
-#ifndef SDD_PF
-#define SDD_PF 1
-#endif
+constexpr int SDD_SLAB_BLOCKS = 140;             // blocks of one fp32 slab (written, read back) that cost one unit
+constexpr int SDD_STAGE = ((SDD_NQ + SDD_RMAX / 4) * 4 + SDD_WAVES - 1) / SDD_WAVES;       // copy instructions of a wavefront per step
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct SddArgs {
     const int32_t *plan;
@@ -54,40 +59,59 @@ struct SddArgs {
     int64_t lda, ldb, M;
     float *acc;
     uint16_t *out;
-    int32_t Cb, tsplit, steps_per_split, nsteps, nnz, per_xcd;
+    int32_t Cb, tsplit, steps_per_split, nsteps, nnz, per_xcd, n_wg, seg_cb;
 };
 
-__device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0;
-    return (uint16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
-}
-
-// 8 tokens of one feature (= lane & 15) of the block-column (or block-row) whose first token sits at LDS byte `tile`:
+// 8 tokens of one feature (= lane & 15) of the block-column (or block-row) whose first token sits at LDS address `tile`:
 // group g = lane >> 4 gets tokens {8r + g} and {8r + 4 + g}, r = 0..3 - one token of each 8-token chunk per read, which
 // spreads the 32 lanes served together over all banks.  Both operands use the same order, so the contraction is
-// unchanged.  `off` = this lane's row/piece address inside the quad.
-__device__ __forceinline__ bf16x8 read_tr(const char *smem, int tile, int off) {
-    typedef __attribute__((address_space(3))) s16x4 *lds_ptr;
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(smem + tile + off));
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(smem + tile + off + 4 * 128));
-    union { s16x4 h[2]; bf16x8 v; } u;
-    u.h[0] = lo;
-    u.h[1] = hi;
-    return u.v;
+// unchanged.  Written as inline assembly: the caller waits (lds_wait) where the operand is used, so that reads of later
+// tiles stay in flight.
+union SddTile {
+    u32x2_t h[2];
+    bf16x8_t v;
+};
+__device__ __forceinline__ void read_tr(SddTile &t, uint32_t addr) {
+    asm volatile("ds_read_b64_tr_b16 %0, %2\n\tds_read_b64_tr_b16 %1, %2 offset:512" : "=&v"(t.h[0]), "=&v"(t.h[1]) : "v"(addr));
+}
+// The same if bit BIT of the (uniform) flags is set, else `t` stays.
+template <int BIT>
+__device__ __forceinline__ void read_tr_if(SddTile &t, uint32_t addr, uint32_t flags) {
+    asm volatile("s_bitcmp1_b32 %3, %4\n\ts_cbranch_scc0 .Lsame%=\n\tds_read_b64_tr_b16 %0, %2\n\tds_read_b64_tr_b16 %1, %2 offset:512\n.Lsame%=:"
+                 : "+&v"(t.h[0]), "+&v"(t.h[1]) : "v"(addr), "s"(flags), "n"(BIT) : "scc");
+}
+// At most N reads may still be on their way afterwards.
+template <int N>
+__device__ __forceinline__ void lds_wait(SddTile &a, SddTile &b, SddTile &c) {
+    asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(a.h[0]), "+v"(a.h[1]), "+v"(b.h[0]), "+v"(b.h[1]), "+v"(c.h[0]), "+v"(c.h[1]) : "n"(N));
 }
 
-// Asynchronous 16-byte-per-lane copy global -> LDS: lane l's 16 bytes land at lds_base + 16 * l.  Written as inline
-// assembly so that the compiler does not make the LDS reads of the other buffer wait for it; the caller waits with
-// s_waitcnt vmcnt(0) and a barrier before the destination is read.  (One wait state separates the write of M0 from
-// its use as the LDS base.)
-__device__ __forceinline__ void load_to_lds_async(const void *gsrc, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gsrc) : "memory", "m0");
+// Asynchronous 16-byte-per-lane copy global -> LDS from a scalar base and a lane offset: lane l's 16 bytes land at
+// lds_base + 16 * l.  The caller waits with s_waitcnt vmcnt(0) and a barrier before the destination is read.
+__device__ __forceinline__ void load_to_lds_base(const char *base, uint32_t off, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_base), "v"(off), "s"(base) : "memory", "m0");
 }
 
-__device__ __forceinline__ uint32_t lds_addr(const char *p) {
-    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char *)p;
+// Accumulator lane (og = lane >> 4, oc = lane & 15) holds rows 4 og .. 4 og + 3 of column oc; afterwards columns
+// 4 (oc >> 2) .. + 3 of row 4 og + (oc & 3): a 4 x 4 transpose among the four lanes of a quad.
+__device__ __forceinline__ f32x4_t quad_transpose(f32x4_t v, int lane) {
+    const bool o1 = lane & 1, o2 = lane & 2;
+    auto swap = [](float x, auto ctrl) { return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true)); };
+    using xor1 = std::integral_constant<int, 0xB1>;        // quad_perm [1, 0, 3, 2]
+    using xor2 = std::integral_constant<int, 0x4E>;        // quad_perm [2, 3, 0, 1]
+    const float a = swap(o1 ? v[0] : v[1], xor1{}), b = swap(o1 ? v[2] : v[3], xor1{});
+    v = f32x4_t{o1 ? a : v[0], o1 ? v[1] : a, o1 ? b : v[2], o1 ? v[3] : b};
+    const float c = swap(o2 ? v[0] : v[2], xor2{}), d = swap(o2 ? v[1] : v[3], xor2{});
+    return f32x4_t{o2 ? c : v[0], o2 ? d : v[1], o2 ? v[2] : c, o2 ? v[3] : d};
 }
+__device__ __forceinline__ void store_block(uint16_t *out, int64_t j, f32x4_t v, int lane) {
+    const f32x4_t w = quad_transpose(v, lane);
+    const int row = 4 * (lane >> 4) + (lane & 3), c = lane & 12;
+    *reinterpret_cast<u32x2_t *>(out + j * 256 + row * 16 + c) = u32x2_t{bf16_pack2(w[0], w[1]), bf16_pack2(w[2], w[3])};
+}
+
+template <int... I, typename F>
+__device__ __forceinline__ void sdd_unroll(std::integer_sequence<int, I...>, F f) { (f(std::integral_constant<int, I>{}), ...); }
 
 template <int SDD_NB>
 __global__ __launch_bounds__(SDD_WAVES * 64) void sdd_kernel(SddArgs p) {
@@ -99,8 +123,8 @@ __global__ __launch_bounds__(SDD_WAVES * 64) void sdd_kernel(SddArgs p) {
     // L2.  The (token range, workgroup) items, workgroups in the plan's order (row groups of about the same rows side by
     // side over the K segments), are cut into 8 equal runs, one per XCD: the slice of a is then fetched from HBM once
     // (its nseg readers share an L2) and a slice of b only by the few XCDs that hold its token range.
-    const int n_wg = p.plan[0];
-    const int32_t *order = p.plan + p.plan[3];
+    const int n_wg = p.n_wg;
+    const int32_t *order = p.plan + 4 + n_wg * 4 + (int64_t)n_wg * SDD_G * 2;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     const int item = xcd * p.per_xcd + slot;
     if (slot >= p.per_xcd || item >= p.tsplit * n_wg) return;
@@ -108,117 +132,125 @@ __global__ __launch_bounds__(SDD_WAVES * 64) void sdd_kernel(SddArgs p) {
     const int wg = order[item - ts * n_wg];
     const int32_t *desc = p.plan + 4 + wg * 4;
     const int row0 = desc[0], nrows = desc[1], seg = desc[2];
-    const int seg_cb = p.plan[1];
+    const int seg_cb = p.seg_cb;
     const int c0 = seg * seg_cb;
     const int ncb = min(seg_cb, p.Cb - c0);
     const int nq = (ncb + 3) >> 2, nrq = (nrows + 3) >> 2;          // quads of block-columns / block-rows
-    // this wavefront's blocks: block index (-1 = none) and (row slot << 20 | LDS byte offset of the column's tile);
-    // the second list stays in scalar registers for the whole kernel
-    const int32_t *ent_j = p.plan + 4 + n_wg * 4 + (int64_t)(wg * SDD_WAVES + wave) * SDD_NB;
-    const int32_t *ent_o = ent_j + (int64_t)n_wg * SDD_G;
-    int eo[SDD_NB];
+    f32x4_t acc[SDD_NB];
 #pragma unroll
-    for (int b = 0; b < SDD_NB; ++b) eo[b] = __builtin_amdgcn_readfirstlane(ent_o[b]);
-    uint32_t new_row = 1u;                // bit b: slot b is in another block-row than slot b - 1 (reload the a operand)
-#pragma unroll
-    for (int b = 1; b < SDD_NB; ++b) new_row |= (uint32_t)((eo[b] >> 20) != (eo[b - 1] >> 20)) << b;
-    new_row = __builtin_amdgcn_readfirstlane(new_row);
-    f32x4 acc[SDD_NB];
-#pragma unroll
-    for (int b = 0; b < SDD_NB; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int tr_off = ((lane & 15) >> 2) * SDD_CS + (lane >> 4) * 128 + (lane & 3) * 8;
+    for (int b = 0; b < SDD_NB; ++b) acc[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const uint32_t tr_off = ((lane & 15) >> 2) * SDD_CS + (lane >> 4) * 128 + (lane & 3) * 8;
     // staging role of this lane inside one instruction: token 8c + (lane >> 3), 16-byte piece lane & 7 of the 128-byte line
     const int st_tok = lane >> 3, st_piece = lane & 7;
     const int s_begin = ts * p.steps_per_split, s_end = min(p.nsteps, s_begin + p.steps_per_split);
 
-    // Stage the slices of step s into buffer `buf` with direct global->LDS loads (asynchronous, no registers held).
-    // One wavefront instruction moves 8 tokens x one 128-byte line (4 block-columns, or 4 block-rows of a) into 1 KB
-    // of contiguous LDS.  Rows past M are not loaded; in the one partial step they are cleared with plain stores
-    // (disjoint addresses from the loads).
+    // Staging: one wavefront instruction moves 8 tokens x one 128-byte line (4 block-columns, or 4 block-rows of a) into
+    // 1 KB of contiguous LDS.  What an instruction reads and where it lands is fixed over the steps: a scalar base that
+    // moves on by one step, a lane offset, an LDS address.  Columns and rows past the slice's end read its first one of
+    // the quad (no block refers to them).
+    const int n_copy = (nq + nrq) * 4;
+    const char *base[SDD_STAGE];
+    uint32_t voff[SDD_STAGE];
+    int dst[SDD_STAGE];
+#pragma unroll
+    for (int k = 0; k < SDD_STAGE; ++k) {
+        const int i = wave + k * SDD_WAVES, c = i & 3;
+        const bool is_b = i < nq * 4;
+        const int q = is_b ? i >> 2 : (i >> 2) - nq;
+        const int piece = 4 * q + (st_piece >> 1) < (is_b ? ncb : nrows) ? st_piece : st_piece & 1;
+        base[k] = is_b ? reinterpret_cast<const char *>(p.b + (int64_t)s_begin * SDD_STEP * p.ldb + (int64_t)(c0 + 4 * q) * 16)
+                       : reinterpret_cast<const char *>(p.a + (int64_t)s_begin * SDD_STEP * p.lda + (int64_t)(row0 + 4 * q) * 16);
+        voff[k] = (uint32_t)((8 * c + st_tok) * (is_b ? p.ldb : p.lda) * 2 + piece * 16);
+        dst[k] = (is_b ? q : SDD_NQ + q) * SDD_QS + c * SDD_CS;
+    }
+    // Stages step s (the steps come in order) into buffer `buf`.  Rows past M are not loaded: in the one partial step
+    // they are cleared with plain stores (disjoint addresses from the loads).
     auto stage = [&](int s, int buf) {
-        const int64_t t0 = (int64_t)s * SDD_STEP;
-        char *dst = smem + buf * SDD_BUF;
-        const bool partial = t0 + SDD_STEP > p.M;
-        for (int i = wave; i < (nq + nrq) * 4; i += SDD_WAVES) {
-            const int q = i >> 2, c = i & 3;
-            const int64_t t = t0 + 8 * c + st_tok;
-            const int qq = q < nq ? q : SDD_NQ + q - nq;
-            if (partial && t >= p.M)
-                *reinterpret_cast<u32x4 *>(dst + qq * SDD_QS + c * SDD_CS + lane * 16) = u32x4{0u, 0u, 0u, 0u};
-            if (q < nq) {
-                if (t < p.M && 4 * q + (st_piece >> 1) < ncb)
-                    load_to_lds_async(p.b + t * p.ldb + (int64_t)(c0 + 4 * q) * 16 + st_piece * 8,
-                                      __builtin_amdgcn_readfirstlane(lds_addr(dst + qq * SDD_QS + c * SDD_CS)));
-            } else {
-                if (t < p.M && 4 * (q - nq) + (st_piece >> 1) < nrows)
-                    load_to_lds_async(p.a + t * p.lda + (int64_t)(row0 + 4 * (q - nq)) * 16 + st_piece * 8,
-                                      __builtin_amdgcn_readfirstlane(lds_addr(dst + qq * SDD_QS + c * SDD_CS)));
+        const int64_t left = p.M - (int64_t)s * SDD_STEP;
+#pragma unroll
+        for (int k = 0; k < SDD_STAGE; ++k) {
+            const int i = wave + k * SDD_WAVES;
+            if (i < n_copy) {
+                char *d = smem + buf * SDD_BUF + dst[k];
+                const uint32_t la = __builtin_amdgcn_readfirstlane(mortar_lds_addr(d));
+                if (left >= SDD_STEP) load_to_lds_base(base[k], voff[k], la);
+                else if (8 * (i & 3) + st_tok < left) load_to_lds_base(base[k], voff[k], la);
+                else *reinterpret_cast<u32x4_t *>(d + lane * 16) = u32x4_t{0u, 0u, 0u, 0u};
+                base[k] += (i < nq * 4 ? p.ldb : p.lda) * (2 * SDD_STEP);
             }
         }
     };
 
     if (s_begin < s_end) stage(s_begin, 0);
+    // this wavefront's blocks: block index (-1 = none) and (row slot << 20 | LDS byte offset of the column's tile)
+    const int32_t *ent_j = p.plan + 4 + n_wg * 4 + (int64_t)(wg * SDD_WAVES + wave) * SDD_NB;
+    const int32_t *ent_o = ent_j + (int64_t)n_wg * SDD_G;
+    const int my_j = lane < SDD_NB ? ent_j[lane] : -1;
+    // slots come in pairs of one block-row: per pair one tile of a (read again only where the row changes), per slot one of b
+    int bo[SDD_NB], ao[SDD_NB / 2];
+#pragma unroll
+    for (int b = 0; b < SDD_NB; ++b) {
+        const int e = __builtin_amdgcn_readfirstlane(ent_o[b]), rs = e >> 20;
+        bo[b] = e & 0xfffff;
+        if (b % 2 == 0) ao[b / 2] = SDD_NQ * SDD_QS + (rs >> 2) * SDD_QS + (rs & 3) * 32;
+    }
+    uint32_t new_row = 0;                 // bit k: pair k is in another block-row than pair k - 1
+#pragma unroll
+    for (int k = 1; k < SDD_NB / 2; ++k) new_row |= (uint32_t)(ao[k] != ao[k - 1]) << k;
+    new_row = __builtin_amdgcn_readfirstlane(new_row);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     int buf = 0;
     for (int s = s_begin; s < s_end; ++s) {
         if (s + 1 < s_end) stage(s + 1, buf ^ 1);            // in flight while this step multiplies
         const char *cur = smem + buf * SDD_BUF;
-        // re-materialise the flag word every step: otherwise the 22 loop-invariant tests are hoisted as 22 lane masks
-        uint32_t nr = new_row;
-        asm volatile("" : "+s"(nr));
-        nr = __builtin_amdgcn_readfirstlane(nr);
-        bf16x8 A = {};
-        // the b operand is fetched SDD_PF blocks ahead of its MFMA
-        bf16x8 Bq[SDD_PF];
-#pragma unroll
-        for (int k = 0; k < SDD_PF; ++k) Bq[k] = read_tr(cur, eo[k] & 0xfffff, tr_off);
-#pragma unroll
-        for (int b = 0; b < SDD_NB; ++b) {
-            if (nr & (1u << b)) {                 // (an empty slot repeats a valid tile: its sum is never stored)
-                const int rs = eo[b] >> 20;
-                A = read_tr(cur, SDD_NQ * SDD_QS + (rs >> 2) * SDD_QS + (rs & 3) * 32, tr_off);
+        // b is read one pair of slots ahead of its MFMAs (an empty slot repeats a valid tile: its sum is never stored)
+        const uint32_t at = mortar_lds_addr(cur) + tr_off;
+        SddTile A, B[4];
+        read_tr(A, at + ao[0]);
+        read_tr(B[0], at + bo[0]);
+        read_tr(B[1], at + bo[1]);
+        sdd_unroll(std::make_integer_sequence<int, SDD_NB / 2>{}, [&](auto kc) {
+            constexpr int k = decltype(kc)::value, c = 2 * (k & 1), n = c ^ 2;
+            if constexpr (k + 1 < SDD_NB / 2) {
+                read_tr(B[n], at + bo[2 * k + 2]);
+                read_tr(B[n + 1], at + bo[2 * k + 3]);
+                lds_wait<4>(A, B[c], B[c + 1]);
+            } else {
+                lds_wait<0>(A, B[c], B[c + 1]);
             }
-            const bf16x8 B = Bq[b % SDD_PF];
-            if (b + SDD_PF < SDD_NB) Bq[b % SDD_PF] = read_tr(cur, eo[b + SDD_PF] & 0xfffff, tr_off);
-            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[b], 0, 0, 0);
-        }
+            acc[2 * k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A.v, B[c].v, acc[2 * k], 0, 0, 0);
+            acc[2 * k + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A.v, B[c + 1].v, acc[2 * k + 1], 0, 0, 0);
+            if constexpr (k + 1 < SDD_NB / 2) read_tr_if<k + 1>(A, at + ao[k + 1], new_row);
+        });
         __builtin_amdgcn_s_waitcnt(0);                       // the next step's slices have landed
         __syncthreads();                                     // ... for every wavefront, and this buffer is free again
         buf ^= 1;
     }
-    // accumulator register r of lane (column = lane & 15, g = lane >> 4) is out[4g + r][column]
-    const int oc = lane & 15, og = lane >> 4;
+    // a slab keeps a block's sums in accumulator order (64 lanes x 16 bytes)
     float *part = p.acc + (int64_t)ts * p.nnz * 256;
 #pragma unroll
     for (int b = 0; b < SDD_NB; ++b) {
-        const int j = __builtin_amdgcn_readfirstlane(ent_j[b]);
+        const int j = __builtin_amdgcn_readlane(my_j, b);
         if (j >= 0) {
-            const int64_t base = (int64_t)j * 256 + (4 * og) * 16 + oc;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (p.tsplit > 1) part[base + r * 16] = acc[b][r];
-                else p.out[base + r * 16] = f32_to_bf16(acc[b][r]);
-            }
+            if (p.tsplit > 1) *reinterpret_cast<f32x4_t *>(part + (int64_t)j * 256 + lane * 4) = acc[b];
+            else store_block(p.out, j, acc[b], lane);
         }
     }
 }
 
 __global__ __launch_bounds__(256) void sdd_zero_kernel(float *acc, int64_t n4) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n4) reinterpret_cast<f32x4 *>(acc)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (i < n4) reinterpret_cast<f32x4_t *>(acc)[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 }
 
-// out = bf16(sum over the token ranges, in range order)
+// out = bf16(sum over the token ranges, in range order), one wavefront per block
 __global__ __launch_bounds__(256) void sdd_round_kernel(const float *acc, uint16_t *out, int64_t n4, int tsplit) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n4) {
-        f32x4 v = reinterpret_cast<const f32x4 *>(acc)[i];
-        for (int t = 1; t < tsplit; ++t) v += reinterpret_cast<const f32x4 *>(acc)[i + (int64_t)t * n4];
-        uint2 o;
-        o.x = (uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16);
-        o.y = (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16);
-        reinterpret_cast<uint2 *>(out)[i] = o;
+        f32x4_t v = reinterpret_cast<const f32x4_t *>(acc)[i];
+        for (int t = 1; t < tsplit; ++t) v += reinterpret_cast<const f32x4_t *>(acc)[i + (int64_t)t * n4];
+        store_block(out, i >> 6, v, threadIdx.x & 63);
     }
 }
 
@@ -226,24 +258,28 @@ __global__ __launch_bounds__(256) void sdd_round_kernel(const float *acc, uint16
 
 // Workgroups of a plan with `nb` blocks per wavefront: per K segment, runs of consecutive block-rows holding at most
 // 16 * nb blocks of the segment and at most SDD_RMAX rows.
-struct SddGroup { int row0, nrows, seg; std::vector<int32_t> j, o; };
+struct SddGroup { int row0, nrows, seg, blocks; std::vector<int32_t> j, o; };
 
 static bool sdd_nb_built(int nb) {
     for (int v : SDD_NB_SIZES) if (v == nb) return true;
     return false;
 }
 
+static void sdd_segments(int Cb, int &nseg, int &seg_cb) {
+    nseg = (Cb + SDD_SEG - 1) / SDD_SEG;
+    seg_cb = ((Cb + nseg - 1) / nseg + 3) & ~3;                    // whole 128-byte lines
+}
+
 static void sdd_groups(const int32_t *row_ptr, const int16_t *col, int Rb, int Cb, int nb, bool fill,
                        std::vector<SddGroup> &wgs, int &nseg, int &seg_cb) {
     const int G = SDD_WAVES * nb;
-    nseg = (Cb + SDD_SEG - 1) / SDD_SEG;
-    seg_cb = ((Cb + nseg - 1) / nseg + 3) & ~3;                    // whole 128-byte lines
+    sdd_segments(Cb, nseg, seg_cb);
     for (int sg = 0; sg < nseg; ++sg) {
-        SddGroup cur{0, 0, sg, {}, {}};
+        SddGroup cur{0, 0, sg, 0, {}, {}};
         int held = 0;
         auto flush = [&]() {
             if (held) wgs.push_back(cur);
-            cur = SddGroup{0, 0, sg, {}, {}};
+            cur = SddGroup{0, 0, sg, 0, {}, {}};
             held = 0;
         };
         for (int r = 0; r < Rb; ++r) {
@@ -253,15 +289,21 @@ static void sdd_groups(const int32_t *row_ptr, const int16_t *col, int Rb, int C
             int hi = lo;
             while (hi < e && col[hi] < (sg + 1) * seg_cb) ++hi;
             if (hi == lo) continue;
-            if (held && (held + (hi - lo) > G || r - cur.row0 + 1 > SDD_RMAX)) flush();
+            const int slots = (hi - lo + 1) & ~1;              // pairs of slots share a block-row
+            if (held && (held + slots > G || r - cur.row0 + 1 > SDD_RMAX)) flush();
             if (!held) cur.row0 = r;
             cur.nrows = r - cur.row0 + 1;
-            held += hi - lo;
+            cur.blocks += hi - lo;
+            held += slots;
             if (!fill) continue;
             for (int j = lo; j < hi; ++j) {
                 cur.j.push_back(j);
                 const int cr = col[j] - sg * seg_cb;
                 cur.o.push_back(((r - cur.row0) << 20) | ((cr >> 2) * SDD_QS + (cr & 3) * 32));
+            }
+            if (slots > hi - lo) {
+                cur.j.push_back(-1);
+                cur.o.push_back(cur.o.back());
             }
         }
         flush();
@@ -270,24 +312,28 @@ static void sdd_groups(const int32_t *row_ptr, const int16_t *col, int Rb, int C
 
 // Token ranges for M tokens over the n_wg workgroups of a plan with nb blocks per wavefront.  One workgroup runs per
 // CU and the (range, workgroup) items are dealt evenly over the XCDs, so the launch takes
-// ceil(items per XCD / CUs per XCD) rounds of ceil(steps / ranges) + 1 steps, a step costing nb + 7 units (one per
-// block and wavefront, plus staging and the barrier); every extra range adds one slab of fp32 sums to write and to
-// read back, priced per block.  The constants are a fit to launch times over group sizes, range counts and 1024 to
-// 16384 tokens (4.5 % rms).  Returns the cost of the cheapest count of ranges.
-static int64_t sdd_split(int32_t n_wg, int32_t nnz, int nb, int64_t M, int &nsteps, int &steps_per_split, int &tsplit) {
+// ceil(items per XCD / CUs per XCD) rounds of ceil(steps / ranges) steps.  A step costs nb + 7 units (a block and wavefront
+// one each, the barrier) plus a tenth per staged tile (block-rows + block-columns), a round 2.5 nb + 8 (the first slices, the
+// stores); more than one range costs the pass that adds the slabs and, per range, a slab of fp32 sums to write and to read
+// back.  A unit is 36 ns; the constants are a fit to 1022 launch times over six topologies, all group sizes, 1 to 16 ranges
+// and 512 to 16384 tokens (6.5 % rms; the choice is within 2 % of the best on average).  The ranges are chosen for 60 staged
+// tiles, whatever the plan; the returned cost of that choice counts the `tiles` given.
+constexpr int SDD_TILES = 60;
+static int64_t sdd_split(int32_t n_wg, int32_t nnz, int nb, int64_t M, int tiles, int &nsteps, int &steps_per_split, int &tsplit) {
     nsteps = (int)((M + SDD_STEP - 1) / SDD_STEP);
-    int best = 1;
-    int64_t best_cost = INT64_MAX;
-    for (int t = 1; t <= std::min(nsteps, 16); ++t) {
+    auto cost = [&](int t, int tl) {
         const int sps = (nsteps + t - 1) / t, tt = (nsteps + sps - 1) / sps;
         const int64_t per_xcd = ((int64_t)n_wg * tt + 7) / 8;
         const int64_t rounds = (per_xcd + SDD_TARGET_WGS / 8 - 1) / (SDD_TARGET_WGS / 8);
-        const int64_t cost = rounds * (sps + 1) * (nb + 7) + (tt > 1 ? (int64_t)tt * nnz / SDD_SLAB_BLOCKS : 0);
-        if (cost < best_cost) { best_cost = cost; best = t; }
-    }
+        return rounds * (sps * (10 * nb + 70 + tl) + 25 * nb + 80) + (tt > 1 ? (int64_t)tt * nnz * 10 / SDD_SLAB_BLOCKS + 530 : 0);
+    };
+    int best = 1;
+    if (nsteps > 0)
+        for (int t = 2; t <= std::min(nsteps, 16); ++t)
+            if (cost(t, SDD_TILES) < cost(best, SDD_TILES)) best = t;
     steps_per_split = std::max(1, (nsteps + best - 1) / best);
     tsplit = std::max(1, (nsteps + steps_per_split - 1) / steps_per_split);
-    return best_cost;
+    return nsteps > 0 ? cost(best, tiles) : 0;
 }
 
 // Blocks per wavefront for this topology at M tokens: the built size whose plan is cheapest by sdd_split's measure.
@@ -303,7 +349,10 @@ extern "C" int32_t mortar_sdd_blocks_per_wave_host(const int32_t *row_ptr, const
         std::vector<SddGroup> wgs;
         int nseg, seg_cb, nsteps, sps, tsplit;
         sdd_groups(row_ptr, col, Rb, Cb, nb, false, wgs, nseg, seg_cb);
-        const int64_t cost = sdd_split((int32_t)wgs.size(), row_ptr[Rb], nb, M, nsteps, sps, tsplit);
+        int64_t rows = 0;
+        for (const SddGroup &g : wgs) rows += g.nrows;
+        const int tiles = seg_cb + (int)(rows / (int64_t)std::max<size_t>(1, wgs.size()));
+        const int64_t cost = sdd_split((int32_t)wgs.size(), row_ptr[Rb], nb, M, tiles, nsteps, sps, tsplit);
         if (cost <= best_cost) { best_cost = cost; best = nb; }      // ties: the larger group (fewer staged bytes)
     }
     return best;
@@ -345,7 +394,7 @@ extern "C" int64_t mortar_sdd_plan_host(const int32_t *row_ptr, const int16_t *c
     int32_t *ent_j = plan_out + 4 + n_wg * 4, *ent_o = ent_j + n_wg * SDD_G;
     for (int64_t w = 0; w < n_wg; ++w) {
         int32_t *d = plan_out + 4 + w * 4;
-        d[0] = wgs[w].row0; d[1] = wgs[w].nrows; d[2] = wgs[w].seg; d[3] = (int32_t)wgs[w].j.size();
+        d[0] = wgs[w].row0; d[1] = wgs[w].nrows; d[2] = wgs[w].seg; d[3] = wgs[w].blocks;
         for (int i = 0; i < SDD_G; ++i) {
             const bool ok = i < (int)wgs[w].j.size();
             ent_j[w * SDD_G + i] = ok ? wgs[w].j[i] : -1;
@@ -359,7 +408,7 @@ extern "C" int64_t mortar_sdd_workspace_bytes(int32_t n_wg, int32_t nnz, int32_t
     if (n_wg <= 0 || nnz <= 0 || M < 0 || !sdd_nb_built(blocks_per_wave))
         return mortar_fail(MORTAR_ERR_ARG, "sdd_workspace_bytes: bad argument");
     int nsteps, sps, tsplit;
-    sdd_split(n_wg, nnz, blocks_per_wave, M, nsteps, sps, tsplit);
+    sdd_split(n_wg, nnz, blocks_per_wave, M, SDD_TILES, nsteps, sps, tsplit);
     return (int64_t)tsplit * nnz * 256 * (int64_t)sizeof(float);
 }
 
@@ -396,11 +445,15 @@ extern "C" int mortar_sdd_bf16(const int32_t *plan, int32_t n_wg, int32_t blocks
         (reinterpret_cast<uintptr_t>(a) & 15) || (reinterpret_cast<uintptr_t>(b) & 15) ||
         (reinterpret_cast<uintptr_t>(acc) & 15))
         return mortar_fail(MORTAR_ERR_ARG, "sdd: operands need 16-byte aligned rows (leading dimensions multiples of 8)");
+    if (lda > (1 << 26) || ldb > (1 << 26))
+        return mortar_fail(MORTAR_ERR_LIMIT, "sdd: leading dimensions above 2^26 elements (32 tokens are addressed with 32 bits)");
     const int64_t n4 = (int64_t)nnz * 64;
     SddArgs p;
     p.plan = plan; p.a = a; p.b = b; p.lda = lda; p.ldb = ldb; p.M = M; p.acc = acc; p.out = out;
-    p.Cb = Cb; p.nnz = nnz;
-    sdd_split(n_wg, nnz, blocks_per_wave, M, p.nsteps, p.steps_per_split, p.tsplit);
+    p.Cb = Cb; p.nnz = nnz; p.n_wg = n_wg;
+    int nseg;
+    sdd_segments(Cb, nseg, p.seg_cb);
+    sdd_split(n_wg, nnz, blocks_per_wave, M, SDD_TILES, p.nsteps, p.steps_per_split, p.tsplit);
     p.per_xcd = (p.tsplit * n_wg + 7) / 8;
     hipError_t e = hipSuccess;
     switch (blocks_per_wave) {
