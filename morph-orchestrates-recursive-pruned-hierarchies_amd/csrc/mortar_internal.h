@@ -14,4 +14,9 @@ int mortar_check_bcsr_host(const int32_t *row_ptr, const int16_t *col, int32_t R
 __attribute__((visibility("hidden"))) int mortar_spmm_codes_f32(const mortar_bcsr_t *W, const int32_t *sched, const uint16_t *x,
                                                                  int64_t M, int64_t ldx, float *y32, int64_t ldy, void *stream);
 
+// qv[m, :] = x[m, :] W^T + bias for few tokens (bias may be null): K shared by the waves of a workgroup.  The caller has checked
+// the shapes: d_in % 8 == 0, d_out % 4 == 0, all pointers and rows 16-byte aligned.
+__attribute__((visibility("hidden"))) int mortar_router_project_skinny(const uint16_t *x, int64_t M, int32_t d_in, int64_t ldx, const float *wq,
+                                                                       int32_t d_out, const float *bias, float *qv, int64_t ldq, void *stream);
+
 #endif

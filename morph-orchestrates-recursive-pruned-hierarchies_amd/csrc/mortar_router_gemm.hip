@@ -165,6 +165,110 @@ int launch_gemm(const uint16_t *x, int M, int K, int64_t ldx, const float *W, in
     return MORTAR_OK;
 }
 
+// The same product for fewer tokens, K <= 2048.  The kernel above gives a workgroup all of K, 32 steps behind a barrier each, and
+// has too few workgroups; here the eight waves of a workgroup share K: 16 outputs per workgroup, wave w holds the three terms of
+// 32 CH values of their rows in registers (one burst of loads, split once) and the workgroup's token tiles pass over them.
+// Activations travel two tiles ahead through LDS regions that belong to one wave (no barrier), in copies of whole 64 CH-byte row
+// pieces: operand loads straight from L2 (16 rows of 64 bytes at a power-of-two stride) took 2 us per tile.  The eight partial sums
+// of a group of 64 tokens meet in LDS.  The high terms have accumulators of their own, four chains per tile: the error stays that
+// of the wave-wide fp32 sums that this replaces.
+constexpr int RS_TG = 4;                  // token tiles of 16 per group
+
+template <int CH>
+__global__ void __launch_bounds__(512) router_skinny_kernel(const uint16_t *x, int M, int K, int64_t ldx, const float *W, int N, const float *bias,
+                                                            float *qv, int64_t ldq) {
+    constexpr int WU = 8 * CH, XU = 4 * CH, XT = 16 * XU * 16;      // 16-byte units of a row piece (weights, activations); bytes of a tile
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];       // 8 waves x 2 tiles (first the weights) | partial sums
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, g = lane >> 4;
+    const int o0 = blockIdx.x * 16, kw = wave * 32 * CH;
+    unsigned char *own = lds + wave * 2 * XT;
+    f32x4_t *part = reinterpret_cast<f32x4_t *>(lds + 16 * XT);
+    // token tiles of this workgroup in order: tile t is tile t % RS_TG of its group t / RS_TG
+    auto tile_row = [&](int t) { return ((int)blockIdx.y + t / RS_TG * (int)gridDim.y) * 16 * RS_TG + t % RS_TG * 16; };
+    // Slot s of a tile (weights: of the 16 rows) holds unit (s % units) ^ row of row s / units: the operand reads then touch every bank
+    // once.  K % 8 == 0: a unit lies in the row or past its end as a whole; past the end the row's first values are copied and
+    // cleared after the read.
+    auto x_src = [&](int t, int i) {
+        const int s = i * 64 + lane, r = s / XU, k = kw + ((s % XU) ^ r) * 8, row = tile_row(t) + r;
+        return x + (int64_t)(row < M ? row : M - 1) * ldx + (k < K ? k : 0);
+    };
+    auto x_copy = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+            mortar_load_to_lds((const MORTAR_GLOBAL char *)x_src(t, i), __builtin_amdgcn_readfirstlane(mortar_lds_addr(own + (t & 1) * XT + i * 1024)));
+    };
+#pragma unroll
+    for (int i = 0; i < 2 * CH; ++i) {
+        const int s = i * 64 + lane, r = s / WU, k = kw + ((s % WU) ^ r) * 4, row = o0 + r;
+        mortar_load_to_lds((const MORTAR_GLOBAL char *)(W + (int64_t)(row < N ? row : N - 1) * K + (k < K ? k : 0)),
+                           __builtin_amdgcn_readfirstlane(mortar_lds_addr(own + i * 1024)));
+    }
+    u32x4_t x0[CH];                        // the first tile waits in registers: its LDS holds the weights
+#pragma unroll
+    for (int i = 0; i < CH; ++i) x0[i] = *reinterpret_cast<const u32x4_t *>(x_src(0, i));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    u32x4_t p[CH][3];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const float4 w = *reinterpret_cast<const float4 *>(own + (n * WU + ((8 * c + 2 * g + j) ^ n)) * 16);
+            v[4 * j] = w.x; v[4 * j + 1] = w.y; v[4 * j + 2] = w.z; v[4 * j + 3] = w.w;
+        }
+        split3(v, p[c]);
+        if (kw + 32 * c + 8 * g >= K) p[c][0] = p[c][1] = p[c][2] = u32x4_t{0u, 0u, 0u, 0u};
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < CH; ++i) *reinterpret_cast<u32x4_t *>(own + i * 1024 + lane * 16) = x0[i];
+    if (tile_row(1) < M) x_copy(1);
+    for (int t0 = 0; tile_row(t0) < M; t0 += RS_TG) {
+        f32x4_t acc[RS_TG];
+#pragma unroll
+        for (int i = 0; i < RS_TG; ++i) {
+            const int t = t0 + i;
+            f32x4_t hi[4], lo = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) hi[c] = lo;
+            if (tile_row(t) < M) {
+                // tile t has landed: the copies of tile t + 1, where there is one, are all that may be in flight
+                if (tile_row(t + 1) < M) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(CH) : "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                u32x4_t b[CH];
+#pragma unroll
+                for (int c = 0; c < CH; ++c) b[c] = *reinterpret_cast<const u32x4_t *>(own + (t & 1) * XT + (n * XU + ((4 * c + g) ^ n)) * 16);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if (tile_row(t + 2) < M) x_copy(t + 2);
+#pragma unroll
+                for (int c = 0; c < CH; ++c) {
+                    if (kw + 32 * c + 8 * g >= K) b[c] = u32x4_t{0u, 0u, 0u, 0u};
+                    lo = mortar_mfma(p[c][2], b[c], lo);
+                    hi[c & 3] = mortar_mfma(p[c][0], b[c], hi[c & 3]);
+                    lo = mortar_mfma(p[c][1], b[c], lo);
+                }
+            }
+            acc[i] = lo + ((hi[0] + hi[1]) + (hi[2] + hi[3]));
+        }
+#pragma unroll
+        for (int i = 0; i < RS_TG; ++i) part[(wave * RS_TG + i) * 64 + lane] = acc[i];
+        __syncthreads();
+        if (wave < RS_TG) {                                   // wave i finishes tile i: a lane holds outputs o0 + 4 g .. + 3 of token n
+            f32x4_t s = part[wave * 64 + lane];
+#pragma unroll
+            for (int k = 1; k < 8; ++k) s += part[(k * RS_TG + wave) * 64 + lane];
+            const int m = tile_row(t0 + wave) + n, o = o0 + 4 * g;
+            if (m < M && o < N) {
+                if (bias) s += *reinterpret_cast<const f32x4_t *>(bias + o);
+                *reinterpret_cast<f32x4_t *>(qv + (int64_t)m * ldq + o) = s;
+            }
+        }
+        __syncthreads();
+    }
+}
+
 // ---- load statistics -----------------------------------------------------------------------------------------------
 
 constexpr int ST_ROWS = 64;          // tokens per workgroup of the first pass
@@ -244,6 +348,39 @@ int check_launch(const char *what) {
 
 }  // namespace
 
+namespace {
+template <int CH>
+int launch_skinny(dim3 grid, const uint16_t *x, int M, int K, int64_t ldx, const float *W, int N, const float *bias, float *qv, int64_t ldq, hipStream_t st) {
+    constexpr int smem = 16 * (16 * 4 * CH * 16) + 8 * RS_TG * 1024;
+    static_assert(smem <= 160 * 1024, "LDS of a CU");
+    static bool done = false;
+    if (!done) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(router_skinny_kernel<CH>), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "router projection: %s", hipGetErrorString(e));
+        done = true;
+    }
+    hipLaunchKernelGGL(router_skinny_kernel<CH>, grid, dim3(512), smem, st, x, M, K, ldx, W, N, bias, qv, ldq);
+    return check_launch("router projection");
+}
+}  // namespace
+
+// One workgroup per CU: 16 outputs each, the token groups of 64 dealt over what is left of the chip.
+static int64_t skinny_rounds(int64_t M, int32_t d_out) {
+    const int64_t groups = (M + 16 * RS_TG - 1) / (16 * RS_TG), gy = d_out > 4096 ? 1 : 256 / ((d_out + 15) / 16);
+    return (groups + gy - 1) / gy;
+}
+
+int mortar_router_project_skinny(const uint16_t *x, int64_t M, int32_t d_in, int64_t ldx, const float *wq, int32_t d_out, const float *bias,
+                                 float *qv, int64_t ldq, void *stream) {
+    const int nt = (d_out + 15) / 16;
+    const int64_t groups = (M + 16 * RS_TG - 1) / (16 * RS_TG), rounds = skinny_rounds(M, d_out);
+    const int64_t gy = (groups + rounds - 1) / rounds;
+    const dim3 grid((unsigned)nt, (unsigned)gy);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (d_in <= 1024) return launch_skinny<4>(grid, x, (int)M, d_in, ldx, wq, d_out, bias, qv, ldq, st);
+    return launch_skinny<8>(grid, x, (int)M, d_in, ldx, wq, d_out, bias, qv, ldq, st);
+}
+
 extern "C" int mortar_router_project_bf16(const uint16_t *x, int64_t M, int32_t d_in, int64_t ldx, const float *wq, int32_t d_out, float *qv,
                                           int64_t ldq, void *stream) {
     if (!x || !wq || !qv) return mortar_fail(MORTAR_ERR_ARG, "router projection: null pointer");
@@ -258,6 +395,12 @@ extern "C" int mortar_router_project_bf16(const uint16_t *x, int64_t M, int32_t 
     const int64_t nt8 = (d_out + 127) / 128, w64 = (M + 63) / 64 * ((d_out + 63) / 64);
     const int64_t c256 = ((M + 255) / 256 * nt8 + 255) / 256 * 356, c128 = ((M + 127) / 128 * nt8 + 255) / 256 * 228;
     const int64_t c64 = w64 <= 256 ? 131 : (w64 + 511) / 512 * 164;
+    // The kernel that shares K takes 30 + 17 units per round of 64-token groups where a wave holds 256 values of K (6.5 + 3.7 us) and,
+    // where it holds 128, 37 + 20 units of a K of 1024.  Against the tiles: 65 tokens x 2048 x 2048 27.4 -> 9.4 us, 300 28 -> 17,
+    // 700 34 -> 28, 1000 35 against 36; at 1024 values 65 15.1 -> 5.8, 1000 16.1 -> 13.0, 2000 20 against 21.
+    const int64_t rs = skinny_rounds(M, d_out);
+    const int64_t csk = d_in > 2048 ? INT64_MAX : d_in > 1024 ? (30 + 17 * rs) * 2048 / d_in : (37 + 20 * rs) * 1024 / d_in;
+    if (csk <= c64 && csk <= c128 && csk <= c256) return mortar_router_project_skinny(x, M, d_in, ldx, wq, d_out, nullptr, qv, ldq, stream);
     int rc;
     if (c256 <= c128 && c256 <= c64) rc = launch_gemm<256, 8, 2>(x, (int)M, d_in, ldx, wq, d_out, qv, ldq, st);
     else if (c128 <= c64) rc = launch_gemm<128, 8, 2>(x, (int)M, d_in, ldx, wq, d_out, qv, ldq, st);

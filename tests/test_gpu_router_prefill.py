@@ -27,6 +27,30 @@ def test_projection_has_fp32_accuracy(dev, M, d_in, d_out):
     assert ((qv - ref).abs() <= bound).all(), (qv - ref).abs().max().item()
 
 
+@pytest.mark.parametrize("M", [65, 129, 300])                             # the kernel that shares K: whole and ragged K, outputs, token groups
+@pytest.mark.parametrize("d_in,d_out", [(1000, 1024), (1032, 260), (2040, 2044)])
+def test_shared_k_projection_has_fp32_accuracy(dev, M, d_in, d_out):
+    test_projection_has_fp32_accuracy(dev, M, d_in, d_out)
+
+
+@pytest.mark.parametrize("B", [5, 16, 17, 33, 64])
+@pytest.mark.parametrize("d", [8, 136, 1032, 2040])
+def test_decode_projection_on_the_matrix_cores(dev, B, d):
+    g = torch.Generator(device=dev).manual_seed(B + d)
+    x = torch.randn(B, d + 8, device=dev, generator=g).to(torch.bfloat16)[:, :d]
+    w, iv = torch.randn(d, d, device=dev, generator=g) * 0.05, torch.randn(d, device=dev, generator=g)
+    qv, gates = torch.full((B, d), float("nan"), device=dev), torch.empty(B, 4, device=dev)
+    one, keys = torch.ones(d, device=dev), torch.randn(2, 2, d // 2, device=dev, generator=g)
+    for bias in (None, iv):
+        rc = _lib.lib().mortar_router_bf16(x.data_ptr(), 0, B, d, x.stride(0), w.data_ptr(), bias.data_ptr() if bias is not None else None,
+                                           one.data_ptr(), one.data_ptr(), 1e-5, keys[0].data_ptr(), keys[1].data_ptr(), 2, one.data_ptr(), 4, 2,
+                                           qv.data_ptr(), None, gates.data_ptr(), None, torch.cuda.current_stream().cuda_stream)
+        _lib.check(rc, "router")
+        ref = x.double() @ w.double().t() + (0 if bias is None else iv.double())
+        bound = (x.double().abs() @ w.double().abs().t() + iv.double().abs()) * 2.0 ** -22
+        assert ((qv.double() - ref).abs() <= bound).all(), (qv.double() - ref).abs().max().item()
+
+
 def test_projection_is_exact_on_small_integers(dev):
     x = torch.randint(-8, 9, (300, 128), device=dev).to(torch.bfloat16)
     w = torch.randint(-2 ** 15, 2 ** 15, (96, 128), device=dev).float()       # needs two of the three terms; every sum fits 24 bits
