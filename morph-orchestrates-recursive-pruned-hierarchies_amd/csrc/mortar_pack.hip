@@ -4,8 +4,8 @@
 // block_sparse.py:909-919 on every QAT forward: scale = mean|w|, q = sign(w/s) * (|w/s| > threshold)) and keeps the
 // transposed topology for the dX product as index arrays over the same data (stk matrix.py:107-125).  Here the
 // topology of a pack (columns, offsets, octet positions) is fixed once on the host, and this kernel refreshes the
-// values: one wavefront per block reads the 256 values (optionally of another block, transposed: the dX pack),
-// forms the scale, and writes the row dwords into `codes`, the octet stream and its 4-bit copy.
+// values: a wavefront reads four blocks (optionally other blocks, transposed: the dX pack), forms the scale, and writes the row
+// dwords into `codes`, the octet stream and its 4-bit copy.
 #include <hip/hip_runtime.h>
 
 #include "mortar_internal.h"
@@ -13,11 +13,6 @@
 namespace {
 
 constexpr int PARTIALS = 256;           // workgroups of the |w| reduction; the workspace holds one double each
-
-__device__ __forceinline__ float load_val(const void *v, int64_t i, bool f32) {
-    if (f32) return reinterpret_cast<const float *>(v)[i];
-    return __uint_as_float((uint32_t) reinterpret_cast<const uint16_t *>(v)[i] << 16);
-}
 
 __device__ __forceinline__ double wave_sum(double x) {
 #pragma unroll
@@ -32,8 +27,7 @@ __global__ __launch_bounds__(256) void abs_sum_kernel(const void *values, int64_
     double s = 0.0;
     const int per = f32 ? 4 : 8;                                     // values per 16-byte piece
     const uint4 *v = reinterpret_cast<const uint4 *>(values);
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n / per; i += (int64_t)PARTIALS * 256) {
-        const uint4 q = v[i];
+    auto add = [&](uint4 q) {
         const uint32_t w[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -44,6 +38,17 @@ __global__ __launch_bounds__(256) void abs_sum_kernel(const void *values, int64_
                 s += (double)fabsf(__uint_as_float(w[e] & 0xffff0000u));
             }
         }
+    };
+    // eight pieces in flight per thread: with one wave per SIMD, a load per turn of the loop waits out its latency
+    constexpr int64_t STEP = (int64_t)PARTIALS * 256;
+    const int64_t m = n / per;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < m; i += 8 * STEP) {
+        uint4 q[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) q[u] = v[i + u * STEP < m ? i + u * STEP : i];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (i + u * STEP < m) add(q[u]);
     }
     s = wave_sum(s);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = s;
@@ -68,38 +73,65 @@ struct RequantArgs {
     float ternary_tol;      // > 0: with a given scale, flag values that are neither 0 nor +-s within this relative bound
 };
 
-// mode 0: one scale per matrix from the partial sums, 1: one per block, 2: scale_in[0], 3: scale_in[source block]
+// The smallest float c > 0 with RN(c / s) > threshold, so that |w / s| > threshold is |w| >= c without a division per value (the
+// rounded quotient does not fall as w grows).  Lane l tries the float l - 32 steps from threshold * s; false when the change does not lie
+// between those (a quotient that underflows), and the caller divides.
+__device__ __forceinline__ bool code_cut(float s, float threshold, int lane, float &cut) {
+    const int b = (int)__float_as_uint(threshold * s) + lane - 32;
+    const float c = __uint_as_float(b > 0 ? (uint32_t)b : 0u);
+    const uint64_t above = __ballot(c / s > threshold);
+    cut = __shfl(c, above ? __builtin_ctzll(above) : 0);
+    return above != 0 && (above & 1) == 0 && (above & (above + (above & -above))) == 0 && (above >> 63) != 0;
+}
+
+// mode 0: one scale per matrix from the partial sums, 1: one per block, 2: scale_in[0], 3: scale_in[source block].
+// A wavefront takes four blocks, a lane one row of one of them: 32 or 64 bytes of values in, and one dword for each of the arrays out.
+// One wave per block with the quotients of four values per lane was bound by its vector instructions (gate_up and down at
+// 2048 x 5632 and 25 %, both orientations: 12.5 us on average): a row is encoded by one comparison per value, and a transposed
+// block is turned as 16 x 16 two-bit codes in registers, four exchanges between the 16 lanes of a block (now 6.6 us).
+template <bool F32>
 __global__ __launch_bounds__(256) void requant_kernel(RequantArgs a) {
-    __shared__ float tr[4][16][17];                     // per wavefront: one block, for the transposed read
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int j = blockIdx.x * 4 + wv;
-    if (j >= a.nnz) return;
-    const int src = a.src_block ? a.src_block[j] : j;
-    const int n = lane >> 2, q = lane & 3;
-    // the lane's four consecutive values of row n of the source block, in one load
-    float w[4];
-    if (a.f32) {
-        const float4 v = reinterpret_cast<const float4 *>(a.values)[(int64_t)src * 64 + lane];
-        w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+    const int lane = threadIdx.x & 63, n = lane & 15;
+    const int j0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 4, j = j0 + (lane >> 4);
+    if (j0 >= a.nnz) return;
+    const bool on = j < a.nnz;
+    const int jc = on ? j : a.nnz - 1;
+    const int src = a.src_block ? a.src_block[jc] : jc;
+    const int P = a.pos[jc];
+    float w[16];
+    if (F32) {
+        const float4 *v = reinterpret_cast<const float4 *>(a.values) + (int64_t)src * 64 + n * 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float4 x = v[e];
+            w[4 * e] = x.x; w[4 * e + 1] = x.y; w[4 * e + 2] = x.z; w[4 * e + 3] = x.w;
+        }
     } else {
-        const uint2 v = reinterpret_cast<const uint2 *>(a.values)[(int64_t)src * 64 + lane];
-        w[0] = __uint_as_float(v.x << 16); w[1] = __uint_as_float(v.x & 0xffff0000u);
-        w[2] = __uint_as_float(v.y << 16); w[3] = __uint_as_float(v.y & 0xffff0000u);
-    }
-    if (a.transpose) {                                  // element (n, 4q + e) of the result is element (4q + e, n) of the source
+        const uint4 *v = reinterpret_cast<const uint4 *>(a.values) + (int64_t)src * 32 + n * 2;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) tr[wv][n][4 * q + e] = w[e];
-        __builtin_amdgcn_wave_barrier();
+        for (int e = 0; e < 2; ++e) {
+            const uint4 x = v[e];
+            const uint32_t u[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] = tr[wv][4 * q + e][n];
+            for (int k = 0; k < 4; ++k) {
+                w[8 * e + 2 * k] = __uint_as_float(u[k] << 16);
+                w[8 * e + 2 * k + 1] = __uint_as_float(u[k] & 0xffff0000u);
+            }
+        }
     }
     float s;
     if (a.mode == 0) {
         const double t = wave_sum((a.partial[lane] + a.partial[lane + 64]) + (a.partial[lane + 128] + a.partial[lane + 192]));
         s = fmaxf((float)(t / ((double)a.nnz * 256.0)), 1e-8f);
     } else if (a.mode == 1) {
-        const double t = wave_sum(((double)fabsf(w[0]) + (double)fabsf(w[1])) + ((double)fabsf(w[2]) + (double)fabsf(w[3])));
-        s = fmaxf((float)(t * (1.0 / 256.0)), 1e-6f);
+        double t[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            t[q] = ((double)fabsf(w[4 * q]) + (double)fabsf(w[4 * q + 1])) + ((double)fabsf(w[4 * q + 2]) + (double)fabsf(w[4 * q + 3]));
+#pragma unroll
+            for (int o = 8; o > 0; o >>= 1) t[q] += __shfl_xor(t[q], o);
+        }
+        s = fmaxf((float)(((t[0] + t[2]) + (t[1] + t[3])) * (1.0 / 256.0)), 1e-6f);
     } else {
         s = a.scale_in[a.mode == 2 ? 0 : src];
     }
@@ -110,7 +142,7 @@ __global__ __launch_bounds__(256) void requant_kernel(RequantArgs a) {
     if ((sb & 0x7fffu) != 0) {
         const uint32_t e8 = (sb >> 7) & 0xffu;
         if (e8 < 27 || e8 > 227) {
-            if (lane == 0 && a.status) a.status[0] = 1;
+            if (on && n == 0 && a.status) a.status[0] = 1;
         } else {
             const uint32_t adj = sb - 0x0400u;
             sd = adj | (adj << 16);
@@ -120,33 +152,56 @@ __global__ __launch_bounds__(256) void requant_kernel(RequantArgs a) {
         // every value must be 0 or +-s up to the bound (a bf16 cast of +-s(1 + rounding) may land one step beside bf16(s))
         bool bad = false;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < 16; ++e) {
             const float m = fabsf(w[e]);
             bad = bad || !(m <= a.ternary_tol * s || fabsf(m - s) <= a.ternary_tol * s);
         }
-        if (bad) a.status[1] = 1;
+        if (on && bad) a.status[1] = 1;
     }
+    // two bits per value in column order: 1 = +, 3 = -
     uint32_t row = 0;
+    float cut;
+    const uint32_t flip = u & 0x80000000u;                       // a given scale may be negative
+    if (!(a.mode & 1) && code_cut(fabsf(s), a.threshold, lane, cut)) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int c = 4 * q + e;
-        const float wn = w[e] / s;
-        const uint32_t enc = (fabsf(wn) > a.threshold && wn != 0.f && sd != 0) ? (wn < 0.f ? 3u : 1u) : 0u;
-        row |= enc << (2 * (c < 8 ? 2 * c + 1 : 2 * (c - 8)));
+        for (int e = 0; e < 16; ++e) {
+            const uint32_t enc = 1u | ((__float_as_uint(w[e]) ^ flip) >> 30 & 2u);
+            row |= (fabsf(w[e]) >= cut ? enc : 0u) << (2 * e);
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const float wn = w[e] / s;
+            row |= (fabsf(wn) > a.threshold && wn != 0.f ? (wn < 0.f ? 3u : 1u) : 0u) << (2 * e);
+        }
     }
-    row |= __shfl_xor(row, 1);
-    row |= __shfl_xor(row, 2);
-    const int P = a.pos[j];
-    if (q == 0) {
-        a.codes[(int64_t)j * 16 + n] = row;
-    } else if (q == 1) {
-        a.codes_o[(int64_t)(P >> 2) * 64 + n * 4 + (P & 3)] = row;
-    } else if (a.codes4_o) {
-        const int h = q - 2;
-        const int64_t g = P >> 3, s2 = (P >> 2) & 1;
-        a.codes4_o[((g * 4 + 2 * s2 + h) * 16 + n) * 4 + (P & 3)] = (row << (2 * h)) & 0xCCCCCCCCu;
+    if (sd == 0) row = 0;
+    if (a.transpose) {                                  // 16 x 16 codes across the 16 lanes of the block
+        auto turn = [&](int o, int bits, uint32_t low) {        // swaps the off-diagonal halves of every 2 o x 2 o square
+            const uint32_t other = (uint32_t)__shfl_xor((int)row, o);
+            row = (n & o) ? (row & ~low) | ((other & ~low) >> bits) : (row & low) | ((other & low) << bits);
+        };
+        turn(8, 16, 0x0000ffffu);
+        turn(4, 8, 0x00ff00ffu);
+        turn(2, 4, 0x0f0f0f0fu);
+        turn(1, 2, 0x33333333u);
     }
-    if (lane == 0) {
+    // device order of a row: column c < 8 in field 2 c + 1, column c >= 8 in field 2 (c - 8)
+    auto spread = [](uint32_t x) {
+        x = (x | (x << 8)) & 0x00ff00ffu;
+        x = (x | (x << 4)) & 0x0f0f0f0fu;
+        return (x | (x << 2)) & 0x33333333u;
+    };
+    row = (spread(row & 0xffffu) << 2) | spread(row >> 16);
+    if (!on) return;
+    a.codes[(int64_t)j * 16 + n] = row;
+    a.codes_o[(int64_t)(P >> 2) * 64 + n * 4 + (P & 3)] = row;
+    if (a.codes4_o) {
+        const int64_t o4 = (((int64_t)(P >> 3) * 4 + 2 * ((P >> 2) & 1)) * 16 + n) * 4 + (P & 3);
+        a.codes4_o[o4] = row & 0xCCCCCCCCu;
+        a.codes4_o[o4 + 64] = (row << 2) & 0xCCCCCCCCu;
+    }
+    if (n == 0) {
         a.sdup[j] = sd;
         a.sd_o[P] = sd;
         if (a.scale_out) a.scale_out[(a.mode == 0 || a.mode == 2) ? 0 : j] = s;
@@ -217,7 +272,9 @@ extern "C" int mortar_requantize(const mortar_bcsr_t *W, const void *values, int
     a.mode = scale_mode;
     a.threshold = threshold;
     a.ternary_tol = ternary_tol;
-    hipLaunchKernelGGL(requant_kernel, dim3((W->nnz + 3) / 4), dim3(256), 0, st, a);
+    const dim3 grid((W->nnz + 15) / 16);
+    if (values_f32) hipLaunchKernelGGL(requant_kernel<true>, grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(requant_kernel<false>, grid, dim3(256), 0, st, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "requantize: %s", hipGetErrorString(e));
     return MORTAR_OK;

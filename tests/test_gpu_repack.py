@@ -87,6 +87,29 @@ def test_requantize_threshold_is_strict(dev):
     assert s.tolist() == [4.0] and (q[:, 0, :] == 0).all() and (q[:, 1:, :] == 1).all()
 
 
+@pytest.mark.parametrize("scale", [0.037, -0.037, 1e-12, 3e20])
+@pytest.mark.parametrize("thr", [0.0, 0.5, 1 / 3, 0.7, 5.0, 1e-30])
+def test_requantize_codes_are_those_of_the_rounded_quotient(dev, scale, thr):
+    """One scale per matrix: values from 40 floats below to 40 above threshold * scale, an odd number of blocks, both orientations."""
+    m = synth.synth_matrix(16 * 3, 16 * 9, 0.4, seed=5)
+    nnz = m["col_idx"].size
+    s, t = np.float32(scale), np.float32(thr)
+    base = int(np.float32(t * abs(s)).view(np.uint32))
+    bits = np.clip(base + np.arange(-40, 41, dtype=np.int64), 0, 0x7f7fffff).astype(np.uint32)
+    rng = np.random.Generator(np.random.PCG64(6))
+    v = rng.choice(bits.view(np.float32), size=(nnz, 16, 16)) * rng.choice(np.array([-1, 1], np.float32), size=(nnz, 16, 16))
+    v[0, 0, :4] = [0.0, -0.0, np.inf, -np.inf]
+    with np.errstate(under="ignore"):
+        q = _rule(v, s, t)
+    W = MortarPack(None, None, m["col_idx"], m["offsets"], 16 * 3, 16 * 9, dev)
+    vt, st = torch.from_numpy(v).to(dev), torch.tensor([s])
+    W.requantize(vt, scale=st, threshold=thr, sync=False)
+    assert np.array_equal(decode_blocks(W.codes.cpu().numpy().view(np.uint32)), q)
+    Wt = W.transposed()
+    Wt.requantize(vt, scale=st, threshold=thr, transpose=True, sync=False)
+    assert np.array_equal(decode_blocks(Wt.codes.cpu().numpy().view(np.uint32)), q[Wt.src_block.cpu().numpy()].transpose(0, 2, 1))
+
+
 def test_requantize_given_scales_and_refresh(dev):
     """Given scales (one or per block), a second refresh with other values, and the asynchronous form."""
     m = synth.synth_matrix(16 * 8, 16 * 24, 0.3, seed=21)
