@@ -286,14 +286,14 @@ __device__ __attribute__((noinline)) void ranked_logits(const float *sct, int ns
 // (LayerNorm weights, its slices of the sub-key rows of its wave) is fetched into registers before the first reduction,
 // so the kernel pays one memory round trip instead of one per phase and key row.
 template <int MAXPL, int PRE>
-__global__ void __launch_bounds__(256) router_tail_kernel(const float *qv, int d, const float *ln_w, const float *ln_b,
+__global__ void __launch_bounds__(256) router_tail_kernel(const float *qv, int d, int64_t ldq, const float *iter_vec, const float *ln_w, const float *ln_b,
                                                            float ln_eps, const float *ka, const float *kb, int nsk,
                                                            const float *bias, int n, int k, float *logits_out,
                                                            float *gates, uint8_t *active) {
     extern __shared__ __attribute__((aligned(16))) float sm[];       // qn[d] | s[2 * nsk] | logits[n] | red[4] | sort keys
     float *qn = sm, *sc = sm + d, *lg = sc + 2 * nsk, *red = lg + n;
     const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const float *q = qv + (int64_t)b * d;
+    const float *q = qv + (int64_t)b * ldq;
     const int d2 = d / 2, n4 = d2 / 4;          // d % 8 == 0: both halves are whole float4 runs
     constexpr int QE = 8, DPW = PRE > 0 ? PRE : 1, KU = 4;      // PRE: entries per thread, sub-key dots per wave, float4 per lane and dot
     float qe[QE], lw[QE], lbv[QE];
@@ -304,6 +304,13 @@ __global__ void __launch_bounds__(256) router_tail_kernel(const float *qv, int d
             const int i = tid + 256 * j, ic = i < d ? i : d - 1;
             qe[j] = q[ic]; lw[j] = ln_w[ic]; lbv[j] = ln_b[ic];
         }
+        float iv[QE];
+#pragma unroll
+        for (int j = 0; j < QE; ++j) iv[j] = 0.f;
+        if (iter_vec) {
+#pragma unroll
+            for (int j = 0; j < QE; ++j) iv[j] = iter_vec[tid + 256 * j < d ? tid + 256 * j : d - 1];
+        }
 #pragma unroll
         for (int cc = 0; cc < DPW; ++cc) {
             int c = wave + 4 * cc;
@@ -312,13 +319,17 @@ __global__ void __launch_bounds__(256) router_tail_kernel(const float *qv, int d
 #pragma unroll
             for (int u = 0; u < KU; ++u) kreg[cc][u] = lane + 64 * u < n4 ? kr[lane + 64 * u] : float4{0.f, 0.f, 0.f, 0.f};
         }
+        if (iter_vec) {
+#pragma unroll
+            for (int j = 0; j < QE; ++j) qe[j] += iv[j];
+        }
     }
     float s = 0.f;
     if (PRE) {
 #pragma unroll
         for (int j = 0; j < QE; ++j) s += tid + 256 * j < d ? qe[j] : 0.f;
     } else {
-        for (int i = tid; i < d; i += 256) { const float t = q[i]; qn[i] = t; s += t; }      // a thread re-reads its own entries
+        for (int i = tid; i < d; i += 256) { const float t = iter_vec ? q[i] + iter_vec[i] : q[i]; qn[i] = t; s += t; }      // a thread re-reads its own entries
     }
     const float mean = block_sum256(s, red) / (float)d;
     float v = 0.f;
@@ -655,12 +666,18 @@ __global__ void __launch_bounds__(512) router_scores_kernel(const float *qv, int
 #pragma unroll
     for (int j = 0; j < PF; ++j) fetch(j);
     float s = 0.f;
+    if (iv) {                        // eight loads in flight (one test per chunk made each wait for the one before)
+#pragma unroll
+        for (int j0 = 0; j0 < CH; j0 += 8) {
+            float4 c[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) c[j] = *reinterpret_cast<const float4 *>(iv + (at(j0 + j) < d2 ? at(j0 + j) : 0));
+#pragma unroll
+            for (int j = 0; j < 8; ++j) { v[j0 + j].x += c[j].x; v[j0 + j].y += c[j].y; v[j0 + j].z += c[j].z; v[j0 + j].w += c[j].w; }
+        }
+    }
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
-        if (iv) {
-            const float4 c = *reinterpret_cast<const float4 *>(iv + (at(j) < d2 ? at(j) : 0));
-            v[j].x += c.x; v[j].y += c.y; v[j].z += c.z; v[j].w += c.w;
-        }
         if (at(j) >= d2) v[j] = zero4;
         s += (v[j].x + v[j].y) + (v[j].z + v[j].w);
     }
@@ -869,6 +886,30 @@ extern "C" int mortar_remoe_gates(const float *logits, int64_t M, int32_t n, int
     return check_launch("remoe_gates");
 }
 
+// One workgroup per token.
+static int launch_tail(const float *qv, int64_t N, int32_t d, int64_t ldq, const float *iter_vec, const float *ln_w, const float *ln_b, float ln_eps,
+                       const float *ka, const float *kb, int32_t nsk, const float *bias, int32_t n, int32_t k, float *logits_out, float *gates,
+                       uint8_t *active, hipStream_t st) {
+    size_t sort_keys = 0;                          // nsk^2 > n: room for the product scores, padded to a power of two
+    if ((int64_t)nsk * nsk > n) { sort_keys = 1; while (sort_keys < (size_t)nsk * nsk) sort_keys <<= 1; }
+    const size_t smem = (size_t)(d + 2 * nsk + n + 4 + sort_keys) * sizeof(float);
+    const dim3 tg((unsigned)N), blk(256);
+    const int npl = (n + 63) / 64;
+    const int pre = d > 2048 ? 0 : nsk <= 4 ? 2 : nsk <= 20 ? 10 : 0;      // sub-key dots per wave with their rows in registers
+#define MORTAR_TAILP(PL, PR) hipLaunchKernelGGL((router_tail_kernel<PL, PR>), tg, blk, smem, st, qv, d, ldq, iter_vec, ln_w, ln_b, ln_eps, \
+                                               ka, kb, nsk, bias, n, k, logits_out, gates, active)
+#define MORTAR_TAIL(PL) do { if (pre == 2) MORTAR_TAILP(PL, 2); else if (pre == 10) MORTAR_TAILP(PL, 10); else MORTAR_TAILP(PL, 0); } while (0)
+    if (npl <= 1) MORTAR_TAIL(1);
+    else if (npl <= 2) MORTAR_TAIL(2);
+    else if (npl <= 4) MORTAR_TAIL(4);
+    else if (npl <= 6) MORTAR_TAIL(6);
+    else if (npl <= 8) MORTAR_TAIL(8);
+    else MORTAR_TAIL(16);
+#undef MORTAR_TAILP
+#undef MORTAR_TAIL
+    return check_launch("router tail");
+}
+
 extern "C" int mortar_router_bf16(const void *x, int32_t x_is_f32, int64_t B, int32_t d, int64_t ldx, const float *wq,
                                   const float *iter_vec, const float *ln_w, const float *ln_b, float ln_eps,
                                   const float *ka, const float *kb, int32_t nsk, const float *bias, int32_t n,
@@ -901,24 +942,7 @@ extern "C" int mortar_router_bf16(const void *x, int32_t x_is_f32, int64_t B, in
         rc = check_launch("router projection");
     }
     if (rc) return rc;
-    size_t sort_keys = 0;                          // nsk^2 > n: room for the product scores, padded to a power of two
-    if ((int64_t)nsk * nsk > n) { sort_keys = 1; while (sort_keys < (size_t)nsk * nsk) sort_keys <<= 1; }
-    const size_t smem = (size_t)(d + 2 * nsk + n + 4 + sort_keys) * sizeof(float);
-    const dim3 tg((unsigned)B);
-    const int npl = (n + 63) / 64;
-    const int pre = d > 2048 ? 0 : nsk <= 4 ? 2 : nsk <= 20 ? 10 : 0;      // sub-key dots per wave with their rows in registers
-#define MORTAR_TAILP(PL, PR) hipLaunchKernelGGL((router_tail_kernel<PL, PR>), tg, blk, smem, st, qv, d, ln_w, ln_b, ln_eps, \
-                                               ka, kb, nsk, bias, n, k, logits_out, gates, active)
-#define MORTAR_TAIL(PL) do { if (pre == 2) MORTAR_TAILP(PL, 2); else if (pre == 10) MORTAR_TAILP(PL, 10); else MORTAR_TAILP(PL, 0); } while (0)
-    if (npl <= 1) MORTAR_TAIL(1);
-    else if (npl <= 2) MORTAR_TAIL(2);
-    else if (npl <= 4) MORTAR_TAIL(4);
-    else if (npl <= 6) MORTAR_TAIL(6);
-    else if (npl <= 8) MORTAR_TAIL(8);
-    else MORTAR_TAIL(16);
-#undef MORTAR_TAILP
-#undef MORTAR_TAIL
-    return check_launch("router tail");
+    return launch_tail(qv, B, d, d, nullptr, ln_w, ln_b, ln_eps, ka, kb, nsk, bias, n, k, logits_out, gates, active, st);
 }
 
 extern "C" int mortar_router_tail_f32(const float *qv, int64_t N, int32_t d, int64_t ldq, const float *iter_vec,
@@ -937,6 +961,11 @@ extern "C" int mortar_router_tail_f32(const float *qv, int64_t N, int32_t d, int
     if ((int64_t)nsk * nsk > n && (int64_t)nsk * nsk > 1024)
         return mortar_fail(MORTAR_ERR_LIMIT, "router tail: %d x %d product keys for %d groups exceed the 1024 the kernel ranks", nsk, nsk, n);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    // One workgroup per token, its sub-key rows in registers, while that is one round of the chip: a chain of 6 to 16 us against the
+    // 12 to 25 us of the launches below, whatever the number of tokens (65 tokens, 2048 values: 19 x 19 keys for 352 groups 24.5 ->
+    // 15.5 us, 4 x 4 for 16 16.1 -> 6.5; 512: 24.9 -> 17.6; 700: 25.3 against 27.7; 2000 with 4 x 4: 17.4 -> 12.6).
+    if (d <= 2048 && (nsk <= 4 ? N <= 2048 : nsk <= 20 && N <= 512))
+        return launch_tail(qv, N, d, ldq, iter_vec, ln_w, ln_b, ln_eps, ka, kb, nsk, bias, n, k, logits_out, gates, active, st);
     if (d <= 4096 && nsk <= 32 && 2 * nsk <= n) {      // two launches; wider rows, more keys or fewer groups than scores: one
         const dim3 sg((unsigned)((N + 15) / 16)), rg((unsigned)((N + 3) / 4));
         const int ch = (d / 2 + 63) / 64;

@@ -92,6 +92,13 @@ def test_tail_against_float64(dev, N, d, nsk, n, iter_vec):
     assert torch.equal(active.bool(), gates > 0)
 
 
+@pytest.mark.parametrize("N,d,nsk,n", [(512, 2048, 20, 390), (513, 2048, 20, 390), (2048, 136, 4, 13), (2049, 136, 4, 13), (600, 1032, 16, 256),
+                                       (65, 2048, 4, 16), (65, 2056, 4, 16), (66, 768, 21, 441)])     # either side of the one-token workgroups
+@pytest.mark.parametrize("iter_vec", [False, True])
+def test_tail_dispatch_against_float64(dev, N, d, nsk, n, iter_vec):
+    test_tail_against_float64(dev, N, d, nsk, n, iter_vec)
+
+
 @pytest.mark.parametrize("M", [64, 65, 600])
 def test_router_module_call_equals_the_torch_ops(dev, M):
     torch.manual_seed(2)
