@@ -91,10 +91,30 @@ int segmented_upw(const SpmmParams &p) {
 
 // Plain product of a `down` whose input is stored in tile order (mortar_mlp_bf16): the instantiations that copy their
 // token tiles straight into LDS.  The caller has checked that the matrix runs 32-token tiles.
+// Gate/up unit pairs per wave of the K-segmented gate_up: 1, 2 or 3 (four spill), the choice with the least rounds of 256
+// workgroups x (staging + units).  A unit pair takes about 6.7 us and staging the segments 5 us (d_model 3072 and 4096), so a round
+// weighs 3 + 4 upw.  With two units per wave throughout, 400 rows of d_model 4096 were 286 workgroups: 83 -> 70 us for the MLP; 150
+// rows 52 -> 44, 1999 rows (1386 workgroups, 5.4 rounds) 236 -> 227; d_model 3072 at 200 rows 40.9 -> 34.6, at 600 64 -> 52.5.
+int gateup_upw(const SpmmParams &p) {
+    const int64_t tiles = (p.M + 31) / 32;
+    int best = 2;
+    int64_t best_cost = INT64_MAX;
+    for (int upw : {2, 3, 1}) {
+        const int64_t wgs = tiles * ((p.n_units + SEG_WAVES * upw - 1) / (SEG_WAVES * upw));
+        const int64_t cost = (wgs + 255) / 256 * (3 + 4 * upw);
+        if (cost < best_cost) { best = upw; best_cost = cost; }
+    }
+    return best;
+}
+
 template <int CODE>
 int dispatch_gateup_tiled(SpmmParams &p, hipStream_t st) {     // gate_up + SwiGLU storing tile-ordered hidden activations
     if (p.nseg == 1) return launch_resident_any<2, false, CODE, true>(p, st);
-    return mortar_launch_segmented<32, 2, false, SEG_WAVES, 2, false, CODE, true>(p, nullptr, 1, st);
+    switch (gateup_upw(p)) {
+        case 2: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 2, false, CODE, true>(p, nullptr, 1, st);
+        case 3: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 3, false, CODE, true>(p, nullptr, 1, st);
+    }
+    return mortar_launch_segmented<32, 2, false, SEG_WAVES, 1, false, CODE, true>(p, nullptr, 1, st);
 }
 
 template <int CODE>
@@ -119,7 +139,11 @@ int dispatch_prefill(int kind, SpmmParams &p, hipStream_t st) {
             return mortar_launch_segmented<32, 1, false, SEG_WAVES, SEG_UPW, false, CODE>(p, nullptr, 1, st);
         case 1:
             if (p.nseg == 1) return launch_resident_any<2, false, CODE>(p, st);
-            return mortar_launch_segmented<32, 2, false, SEG_WAVES, 2, false, CODE>(p, nullptr, 1, st);
+            switch (gateup_upw(p)) {
+                case 2: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 2, false, CODE>(p, nullptr, 1, st);
+                case 3: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 3, false, CODE>(p, nullptr, 1, st);
+            }
+            return mortar_launch_segmented<32, 2, false, SEG_WAVES, 1, false, CODE>(p, nullptr, 1, st);
         case 2:
             return launch_resident_any<2, true, CODE>(p, st);
         default:

@@ -6,6 +6,7 @@ import torch
 
 import mortar_amd
 from mortar_amd import ops, synth
+from mortar_amd.pack import MortarPack, decode_blocks
 from oracle import mortar_oracle as O
 from util import assert_close_bf16, oracle_spmm, to_dev, to_np
 
@@ -1283,3 +1284,24 @@ def test_raw_c_abi_refuses_bad_calls_of_the_newer_entry_points(dev):
     torch.cuda.synchronize()
     assert bool((g == 7.0).all())
 
+
+@pytest.mark.parametrize("per_block", [False, True])
+@pytest.mark.parametrize("M", [1400, 2801, 5473])          # one, two and three unit pairs per wave
+def test_wide_gate_up_units_per_wave(dev, M, per_block):
+    """gate_up over two K segments of more rows than the 16-token tiles take, 47 unit pairs: a row is computed alike by all three forms, so
+    a long batch equals its head; the last rows are checked against the dense product."""
+    d, f = 2560, 752
+    m = synth.synth_matrix(2 * f, d, 0.1, seed=41)
+    nnz = m["col_idx"].size
+    g = torch.Generator(device=dev).manual_seed(M)
+    W = MortarPack(None, None, m["col_idx"], m["offsets"], 2 * f, d, dev)
+    vals = torch.randn(nnz, 16, 16, device=dev, generator=g) * 0.05
+    s = W.requantize(vals, per_block=per_block).expand(nnz).cpu().numpy()
+    x = torch.randn(M, d, device=dev, generator=g).to(torch.bfloat16)
+    h = ops.gateup_swiglu(x, W)
+    assert torch.equal(h[:1400], ops.gateup_swiglu(x[:1400], W))
+    codes = decode_blocks(W.codes.cpu().numpy().view(np.uint32)).astype(np.float32) * O.bf16_round(s)[:, None, None]
+    dense = torch.from_numpy(O.to_dense(codes, m["row_idx"], m["col_idx"], (2 * f, d))).to(dev)
+    gu = (x[-161:].float() @ dense.float().t()).to(torch.bfloat16)
+    ref = (torch.nn.functional.silu(gu[:, :f]) * gu[:, f:]).float()
+    assert (h[-161:].float() - ref).norm() <= 1e-2 * ref.norm()
