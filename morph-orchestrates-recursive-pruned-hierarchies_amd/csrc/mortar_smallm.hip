@@ -211,11 +211,19 @@ static int smallm_launch_code(int kind, SpmmParams &p, const SpmmParams *table, 
     if (!table && layers == 1 && w == 2) {      // one matrix over the whole chip: latency form
         int rc = -1;
         if (resident) {
-            rc = t == 4 ? launch_partsplit<4, CODE>(kind, p, st) : launch_partsplit<16, CODE>(kind, p, st);
+            // gate_up of 5..32 rows: 8-token tiles, which stage (and normalise) half as much per workgroup and put twice the
+            // workgroups on the chip, up to 360 of them (MLP of d_model 2048, graph replay: 8 rows 13.7 -> 12.4 us, 13 rows 14.5 ->
+            // 12.5, 32 rows 15.0 -> 13.4; 352 workgroups are faster, 384 and 516 slower: d_model 3072 at 24 rows 19.1 against 19.9 us)
+            const bool eight = kind == 1 && t == 16 && p.M <= 32 && (p.M + 7) / 8 * (int64_t)((p.n_units + 3) / 4) <= 360;
+            rc = t == 4 ? launch_partsplit<4, CODE>(kind, p, st) : eight ? launch_partsplit<8, CODE>(kind, p, st) : -1;
+            if (rc < 0 && t != 4) rc = launch_partsplit<16, CODE>(kind, p, st);
             if (rc < 0 && t == 16 && kind == 1) rc = wide_gate_up();
             if (rc < 0 && t == 16 && kind != 2) rc = narrow_tiles();      // (fails as well where a row is one part)
         } else {
-            if (fits(8, p.Cb)) rc = launch_partsplit<8, CODE>(kind, p, st);      // 8-token tiles of all K instead of K segments
+            // tiles of all K instead of K segments: 4 tokens while their workgroups are one round of the chip (`down` of d_model 2048,
+            // with its gate_up: 8 rows 12.4 -> 11.8 us, 16 rows 14.6 -> 13.9, 32 rows 14.7 -> 14.2; two rounds 15.1 against 16.8), else 8
+            if (fits(4, p.Cb) && (p.M + 3) / 4 * (int64_t)((p.n_units + 3) / 4) <= 256) rc = launch_partsplit<4, CODE>(kind, p, st);
+            if (rc < 0 && fits(8, p.Cb)) rc = launch_partsplit<8, CODE>(kind, p, st);
             if (rc < 0) rc = narrow_tiles();
         }
         if (rc >= 0) return rc;

@@ -1305,3 +1305,23 @@ def test_wide_gate_up_units_per_wave(dev, M, per_block):
     gu = (x[-161:].float() @ dense.float().t()).to(torch.bfloat16)
     ref = (torch.nn.functional.silu(gu[:, :f]) * gu[:, f:]).float()
     assert (h[-161:].float() - ref).norm() <= 1e-2 * ref.norm()
+
+
+@pytest.mark.parametrize("M", [5, 8, 9, 16, 17, 32, 33])
+@pytest.mark.parametrize("f,norm", [(1408, False), (1408, True), (5632, True)])
+def test_decode_tiles_of_eight_and_four_tokens(dev, M, f, norm):
+    """gate_up (one K segment) and down (several) around the row counts at which their token tiles change."""
+    d = 2048 if f == 5632 else 512
+    gu, dn = synth.synth_matrix(2 * f, d, 0.1, seed=51), synth.synth_matrix(64, 5632, 0.1, seed=52)
+    x = synth.synth_x(M, d, seed=M)
+    w = (1.0 + 0.1 * np.sin(np.arange(d))).astype(np.float32)
+    W = MortarPack(synth.flat_pack(gu["codes"]), gu["scales"], gu["col_idx"], gu["offsets"], 2 * f, d, dev)
+    h = ops.gateup_swiglu(to_dev(x, dev), W, norm=(to_dev(w, dev), 1e-6) if norm else None)
+    xn = ops.rmsnorm(to_dev(x, dev), to_dev(w, dev), 1e-6) if norm else to_dev(x, dev)
+    g = ops.spmm(xn, W)
+    ref = (torch.nn.functional.silu(g[:, :f]) * g[:, f:]).float()
+    assert (h.float() - ref).norm() <= 1e-2 * ref.norm()
+    assert_close_bf16(to_np(g), oracle_spmm(to_np(xn), gu), "gate_up")
+    D = MortarPack(synth.flat_pack(dn["codes"]), dn["scales"], dn["col_idx"], dn["offsets"], 64, 5632, dev)
+    z = synth.synth_x(M, 5632, seed=M + 1)
+    assert_close_bf16(to_np(ops.spmm(to_dev(z, dev), D)), oracle_spmm(z, dn), "down")
