@@ -7,10 +7,11 @@ import torch
 from torch import Tensor
 
 from . import _lib, ops
+from .mlp import _SwiGLUMortar, call_is_forward
 from .pack import MortarPack
 from .routing import TileRouter
 
-_module = torch.nn.modules.module
+_mlp_forward = _SwiGLUMortar.forward
 
 
 def mortar_pack_strips(cms) -> MortarPack:
@@ -56,7 +57,7 @@ class MortarDecodeMLP:
 
     def __call__(self, x: Tensor, gates: Tensor | None = None) -> Tensor:
         mlp = self.mlp
-        if gates is None and not (mlp._forward_hooks or mlp._forward_pre_hooks or _module._global_forward_hooks or _module._global_forward_pre_hooks):
+        if gates is None and call_is_forward(mlp, _mlp_forward):
             y = self._native(mlp, x)
             if y is not None:
                 return y

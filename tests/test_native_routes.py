@@ -1,0 +1,60 @@
+"""Which calls the native call layer may take, decided in Python before any launch: the layer is replaced by a recorder and the
+packs stand on the CPU, so every test here asks only which path a call takes."""
+import pytest
+import torch
+
+from mortar_amd import _lib, synth
+from mortar_amd.engine import MortarDecodeMLP
+from mortar_amd.mlp import _SwiGLUMortar
+
+
+class _Native:
+    """Answers every entry point of the native layer with TAKEN."""
+    TAKEN = torch.full((1,), 7.0)
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def call(*a):
+            self.calls.append((name, a))
+            return self.TAKEN
+        return call
+
+
+@pytest.fixture
+def native(monkeypatch):
+    n = _Native()
+    monkeypatch.setattr(_lib, "_native", n)
+    monkeypatch.setattr(_SwiGLUMortar, "native_pair", lambda self: (self.gate_up._cms._pack, self.down._cms._pack))
+    return n
+
+
+def _mlp(cls=_SwiGLUMortar):
+    mlp = synth.mlp_module(synth.synth_mlp(64, 128, 0.5, seed=1), torch.device("cpu"))
+    mlp.__class__ = cls
+    return mlp
+
+
+X = torch.zeros(2, 64, dtype=torch.bfloat16)
+
+
+class _Adapter(_SwiGLUMortar):
+    def forward(self, x, **kw):
+        return x + 1
+
+
+def _instance_forward():
+    mlp = _mlp()
+    mlp.forward = lambda x, **kw: x + 1
+    return mlp
+
+
+def test_decode_call_of_the_plain_module_is_native(native):
+    assert MortarDecodeMLP(_mlp())(X) is native.TAKEN
+
+
+@pytest.mark.parametrize("make", [lambda: _mlp(_Adapter), _instance_forward])
+def test_decode_call_runs_an_overridden_forward(native, make):
+    y = MortarDecodeMLP(make())(X)
+    assert torch.equal(y, torch.ones(2, 1, 64, dtype=torch.bfloat16)) and not native.calls
