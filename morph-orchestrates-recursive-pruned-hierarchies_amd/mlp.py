@@ -17,10 +17,11 @@ from .sparsity import MortarLinear
 _module = nn.modules.module
 
 
-def call_is_forward(m: nn.Module, forward) -> bool:
-    """True if calling the module ``m`` runs the method ``forward`` and nothing else: not overridden by a subclass or on the
-    instance, no hooks of its own or global ones.  Whoever does a module's work without calling it has to ask first."""
-    return (type(m).forward is forward and type(m).__call__ is nn.Module.__call__ and "forward" not in m.__dict__
+def call_is_forward(m, forward) -> bool:
+    """True if calling ``m`` is the module method ``forward`` and nothing else: not another kind of object, not overridden by a
+    subclass or on the instance, no hooks of its own or global ones.  Whoever does a module's work without calling it has to
+    ask first."""
+    return (getattr(type(m), "forward", None) is forward and type(m).__call__ is nn.Module.__call__ and "forward" not in m.__dict__
             and not (m._forward_hooks or m._forward_pre_hooks or _module._global_forward_hooks or _module._global_forward_pre_hooks))
 
 

@@ -58,3 +58,17 @@ def test_decode_call_of_the_plain_module_is_native(native):
 def test_decode_call_runs_an_overridden_forward(native, make):
     y = MortarDecodeMLP(make())(X)
     assert torch.equal(y, torch.ones(2, 1, 64, dtype=torch.bfloat16)) and not native.calls
+
+
+class _Host:
+    """What MortarDecodeMLP reads of its host, without being a module."""
+    def __init__(self, mlp):
+        self.gate_up, self.down, self.d_ff, self.router = mlp.gate_up, mlp.down, mlp.d_ff, None
+
+    def __call__(self, x, iter_idx=0, gates=None, norm=None):
+        return x + 2
+
+
+def test_decode_call_serves_a_host_that_is_no_module(native):
+    y = MortarDecodeMLP(_Host(_mlp()))(X)
+    assert torch.equal(y, torch.full((2, 1, 64), 2, dtype=torch.bfloat16)) and not native.calls
