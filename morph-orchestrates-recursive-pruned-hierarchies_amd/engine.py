@@ -68,7 +68,7 @@ class MortarDecodeMLP:
         pair = mlp.native_pair()
         if pair is None:
             return None
-        rt = mlp._modules.get("router")
+        rt = mlp.router
         if rt is None:
             return _lib.native().mlp(x, *pair, True, True, self.norm_weight, self.eps, None)
         if type(rt) is not TileRouter or mlp.gate_up._cms._pack is not self.Mgu or mlp.down._cms._pack is not self.Mdown:

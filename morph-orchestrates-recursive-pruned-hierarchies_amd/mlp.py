@@ -151,7 +151,7 @@ class _SwiGLUMortar(nn.Module):
         it exists so that a caller which already evaluated the router (or holds seeded logits) can feed it.
         ``norm`` = (weight or None, eps): x is the activation BEFORE the block's RMSNorm (norm_mlp) and the norm is
         applied here, inside the gate_up launch when the matrix allows it; same result as mlp(rmsnorm(x))."""
-        if gates is None and "router" not in self._modules:
+        if gates is None and self.router is None:
             pair = self.native_pair()
             if pair is not None:
                 nw, eps = norm if norm is not None else (None, 0.0)

@@ -72,3 +72,22 @@ class _Host:
 def test_decode_call_serves_a_host_that_is_no_module(native):
     y = MortarDecodeMLP(_Host(_mlp()))(X)
     assert torch.equal(y, torch.full((2, 1, 64), 2, dtype=torch.bfloat16)) and not native.calls
+
+
+class _Router:
+    """A router that is no module: the MLP only calls it."""
+    def __call__(self, x, iter_idx=0):
+        return torch.zeros(x.shape[0], 4), None
+
+    def route(self, x, iter_idx=0):
+        return torch.zeros(x.shape[0], 4), None
+
+
+def test_a_router_that_is_no_module_is_not_left_out(native):
+    mlp = _mlp()
+    dec = MortarDecodeMLP(mlp)
+    mlp.router = _Router()
+    for call in (mlp, dec):
+        with pytest.raises(RuntimeError, match="ROCm device"):       # the general path, which needs the GPU
+            call(X)
+    assert not native.calls
