@@ -64,14 +64,15 @@ class MortarDecodeMLP:
         return self._general(x, gates)
 
     def _native(self, mlp, x: Tensor):
-        """The whole step as one native call; None when the layers are not deployed packs or the call is not covered."""
+        """The whole step as one native call; None when the layers are not deployed packs (or no longer those of the
+        constructor, which the general path multiplies with where it does not call the module) or the call is not covered."""
         pair = mlp.native_pair()
-        if pair is None:
+        if pair is None or mlp.gate_up._cms._pack is not self.Mgu or mlp.down._cms._pack is not self.Mdown:
             return None
         rt = mlp.router
         if rt is None:
             return _lib.native().mlp(x, *pair, True, True, self.norm_weight, self.eps, None)
-        if type(rt) is not TileRouter or mlp.gate_up._cms._pack is not self.Mgu or mlp.down._cms._pack is not self.Mdown:
+        if type(rt) is not TileRouter:
             return None
         proj, norm = rt._modules["query_proj"], rt._modules["query_norm"]
         return _lib.native().routed_decode(x, *pair, self.norm_weight, self.eps, rt._parameters, proj._parameters, norm._parameters,

@@ -91,3 +91,14 @@ def test_a_router_that_is_no_module_is_not_left_out(native):
         with pytest.raises(RuntimeError, match="ROCm device"):       # the general path, which needs the GPU
             call(X)
     assert not native.calls
+
+
+def test_decode_call_keeps_the_packs_it_was_built_with(native):
+    """Where the general path multiplies with the packs of the constructor (no router, but a norm in its own launch; or a
+    router), so does the native one: not with those of weights that were loaded since."""
+    mlp = _mlp()
+    dec = MortarDecodeMLP(mlp)
+    mlp.to(torch.device("cpu"))                      # drops the packs
+    mlp.gate_up._cms.mortar_pack(), mlp.down._cms.mortar_pack()
+    dec._general = lambda x, gates: "general"
+    assert dec(X) == "general" and not native.calls
