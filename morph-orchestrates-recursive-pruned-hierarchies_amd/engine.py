@@ -67,15 +67,16 @@ class MortarDecodeMLP:
         """The whole step as one native call; None when the layers are not deployed packs (or no longer those of the
         constructor, which the general path multiplies with where it does not call the module) or the call is not covered."""
         pair = mlp.native_pair()
-        if pair is None or mlp.gate_up._cms._pack is not self.Mgu or mlp.down._cms._pack is not self.Mdown:
+        if pair is None or pair[0] is not self.Mgu or pair[1] is not self.Mdown:
             return None
+        gu, dn = pair[0].address, pair[1].address
         rt = mlp.router
         if rt is None:
-            return _lib.native().mlp(x, *pair, True, True, self.norm_weight, self.eps, None)
+            return _lib.native().mlp(x, gu, dn, True, True, self.norm_weight, self.eps, None)
         if type(rt) is not TileRouter:
             return None
         proj, norm = rt._modules["query_proj"], rt._modules["query_norm"]
-        return _lib.native().routed_decode(x, *pair, self.norm_weight, self.eps, rt._parameters, proj._parameters, norm._parameters,
+        return _lib.native().routed_decode(x, gu, dn, self.norm_weight, self.eps, rt._parameters, proj._parameters, norm._parameters,
                                            (rt.n_iters, rt.n_sub_keys, rt.n_tile_groups, rt.activation_k), norm.eps, self.iter_idx)
 
     @torch.no_grad()

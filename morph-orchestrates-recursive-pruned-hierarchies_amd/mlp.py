@@ -6,6 +6,8 @@ epilogue, then down.  Before carving the layers run their dense forward.
 """
 from __future__ import annotations
 
+import weakref
+
 import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
@@ -133,18 +135,22 @@ class _SwiGLUMortar(nn.Module):
                    and "mortar_packed" not in m._cms._buffers for m in (self.gate_up, self.down))
 
     def native_pair(self) -> tuple | None:
-        """Handles (gate_up, down) for the native call layer when both layers hold a deployed pack (mortar_packed) in the
-        runtime's blocking, else None.  A pack that was dropped (moved, loaded again) or a layer that was replaced is
-        noticed by identity."""
+        """The packs (gate_up, down) for the native call layer when both layers hold a deployed one (mortar_packed) in the
+        runtime's blocking, else None; their schedules are in place and the caller's reference keeps them alive over the call.
+        What was found out stands in the gate_up pack, with a weak reference to its partner: nothing of it is in the module,
+        which has to copy and save, and a pack that the layer drops (moved, loaded again) is freed with it."""
         gu, dn = self._modules["gate_up"]._modules["_cms"], self._modules["down"]._modules["_cms"]
-        c = self.__dict__.get("_native_cache")
-        if c is None or c[0] is not gu._pack or c[1] is not dn._pack or c[2] is not gu or c[3] is not dn:
-            if not all(m._mortar and m._mortar_blocking == 16 and "mortar_packed" in m._buffers and m._pack is not None for m in (gu, dn)):
+        p, q = gu._pack, dn._pack
+        if p is None or q is None:
+            return None
+        if p.mate is None or p.mate() is not q:
+            if not all(m._mortar and m._mortar_blocking == 16 and "mortar_packed" in m._buffers for m in (gu, dn)):
                 return None
-            if gu._pack.Rb % 2 or gu._pack.Rb != 2 * dn._pack.Cb or not gu._pack.codes.is_cuda:
+            if p.Rb % 2 or p.Rb != 2 * q.Cb or not p.on_gpu:
                 return None
-            c = self.__dict__["_native_cache"] = (gu._pack, dn._pack, gu, dn, (gu._pack.handle(2), dn._pack.handle(1)))
-        return c[4]
+            p.sched(2), q.sched(1)
+            p.mate = weakref.ref(q)
+        return p, q
 
     def forward(self, x: Tensor, iter_idx: int = 0, gates: Tensor | None = None, norm: tuple | None = None) -> Tensor:
         """x [..., d_model] -> [..., d_model].  ``gates`` overrides the router output (fp32 [N, n_clusters]);
@@ -155,7 +161,7 @@ class _SwiGLUMortar(nn.Module):
             pair = self.native_pair()
             if pair is not None:
                 nw, eps = norm if norm is not None else (None, 0.0)
-                y = _lib.native().mlp(x, *pair, False, norm is not None, nw, eps, None)
+                y = _lib.native().mlp(x, pair[0].address, pair[1].address, False, norm is not None, nw, eps, None)
                 if y is not None:
                     return y
         train = self._carved() and self._wants_grad(x)
@@ -178,7 +184,7 @@ class _SwiGLUMortar(nn.Module):
                 r = rt.forward_native(rx, iter_idx) if type(rt) is TileRouter and not (rt._forward_hooks or rt._forward_pre_hooks) else None
                 gates, self._last_aux_loss = r if r is not None else rt(rx, iter_idx=iter_idx)
                 gates = gates.detach()
-            y = _lib.native().mlp(x, *pair, False, False, None, 0.0, gates)
+            y = _lib.native().mlp(x, pair[0].address, pair[1].address, False, False, None, 0.0, gates)
             if y is not None:
                 return y
         if (train and x.is_cuda and self.router is None and gates is None and norm is None

@@ -300,11 +300,11 @@ class MortarPack:
         self.address = C.addressof(self._handle)
         for rpu, t in self._scheds.items():
             setattr(self._handle, f"sched{rpu}", t.data_ptr())
+        self.mate = None      # weak reference to the `down` pack that this gate_up pack was found to chain with (native_pair)
 
-    def handle(self, rows_per_unit: int) -> int:
-        """Address of the native call layer's handle, with the schedule for plain (1) or gate/up (2) units in place."""
-        self.sched(rows_per_unit)
-        return self.address
+    @property
+    def on_gpu(self) -> bool:
+        return self.device.type == "cuda"
 
     def _make_struct(self):
         return _lib.BcsrStruct(self.codes.data_ptr(), self.sdup.data_ptr(), self.col.data_ptr(),

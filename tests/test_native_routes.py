@@ -1,5 +1,10 @@
 """Which calls the native call layer may take, decided in Python before any launch: the layer is replaced by a recorder and the
 packs stand on the CPU, so every test here asks only which path a call takes."""
+import copy
+import io
+import pickle
+import weakref
+
 import pytest
 import torch
 
@@ -102,3 +107,47 @@ def test_decode_call_keeps_the_packs_it_was_built_with(native):
     mlp.gate_up._cms.mortar_pack(), mlp.down._cms.mortar_pack()
     dec._general = lambda x, gates: "general"
     assert dec(X) == "general" and not native.calls
+
+
+@pytest.fixture
+def pair_of(monkeypatch):
+    """native_pair() as on a GPU: the packs of a CPU module taken for resident ones."""
+    from mortar_amd.pack import MortarPack
+    monkeypatch.setattr(MortarPack, "on_gpu", True)
+    monkeypatch.setattr(_lib, "_native", _Native())
+
+    def build(cls=_SwiGLUMortar):
+        mlp = _mlp(cls)
+        mlp.gate_up._cms.mortar_pack(), mlp.down._cms.mortar_pack()
+        assert mlp.native_pair() is not None
+        return mlp
+    return build
+
+
+def test_a_module_copies_and_saves_after_a_native_call(pair_of):
+    mlp = pair_of()
+    mlp.to(torch.device("cpu"))                      # (a move drops the packs, which hold device addresses)
+    again = copy.deepcopy(mlp)
+    torch.save(mlp, io.BytesIO())
+    pickle.dumps(mlp)
+    assert again.native_pair() is None
+    again.gate_up._cms.mortar_pack(), again.down._cms.mortar_pack()
+    assert again.native_pair() == (again.gate_up._cms._pack, again.down._cms._pack)
+
+
+@pytest.mark.parametrize("layer", ["gate_up", "down"])
+def test_a_dropped_pack_is_freed(pair_of, layer):
+    mlp = pair_of()
+    packs = [weakref.ref(m._cms._pack) for m in (mlp.gate_up, mlp.down)]
+    getattr(mlp, layer).to(torch.device("cpu"))
+    assert mlp.native_pair() is None
+    assert [p() is None for p in packs] == [layer == "gate_up", layer == "down"]
+
+
+def test_a_copied_pack_hands_out_its_own_addresses(pair_of):
+    """clone_weights() copies the pack's attributes: not what was found out for the original's pair."""
+    mlp = pair_of()
+    cms = mlp.gate_up._cms
+    old, cms._pack = cms._pack, cms._pack.clone_weights()
+    new = mlp.native_pair()
+    assert new[0] is cms._pack and new[0].address != old.address and new[0]._handle.sched2 != old._handle.sched2
