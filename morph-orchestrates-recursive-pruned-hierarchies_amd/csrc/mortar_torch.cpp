@@ -37,6 +37,13 @@ const at::Tensor *tensor_of(PyObject *o) { return THPVariable_CheckExact(o) ? &T
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// Truth of any Python object as `if o:` has it (True, 1, numpy.True_, ...); false with the Python error set where it has none.
+bool truth(PyObject *o, bool &v) {
+    const int t = PyObject_IsTrue(o);
+    v = t > 0;
+    return t >= 0;
+}
+
 PyObject *raise_rc(int rc, const char *what) {
     PyErr_Format(rc == MORTAR_ERR_HIP ? PyExc_RuntimeError : PyExc_ValueError, "%s failed (%d): %s", what, rc, mortar_last_error());
     return nullptr;
@@ -110,7 +117,8 @@ PyObject *py_mlp(PyObject *, PyObject *const *a, Py_ssize_t na) {
     const at::Tensor *xt = tensor_of(a[0]);
     const PackHandle *gu = handle_of(a[1]), *dn = handle_of(a[2]);
     if (PyErr_Occurred()) return nullptr;
-    const bool decode = a[3] == Py_True, norm = a[4] == Py_True;
+    bool decode, norm;
+    if (!truth(a[3], decode) || !truth(a[4], norm)) return nullptr;
     if (!xt || !gu || !dn || !gu->sched2 || !dn->sched1) Py_RETURN_NONE;
     const at::Tensor &x = *xt;
     const int64_t d = (int64_t)gu->w->Cb * 16;
@@ -305,10 +313,10 @@ PyObject *py_gemv_f32(PyObject *, PyObject *const *a, Py_ssize_t na) {
     }
     const at::Tensor *xt = tensor_of(a[0]), *sc = tensor_of(a[2]);
     const PackHandle *h = handle_of(a[1]);
-    if (PyErr_Occurred()) return nullptr;
+    bool swx, swo;
+    if (PyErr_Occurred() || !truth(a[3], swx) || !truth(a[4], swo)) return nullptr;
     if (!xt || !sc || !h || sc->numel() != 1 || sc->scalar_type() != at::kFloat) Py_RETURN_NONE;
     const at::Tensor &x = *xt;
-    const bool swx = a[3] == Py_True, swo = a[4] == Py_True;
     const int64_t K = (int64_t)h->w->Cb * 16, nout = (int64_t)h->w->Rb * (swo ? 8 : 16);
     if (!x.is_cuda() || sc->device() != x.device() || x.scalar_type() != at::kFloat || x.dim() != 2 || x.size(1) != K * (swx ? 2 : 1) ||
         !x.is_contiguous() || !aligned16(x.const_data_ptr()) || (swo && (h->w->Rb & 1)))

@@ -1,5 +1,6 @@
 """The native call layer (csrc/mortar_torch.cpp) against the general Python path of the same modules: same bits where both
 serve a call, and the general path where the layer declines."""
+import numpy as np
 import pytest
 import torch
 
@@ -88,3 +89,14 @@ def test_one_launch_fp32_decode_product(dev, K_blocks, seg, B):
     want = torch.nn.functional.silu(gu[:, :80]) * gu[:, 80:] * gates.double().repeat_interleave(16, 1)
     got = mortar_amd.mortar_gemv(x, W, swiglu_out=True, gates=gates)
     assert torch.allclose(got.double(), want, rtol=1e-4, atol=1e-5 * want.abs().max().item() + 1e-12)
+
+
+@pytest.mark.parametrize("flag", [1, np.True_, torch.tensor(True)])
+def test_fp32_decode_product_takes_any_true_flag(dev, flag):
+    m = synth.synth_matrix(16 * 4, 16 * 8, 0.5, seed=9, per_tensor_scale=True)
+    W = synth.to_pack(m, dev)
+    x = torch.randn(3, 256, device=dev)
+    assert torch.equal(mortar_amd.mortar_gemv(x, W, swiglu_x=flag), mortar_amd.mortar_gemv(x, W, swiglu_x=True))
+    x = x[:, :128].contiguous()
+    h = mortar_amd.mortar_gemv(x, W, swiglu_out=flag)
+    assert h.shape == (3, 32) and torch.equal(h, mortar_amd.mortar_gemv(x, W, swiglu_out=True))

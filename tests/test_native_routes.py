@@ -151,3 +151,19 @@ def test_a_copied_pack_hands_out_its_own_addresses(pair_of):
     old, cms._pack = cms._pack, cms._pack.clone_weights()
     new = mlp.native_pair()
     assert new[0] is cms._pack and new[0].address != old.address and new[0]._handle.sched2 != old._handle.sched2
+
+
+def test_flags_of_the_native_layer_are_read_by_their_truth():
+    """numpy.True_, 1 and other true objects are true: the layer asks them, it does not look for the object True."""
+    class Flag:
+        asked = 0
+
+        def __bool__(self):
+            Flag.asked += 1
+            return True
+
+    n, x = _lib.native(), torch.zeros(2, 64)               # a CPU tensor: declined, once the arguments are read
+    assert n.gemv_f32(x, 0, x[0, :1], Flag(), Flag(), None, None, None) is None and Flag.asked == 2
+    assert n.mlp(x, 0, 0, Flag(), Flag(), None, 0.0, None) is None and Flag.asked == 4
+    with pytest.raises(ValueError, match="ambiguous"):
+        n.gemv_f32(x, 0, x[0, :1], torch.zeros(2).numpy(), False, None, None, None)
