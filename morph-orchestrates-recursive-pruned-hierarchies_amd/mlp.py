@@ -17,6 +17,7 @@ from .routing import TileRouter
 from .sparsity import MortarLinear
 
 _module = nn.modules.module
+_router_forward = TileRouter.forward
 
 
 def call_is_forward(m, forward) -> bool:
@@ -152,6 +153,12 @@ class _SwiGLUMortar(nn.Module):
             p.mate = weakref.ref(q)
         return p, q
 
+    def _routed(self, x: Tensor, iter_idx: int):
+        """(gates, auxiliary loss) of the module's router: one native call where calling it is nothing but its forward."""
+        rt = self.router
+        r = rt.forward_native(x, iter_idx) if type(rt) is TileRouter and call_is_forward(rt, _router_forward) else None
+        return r if r is not None else rt(x, iter_idx=iter_idx)
+
     def forward(self, x: Tensor, iter_idx: int = 0, gates: Tensor | None = None, norm: tuple | None = None) -> Tensor:
         """x [..., d_model] -> [..., d_model].  ``gates`` overrides the router output (fp32 [N, n_clusters]);
         it exists so that a caller which already evaluated the router (or holds seeded logits) can feed it.
@@ -180,9 +187,7 @@ class _SwiGLUMortar(nn.Module):
                 norm = (norm[0].to(torch.bfloat16), norm[1])
         if self._carved() and not train and x.is_cuda and norm is None and not self.route_skip and (pair := self.native_pair()) is not None:
             if gates is None and self.router is not None:
-                rx, rt = (x.detach() if self._aux_detach_input else x), self.router
-                r = rt.forward_native(rx, iter_idx) if type(rt) is TileRouter and not (rt._forward_hooks or rt._forward_pre_hooks) else None
-                gates, self._last_aux_loss = r if r is not None else rt(rx, iter_idx=iter_idx)
+                gates, self._last_aux_loss = self._routed(x.detach() if self._aux_detach_input else x, iter_idx)
                 gates = gates.detach()
             y = _lib.native().mlp(x, pair[0].address, pair[1].address, False, False, None, 0.0, gates)
             if y is not None:

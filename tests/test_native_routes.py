@@ -167,3 +167,33 @@ def test_flags_of_the_native_layer_are_read_by_their_truth():
     assert n.mlp(x, 0, 0, Flag(), Flag(), None, 0.0, None) is None and Flag.asked == 4
     with pytest.raises(ValueError, match="ambiguous"):
         n.gemv_f32(x, 0, x[0, :1], torch.zeros(2).numpy(), False, None, None, None)
+
+
+def _instance_forward_of(router, called):
+    def forward(x, iter_idx=0):
+        called.append(1)
+        return None, None
+    router.forward = forward
+
+
+@pytest.mark.parametrize("change", [lambda r, called: torch.nn.modules.module.register_module_forward_pre_hook(lambda m, a: called.append(1)),
+                                    lambda r, called: r.register_forward_hook(lambda m, a, o: called.append(1)), _instance_forward_of])
+def test_the_modules_router_is_called_where_a_call_is_more_than_its_forward(monkeypatch, change):
+    mlp = _mlp()
+    mlp.enable_routing(n_clusters=4)
+    monkeypatch.setattr(type(mlp.router), "forward_native", lambda self, x, iter_idx=0: ("native", None))
+    called = []
+    handle = change(mlp.router, called)
+    try:
+        mlp._routed(X, 0)
+        assert called == [1]
+    finally:
+        if handle is not None:
+            handle.remove()
+
+
+def test_the_modules_router_is_left_to_the_native_layer_otherwise(monkeypatch):
+    mlp = _mlp()
+    mlp.enable_routing(n_clusters=4)
+    monkeypatch.setattr(type(mlp.router), "forward_native", lambda self, x, iter_idx=0: ("native", None))
+    assert mlp._routed(X, 0)[0] == "native"
