@@ -73,7 +73,7 @@ class MortarDecodeMLP:
         rt = mlp.router
         if rt is None:
             return _lib.native().mlp(x, gu, dn, True, True, self.norm_weight, self.eps, None)
-        if type(rt) is not TileRouter:
+        if type(rt) is not TileRouter or not rt.route_is_own():
             return None
         proj, norm = rt._modules["query_proj"], rt._modules["query_norm"]
         return _lib.native().routed_decode(x, gu, dn, self.norm_weight, self.eps, rt._parameters, proj._parameters, norm._parameters,

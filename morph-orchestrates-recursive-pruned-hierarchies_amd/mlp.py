@@ -156,7 +156,8 @@ class _SwiGLUMortar(nn.Module):
     def _routed(self, x: Tensor, iter_idx: int):
         """(gates, auxiliary loss) of the module's router: one native call where calling it is nothing but its forward."""
         rt = self.router
-        r = rt.forward_native(x, iter_idx) if type(rt) is TileRouter and call_is_forward(rt, _router_forward) else None
+        own = type(rt) is TileRouter and rt.route_is_own() and call_is_forward(rt, _router_forward)
+        r = rt.forward_native(x, iter_idx) if own else None
         return r if r is not None else rt(x, iter_idx=iter_idx)
 
     def forward(self, x: Tensor, iter_idx: int = 0, gates: Tensor | None = None, norm: tuple | None = None) -> Tensor:

@@ -85,6 +85,10 @@ class TileRouter(nn.Module):
         self.last_active = r[1]
         return r[0], r[2]
 
+    def route_is_own(self) -> bool:
+        """route() is this class's: only then may a native call do its work (a subclass or the instance may have another)."""
+        return type(self).route is _route and "route" not in self.__dict__
+
     def _fused_ok(self, x_flat: Tensor) -> bool:
         """Decode-sized inference calls on the GPU with fp32 router parameters go through the two-launch HIP router."""
         return (x_flat.is_cuda and 0 < x_flat.shape[0] <= ops.ROUTER_MAX_TOKENS and not torch.is_grad_enabled()
@@ -124,7 +128,7 @@ class TileRouter(nn.Module):
 
     def forward(self, x: Tensor, iter_idx: int = 0) -> Tuple[Tensor, Tensor]:
         orig_shape = x.shape
-        if x.numel() <= ops.ROUTER_MAX_TOKENS * orig_shape[-1]:
+        if x.numel() <= ops.ROUTER_MAX_TOKENS * orig_shape[-1] and self.route_is_own():
             r = self.forward_native(x, iter_idx)
             if r is not None:
                 return (r[0].view(orig_shape[0], orig_shape[1], -1) if len(orig_shape) == 3 else r[0]), r[1]
@@ -157,3 +161,6 @@ class TileRouter(nn.Module):
         if len(orig_shape) == 3:
             gates = gates.reshape(orig_shape[0], orig_shape[1], self.n_tile_groups)
         return gates, aux_loss
+
+
+_route = TileRouter.route

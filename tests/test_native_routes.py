@@ -197,3 +197,31 @@ def test_the_modules_router_is_left_to_the_native_layer_otherwise(monkeypatch):
     mlp.enable_routing(n_clusters=4)
     monkeypatch.setattr(type(mlp.router), "forward_native", lambda self, x, iter_idx=0: ("native", None))
     assert mlp._routed(X, 0)[0] == "native"
+
+
+@pytest.mark.parametrize("on_instance", [False, True])
+def test_an_overridden_route_is_called(native, monkeypatch, on_instance):
+    """TileRouter.forward goes through route() for the calls that the kernels cover: a route() of a subclass or of the
+    instance is what runs, from the router's forward, the module and the decode call alike."""
+    from mortar_amd.routing import TileRouter
+    called = []
+
+    def route(self, x_flat, iter_idx=0):
+        called.append(1)
+        return torch.zeros(x_flat.shape[0], 4), torch.zeros(x_flat.shape[0], 4, dtype=torch.uint8)
+
+    mlp = _mlp()
+    mlp.enable_routing(n_clusters=4)
+    if on_instance:
+        mlp.router.route = route.__get__(mlp.router)
+    else:
+        mlp.router.__class__ = type("Router", (TileRouter,), {"route": route})
+    monkeypatch.setattr(TileRouter, "forward_native", lambda self, x, iter_idx=0: ("native", None))
+    monkeypatch.setattr(TileRouter, "_fused_ok", lambda self, x: True)
+    mlp.router(X)
+    assert len(called) == 1
+    mlp._routed(X, 0)
+    assert len(called) == 2
+    dec = MortarDecodeMLP(mlp)
+    dec._general = lambda x, gates: "general"
+    assert dec(X) == "general" and not native.calls
