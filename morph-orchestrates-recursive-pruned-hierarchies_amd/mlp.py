@@ -140,7 +140,9 @@ class _SwiGLUMortar(nn.Module):
         runtime's blocking, else None; their schedules are in place and the caller's reference keeps them alive over the call.
         What was found out stands in the gate_up pack, with a weak reference to its partner: nothing of it is in the module,
         which has to copy and save, and a pack that the layer drops (moved, loaded again) is freed with it."""
-        gu, dn = self._modules["gate_up"]._modules["_cms"], self._modules["down"]._modules["_cms"]
+        gu, dn = self._modules["gate_up"]._modules.get("_cms"), self._modules["down"]._modules.get("_cms")
+        if gu is None or dn is None:                    # a layer inside another module, which hands on its _cms
+            return None
         p, q = gu._pack, dn._pack
         if p is None or q is None:
             return None

@@ -225,3 +225,25 @@ def test_an_overridden_route_is_called(native, monkeypatch, on_instance):
     dec = MortarDecodeMLP(mlp)
     dec._general = lambda x, gates: "general"
     assert dec(X) == "general" and not native.calls
+
+
+class _Wrapped(torch.nn.Module):
+    """A carved linear layer inside another module, which hands on what the MLP reads of it."""
+    def __init__(self, layer):
+        super().__init__()
+        self.inner = layer
+
+    @property
+    def _cms(self):
+        return self.inner._cms
+
+
+def test_wrapped_layers_take_the_general_path(monkeypatch):
+    monkeypatch.setattr(_lib, "_native", _Native())
+    mlp = _mlp()
+    mlp.down = _Wrapped(mlp.down)
+    dec = MortarDecodeMLP(mlp)
+    for call in (mlp, dec):
+        with pytest.raises(RuntimeError, match="ROCm device"):
+            call(X)
+    assert not _lib._native.calls
