@@ -116,7 +116,10 @@ struct ValOut {
         r = val_rsrc(a.y + (int64_t)m0 * a.ldy, (int)((nt - 1) * a.ldy * 2 + a.Rb * 32));
         odd = g & 1;
 #pragma unroll
-        for (int ms = 0; ms < MT / 16; ++ms) off[ms] = (uint32_t)((ms * 16 + n) * a.ldy * 2) + odd * 32 + (g >> 1) * 16;
+        for (int ms = 0; ms < MT / 16; ++ms) {
+            const int t = ms * 16 + n;
+            off[ms] = t < nt ? (uint32_t)(t * a.ldy * 2) + odd * 32 + (g >> 1) * 16 : 0xfffffff0u;
+        }
     }
     __device__ __forceinline__ void store(int row, bool both, const f32x4_t (&a0)[MT / 16], const f32x4_t (&a1)[MT / 16]) const {
 #pragma unroll
@@ -368,6 +371,29 @@ int launch_segmented(ValArgs &a, hipStream_t st) {
 // LDS bytes a tile of all K may take (16 bytes stay for the row counter).
 bool val_fits(int mt, int Cb) { return (Cb + 1) / 2 * (mt * 64) + 16 <= LDS_BUDGET; }
 
+// The launch for the tokens of `a` (seg_cb and nfine are set).
+int val_dispatch(ValArgs &a, hipStream_t st) {
+    // the largest token tile of all K: a block's values are read from L2 once per tile
+    if (a.nfine == 1) return val_fits(64, a.Cb) ? launch_resident<64>(a, st) : launch_resident<32>(a, st);
+    // Tokens per tile and block-rows per wave: the choice with the least rounds of workgroups x (staging + rows), staging
+    // weighing about three rows; a 64-token row costs 1.7 of a 32-token one (its values are fetched once for both halves).
+    int best = 0;
+    int64_t best_cost = INT64_MAX;
+    const struct { int mt, upw, unit; } shape[5] = {{64, 4, 17}, {64, 2, 17}, {32, 4, 10}, {32, 2, 10}, {32, 1, 10}};
+    for (int i = 0; i < 5; ++i) {
+        const int64_t wgs = ((int64_t)a.M + shape[i].mt - 1) / shape[i].mt * ((a.Rb + VAL_CW * shape[i].upw - 1) / (VAL_CW * shape[i].upw));
+        const int64_t cost = (wgs + 255) / 256 * (3 + shape[i].upw) * shape[i].unit;
+        if (cost < best_cost) { best_cost = cost; best = i; }
+    }
+    switch (best) {
+        case 0: return launch_segmented<64, 4>(a, st);
+        case 1: return launch_segmented<64, 2>(a, st);
+        case 2: return launch_segmented<32, 4>(a, st);
+        case 3: return launch_segmented<32, 2>(a, st);
+    }
+    return launch_segmented<32, 1>(a, st);
+}
+
 }  // namespace
 
 extern "C" int32_t mortar_values_seg_cb(int32_t Cb) {
@@ -402,7 +428,7 @@ extern "C" int mortar_dds_values_bf16(const int32_t *row_ptr, const int16_t *col
         return mortar_fail(MORTAR_ERR_ARG, "dds_values: bad leading dimension (ldx %% 8 == 0, ldy %% 4 == 0)");
     if ((reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(y) & 7) || (reinterpret_cast<uintptr_t>(data) & 15))
         return mortar_fail(MORTAR_ERR_ARG, "dds_values: x and data must be 16-byte and y 8-byte aligned");
-    if (ldy > (1 << 23)) return mortar_fail(MORTAR_ERR_LIMIT, "dds_values: ldy=%lld exceeds 2^23 (a tile's results are addressed with 32 bits)", (long long)ldy);
+    if (Rb >= 1 << 26) return mortar_fail(MORTAR_ERR_LIMIT, "dds_values: %d block-rows (a token's results are addressed with 31 bits)", Rb);
     const int seg_cb = mortar_values_seg_cb(Cb);
     const int nseg = (Cb + seg_cb - 1) / seg_cb;
     if (nseg > 1 && !seg_ptr) return mortar_fail(MORTAR_ERR_ARG, "dds_values: %d K segments need seg_ptr (mortar_segment_ptr_host)", nseg);
@@ -413,28 +439,19 @@ extern "C" int mortar_dds_values_bf16(const int32_t *row_ptr, const int16_t *col
         return e == hipSuccess ? MORTAR_OK : mortar_fail(MORTAR_ERR_HIP, "dds_values launch: %s", hipGetErrorString(e));
     }
     ValArgs a{};
-    a.row_ptr = row_ptr; a.seg_ptr = seg_ptr; a.col = col; a.data = data; a.x = x; a.y = y; a.ldx = ldx; a.ldy = ldy;
-    a.M = (int)M; a.Rb = Rb; a.Cb = Cb; a.nnz = (int)nnz; a.seg_cb = seg_cb; a.nfine = nseg; a.sub = 1;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    // the largest token tile of all K: a block's values are read from L2 once per tile
-    if (nseg == 1) return val_fits(64, Cb) ? launch_resident<64>(a, st) : launch_resident<32>(a, st);
-    // Tokens per tile and block-rows per wave: the choice with the least rounds of workgroups x (staging + rows), staging
-    // weighing about three rows; a 64-token row costs 1.7 of a 32-token one (its values are fetched once for both halves).
-    int best = 0;
-    int64_t best_cost = INT64_MAX;
-    const struct { int mt, upw, unit; } shape[5] = {{64, 4, 17}, {64, 2, 17}, {32, 4, 10}, {32, 2, 10}, {32, 1, 10}};
-    for (int i = 0; i < 5; ++i) {
-        const int64_t wgs = (M + shape[i].mt - 1) / shape[i].mt * ((Rb + VAL_CW * shape[i].upw - 1) / (VAL_CW * shape[i].upw));
-        const int64_t cost = (wgs + 255) / 256 * (3 + shape[i].upw) * shape[i].unit;
-        if (cost < best_cost) { best_cost = cost; best = i; }
+    a.row_ptr = row_ptr; a.seg_ptr = seg_ptr; a.col = col; a.data = data; a.ldx = ldx; a.ldy = ldy;
+    a.Rb = Rb; a.Cb = Cb; a.nnz = (int)nnz; a.seg_cb = seg_cb; a.nfine = nseg; a.sub = 1;
+    // A tile's results are addressed with 31 bits from its first token: where 64 rows of y do not fit that (rows more than
+    // 16.7 M values apart), as many tokens per launch as do.
+    const int64_t reach = 1 + (0x7fffffff - (int64_t)Rb * 32) / (2 * ldy), step = reach >= 64 ? M : reach;
+    for (int64_t m = 0; m < M; m += step) {
+        a.x = x + m * ldx;
+        a.y = y + m * ldy;
+        a.M = (int)(M - m < step ? M - m : step);
+        const int rc = val_dispatch(a, static_cast<hipStream_t>(stream));
+        if (rc) return rc;
     }
-    switch (best) {
-        case 0: return launch_segmented<64, 4>(a, st);
-        case 1: return launch_segmented<64, 2>(a, st);
-        case 2: return launch_segmented<32, 4>(a, st);
-        case 3: return launch_segmented<32, 2>(a, st);
-    }
-    return launch_segmented<32, 1>(a, st);
+    return MORTAR_OK;
 }
 
 extern "C" int mortar_transpose_blocks_bf16(const uint16_t *data, const int32_t *src_block, int64_t nnz, uint16_t *out, void *stream) {

@@ -36,3 +36,20 @@ def test_values_product_edges(dev, Rb, Cb, M, density):
     if T.nnz:
         _, src = T.transposed()
         assert torch.equal(ops.transpose_blocks(data, src), data[src.long()].transpose(1, 2))
+
+
+@pytest.mark.parametrize("Rb,Cb", [(5, 3), (33, 170)])                 # all of K in one tile, K segments
+@pytest.mark.parametrize("ld,M", [(2 ** 23 + 8, 70), (2 ** 26, 19), (2 ** 30, 3)])      # 64 rows of y in 31 bits; 16 of them; one
+def test_values_product_into_rows_far_apart(dev, Rb, Cb, ld, M):
+    rng = np.random.default_rng(7)
+    mask = rng.random((Rb, Cb)) < 0.4
+    T = BcsrTopology(np.concatenate([[0], np.cumsum(mask.sum(1))]).astype(np.int32), np.nonzero(mask)[1].astype(np.int16), Rb * 16, Cb * 16, dev)
+    data = torch.randn(T.nnz, 16, 16, device=dev).bfloat16()
+    x = torch.randn(M, Cb * 16, device=dev).bfloat16()
+    buf = torch.empty((M - 1) * ld + Rb * 16 + 16, device=dev, dtype=torch.bfloat16)
+    out = buf.as_strided((M, Rb * 16 + 16), (ld, 1))
+    out.fill_(7.0)
+    ops.dds_values(x, data, T, out=out[:, :Rb * 16])
+    # other tiles pair the blocks of a row differently: one bf16 step apart, and 2^-20 of at most 2720 * 0.4 products of size 1
+    assert torch.allclose(out[:, :Rb * 16].float(), ops.dds_values(x, data, T).float(), rtol=2.0 ** -7, atol=1e-3)
+    assert (out[:, Rb * 16:] == 7.0).all()
