@@ -113,7 +113,8 @@ __device__ __forceinline__ void store_block(uint16_t *out, int64_t j, f32x4_t v,
 template <int... I, typename F>
 __device__ __forceinline__ void sdd_unroll(std::integer_sequence<int, I...>, F f) { (f(std::integral_constant<int, I>{}), ...); }
 
-template <int SDD_NB>
+// WIDE: 32 tokens of an operand do not fit a 32-bit offset (rows more than 2^26 values apart): 64-bit lane addresses.
+template <int SDD_NB, bool WIDE>
 __global__ __launch_bounds__(SDD_WAVES * 64) void sdd_kernel(SddArgs p) {
     constexpr int SDD_G = SDD_WAVES * SDD_NB;        // blocks per workgroup
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -160,7 +161,7 @@ __global__ __launch_bounds__(SDD_WAVES * 64) void sdd_kernel(SddArgs p) {
         const int piece = 4 * q + (st_piece >> 1) < (is_b ? ncb : nrows) ? st_piece : st_piece & 1;
         base[k] = is_b ? reinterpret_cast<const char *>(p.b + (int64_t)s_begin * SDD_STEP * p.ldb + (int64_t)(c0 + 4 * q) * 16)
                        : reinterpret_cast<const char *>(p.a + (int64_t)s_begin * SDD_STEP * p.lda + (int64_t)(row0 + 4 * q) * 16);
-        voff[k] = (uint32_t)((8 * c + st_tok) * (is_b ? p.ldb : p.lda) * 2 + piece * 16);
+        voff[k] = (uint32_t)((WIDE ? 0 : (8 * c + st_tok) * (is_b ? p.ldb : p.lda) * 2) + piece * 16);
         dst[k] = (is_b ? q : SDD_NQ + q) * SDD_QS + c * SDD_CS;
     }
     // Stages step s (the steps come in order) into buffer `buf`.  Rows past M are not loaded: in the one partial step
@@ -173,8 +174,16 @@ __global__ __launch_bounds__(SDD_WAVES * 64) void sdd_kernel(SddArgs p) {
             if (i < n_copy) {
                 char *d = smem + buf * SDD_BUF + dst[k];
                 const uint32_t la = __builtin_amdgcn_readfirstlane(mortar_lds_addr(d));
-                if (left >= SDD_STEP) load_to_lds_base(base[k], voff[k], la);
-                else if (8 * (i & 3) + st_tok < left) load_to_lds_base(base[k], voff[k], la);
+                auto copy = [&]() {
+                    if constexpr (WIDE) {
+                        const int64_t row = (int64_t)(8 * (i & 3) + st_tok) * (i < nq * 4 ? p.ldb : p.lda) * 2;
+                        mortar_load_to_lds((const MORTAR_GLOBAL char *)(base[k] + row + voff[k]), la);
+                    } else {
+                        load_to_lds_base(base[k], voff[k], la);
+                    }
+                };
+                if (left >= SDD_STEP) copy();
+                else if (8 * (i & 3) + st_tok < left) copy();
                 else *reinterpret_cast<u32x4_t *>(d + lane * 16) = u32x4_t{0u, 0u, 0u, 0u};
                 base[k] += (i < nq * 4 ? p.ldb : p.lda) * (2 * SDD_STEP);
             }
@@ -412,18 +421,32 @@ extern "C" int64_t mortar_sdd_workspace_bytes(int32_t n_wg, int32_t nnz, int32_t
     return (int64_t)tsplit * nnz * 256 * (int64_t)sizeof(float);
 }
 
-template <int NB>
+template <int NB, bool WIDE>
 static hipError_t sdd_launch(const SddArgs &p, hipStream_t st) {
     static bool configured = false;
     const int smem = 2 * SDD_BUF;
     if (!configured) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sdd_kernel<NB>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(sdd_kernel<NB, WIDE>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         if (e != hipSuccess) return e;
         configured = true;
     }
-    hipLaunchKernelGGL(sdd_kernel<NB>, dim3((unsigned)(8 * p.per_xcd)), dim3(SDD_WAVES * 64), smem, st, p);
+    hipLaunchKernelGGL((sdd_kernel<NB, WIDE>), dim3((unsigned)(8 * p.per_xcd)), dim3(SDD_WAVES * 64), smem, st, p);
     return hipSuccess;
+}
+
+template <bool WIDE>
+static hipError_t sdd_launch_nb(int nb, const SddArgs &p, hipStream_t st) {
+    switch (nb) {
+        case 8: return sdd_launch<8, WIDE>(p, st);
+        case 10: return sdd_launch<10, WIDE>(p, st);
+        case 12: return sdd_launch<12, WIDE>(p, st);
+        case 14: return sdd_launch<14, WIDE>(p, st);
+        case 16: return sdd_launch<16, WIDE>(p, st);
+        case 18: return sdd_launch<18, WIDE>(p, st);
+        case 20: return sdd_launch<20, WIDE>(p, st);
+    }
+    return sdd_launch<22, WIDE>(p, st);
 }
 
 extern "C" int mortar_sdd_bf16(const int32_t *plan, int32_t n_wg, int32_t blocks_per_wave,
@@ -445,8 +468,6 @@ extern "C" int mortar_sdd_bf16(const int32_t *plan, int32_t n_wg, int32_t blocks
         (reinterpret_cast<uintptr_t>(a) & 15) || (reinterpret_cast<uintptr_t>(b) & 15) ||
         (reinterpret_cast<uintptr_t>(acc) & 15))
         return mortar_fail(MORTAR_ERR_ARG, "sdd: operands need 16-byte aligned rows (leading dimensions multiples of 8)");
-    if (lda > (1 << 26) || ldb > (1 << 26))
-        return mortar_fail(MORTAR_ERR_LIMIT, "sdd: leading dimensions above 2^26 elements (32 tokens are addressed with 32 bits)");
     const int64_t n4 = (int64_t)nnz * 64;
     SddArgs p;
     p.plan = plan; p.a = a; p.b = b; p.lda = lda; p.ldb = ldb; p.M = M; p.acc = acc; p.out = out;
@@ -455,17 +476,7 @@ extern "C" int mortar_sdd_bf16(const int32_t *plan, int32_t n_wg, int32_t blocks
     sdd_segments(Cb, nseg, p.seg_cb);
     sdd_split(n_wg, nnz, blocks_per_wave, M, SDD_TILES, p.nsteps, p.steps_per_split, p.tsplit);
     p.per_xcd = (p.tsplit * n_wg + 7) / 8;
-    hipError_t e = hipSuccess;
-    switch (blocks_per_wave) {
-        case 8: e = sdd_launch<8>(p, st); break;
-        case 10: e = sdd_launch<10>(p, st); break;
-        case 12: e = sdd_launch<12>(p, st); break;
-        case 14: e = sdd_launch<14>(p, st); break;
-        case 16: e = sdd_launch<16>(p, st); break;
-        case 18: e = sdd_launch<18>(p, st); break;
-        case 20: e = sdd_launch<20>(p, st); break;
-        default: e = sdd_launch<22>(p, st); break;
-    }
+    hipError_t e = lda > (1 << 26) || ldb > (1 << 26) ? sdd_launch_nb<true>(blocks_per_wave, p, st) : sdd_launch_nb<false>(blocks_per_wave, p, st);
     if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
     if (p.tsplit > 1)
         hipLaunchKernelGGL(sdd_round_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st, acc, out, n4, p.tsplit);

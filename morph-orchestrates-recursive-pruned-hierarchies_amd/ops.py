@@ -360,9 +360,9 @@ def sdd(a: Tensor, b: Tensor, W: MortarPack, out: Tensor | None = None, blocks_p
     a, b = _bf16_2d(a, "sdd"), _bf16_2d(b, "sdd")
     if a.shape[0] != b.shape[0] or a.shape[1] != W.out_features or b.shape[1] != W.in_features:
         raise ValueError(f"sdd: a {tuple(a.shape)} / b {tuple(b.shape)} do not match the matrix [{W.out_features}, {W.in_features}]")
-    if a.stride(0) % 8 or a.data_ptr() % 16 or a.stride(0) > 1 << 26:
+    if a.stride(0) % 8 or a.data_ptr() % 16:
         a = a.contiguous()
-    if b.stride(0) % 8 or b.data_ptr() % 16 or b.stride(0) > 1 << 26:
+    if b.stride(0) % 8 or b.data_ptr() % 16:
         b = b.contiguous()
     plan, n_wg, nb = W.sdd_plan(a.shape[0], blocks_per_wave)
     if out is None:

@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 import torch
 
-from mortar_amd import ops
+from mortar_amd import ops, synth
 from mortar_amd.pack import BcsrTopology
 
 pytestmark = pytest.mark.gpu
@@ -53,3 +53,19 @@ def test_values_product_into_rows_far_apart(dev, Rb, Cb, ld, M):
     # other tiles pair the blocks of a row differently: one bf16 step apart, and 2^-20 of at most 2720 * 0.4 products of size 1
     assert torch.allclose(out[:, :Rb * 16].float(), ops.dds_values(x, data, T).float(), rtol=2.0 ** -7, atol=1e-3)
     assert (out[:, Rb * 16:] == 7.0).all()
+
+
+@pytest.mark.parametrize("lda,ldb", [(2 ** 26 + 8, None), (None, 2 ** 26 + 8)])
+def test_weight_gradient_of_rows_far_apart(dev, lda, ldb):
+    """Leading dimensions beyond 2^26 values, where 32 tokens no longer fit a 32-bit offset; a whole step and a part of one."""
+    W = synth.to_pack(synth.synth_matrix(16 * 9, 16 * 50, 0.3, seed=8), dev)
+    M = 37
+
+    def far(t, ld):
+        if ld is None:
+            return t
+        out = torch.empty((M - 1) * ld + t.shape[1], device=dev, dtype=torch.bfloat16).as_strided(t.shape, (ld, 1))
+        return out.copy_(t)
+
+    a, b = (torch.randn(M, n, device=dev).bfloat16() for n in (W.out_features, W.in_features))
+    assert torch.equal(ops.sdd(far(a, lda), far(b, ldb), W), ops.sdd(a, b, W))
