@@ -13,6 +13,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -234,7 +235,8 @@ PyObject *py_routed_decode(PyObject *, PyObject *const *a, Py_ssize_t na) {
 
 // route(x, own, proj, norm, shape, ln_eps, iter_idx, ema, alpha, coeff) -> (gates [M, n], active [M, n], aux): the router of
 // the M rows of x, without autograd.  With ema (the load statistics buffer, fp32 [n]) the statistics are updated in place
-// and aux is the load-balance loss; with ema = None aux is None.
+// and aux is the load-balance loss; with ema = None aux is None.  The in-place update counts as one for autograd and others
+// who look at the version of the buffer.
 PyObject *py_route(PyObject *, PyObject *const *a, Py_ssize_t na) {
     if (na != 10 || !PyTuple_Check(a[4]) || PyTuple_GET_SIZE(a[4]) != 4) {
         PyErr_SetString(PyExc_TypeError, "route: 10 arguments");
@@ -257,8 +259,8 @@ PyObject *py_route(PyObject *, PyObject *const *a, Py_ssize_t na) {
     if (!read_router(a[1], a[2], a[3], it, sh[0], nsk, n, d, x, r)) Py_RETURN_NONE;
     const at::Tensor *ema = a[7] == Py_None ? nullptr : tensor_of(a[7]);
     if (a[7] != Py_None && (!ema || ema->scalar_type() != at::kFloat || ema->device() != x.device() || ema->dim() != 1 || ema->size(0) != n ||
-                            !ema->is_contiguous()))
-        Py_RETURN_NONE;
+                            !ema->is_contiguous() || (ema->is_inference() && !c10::InferenceMode::is_enabled())))
+        Py_RETURN_NONE;          // (an inference tensor outside inference mode: torch's in-place operators word that error)
     const c10::DeviceGuard guard(x.device());
     void *st = stream_of(x);
     const auto f32 = x.options().dtype(at::kFloat).requires_grad(false);
@@ -282,6 +284,7 @@ PyObject *py_route(PyObject *, PyObject *const *a, Py_ssize_t na) {
         const at::Tensor ws = at::empty({mortar_router_stats_workspace_bytes(M, r.n)}, f32.dtype(at::kByte));
         rc = mortar_router_stats(gp, M, r.n, (float)alpha, (float)(1.0 - alpha), (float)coeff, static_cast<float *>(ema->data_ptr()),
                                  static_cast<float *>(aux.data_ptr()), ws.data_ptr(), st);
+        if (rc == MORTAR_OK && !ema->is_inference()) ema->unsafeGetTensorImpl()->bump_version();      // written through its address
     }
     if (rc) return raise_rc(rc, "mortar_route");
     PyObject *g = THPVariable_Wrap(std::move(gates)), *ac = THPVariable_Wrap(std::move(active));

@@ -113,3 +113,19 @@ def test_router_module_call_equals_the_torch_ops(dev, M):
     assert gates.shape == (flat.shape[0], 44) and torch.allclose(gates.reshape(-1, 44), want, rtol=1e-3, atol=1e-4)
     assert torch.allclose(rt.group_load_ema, ema, rtol=1e-3, atol=1e-4) and rt.last_active.shape == (flat.shape[0], 44)
     assert torch.allclose(aux, rt.aux_loss_coeff * want.mean(0).var(), rtol=1e-2)
+
+
+@pytest.mark.parametrize("M", [3, 300])
+def test_load_statistics_are_an_in_place_update_for_torch(dev, M):
+    rt = TileRouter(16, 256).to(dev)
+    x = torch.randn(M, 256, device=dev).to(torch.bfloat16)
+    before = rt.group_load_ema._version
+    with torch.no_grad():
+        assert rt.forward_native(x) is not None
+    assert rt.group_load_ema._version > before
+    with torch.inference_mode():
+        rt = TileRouter(16, 256).to(dev)
+        x = x.clone()
+        assert rt.forward_native(x) is not None
+    with torch.no_grad(), pytest.raises(RuntimeError, match="[Ii]nference"):      # as any in-place operator on such a buffer
+        rt(x)
