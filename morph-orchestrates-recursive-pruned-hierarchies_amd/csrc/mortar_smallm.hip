@@ -69,16 +69,25 @@ static int pick_waves(int t, const SpmmParams &p, int layers) {
     return bytes > 40 * 1024 ? 16 : 8;
 }
 
-// Part-split launch for one matrix: PW waves per unit, PW = 4, 3 or 2, dividing the unit's part count where one does.
+// Waves that share the parts of a unit in the part-split form: 4, 3 or 2, dividing the part count where one does; 0: none.
+// A part count no wave count divides (5, 7, 11 ... K segments): the waves of a unit take parts q, q + PW, ... and some take
+// one more than others - still far better than one wave per unit ([4096, 11008] at one row: 9.0 -> 5.6 us).
+static int partsplit_waves(int nparts) {
+    const int pw = nparts % 4 == 0 ? 4 : (nparts % 3 == 0 ? 3 : (nparts % 2 == 0 ? 2 : 0));
+    if (pw == 0 && nparts >= 5) return (nparts + 3) / 4 < (nparts + 2) / 3 ? 4 : 3;
+    return pw;
+}
+// LDS: the tile, then the partial sums of the workgroup's PW * 4 waves (1 KB per wave, accumulator and sub-tile).
+static bool partsplit_fits(int mt, int nacc, const SpmmParams &p) {
+    const int pw = partsplit_waves(p.nseg * nacc);
+    return pw != 0 && tile_bytes(mt, p.Cb) + pw * 4 * nacc * ((mt + 15) / 16) * 1024 <= 160 * 1024;
+}
+
+// Part-split launch for one matrix.
 template <int MT, int CODE>
 static int launch_partsplit(int kind, SpmmParams &p, hipStream_t st) {
-    const int nacc = (kind == 0 || kind == 3) ? 1 : 2, nparts = p.nseg * nacc;
-    // a part count no wave count divides (5, 7, 11 ... K segments): the waves of a unit take parts q, q + PW, ... and
-    // some take one more than others - still far better than one wave per unit ([4096, 11008] at one row: 9.0 -> 5.6 us)
-    int pw = nparts % 4 == 0 ? 4 : (nparts % 3 == 0 ? 3 : (nparts % 2 == 0 ? 2 : 0));
-    if (pw == 0 && nparts >= 5) pw = (nparts + 3) / 4 < (nparts + 2) / 3 ? 4 : 3;
-    // LDS: the tile, then the partial sums of the workgroup's PW * 4 waves (1 KB per wave, accumulator and sub-tile)
-    if (pw == 0 || tile_bytes(MT, p.Cb) + pw * 4 * nacc * ((MT + 15) / 16) * 1024 > 160 * 1024) return -1;
+    const int nacc = (kind == 0 || kind == 3) ? 1 : 2, nparts = p.nseg * nacc, pw = partsplit_waves(nparts);
+    if (!partsplit_fits(MT, nacc, p)) return -1;
     // more tiles x 4-unit workgroups than one round holds (one workgroup fills a CU): 8 units per workgroup, two waves
     // each (gate_up of d_model 2048 at 33..64 rows: 8.3 -> 6.1 us)
     if (kind != 2 && nparts >= 2 && (p.M + MT - 1) / MT * (int64_t)((p.n_units + 3) / 4) > 256 &&
@@ -211,10 +220,16 @@ static int smallm_launch_code(int kind, SpmmParams &p, const SpmmParams *table, 
     if (!table && layers == 1 && w == 2) {      // one matrix over the whole chip: latency form
         int rc = -1;
         if (resident) {
-            // gate_up of 5..32 rows: 8-token tiles, which stage (and normalise) half as much per workgroup and put twice the
-            // workgroups on the chip, up to 360 of them (MLP of d_model 2048, graph replay: 8 rows 13.7 -> 12.4 us, 13 rows 14.5 ->
-            // 12.5, 32 rows 15.0 -> 13.4; 352 workgroups are faster, 384 and 516 slower: d_model 3072 at 24 rows 19.1 against 19.9 us)
-            const bool eight = kind == 1 && t == 16 && p.M <= 32 && (p.M + 7) / 8 * (int64_t)((p.n_units + 3) / 4) <= 360;
+            // gate_up of 5 rows and more: 8-token tiles stage (and normalise) half as much per workgroup and put twice the
+            // workgroups on the chip.  While their 4-unit workgroups are one round of it (256) they are faster than 16-token
+            // tiles at every width (d_model 2048 with the norm 8.2 -> 6.2 us, without 4.65 -> 4.4; 768 5.9 -> 4.75, 3.65 -> 3.55).
+            // Beyond, the launcher packs 8 units into a workgroup, two waves each: still faster for up to a round of those
+            // (512) where the staging is long, that is with the norm in it (d_model 2048, 25..32 rows 8.2 -> 6.9) or where
+            // no 16-token tile leaves room for the partial sums (d_model 4096, d_ff 8192, 17..32 rows 10.3 -> 8.6..9.1), but not
+            // otherwise (d_model 2048 without the norm, 17..32 rows: 4.7 against 5.6..5.8; 3072 6.4 against 7.2), and in a second
+            // round never (d_model 2048, 48 rows: 8.3 against 12.0).
+            const int64_t w8 = (p.M + 7) / 8 * (int64_t)((p.n_units + 3) / 4);
+            const bool eight = kind == 1 && t == 16 && w8 <= (p.norm || !partsplit_fits(16, 2, p) ? 512 : 256);
             rc = t == 4 ? launch_partsplit<4, CODE>(kind, p, st) : eight ? launch_partsplit<8, CODE>(kind, p, st) : -1;
             if (rc < 0 && t != 4) rc = launch_partsplit<16, CODE>(kind, p, st);
             if (rc < 0 && t == 16 && kind == 1) rc = wide_gate_up();

@@ -1325,3 +1325,19 @@ def test_decode_tiles_of_eight_and_four_tokens(dev, M, f, norm):
     D = MortarPack(synth.flat_pack(dn["codes"]), dn["scales"], dn["col_idx"], dn["offsets"], 64, 5632, dev)
     z = synth.synth_x(M, 5632, seed=M + 1)
     assert_close_bf16(to_np(ops.spmm(to_dev(z, dev), D)), oracle_spmm(z, dn), "down")
+
+
+@pytest.mark.parametrize("d,f,norm,M", [(2048, 5632, False, 16), (2048, 5632, False, 17), (2048, 5632, True, 40), (2048, 5632, True, 41),
+                                        (64, 2048, False, 64), (64, 2064, False, 64), (64, 4096, True, 64), (64, 4112, True, 64),
+                                        (4096, 1024, False, 64), (4096, 8192, False, 32), (4096, 8192, False, 33)])
+def test_gate_up_tiles_around_one_round_of_workgroups(dev, d, f, norm, M):
+    """gate_up of up to 64 rows on either side of the workgroup counts at which its token tile changes."""
+    gu = synth.synth_matrix(2 * f, d, 0.1, seed=53)
+    x = synth.synth_x(M, d, seed=M)
+    W = synth.to_pack(gu, dev)
+    w = to_dev((1.0 + 0.1 * np.sin(np.arange(d))).astype(np.float32), dev)
+    h = ops.gateup_swiglu(to_dev(x, dev), W, norm=(w, 1e-6) if norm else None)
+    xn = ops.rmsnorm(to_dev(x, dev), w, 1e-6) if norm else to_dev(x, dev)
+    g = oracle_spmm(to_np(xn), gu)
+    g = torch.from_numpy(g).to(torch.bfloat16).float()
+    assert_close_bf16(to_np(h), (torch.nn.functional.silu(g[:, :f]) * g[:, f:]).numpy(), "gate_up", ulps=4)
