@@ -355,17 +355,10 @@ int mortar_gemv_bf16(const mortar_bcsr_t *W, const int32_t *entries, int64_t n_e
  *   part       device workspace of part_bytes >= mortar_gemv_f32_workspace_bytes(W, B, nslots) bytes, 16-byte aligned
  *              (may be NULL when nslots == 1; then only the work-list kernel runs)
  *   other arguments as mortar_gemv_bf16.  Agreement with a float64 evaluation: fp32 rounding of the sums only.
- * With one scale (scale_count = 1, the reference's format) and a schedule, the product runs as mortar_gemv_f32_one instead
- * of the work list: the same exact products and fp32 sums in another order of addition.  Flags keep their per-stream
- * meaning there: a chunk of x whose column is off for its stream enters as zeros, and the sum of a row that is off for a
- * stream is written as zero. */
-/* The one-scale form of that product in one launch, without schedule, work list or workspace: scale fp32 [1], other
- * arguments as mortar_gemv_f32 with x rows 16-byte aligned.  Returns MORTAR_NO_KERNEL (-100, nothing launched) for rows too wide for
- * any tile of all K (in_features > 27000); mortar_gemv_f32 uses it by itself where it is the faster form. */
-#define MORTAR_NO_KERNEL (-100)
-int mortar_gemv_f32_one(const mortar_bcsr_t *W, const float *scale, int32_t mode, int32_t swiglu_x, const float *x, int32_t B,
-                        int64_t ldx, float *y, int64_t ldy, const float *gates, int32_t n_clusters, int64_t ldg,
-                        const int32_t *row_act, int64_t ldr, const int32_t *col_act, int64_t ldc, void *stream);
+ * With one scale (scale_count = 1, the reference's format) and a schedule, the product runs as mortar_gemv_f32_one or, on
+ * 3 B rows of bf16 terms, on the SpMM kernels instead of the work list: the same exact products and fp32 sums in another
+ * order of addition.  Flags keep their per-stream meaning there: a chunk of x whose column is off for its stream enters as
+ * zeros, and the sum of a row that is off for a stream is written as zero. */
 int64_t mortar_gemv_f32_workspace_bytes(const mortar_bcsr_t *W, int32_t B, int32_t nslots);
 int mortar_gemv_f32(const mortar_bcsr_t *W, const float *scale, int64_t scale_count, const int32_t *sched,
                     const int32_t *entries,
@@ -373,6 +366,15 @@ int mortar_gemv_f32(const mortar_bcsr_t *W, const float *scale, int64_t scale_co
                     int32_t swiglu_x, const float *x, int32_t B, int64_t ldx, float *y, int64_t ldy, float *part,
                     int64_t part_bytes, const float *gates, int32_t n_clusters, int64_t ldg,
                     const int32_t *row_act, int64_t ldr, const int32_t *col_act, int64_t ldc, void *stream);
+/* The one-scale form of that product in one launch, without schedule, work list or workspace: scale fp32 [1], other
+ * arguments as mortar_gemv_f32 with x rows 16-byte aligned.  Returns MORTAR_NO_KERNEL (-100, nothing launched) for rows too wide for
+ * any tile of all K (in_features above about 24800, with mode 1 22300).  mortar_gemv_f32 uses it where mortar_gemv_f32_one_better
+ * says 1: while its workgroups make three (mode 1) or four rounds of the chip; otherwise three launches on the SpMM kernels. */
+#define MORTAR_NO_KERNEL (-100)
+int mortar_gemv_f32_one_better(const mortar_bcsr_t *W, int32_t mode, int32_t B);
+int mortar_gemv_f32_one(const mortar_bcsr_t *W, const float *scale, int32_t mode, int32_t swiglu_x, const float *x, int32_t B,
+                        int64_t ldx, float *y, int64_t ldy, const float *gates, int32_t n_clusters, int64_t ldg,
+                        const int32_t *row_act, int64_t ldr, const int32_t *col_act, int64_t ldc, void *stream);
 
 /* mortar_gemv_bf16 for callers that cannot allocate device memory or hand in a workspace: code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments and

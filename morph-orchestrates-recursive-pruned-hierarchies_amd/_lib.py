@@ -85,6 +85,7 @@ _SIGS = {
     "mortar_gemv_f32_workspace_bytes": (c_i64, [c_vp, c_i32, c_i32]),
     "mortar_gemv_f32": (C.c_int, [c_vp, c_vp, c_i64, c_vp, c_vp, c_i64, c_i32, c_vp, c_i32, c_i32, c_i32, c_vp, c_i32, c_i64, c_vp, c_i64,
                                   c_vp, c_i64, c_vp, c_i32, c_i64, c_vp, c_i64, c_vp, c_i64, c_vp]),
+    "mortar_gemv_f32_one_better": (C.c_int, [c_vp, c_i32, c_i32]),
     "mortar_gemv_f32_one": (C.c_int, [c_vp, c_vp, c_i32, c_i32, c_vp, c_i32, c_i64, c_vp, c_i64, c_vp, c_i32, c_i64, c_vp, c_i64, c_vp, c_i64,
                                       c_vp]),
     "mortar_gemv_noalloc_max_floats": (c_i64, []),

@@ -473,7 +473,7 @@ int launch_gemv_f32(const GemvF32Params &p, hipStream_t st) {
     return MORTAR_OK;
 }
 
-// ---- one scale for the whole matrix, no flags: the product runs on the bandwidth-bound SpMM kernels ----------------
+// ---- one scale for the whole matrix: the product runs on the bandwidth-bound SpMM kernels ----------------
 // The three bf16 terms of every activation row become three rows of a bf16 matrix [3B, in_features] (hi rows, then
 // mid, then lo); the SpMM kernels for matrices with one scale contract them with the +-2 / 0 blocks (every product
 // exact, fp32 sums in the matrix pipe) and store the sums unrounded; a last kernel adds the three sums of a row, applies
@@ -547,7 +547,9 @@ int64_t gemv_f32_fast_bytes(const mortar_bcsr_t *W, int B) {
     return (int64_t)3 * B * ((int64_t)W->Rb * 16 * 4 + (int64_t)W->Cb * 16 * 2);
 }
 
-// Rows too wide for a tile of all K of even one token (mortar_gemv_f32_one): split, SpMM on the 3 B term rows, combine.
+// Split, SpMM on the 3 B term rows, combine: for calls that mortar_gemv_f32_one would serve in many rounds of workgroups, or not
+// at all (rows too wide for a tile of all K of even one token: [8192, 28672] at 8 rows 50 us against 132 on the work list, relative
+// error 7e-8 against 1.3e-7).
 // Returns MORTAR_NO_KERNEL when the SpMM kernels cannot serve the shape (the caller then runs the work-list kernel).
 int gemv_f32_fast(const mortar_bcsr_t *W, const int32_t *sched, const GemvF32Params &p, void *ws, hipStream_t st) {
     const int K = W->Cb * 16, N = W->Rb * 16;
@@ -609,13 +611,17 @@ extern "C" int mortar_gemv_f32(const mortar_bcsr_t *W, const float *scale, int64
     if (nslots > 1 && part_bytes < (int64_t)nslots * B * W->Rb * 16 * 4)
         return mortar_fail(MORTAR_ERR_ARG, "gemv_f32: the partial workspace holds %lld bytes, need %lld", (long long)part_bytes,
                            (long long)nslots * B * W->Rb * 16 * 4);
-    if (scale_count == 1 && sched && W->row_desc && W->codes_o && W->col_o && (B == 1 || ldx % 4 == 0) && !(reinterpret_cast<uintptr_t>(x) & 15)) {
-        const int rc = mortar_gemv_f32_one(W, scale, mode, swiglu_x, x, B, ldx, y, ldy, gates, n_clusters, ldg, row_act, ldr, col_act, ldc, stream);
+    // one scale: one launch (mortar_gemv_f32_one) where that is the faster form, else the three on the SpMM kernels, else the one
+    const bool one = scale_count == 1 && sched && W->row_desc && W->codes_o && W->col_o && (B == 1 || ldx % 4 == 0) && !(reinterpret_cast<uintptr_t>(x) & 15);
+    const bool three = scale_count == 1 && sched && W->codes_o && part && !(reinterpret_cast<uintptr_t>(part) & 15) &&
+                       part_bytes >= gemv_f32_fast_bytes(W, B) && ldx % 4 == 0 && !(reinterpret_cast<uintptr_t>(x) & 15);
+    const bool better = one && mortar_gemv_f32_one_better(W, mode, B);
+    if (three && !better) {
+        const int rc = gemv_f32_fast(W, sched, p, part, st);
         if (rc != MORTAR_NO_KERNEL) return rc;
     }
-    if (scale_count == 1 && sched && W->codes_o && part && !(reinterpret_cast<uintptr_t>(part) & 15) &&
-        part_bytes >= gemv_f32_fast_bytes(W, B) && ldx % 4 == 0 && !(reinterpret_cast<uintptr_t>(x) & 15)) {
-        const int rc = gemv_f32_fast(W, sched, p, part, st);
+    if (one) {
+        const int rc = mortar_gemv_f32_one(W, scale, mode, swiglu_x, x, B, ldx, y, ldy, gates, n_clusters, ldg, row_act, ldr, col_act, ldc, stream);
         if (rc != MORTAR_NO_KERNEL) return rc;
     }
     int rc = B <= 16 ? launch_gemv_f32<1>(p, st) : (B <= 32 ? launch_gemv_f32<2>(p, st) : launch_gemv_f32<4>(p, st));

@@ -6,7 +6,8 @@
 // term * T + t of the tile is a term of token t), the blocks are contracted as +-2 / 0, and the epilogue adds the three sums
 // of a token (columns of the accumulator, two lane exchanges), scales, and applies SwiGLU and gates.
 // Three launches per product (split, SpMM on 3 B rows, combine) took 11.9 us of GPU time and 16 us of host time at 8 rows of
-// the 2048 -> 11264 matrix; what they moved through memory between them is now in LDS and registers.
+// the 2048 -> 11264 matrix; what they moved through memory between them is now in LDS and registers.  Where this form makes many
+// rounds of workgroups (wide K, many rows) the three launches stay the faster one: mortar_gemv_f32_one_better.
 #include "mortar_spmm_core.h"
 
 namespace {
@@ -154,9 +155,24 @@ __global__ void __launch_bounds__(PW * 4 * 64) gemv_f32_one_kernel(const SpmmPar
     *reinterpret_cast<f32x4_t *>(a.y + (int64_t)tok * a.ldy + pos * 16 + 4 * g) = r[0];
 }
 
+int one_lds(int t, int nacc, int pw, int Cb) { return tile_bytes(3 * t, Cb) + (pw > 1 ? pw * 4 * nacc * 1024 : 0); }
+
+struct OneShape { int t, pw; };        // tokens per tile (0: none fits), waves per unit
+
+OneShape one_shape(const mortar_bcsr_t *W, int mode, int B) {
+    const int seg = W->seg_cb < W->Cb ? W->seg_cb : W->Cb, nacc = mode + 1, nparts = (W->Cb + seg - 1) / seg * nacc;
+    // waves per unit: a divisor of the part count where there is one (as the bf16 part-split launches)
+    const int pw = nparts == 1 ? 1 : nparts % 4 == 0 ? 4 : nparts % 3 == 0 ? 3 : nparts % 2 == 0 ? 2 : (nparts + 3) / 4 < (nparts + 2) / 3 ? 4 : 3;
+    // tokens per tile: all of them where they fit (at most five: 15 of the MFMA's 16 columns), else the most that LDS takes
+    int t = 0;
+    for (int c : {1, 2, 4, 5})
+        if (one_lds(c, nacc, pw, W->Cb) <= 160 * 1024) { t = c; if (c >= B) break; }
+    return {t, pw};
+}
+
 template <int T, int NACC, int PW>
 int launch_one(SpmmParams &p, const GemvOneArgs &a, hipStream_t st) {
-    const int smem = tile_bytes(3 * T, p.Cb) + (PW > 1 ? PW * 4 * NACC * 1024 : 0);
+    const int smem = one_lds(T, NACC, PW, p.Cb);
     static bool done = false;
     int rc = mortar_allow_big_lds(gemv_f32_one_kernel<T, NACC, PW>, done);
     if (rc) return rc;
@@ -191,6 +207,21 @@ int launch_t(int t, int pw, SpmmParams &p, const GemvOneArgs &a, hipStream_t st)
 
 }  // namespace
 
+// Every workgroup stages its tile of all K again, and few tokens fit one where K is wide: a round of workgroups costs 5 us (as
+// many per CU as LDS holds), while the three launches of mortar_gemv_f32 grow slowly with the rows.  They meet at three rounds
+// for the SwiGLU form (d_model 3072, 24 rows: 16.0 against 15.6 us, 64 rows 35 against 22; 4096, 16 rows 17.9 against 21.4, 64 rows
+// 51 against 33) and at four for the plain product (11008 inputs, 32 rows: 26.8 against 31.2, 64 rows 50 against 32.5; 22016 inputs,
+// 8 rows 26.5 against 31.6, 64 rows 192 against 50).
+extern "C" int mortar_gemv_f32_one_better(const mortar_bcsr_t *W, int32_t mode, int32_t B) {
+    if (!W || W->Rb <= 0 || W->Cb <= 0 || W->seg_cb <= 0 || B <= 0 || B > 64 || (mode != 0 && mode != 1)) return 0;
+    const OneShape s = one_shape(W, mode, B);
+    if (s.t == 0) return 0;
+    const int units = mode == 0 ? W->Rb : W->Rb / 2, lds = one_lds(s.t, mode + 1, s.pw, W->Cb);
+    const int by_lds = 160 * 1024 / lds, by_waves = 32 / (4 * s.pw), per_cu = by_lds < by_waves ? by_lds : by_waves;
+    const int64_t wgs = (int64_t)((B + s.t - 1) / s.t) * ((units + 3) / 4), rounds = (wgs + 256 * per_cu - 1) / (256 * per_cu);
+    return rounds <= (mode == 0 ? 4 : 3);
+}
+
 extern "C" int mortar_gemv_f32_one(const mortar_bcsr_t *W, const float *scale, int32_t mode, int32_t swiglu_x, const float *x, int32_t B,
                                    int64_t ldx, float *y, int64_t ldy, const float *gates, int32_t n_clusters, int64_t ldg,
                                    const int32_t *row_act, int64_t ldr, const int32_t *col_act, int64_t ldc, void *stream) {
@@ -214,16 +245,9 @@ extern "C" int mortar_gemv_f32_one(const mortar_bcsr_t *W, const float *scale, i
     p.Rb = W->Rb; p.Cb = W->Cb; p.M = B;
     p.n_units = mode == 0 ? W->Rb : W->Rb / 2;
     p.n_clusters = 1; p.cluster_size = gates ? (int)(nout / n_clusters) : 1 << 30;
-    const int nacc = mode + 1, nparts = p.nseg * nacc;
-    // waves per unit: a divisor of the part count where there is one (as the bf16 part-split launches)
-    const int pw = nparts == 1 ? 1 : nparts % 4 == 0 ? 4 : nparts % 3 == 0 ? 3 : nparts % 2 == 0 ? 2 : (nparts + 3) / 4 < (nparts + 2) / 3 ? 4 : 3;
-    // tokens per tile: all of them where they fit (at most five: 15 of the MFMA's 16 columns), else the most that LDS takes
-    auto fits = [&](int t) { return tile_bytes(3 * t, p.Cb) + (pw > 1 ? pw * 4 * nacc * 1024 : 0) <= 160 * 1024; };
-    int t = 0;
-    for (int c : {1, 2, 4, 5})
-        if (fits(c)) { t = c; if (c >= B) break; }
-    if (t == 0) return MORTAR_NO_KERNEL;
+    const OneShape sh = one_shape(W, mode, B);
+    if (sh.t == 0) return MORTAR_NO_KERNEL;
     const GemvOneArgs a{x, scale, gates, y, row_act, col_act, ldx, ldy, ldg, ldr, ldc, swiglu_x != 0};
     hipStream_t st = static_cast<hipStream_t>(stream);
-    return mode == 0 ? launch_t<1>(t, pw, p, a, st) : launch_t<2>(t, pw, p, a, st);
+    return mode == 0 ? launch_t<1>(sh.t, sh.pw, p, a, st) : launch_t<2>(sh.t, sh.pw, p, a, st);
 }

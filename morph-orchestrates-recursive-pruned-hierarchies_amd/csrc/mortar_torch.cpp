@@ -325,7 +325,7 @@ PyObject *py_gemv_f32(PyObject *, PyObject *const *a, Py_ssize_t na) {
         !x.is_contiguous() || !aligned16(x.const_data_ptr()) || (swo && (h->w->Rb & 1)))
         Py_RETURN_NONE;
     const int64_t B = x.size(0);
-    if (B < 1 || B > DECODE_MAX_ROWS) Py_RETURN_NONE;
+    if (B < 1 || B > DECODE_MAX_ROWS || !mortar_gemv_f32_one_better(h->w, swo, (int32_t)B)) Py_RETURN_NONE;
     const float *gates = nullptr;
     int64_t ncl = 0, ldg = 0;
     if (a[5] != Py_None) {

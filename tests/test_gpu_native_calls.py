@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import mortar_amd
-from mortar_amd import ops, synth
+from mortar_amd import _lib, ops, synth
 from mortar_amd.engine import MortarDecodeMLP
 
 pytestmark = pytest.mark.gpu
@@ -100,3 +100,37 @@ def test_fp32_decode_product_takes_any_true_flag(dev, flag):
     x = x[:, :128].contiguous()
     h = mortar_amd.mortar_gemv(x, W, swiglu_out=flag)
     assert h.shape == (3, 32) and torch.equal(h, mortar_amd.mortar_gemv(x, W, swiglu_out=True))
+
+
+@pytest.mark.parametrize("out_b,K_blocks,B,better", [(10, 1700, 1, 0), (10, 1700, 5, 0), (10, 1700, 22, 0),      # no tile of all K
+                                                     (256, 688, 32, 1), (256, 688, 33, 0),                     # four rounds of workgroups, five
+                                                     (512, 192, 60, 1), (512, 192, 61, 0), (512, 192, 64, 0)])  # SwiGLU form: three rounds, four
+def test_fp32_decode_product_on_either_side_of_the_one_launch_form(dev, out_b, K_blocks, B, better):
+    """mortar_gemv of one-scale matrices where the three launches on the SpMM kernels take over from the one: against float64."""
+    swiglu = out_b == 512
+    m = synth.synth_matrix(16 * out_b, 16 * K_blocks, 0.1, seed=K_blocks, per_tensor_scale=True)
+    W = synth.to_pack(m, dev)
+    assert _lib.lib().mortar_gemv_f32_one_better(W.ref, int(swiglu), B) == better
+    dense = torch.zeros(out_b, K_blocks, 16, 16, dtype=torch.float64, device=dev)
+    dense[torch.from_numpy(m["row_idx"]).long(), torch.from_numpy(m["col_idx"]).long()] = torch.from_numpy(m["codes"]).to(dev).double()
+    dense = dense.permute(0, 2, 1, 3).reshape(16 * out_b, -1) * float(m["scales"][0])
+    g = torch.Generator(device=dev).manual_seed(B)
+    K = 16 * K_blocks
+    x2 = torch.randn(B, 2 * K, device=dev, generator=g)
+    x = x2[:, :K].contiguous()
+    ca = (torch.rand(B, K_blocks, device=dev, generator=g) < 0.6).int()
+    ra = (torch.rand(B, out_b, device=dev, generator=g) < 0.6).int()
+
+    def close(got, want):
+        assert (got.double() - want).abs().max() <= 3e-6 * want.abs().max()
+
+    on = (x.double() * ca.repeat_interleave(16, 1)) @ dense.t() * ra.repeat_interleave(16, 1)
+    if not swiglu:
+        close(mortar_amd.mortar_gemv(x, W), x.double() @ dense.t())
+        close(mortar_amd.mortar_gemv(x, W, row_act=ra, col_act=ca), on)
+        close(mortar_amd.mortar_gemv(x2, W, swiglu_x=True), (torch.nn.functional.silu(x2[:, :K].double()) * x2[:, K:].double()) @ dense.t())
+        return
+    gates = torch.relu(torch.randn(B, 16, device=dev, generator=g))
+    f = 8 * out_b
+    want = torch.nn.functional.silu(on[:, :f]) * on[:, f:] * gates.double().repeat_interleave(f // 16, 1)
+    close(mortar_amd.mortar_gemv(x, W, swiglu_out=True, gates=gates, row_act=ra, col_act=ca), want)
