@@ -129,3 +129,27 @@ def test_load_statistics_are_an_in_place_update_for_torch(dev, M):
         assert rt.forward_native(x) is not None
     with torch.no_grad(), pytest.raises(RuntimeError, match="[Ii]nference"):      # as any in-place operator on such a buffer
         rt(x)
+
+
+@pytest.mark.parametrize("M,d_in,d_out", [(65, 136, 260), (300, 1032, 1024), (129, 2048, 136), (1000, 2056, 260), (4097, 72, 132)])
+def test_projection_keeps_non_finite_values_to_their_row_and_output(dev, M, d_in, d_out):
+    """An infinity or NaN of x makes its row non-finite and no other, one of the weights its output and no other (ragged K
+    and tiles included: what is staged past the end must not come in); weights up to the largest float are exact."""
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn(M, d_in, device=dev, generator=g).to(torch.bfloat16)
+    w = torch.randn(d_out, d_in, device=dev, generator=g) * 0.05
+    ref = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * 2.0 ** -22
+    rows, outs = torch.zeros(M, dtype=torch.bool, device=dev), torch.zeros(d_out, dtype=torch.bool, device=dev)
+    for r, k, v in ((0, 0, float("inf")), (M - 1, d_in - 1, float("nan")), (M // 2, 0, float("-inf"))):
+        x[r, k], rows[r] = v, True
+    for o, k, v in ((0, d_in - 1, float("inf")), (d_out - 1, 0, float("nan")), (d_out // 2, 0, float("-inf"))):
+        w[o, k], outs[o] = v, True
+    qv = _project(x, w)
+    hit = rows[:, None] | outs[None, :]
+    assert not qv[hit].isfinite().any()
+    assert ((qv.double() - ref).abs() <= bound)[~hit].all()
+    x = torch.zeros(M, d_in, device=dev, dtype=torch.bfloat16)
+    x[:, d_in - 1] = 2.0 ** -8
+    w = torch.full((d_out, d_in), torch.finfo(torch.float32).max, device=dev)
+    assert torch.equal(_project(x, w), (w[:, -1] * 2.0 ** -8).expand(M, -1))
