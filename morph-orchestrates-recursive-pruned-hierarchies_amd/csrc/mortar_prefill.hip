@@ -89,8 +89,6 @@ int segmented_upw(const SpmmParams &p) {
     return best;
 }
 
-// Plain product of a `down` whose input is stored in tile order (mortar_mlp_bf16): the instantiations that copy their
-// token tiles straight into LDS.  The caller has checked that the matrix runs 32-token tiles.
 // Gate/up unit pairs per wave of the K-segmented gate_up: 1, 2 or 3 (four spill), the choice with the least rounds of 256
 // workgroups x (staging + units).  A unit pair takes about 6.7 us and staging the segments 5 us (d_model 3072 and 4096), so a round
 // weighs 3 + 4 upw.  With two units per wave throughout, 400 rows of d_model 4096 were 286 workgroups: 83 -> 70 us for the MLP; 150
@@ -117,6 +115,8 @@ int dispatch_gateup_tiled(SpmmParams &p, hipStream_t st) {     // gate_up + SwiG
     return mortar_launch_segmented<32, 2, false, SEG_WAVES, 1, false, CODE, true>(p, nullptr, 1, st);
 }
 
+// Plain product of a `down` whose input is stored in tile order (mortar_mlp_bf16): the instantiations that copy their
+// token tiles straight into LDS.  The caller has checked that the matrix runs 32-token tiles.
 template <int CODE>
 int dispatch_prefill_tiled(SpmmParams &p, hipStream_t st) {
     if (p.nseg == 1) return mortar_launch_resident<32, 1, false, 16, false, CODE, true>(p, nullptr, 1, st);

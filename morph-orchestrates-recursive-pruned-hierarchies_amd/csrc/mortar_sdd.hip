@@ -21,8 +21,8 @@
 // cycles of the matrix core, and the two overlap only in part: three tile reads and two MFMAs per wavefront measured 298
 // cycles beside 217 and 144 alone, two reads 231.  So a is read again only where the block-row changes, nothing but reads and
 // MFMAs stands in the inner loop (a pair of slots never straddles two rows, addresses and copies are fixed over the steps),
-// and the rest is the slabs.  dW of 11264 x 2048 at 25 %, 4096 tokens: 103 -> 84 us; 4096 x 768, 16384 tokens: 68 -> 54 us;
-// 2048 x 5632, 4096 tokens: 65 -> 54 us.
+// and the rest is the slabs.  Both launches, in a loop over the same operands: dW of 11264 x 2048 at 25 %, 4096 tokens 103 -> 84 us
+// (89 over six sets of operands); 4096 x 768, 16384 tokens 68 -> 55 us (71); 2048 x 5632, 4096 tokens 65 -> 54 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

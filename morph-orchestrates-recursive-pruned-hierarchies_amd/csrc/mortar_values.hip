@@ -143,8 +143,9 @@ __device__ __forceinline__ int val_idx(const int32_t *p, int i) {
 
 // All of K in one tile.  The waves draw block-rows (a.unit = 2: pairs of them) from a counter, so that rows of any length keep
 // all of them busy; a wave's batches form one stream across rows, requested two ahead of their products.  Narrow K is bound by
-// the results (16384 x 768 x 4096 at 25 %, 134 MB of them: 84 -> 47 us, of which 21 are a fill of that size; 59 us with rows one
-// at a time), wide K by the values from the L2, once per 32 tokens (4096 x 2048 x 11264: 102 -> 83 us, 18 TB/s of values).
+// the results and the values together (16384 x 768 x 4096 at 25 %, 134 MB of results, a fill of which takes 21 us: 84 -> 51 us in a
+// loop over the same buffers, 57 over six sets of them, 65..69 in the trace of a training step, 153 MB written there; rows one at a
+// time took a quarter longer), wide K by the values from the L2, once per 32 tokens (4096 x 2048 x 11264: 102 -> 83 us, 18 TB/s of values).
 template <int MT>
 __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const ValArgs a) {
     constexpr int MSUB = MT / 16;
@@ -235,8 +236,9 @@ __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const V
 // Wider K: segments through two LDS buffers, one barrier each.  Four loader waves copy the next segment while twelve multiply the
 // current one: a wave's loads complete in order, so a wave that did both would wait for the copies (from beyond the L2) at its
 // next weights.  A consumer keeps the accumulators of its UPW block-rows in registers over the segments.  The values (once per
-// 64 tokens from the L2) and the operand reads from LDS bound it.  16384 x 4096 x 768 at 25 %: 91 -> 51 us; segments of 24
-// columns in three buffers took 54 (short parts leave a batch half empty), batches requested two ahead 60 (registers, moves).
+// 64 tokens from the L2) and the operand reads from LDS bound it.  16384 x 4096 x 768 at 25 %: 91 -> 50 us in a loop over the same
+// buffers, 62 over six sets of them, 61..72 in the trace of a training step.  Segments of 24 columns in three buffers took 6 % longer
+// (short parts leave a batch half empty), batches requested two ahead 18 % (registers, moves).
 template <int MT, int UPW>
 __global__ void __launch_bounds__((VAL_CW + VAL_LOADERS) * 64) values_segmented_kernel(const ValArgs a) {
     constexpr int MSUB = MT / 16;
