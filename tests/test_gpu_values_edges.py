@@ -69,3 +69,9 @@ def test_weight_gradient_of_rows_far_apart(dev, lda, ldb):
 
     a, b = (torch.randn(M, n, device=dev).bfloat16() for n in (W.out_features, W.in_features))
     assert torch.equal(ops.sdd(far(a, lda), far(b, ldb), W), ops.sdd(a, b, W))
+
+
+@pytest.mark.parametrize("Rb,Cb,M", [(33, 78, 65), (12, 77, 130), (70, 155, 97)])      # the widest tiles of all K: 64 tokens, 32 tokens
+@pytest.mark.parametrize("density", [0.04, 0.5])
+def test_values_product_of_the_widest_whole_tiles(dev, Rb, Cb, M, density):
+    test_values_product_edges(dev, Rb, Cb, M, density)
