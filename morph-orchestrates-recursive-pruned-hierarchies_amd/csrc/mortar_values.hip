@@ -370,7 +370,7 @@ int launch_segmented(ValArgs &a, hipStream_t st) {
                       2 * (a.seg_cb * a.sub / 2 * (MT * 64)), st);
 }
 
-// A tile of all K: 155 block-columns for 32 tokens, 78 for 64 (the row counter behind it is outside the tile's budget).
+// A tile of all K: up to 156 block-columns (78 pairs) for 32 tokens, 78 for 64 (the row counter behind it is outside the tile's budget).
 bool val_fits(int mt, int Cb) { return (Cb + 1) / 2 * (mt * 64) <= LDS_BUDGET; }
 
 // The launch for the tokens of `a` (seg_cb and nfine are set).

@@ -71,7 +71,7 @@ def test_weight_gradient_of_rows_far_apart(dev, lda, ldb):
     assert torch.equal(ops.sdd(far(a, lda), far(b, ldb), W), ops.sdd(a, b, W))
 
 
-@pytest.mark.parametrize("Rb,Cb,M", [(33, 78, 65), (12, 77, 130), (70, 155, 97)])      # the widest tiles of all K: 64 tokens, 32 tokens
+@pytest.mark.parametrize("Rb,Cb,M", [(33, 78, 65), (12, 77, 130), (70, 155, 97), (17, 156, 33), (49, 157, 65)])   # the widest tiles of all K (64 tokens, 32), the first K segments
 @pytest.mark.parametrize("density", [0.04, 0.5])
 def test_values_product_of_the_widest_whole_tiles(dev, Rb, Cb, M, density):
     test_values_product_edges(dev, Rb, Cb, M, density)

@@ -550,8 +550,8 @@ def test_layer_carved_at_128_loads_and_packs_on_the_host():
     assert np.array_equal(got, dense)
 
 
-def test_stored_values_of_155_block_columns_are_one_segment():
-    """Rows of up to 2480 values need no segment pointers (the widest 32-token tile of all K): callers may pass NULL there."""
+def test_stored_values_of_156_block_columns_are_one_segment():
+    """Rows of up to 2496 values need no segment pointers (the widest 32-token tile of all K): callers may pass NULL there."""
     from mortar_amd import _lib
     seg = _lib.lib().mortar_values_seg_cb
-    assert [seg(c) for c in (1, 76, 78, 79, 154, 155)] == [1, 76, 78, 79, 154, 155] and 0 < seg(156) < 156
+    assert [seg(c) for c in (1, 76, 78, 79, 154, 155, 156)] == [1, 76, 78, 79, 154, 155, 156] and 0 < seg(157) < 157
