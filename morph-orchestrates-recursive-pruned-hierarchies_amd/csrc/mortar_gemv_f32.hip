@@ -230,6 +230,8 @@ extern "C" int mortar_gemv_f32_one(const mortar_bcsr_t *W, const float *scale, i
     if (mode != 0 && mode != 1) return mortar_fail(MORTAR_ERR_ARG, "gemv_f32_one: mode must be 0 or 1");
     if (W->Rb <= 0 || W->Cb <= 0 || W->nnz <= 0 || W->seg_cb <= 0 || (mode == 1 && (W->Rb & 1)))
         return mortar_fail(MORTAR_ERR_ARG, "gemv_f32_one: bad matrix");
+    const int too_large = mortar_check_octets(W);
+    if (too_large) return too_large;
     const int64_t nout = mode == 0 ? (int64_t)W->Rb * 16 : (int64_t)W->Rb * 8, need = (int64_t)W->Cb * 16 * (swiglu_x ? 2 : 1);
     if (ldx < need || (B > 1 && ldx % 4) || ldy < nout || ldy % 4 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15))
         return mortar_fail(MORTAR_ERR_ARG, "gemv_f32_one: bad leading dimension or alignment (rows 16-byte aligned)");

@@ -9,6 +9,10 @@ int mortar_fail(int code, const char *fmt, ...) __attribute__((format(printf, 2,
 
 int mortar_check_bcsr_host(const int32_t *row_ptr, const int16_t *col, int32_t Rb, int32_t Cb);
 
+// The kernels address the octet stream with 32-bit byte offsets (1 KiB of 4-bit codes per octet): refuses larger matrices.
+// Cb and seg_cb are positive.
+__attribute__((visibility("hidden"))) int mortar_check_octets(const mortar_bcsr_t *W);
+
 // Plain product on the +-1 / 0 codes alone, unrounded: y32[m, :] = sum over the kept blocks of codes . x[m, :] in fp32
 // (the one-scale kernels with the scale left out).  Returns MORTAR_NO_KERNEL when the pack has no such kernel for M rows.
 __attribute__((visibility("hidden"))) int mortar_spmm_codes_f32(const mortar_bcsr_t *W, const int32_t *sched, const uint16_t *x,

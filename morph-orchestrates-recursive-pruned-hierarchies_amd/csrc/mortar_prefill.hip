@@ -10,6 +10,14 @@
 
 #include <vector>
 
+int mortar_check_octets(const mortar_bcsr_t *W) {
+    const int64_t nseg = (W->Cb + W->seg_cb - 1) / W->seg_cb;
+    if ((int64_t)W->nnz / 8 + (int64_t)W->Rb * nseg >= ((int64_t)1 << 22))
+        return mortar_fail(MORTAR_ERR_LIMIT, "spmm: octet stream of %d blocks in %d x %lld row parts exceeds 4 GiB",
+                           W->nnz, W->Rb, (long long)nseg);
+    return MORTAR_OK;
+}
+
 namespace {
 
 int check_common(const mortar_bcsr_t *W, const uint16_t *x, int64_t M, int64_t ldx, const uint16_t *y, int64_t ldy,
@@ -24,12 +32,8 @@ int check_common(const mortar_bcsr_t *W, const uint16_t *x, int64_t M, int64_t l
             return mortar_fail(MORTAR_ERR_ARG, "spmm: K segments of %d block-columns do not fit LDS for %lld rows (max %d; %d up to 16 rows, %d up to 4)",
                                W->seg_cb, (long long)M, mortar_prefill_max_seg_cb(), mortar_decode_max_seg_cb(16), mortar_decode_max_seg_cb(4));
     }
-    {   // the kernels address the octet stream with 32-bit byte offsets (1 KiB of 4-bit codes per octet)
-        const int64_t nseg = (W->Cb + W->seg_cb - 1) / W->seg_cb;
-        if ((int64_t)W->nnz / 8 + (int64_t)W->Rb * nseg >= ((int64_t)1 << 22))
-            return mortar_fail(MORTAR_ERR_LIMIT, "spmm: octet stream of %d blocks in %d x %lld row parts exceeds 4 GiB",
-                               W->nnz, W->Rb, (long long)nseg);
-    }
+    const int rc = mortar_check_octets(W);
+    if (rc) return rc;
     if (M <= 0 || M > (1 << 30)) return mortar_fail(MORTAR_ERR_ARG, "spmm: M=%lld out of range", (long long)M);
     if (ldx < (int64_t)W->Cb * 16 || ldx % 8) return mortar_fail(MORTAR_ERR_ARG, "spmm: ldx=%lld must be >= in_features and a multiple of 8", (long long)ldx);
     if (ldy < out_cols || ldy % 4) return mortar_fail(MORTAR_ERR_ARG, "spmm: ldy=%lld must be >= out_features and a multiple of 4", (long long)ldy);

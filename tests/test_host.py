@@ -555,3 +555,13 @@ def test_stored_values_of_156_block_columns_are_one_segment():
     from mortar_amd import _lib
     seg = _lib.lib().mortar_values_seg_cb
     assert [seg(c) for c in (1, 76, 78, 79, 154, 155, 156)] == [1, 76, 78, 79, 154, 155, 156] and 0 < seg(157) < 157
+
+
+def test_fp32_decode_product_refuses_streams_beyond_32_bit_offsets():
+    """The kernels address the octet stream with 32-bit byte offsets: the one-launch form refuses what the others refuse."""
+    import ctypes as C
+
+    from mortar_amd import _lib
+    W = _lib.BcsrStruct(*[4096] * 9, 1 << 15, 1024, 1 << 25, 128, 1.0, 0)       # never read: refused before any launch
+    rc = _lib.lib().mortar_gemv_f32_one(C.byref(W), 4096, 0, 0, 4096, 1, 16 * 1024, 4096, 16 << 15, None, 0, 0, None, 0, None, 0, None)
+    assert rc == -4 and b"octet stream" in _lib.lib().mortar_last_error()
