@@ -119,7 +119,8 @@ PyObject *py_mlp(PyObject *, PyObject *const *a, Py_ssize_t na) {
     const PackHandle *gu = handle_of(a[1]), *dn = handle_of(a[2]);
     if (PyErr_Occurred()) return nullptr;
     bool decode, norm;
-    if (!truth(a[3], decode) || !truth(a[4], norm)) return nullptr;
+    const double eps = PyFloat_AsDouble(a[6]);
+    if (PyErr_Occurred() || !truth(a[3], decode) || !truth(a[4], norm)) return nullptr;
     if (!xt || !gu || !dn || !gu->sched2 || !dn->sched1) Py_RETURN_NONE;
     const at::Tensor &x = *xt;
     const int64_t d = (int64_t)gu->w->Cb * 16;
@@ -127,8 +128,7 @@ PyObject *py_mlp(PyObject *, PyObject *const *a, Py_ssize_t na) {
     const int64_t M = x.numel() / d;
     if (decode && x.size(0) != M) Py_RETURN_NONE;
     Norm n;
-    if (norm && !read_norm(a[5], PyFloat_AsDouble(a[6]), d, x, n)) Py_RETURN_NONE;
-    if (PyErr_Occurred()) return nullptr;
+    if (norm && !read_norm(a[5], eps, d, x, n)) Py_RETURN_NONE;
     const float *gates = nullptr;
     int64_t ncl = 0;
     if (a[7] != Py_None) {

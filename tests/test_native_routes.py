@@ -247,3 +247,10 @@ def test_wrapped_layers_take_the_general_path(monkeypatch):
         with pytest.raises(RuntimeError, match="ROCm device"):
             call(X)
     assert not _lib._native.calls
+
+
+def test_a_bad_eps_is_a_type_error():
+    """Read before anything else, as float(eps) would: no result may be returned with an exception pending."""
+    n, x = _lib.native(), torch.zeros(2, 64)
+    with pytest.raises(TypeError):
+        n.mlp(x, 0, 0, False, True, None, "1e-6", None)
