@@ -77,7 +77,7 @@ class MortarDecodeMLP:
             return None
         proj, norm = rt._modules["query_proj"], rt._modules["query_norm"]
         return _lib.native().routed_decode(x, gu, dn, self.norm_weight, self.eps, rt._parameters, proj._parameters, norm._parameters,
-                                           (rt.n_iters, rt.n_sub_keys, rt.n_tile_groups, rt.activation_k), norm.eps, self.iter_idx)
+                                           (rt.n_iters, rt.n_sub_keys, rt.n_tile_groups, int(rt.activation_k)), norm.eps, int(self.iter_idx))
 
     @torch.no_grad()
     def _general(self, x: Tensor, gates: Tensor | None = None) -> Tensor:

@@ -71,7 +71,7 @@ class TileRouter(nn.Module):
         if not x.is_cuda:
             return None
         return _lib.native().route(x, self._parameters, self._modules["query_proj"]._parameters, self._modules["query_norm"]._parameters,
-                                   (self.n_iters, self.n_sub_keys, self.n_tile_groups, self.activation_k), self.query_norm.eps, int(iter_idx),
+                                   (self.n_iters, self.n_sub_keys, self.n_tile_groups, int(self.activation_k)), self.query_norm.eps, int(iter_idx),
                                    self._buffers["group_load_ema"] if stats else None, self._load_ema_alpha, self.aux_loss_coeff)
 
     def forward_native(self, x: Tensor, iter_idx: int = 0):

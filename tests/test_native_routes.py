@@ -254,3 +254,17 @@ def test_a_bad_eps_is_a_type_error():
     n, x = _lib.native(), torch.zeros(2, 64)
     with pytest.raises(TypeError):
         n.mlp(x, 0, 0, False, True, None, "1e-6", None)
+
+
+def test_iteration_index_and_k_are_taken_as_integers(native, monkeypatch):
+    """int() of whatever number the caller holds, as the general path takes them."""
+    mlp = _mlp()
+    mlp.enable_routing(n_clusters=4)
+    mlp.router.activation_k = 2.0
+    assert MortarDecodeMLP(mlp, iter_idx=1.0)(X) is native.TAKEN
+    args = native.calls[-1][1]
+    assert type(args[-1]) is int and all(type(v) is int for v in args[-3])
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    mlp.router._native_route(X, 1.0, False)
+    args = native.calls[-1][1]
+    assert type(args[6]) is int and all(type(v) is int for v in args[4])
