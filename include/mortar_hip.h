@@ -75,7 +75,9 @@ typedef struct {
                               multiply +-2 / 0 blocks and scale the fp32 sums once, as the reference's decode kernel
                               does (fused_decode_step.py:1441-1443), instead of scaling every block's weights.
                               0: per-block scales (always valid, also for a uniform matrix). */
-    int32_t reserved_;
+    int32_t one_scale;     /* 1, with uniform_scale == 0: every block has the same scale, but its value is known on the
+                              device only (sdup[0], written by mortar_requantize in modes 0 / 2 with no host wait): the
+                              products run in the same form and read it there.  0 otherwise. */
 } mortar_bcsr_t;
 
 const char *mortar_last_error(void);
@@ -486,8 +488,9 @@ int mortar_rmsnorm_bf16(const uint16_t *x, int64_t M, int32_t d, int64_t ldx, co
  *              stk_dds operator states its restriction: the runtime multiplies ternary blocks only, and data that the
  *              reference's stk_dds would multiply as arbitrary bf16 values is reported instead of silently quantised.
  *   workspace  device, mortar_requantize_workspace_bytes() bytes, 8-byte aligned; needed for scale_mode 0 only
- * mortar_bcsr_t.uniform_scale is host state: after modes 0 / 2 the caller may set it to bf16(s) to select the
- * scale-after-sum kernels, or leave it 0 (per-block kernels, always valid). */
+ * mortar_bcsr_t.uniform_scale and one_scale are host state: after modes 0 / 2 the caller may set uniform_scale to bf16(s), or,
+ * without waiting for the scale, one_scale to 1, to select the scale-after-sum kernels, or leave both 0 (per-block kernels,
+ * always valid); after modes 1 / 3 both have to be 0. */
 int64_t mortar_requantize_workspace_bytes(void);
 int mortar_requantize(const mortar_bcsr_t *W, const void *values, int32_t values_f32, const int32_t *pos,
                       const int32_t *src_block, int32_t transpose, int32_t scale_mode, float threshold,

@@ -20,7 +20,7 @@ class BcsrStruct(C.Structure):
     _fields_ = [("codes", c_vp), ("sdup", c_vp), ("col", c_vp), ("row_ptr", c_vp), ("row_desc", c_vp),
                 ("codes_o", c_vp), ("sd_o", c_vp), ("col_o", c_vp), ("codes4_o", c_vp),
                 ("Rb", c_i32), ("Cb", c_i32), ("nnz", c_i32),
-                ("seg_cb", c_i32), ("uniform_scale", c_f32), ("reserved_", c_i32)]
+                ("seg_cb", c_i32), ("uniform_scale", c_f32), ("one_scale", c_i32)]
 
 
 _SIGS = {

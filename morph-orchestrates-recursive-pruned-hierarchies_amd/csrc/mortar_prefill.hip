@@ -55,6 +55,7 @@ void fill(SpmmParams &p, const mortar_bcsr_t *W, const int32_t *sched, const uin
     p.x = x; p.ldx = ldx; p.M = (int)M; p.y = y; p.ldy = ldy;
     p.n_clusters = 1; p.cluster_size = 1 << 30;
     p.uscale = 0.5f * W->uniform_scale;
+    if (W->uniform_scale == 0.f && W->one_scale && W->sdup) { p.uscale = 1.f; p.scale_dev = W->sdup; }
 }
 
 // Token tile of the resident prefill kernel for a matrix with Cb block-columns (0 = does not fit).
@@ -162,7 +163,7 @@ int dispatch_prefill(int kind, SpmmParams &p, hipStream_t st) {
 // kind: 0 spmm, 1 gate_up + SwiGLU, 2 routed gate_up + SwiGLU, 3 spmm with an input mask.
 // Prefill-sized launches read the 4-bit code stream when the matrix carries one (cheaper unpack: one conversion
 // per register instead of shift + mask); decode-sized launches always stream the 2-bit codes (half the bytes).
-// A matrix with one scale (uniform_scale != 0) runs the kernels that multiply +-2 / 0 blocks and scale the
+// A matrix with one scale (uniform_scale != 0, or one_scale) runs the kernels that multiply +-2 / 0 blocks and scale the
 // accumulators once (decode-sized launches always, prefill-sized ones through the 4-bit stream).
 int dispatch(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
     // products over several K segments have small-tile forms beyond the decode sizes as well (the launcher returns -1
@@ -176,7 +177,7 @@ int dispatch(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
         if (p.uscale != 0.f) return dispatch_prefill<CODE_4BIT | CODE_UNIFORM>(kind, p, st);
         return dispatch_prefill<CODE_4BIT>(kind, p, st);
     }
-    p.uscale = 0.f;      // per-block path: the 2-bit prefill kernels multiply every block by its own pattern
+    p.uscale = 0.f; p.scale_dev = nullptr;      // per-block path: the 2-bit prefill kernels multiply every block by its own pattern
     return dispatch_prefill<CODE_2BIT>(kind, p, st);
 }
 
@@ -214,7 +215,7 @@ int mortar_spmm_codes_f32(const mortar_bcsr_t *W, const int32_t *sched, const ui
     fill(p, W, sched, x, M, ldx, nullptr, ldy);
     p.n_units = W->Rb;
     p.y32 = y32;
-    p.uscale = 0.5f;                       // the kernels multiply the blocks as +-2 / 0
+    p.uscale = 0.5f; p.scale_dev = nullptr;      // the kernels multiply the blocks as +-2 / 0
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (M <= MORTAR_SMALLM_MAX) {
         rc = mortar_smallm_launch(0, p, nullptr, 1, st);
@@ -425,9 +426,9 @@ extern "C" int mortar_stack_prepare(int32_t swiglu, int32_t n_layers, const mort
         if (W[l].Rb != W[0].Rb || W[l].Cb != W[0].Cb || W[l].seg_cb != W[0].seg_cb)
             return mortar_fail(MORTAR_ERR_ARG, "stack_prepare: layer %d differs in shape from layer 0", l);
         if (swiglu && (W[l].Rb & 1)) return mortar_fail(MORTAR_ERR_ARG, "stack_prepare: odd number of block-rows");
-        if ((W[l].uniform_scale != 0.f) != (W[0].uniform_scale != 0.f))
+        if ((W[l].uniform_scale != 0.f || W[l].one_scale) != (W[0].uniform_scale != 0.f || W[0].one_scale))
             return mortar_fail(MORTAR_ERR_ARG, "stack_prepare: layer %d and layer 0 differ in having a uniform scale "
-                               "(set uniform_scale = 0 on all layers to run them together)", l);
+                               "(set uniform_scale = 0 and one_scale = 0 on all layers to run them together)", l);
         const int64_t out_cols = swiglu ? (int64_t)W[l].Rb * 8 : (int64_t)W[l].Rb * 16;
         int rc = check_common(&W[l], x[l], M, ldx, y[l], ldy, out_cols);
         if (rc) return rc;

@@ -36,7 +36,7 @@ struct SpmmParams {
     int xcd_map;              // 1: workgroup ids are renumbered per XCD (grid padded to a multiple of 8)
     int norm;                 // 1: rows of x are RMS-normalised while they are staged (single-segment tiles only)
     float norm_eps;
-    float uscale;             // CODE_UNIFORM kernels: half the matrix's (bf16-rounded) scale
+    float uscale;             // CODE_UNIFORM kernels: half the matrix's (bf16-rounded) scale (any value but 0 with scale_dev)
     float *y32;               // plain products: unrounded fp32 output [M, ldy] in place of the bf16 store, or null
     const uint16_t *norm_w;   // bf16 [in_features] weight of that norm, or null for none
     // hyper-connection POST write in place of the plain store (small tiles, plain products): out[t, i, :] =
@@ -52,7 +52,8 @@ struct SpmmParams {
     // of one (token tile, block-column) are 1 KB of contiguous memory: gate_up's stores of a 16 x 16 result tile are 512
     // contiguous bytes, and `down` stages a K segment of its token tile as one contiguous run, asynchronously, straight
     // into LDS.  y_tiled: the SwiGLU epilogue stores so; x_tiled: the 32-token prefill tiles are staged from it.
-    int x_tiled, y_tiled, pad0_, pad1_;
+    int x_tiled, y_tiled;
+    const uint32_t *scale_dev;   // CODE_UNIFORM kernels: the scale's pattern in device memory (mortar_bcsr_t.one_scale), or null
 };
 
 // Device-side view of the launch parameters: the pointers carry the global address space in their type, so
@@ -71,6 +72,8 @@ struct SpmmView {
     int64_t ldx, ldy;
     int n_units, Cb, M, n_clusters, cluster_size, n_mtiles, n_split, seg_cb, nseg, Rb, xcd_map, norm;
     float norm_eps, uscale;
+    uint32_t scale_pat;                               // pattern behind SpmmParams::scale_dev, 0 without (mortar_resolve_scale)
+    bool scale_on_dev;
     const MORTAR_GLOBAL u32x4_t *norm_w;
     const MORTAR_GLOBAL char *hc_h, *hc_term;
     MORTAR_GLOBAL char *hc_out;
@@ -102,6 +105,8 @@ __device__ __forceinline__ SpmmView mortar_view(const SpmmParams &q) {
     v.hc_out = (MORTAR_GLOBAL char *)q.hc_out; v.hc_res = (const MORTAR_GLOBAL float *)q.hc_res;
     v.hc_post = (const MORTAR_GLOBAL float *)q.hc_post; v.hc_n = q.hc_n; v.hc_f32 = q.hc_f32;
     v.x_tiled = q.x_tiled; v.y_tiled = q.y_tiled;
+    v.scale_on_dev = q.scale_dev != nullptr;
+    v.scale_pat = v.scale_on_dev ? *(const MORTAR_GLOBAL uint32_t *)q.scale_dev : 0u;
     return v;
 }
 
@@ -109,6 +114,17 @@ __device__ __forceinline__ SpmmView mortar_view(const SpmmParams &q) {
 // whole matrix (the reference's per-tensor mortar_scale): the blocks are multiplied as +-2 / 0 and the accumulators
 // are scaled once in the epilogue, which saves the packed multiplies and the scale broadcast of every pair.
 constexpr int CODE_2BIT = 0, CODE_4BIT = 1, CODE_UNIFORM = 2;
+
+// Half the scale from its pattern in device memory, for the CODE_UNIFORM kernels of a matrix whose scale the host does not
+// know.  The pattern is requested with the parameters and taken up here, behind the barrier that ends the staging: a load
+// still in flight in the product loop would make its counted waits full ones.  (Trainable matrices: five of the ten vector
+// instructions of a block pair fall away; the training step of 4096 tokens at 2048 x 5632 went 482 -> 462 us.)
+template <int CODE>
+__device__ __forceinline__ void mortar_resolve_scale(SpmmView &p) {
+    if (!(CODE & CODE_UNIFORM) || !p.scale_on_dev) return;
+    const uint32_t pat = (uint32_t)__builtin_amdgcn_readfirstlane((int)p.scale_pat) & 0xffffu;
+    p.uscale = pat ? 0.5f * bf16_to_f32(pat + 0x0400u) : 0.f;      // the pattern is one fp16 exponent step below the bf16 scale
+}
 
 constexpr int MORTAR_SMALLM_MAX = 64;    // rows up to which the small-tile (decode) instantiations are used
 constexpr int MORTAR_PARTSPLIT_MAX = 128; // rows up to which a plain product over several K segments runs 8-token tiles of all K
@@ -482,7 +498,7 @@ template <int MT, int NACC, bool ROUTED, int WAVES, bool TABLE, int CODE, bool T
 __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmParams p0, const SpmmParams *table) {
     constexpr int MSUB = (MT + 15) / 16;
     constexpr bool XT = TL && NACC == 1, YT = TL && NACC == 2;
-    const SpmmView p = mortar_view(TABLE ? mortar_table_entry(table, blockIdx.y) : p0);
+    SpmmView p = mortar_view(TABLE ? mortar_table_entry(table, blockIdx.y) : p0);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint4 *lx = reinterpret_cast<uint4 *>(smem);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -513,6 +529,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
     if (NACC == 2 && p.norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(next_unit + 4));      // gate_up may carry the norm
     else mortar_stage_tile<MT, WAVES, false, XT>(p, lx, m0, 0, p.Cb, tid);
     __syncthreads();
+    mortar_resolve_scale<CODE>(p);
 
     while (pos < u_end) {
         uint32_t drawn = 0;
@@ -584,7 +601,7 @@ template <int MT, int NACC, bool MASKED, int WAVES, int UPW, bool TABLE, int COD
 __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const SpmmParams p0, const SpmmParams *table) {
     constexpr int MSUB = (MT + 15) / 16, NP = UPW * NACC;
     constexpr bool XT = TL && NACC == 1, YT = TL && NACC == 2;
-    const SpmmView p = mortar_view(TABLE ? mortar_table_entry(table, blockIdx.y) : p0);
+    SpmmView p = mortar_view(TABLE ? mortar_table_entry(table, blockIdx.y) : p0);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint4 *lx = reinterpret_cast<uint4 *>(smem);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -649,6 +666,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
         if (sg > 0) __syncthreads();
         mortar_stage_tile<MT, WAVES, MASKED, XT>(p, lx, m0, c0, ncb, tid);
         __syncthreads();
+        if (sg == 0) mortar_resolve_scale<CODE>(p);
         if (!BATCH_AHEAD) {
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
@@ -705,7 +723,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
 template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE>
 __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const SpmmParams p0) {
     constexpr int MSUB = (MT + 15) / 16, WAVES = PW * UW;
-    const SpmmView p = mortar_view(p0);
+    SpmmView p = mortar_view(p0);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint4 *lx = reinterpret_cast<uint4 *>(smem);
     f32x4_t *red = reinterpret_cast<f32x4_t *>(smem + tile_bytes(MT, p.Cb));   // [WAVES][NACC][MSUB][64]
@@ -759,6 +777,7 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
     if (NACC == 2 && !MASKED && p.norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(red));
     else mortar_stage_tile<MT, WAVES, MASKED>(p, lx, m0, 0, p.Cb, tid);
     __syncthreads();
+    mortar_resolve_scale<CODE>(p);
     bool idle = skip;
     if (GATE_SKIP && valid && has_gates && p.cluster_size % 16 == 0) idle = __ballot(gsk != 0.f) == 0ull;      // NaN and negative gates multiply like any other
 

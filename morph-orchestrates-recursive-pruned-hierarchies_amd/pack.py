@@ -260,6 +260,7 @@ class MortarPack:
         _lib.check(_lib.lib().mortar_uniform_scale_host(_vp(sdup), self.nnz, C.byref(us)), "mortar_uniform_scale_host")
         self.scale_after_sum = bool(scale_after_sum)
         self.uniform_scale = float(us.value) if scale_after_sum else 0.0
+        self.one_scale = 0      # 1: one scale for all blocks, whose value only the device knows (requantize(sync=False))
         dev = self.device
         self.codes = torch.from_numpy(codes.view(np.int32)).to(dev)
         self.sdup = torch.from_numpy(sdup.view(np.int32)).to(dev)
@@ -311,7 +312,7 @@ class MortarPack:
                                self.row_ptr.data_ptr(), self.row_desc.data_ptr(), self.codes_o.data_ptr(),
                                self.sd_o.data_ptr(), self.col_o.data_ptr(),
                                self.codes4_o.data_ptr() if self.codes4_o is not None else None,
-                               self.Rb, self.Cb, self.nnz, self.seg_cb, self.uniform_scale, 0)
+                               self.Rb, self.Cb, self.nnz, self.seg_cb, self.uniform_scale, self.one_scale)
 
     def decode_view(self, rows: int) -> "MortarPack | None":
         """A second stream of this matrix for calls of up to 4 rows: K segments as wide as a 4-token tile allows (one
@@ -352,9 +353,9 @@ class MortarPack:
         block (``per_block``), or the given ``scale`` (fp32 [1] or [nnz], indexed like ``values``); code =
         sign(w/s) * (|w/s| > threshold).  A pack from ``transposed()`` reads the blocks of the original matrix
         (its ``src_block`` map) and pass ``transpose=True``.  Returns the scale tensor (fp32 [1] or [nnz], in this
-        pack's block order).  ``sync=True`` waits, raises if a scale left the representable window, and selects the
-        scale-after-sum kernels for a one-scale matrix; ``sync=False`` only enqueues (per-block kernels) and lets the
-        device status word accumulate: ``poll_status()`` / ``raise_status()`` report it later.
+        pack's block order).  A one-scale matrix (no ``per_block``, no per-block ``scale``) runs the scale-after-sum kernels.
+        ``sync=True`` waits and raises if a scale left the representable window; ``sync=False`` only enqueues (the kernels
+        read the scale on the device) and lets the device status word accumulate: ``poll_status()`` / ``raise_status()`` report it later.
         ``ternary_tol`` > 0 (with a given ``scale``): values that are neither 0 nor +-scale within that relative bound
         are reported as an error (the values are expected to be ternary already)."""
         if values.device != self.device or values.dtype not in (torch.bfloat16, torch.float32):
@@ -395,9 +396,10 @@ class MortarPack:
                 us = float(out.to(torch.bfloat16).float().item())
         elif ternary_tol:
             self._post_status()
-        if us != self.uniform_scale:
-            self.uniform_scale = us
-            self.struct.uniform_scale = us
+        one = int(not sync and mode in (0, 2) and self.scale_after_sum)
+        if us != self.uniform_scale or one != self.one_scale:
+            self.uniform_scale, self.one_scale = us, one
+            self.struct.uniform_scale, self.struct.one_scale = us, one
         return out
 
     # status of asynchronous re-packs: the device words are copied to pinned host memory behind every call; reading them

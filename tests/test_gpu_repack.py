@@ -596,3 +596,27 @@ def test_layer_carved_at_blocking_128_runs_through_the_recut_pack(dev, packed):
     if not packed:
         with pytest.raises(RuntimeError, match="blocking 128"):
             lin(to_dev(x, dev).requires_grad_(True))
+
+
+@pytest.mark.parametrize("M", [1, 13, 40, 70, 300, 545])
+@pytest.mark.parametrize("out_b,in_b", [(12, 48), (20, 128), (24, 160)])          # 64- and 32-token tiles of all K, several K segments
+def test_one_scale_known_on_the_device_only(dev, M, out_b, in_b):
+    """The asynchronous re-pack runs the scale-after-sum kernels with the scale read on the device: the bits of the products are
+    those of the pack that knows it on the host, for a positive and a negative scale, W and W^T, and gate_up + SwiGLU."""
+    m = synth.synth_matrix(16 * out_b, 16 * in_b, 0.25, seed=31)
+    nnz = m["col_idx"].size
+    vt = _values(nnz, 32, torch.bfloat16)[0].to(dev)
+    A, H = (MortarPack(None, None, m["col_idx"], m["offsets"], 16 * out_b, 16 * in_b, dev) for _ in range(2))
+    x = to_dev(synth.synth_x(M, 16 * in_b, 33), dev)
+    dy = to_dev(synth.synth_x(M, 16 * out_b, 34), dev)
+    for scale in (None, torch.tensor([-0.037])):
+        s = A.requantize(vt, scale=scale, sync=False)
+        H.requantize(vt, scale=scale)
+        A.transposed().requantize(vt, scale=s, transpose=True, sync=False)
+        H.transposed().requantize(vt, scale=s, transpose=True)
+        assert (A.one_scale, A.uniform_scale, H.one_scale) == (1, 0.0, 0) and H.uniform_scale != 0
+        assert torch.equal(ops.spmm(x, A), ops.spmm(x, H)) and torch.equal(ops.gateup_swiglu(x, A), ops.gateup_swiglu(x, H))
+        assert torch.equal(ops.spmm(dy, A.transposed()), ops.spmm(dy, H.transposed()))
+    A.requantize(vt, per_block=True, sync=False)
+    H.requantize(vt, per_block=True)
+    assert A.one_scale == 0 and torch.equal(ops.spmm(x, A), ops.spmm(x, H))
