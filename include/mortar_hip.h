@@ -497,6 +497,21 @@ int mortar_requantize(const mortar_bcsr_t *W, const void *values, int32_t values
                       const float *scale_in, float *scale_out, int32_t *status, int32_t flags, float ternary_tol,
                       void *workspace, void *stream);
 
+/* The re-pack of up to two matrices and of their transposes in two launches: what mortar_requantize does for each in mode 0 (flags 1),
+ * the transpose with the scale of its matrix.  Wt NULL leaves a transpose out; scale_out / status / status_t may be NULL.  The
+ * workspaces of the matrices are different buffers. */
+typedef struct {
+    const mortar_bcsr_t *W, *Wt;
+    const int32_t *pos, *pos_t, *src_t;   /* octet positions of W and Wt; block j of Wt is block src_t[j] of W, transposed */
+    const void *values;                   /* [nnz, 16, 16] of W, bf16 or fp32, 16-byte aligned */
+    float *scale_out;
+    int32_t *status, *status_t;
+    void *workspace;
+    int32_t values_f32;
+    float threshold;
+} mortar_repack_t;
+int mortar_requantize_pairs(const mortar_repack_t *m, int32_t n, void *stream);
+
 /* Makes a result unusable when a re-pack reported an error: if status[0] | status[1] != 0 (the words of
  * mortar_requantize, read on the device, no host synchronisation) every 4 bytes of out[0..bytes) become 0x7FC07FC0,
  * NaN both as bf16 pairs and as fp32; otherwise out is not touched.  The stk_dds operator enqueues it behind its

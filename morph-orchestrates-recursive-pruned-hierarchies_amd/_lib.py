@@ -23,6 +23,12 @@ class BcsrStruct(C.Structure):
                 ("seg_cb", c_i32), ("uniform_scale", c_f32), ("one_scale", c_i32)]
 
 
+class RepackStruct(C.Structure):
+    """mortar_repack_t"""
+    _fields_ = [("W", c_vp), ("Wt", c_vp), ("pos", c_vp), ("pos_t", c_vp), ("src_t", c_vp), ("values", c_vp), ("scale_out", c_vp),
+                ("status", c_vp), ("status_t", c_vp), ("workspace", c_vp), ("values_f32", c_i32), ("threshold", c_f32)]
+
+
 _SIGS = {
     "mortar_last_error": (C.c_char_p, []),
     "mortar_abi_version": (C.c_int, []),
@@ -36,6 +42,7 @@ _SIGS = {
     "mortar_requantize_workspace_bytes": (c_i64, []),
     "mortar_requantize": (C.c_int, [c_vp, c_vp, c_i32, c_vp, c_vp, c_i32, c_i32, c_f32, c_vp, c_vp, c_vp, c_i32, c_f32,
                                   c_vp, c_vp]),
+    "mortar_requantize_pairs": (C.c_int, [c_vp, c_i32, c_vp]),
     "mortar_poison_on_status": (C.c_int, [c_vp, c_i64, c_vp, c_vp]),
     "mortar_swiglu_bf16": (C.c_int, [c_vp, c_i64, c_i64, c_i32, c_vp, c_i64, c_vp]),
     "mortar_swiglu_backward_bf16": (C.c_int, [c_vp, c_i64, c_vp, c_i64, c_i64, c_i32, c_vp, c_i64, c_vp]),

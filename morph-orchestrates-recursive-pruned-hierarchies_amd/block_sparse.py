@@ -192,16 +192,21 @@ class CMSBlockLinear(nn.Module):
                 self._pack = MortarPack(pack_ternary_codes(q), scale, self.mortar_column_indices, self.mortar_offsets,
                                         self.out_features, self.in_features, d.device)
             return self._pack
-        if self._pack is None:
-            self._pack = MortarPack(None, None, self.mortar_column_indices, self.mortar_offsets, self.out_features,
-                                    self.in_features, d.device)
-            self._pack_key = None
-            self._pack_gen, self._pack_t_gen = 0, -1
+        self._qat_pack()
         key = (d.data_ptr(), d._version)
         if self._pack_key != key:
             self._pack_scale = self._pack.requantize(self._values(), threshold=self._values_threshold, sync=False)
             self._pack_key = key
             self._pack_gen += 1
+        return self._pack
+
+    def _qat_pack(self) -> MortarPack:
+        """The pack of a layer in values-ternary QAT on the GPU, its values as the last re-pack left them."""
+        if self._pack is None:
+            self._pack = MortarPack(None, None, self.mortar_column_indices, self.mortar_offsets, self.out_features,
+                                    self.in_features, self.mortar_data.device)
+            self._pack_key = None
+            self._pack_gen, self._pack_t_gen = 0, -1
         return self._pack
 
     def _mortar_pack_recut(self) -> MortarPack:
@@ -245,6 +250,17 @@ class CMSBlockLinear(nn.Module):
         (address, version) key alone would miss them; every training forward therefore calls this first (the re-encode
         is two small launches and no synchronisation)."""
         self._pack_key = None
+
+    @staticmethod
+    def repack_for_step(layers: list) -> None:
+        """Re-encodes the values of up to two QAT layers (layer, whether its W^T is needed too) for a training step, in two
+        launches; mortar_pack() and mortar_pack_t() then find them fresh until the values change again."""
+        jobs = [(m._qat_pack(), m._values(), m._values_threshold, with_t) for m, with_t in layers]
+        for (m, with_t), scale in zip(layers, MortarPack.requantize_pairs(jobs)):
+            m._pack_scale, m._pack_key = scale, (m.mortar_data.data_ptr(), m.mortar_data._version)
+            m._pack_gen += 1
+            if with_t:
+                m._pack_t_gen = m._pack_gen
 
     def mortar_pack_t(self) -> MortarPack:
         """The pack of W^T for the dX product (QAT layers on the GPU), refreshed like ``mortar_pack``."""

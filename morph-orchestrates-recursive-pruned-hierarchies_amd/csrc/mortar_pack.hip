@@ -22,7 +22,16 @@ __device__ __forceinline__ double wave_sum(double x) {
 
 // sum |w| over all values -> partial[blockIdx] (fixed order: the result does not depend on timing).  n is a multiple
 // of 256 (whole blocks) and the array is 16-byte aligned, so every thread reads 16-byte pieces.
-__global__ __launch_bounds__(256) void abs_sum_kernel(const void *values, int64_t n, int f32, double *partial) {
+struct AbsSumArgs {
+    const void *values;
+    double *partial;
+    int64_t n;
+    int f32;
+};
+constexpr int MAX_JOBS = 4;
+struct AbsSumJobs { AbsSumArgs job[MAX_JOBS]; };
+
+__device__ __forceinline__ void abs_sum(const void *values, int64_t n, int f32, double *partial) {
     __shared__ double wsum[4];
     double s = 0.0;
     const int per = f32 ? 4 : 8;                                     // values per 16-byte piece
@@ -54,6 +63,10 @@ __global__ __launch_bounds__(256) void abs_sum_kernel(const void *values, int64_
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) partial[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+}
+__global__ __launch_bounds__(256) void abs_sum_kernel(AbsSumJobs a) {
+    const AbsSumArgs &j = a.job[blockIdx.y];
+    abs_sum(j.values, j.n, j.f32, j.partial);
 }
 
 __global__ void clear_status_kernel(int32_t *status) {
@@ -89,17 +102,16 @@ __device__ __forceinline__ bool code_cut(float s, float threshold, int lane, flo
 // One wave per block with the quotients of four values per lane was bound by its vector instructions (gate_up and down at
 // 2048 x 5632 and 25 %, both orientations: 12.5 us on average): a row is encoded by one comparison per value, and a transposed
 // block is turned as 16 x 16 two-bit codes in registers, four exchanges between the 16 lanes of a block (now 6.6 us).
-template <bool F32>
-__global__ __launch_bounds__(256) void requant_kernel(RequantArgs a) {
+__device__ __forceinline__ void requant(const RequantArgs &a, int block) {
     const int lane = threadIdx.x & 63, n = lane & 15;
-    const int j0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 4, j = j0 + (lane >> 4);
+    const int j0 = (block * 4 + (threadIdx.x >> 6)) * 4, j = j0 + (lane >> 4);
     if (j0 >= a.nnz) return;
     const bool on = j < a.nnz;
     const int jc = on ? j : a.nnz - 1;
     const int src = a.src_block ? a.src_block[jc] : jc;
     const int P = a.pos[jc];
     float w[16];
-    if (F32) {
+    if (a.f32) {
         const float4 *v = reinterpret_cast<const float4 *>(a.values) + (int64_t)src * 64 + n * 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -208,6 +220,62 @@ __global__ __launch_bounds__(256) void requant_kernel(RequantArgs a) {
     }
 }
 
+// Several matrices in one launch (a training step re-packs two and their transposes, launches of 4 to 11 us each that the latency of a
+// few dependent loads bounds: 2 + 4 launches 36 us, one of each kind 17 us at 2048 x 5632 and 25 %): workgroups [first[i], first[i + 1]) take the blocks of job i.
+struct RequantJobs {
+    RequantArgs job[MAX_JOBS];
+    int first[MAX_JOBS + 1];
+};
+__global__ __launch_bounds__(256) void requant_kernel(RequantJobs a) {
+    int i = 0;
+#pragma unroll
+    for (int k = 1; k < MAX_JOBS; ++k) i += (int)blockIdx.x >= a.first[k];
+    requant(a.job[i], (int)blockIdx.x - a.first[i]);
+}
+
+// Fills one job from a matrix; the scale comes from `partial` (mode 0) until the caller says otherwise.
+RequantArgs requant_args(const mortar_bcsr_t *W, const void *values, int32_t f32, const int32_t *pos, const int32_t *src_block,
+                         int32_t transpose, float threshold, int32_t *status, const void *partial) {
+    RequantArgs a{};
+    a.codes = const_cast<uint32_t *>(W->codes);
+    a.sdup = const_cast<uint32_t *>(W->sdup);
+    a.codes_o = const_cast<uint32_t *>(W->codes_o);
+    a.sd_o = const_cast<uint32_t *>(W->sd_o);
+    a.codes4_o = const_cast<uint32_t *>(W->codes4_o);
+    a.values = values;
+    a.pos = pos;
+    a.src_block = src_block;
+    a.status = status;
+    a.partial = static_cast<const double *>(partial);
+    a.nnz = W->nnz;
+    a.f32 = f32;
+    a.transpose = transpose;
+    a.threshold = threshold;
+    return a;
+}
+
+// Launches the |w| sums of `ns` value arrays and the re-pack of `n` matrices.
+int launch_requant(const AbsSumJobs &sums, int ns, RequantJobs &jobs, int n, hipStream_t st) {
+    if (ns > 0) hipLaunchKernelGGL(abs_sum_kernel, dim3(PARTIALS, ns), dim3(256), 0, st, sums);
+    jobs.first[0] = 0;
+    for (int i = 0; i < MAX_JOBS; ++i) {
+        if (i < n) jobs.first[i + 1] = jobs.first[i] + (jobs.job[i].nnz + 15) / 16;
+        else jobs.first[i + 1] = INT32_MAX;
+    }
+    hipLaunchKernelGGL(requant_kernel, dim3(jobs.first[n]), dim3(256), 0, st, jobs);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "requantize: %s", hipGetErrorString(e));
+    return MORTAR_OK;
+}
+
+int check_requant(const mortar_bcsr_t *W, const void *values, const int32_t *pos, float threshold) {
+    if (!W || !values || !pos) return mortar_fail(MORTAR_ERR_ARG, "requantize: null pointer");
+    if (!W->codes || !W->sdup || !W->codes_o || !W->sd_o || W->nnz <= 0) return mortar_fail(MORTAR_ERR_ARG, "requantize: incomplete matrix");
+    if (!(threshold >= 0.f)) return mortar_fail(MORTAR_ERR_ARG, "requantize: threshold must be >= 0");
+    if (reinterpret_cast<uintptr_t>(values) & 15) return mortar_fail(MORTAR_ERR_ARG, "requantize: values must be 16-byte aligned");
+    return MORTAR_OK;
+}
+
 // Overwrites out[0..ndw) with quiet-NaN patterns (0x7FC07FC0: NaN as two bf16 and as one fp32) when a status word is set.
 // Every thread reads the two words; the usual case (both 0) ends after that one load.
 __global__ __launch_bounds__(256) void poison_kernel(uint32_t *out, int64_t ndw, const int32_t *status) {
@@ -237,45 +305,43 @@ extern "C" int mortar_requantize(const mortar_bcsr_t *W, const void *values, int
                                  const int32_t *src_block, int32_t transpose, int32_t scale_mode, float threshold,
                                  const float *scale_in, float *scale_out, int32_t *status, int32_t flags,
                                  float ternary_tol, void *workspace, void *stream) {
-    if (!W || !values || !pos) return mortar_fail(MORTAR_ERR_ARG, "requantize: null pointer");
-    if (!W->codes || !W->sdup || !W->codes_o || !W->sd_o || W->nnz <= 0)
-        return mortar_fail(MORTAR_ERR_ARG, "requantize: incomplete matrix");
+    const int rc = check_requant(W, values, pos, threshold);
+    if (rc) return rc;
     if (scale_mode < 0 || scale_mode > 3) return mortar_fail(MORTAR_ERR_ARG, "requantize: scale_mode %d not in 0..3", scale_mode);
     if (scale_mode >= 2 && !scale_in) return mortar_fail(MORTAR_ERR_ARG, "requantize: scale_mode %d needs scale_in", scale_mode);
     if (scale_mode == 0 && !workspace) return mortar_fail(MORTAR_ERR_ARG, "requantize: scale_mode 0 needs the workspace");
-    if (!(threshold >= 0.f)) return mortar_fail(MORTAR_ERR_ARG, "requantize: threshold must be >= 0");
     if (flags & ~1) return mortar_fail(MORTAR_ERR_ARG, "requantize: unknown flags 0x%x", flags);
     if (!(ternary_tol >= 0.f) || (ternary_tol > 0.f && (scale_mode < 2 || !status)))
         return mortar_fail(MORTAR_ERR_ARG, "requantize: ternary_tol needs a given scale (scale_mode 2 or 3) and a status word");
-    if (reinterpret_cast<uintptr_t>(values) & 15) return mortar_fail(MORTAR_ERR_ARG, "requantize: values must be 16-byte aligned");
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (status && !(flags & 1)) hipLaunchKernelGGL(clear_status_kernel, dim3(1), dim3(64), 0, st, status);
-    if (scale_mode == 0)
-        hipLaunchKernelGGL(abs_sum_kernel, dim3(PARTIALS), dim3(256), 0, st, values, (int64_t)W->nnz * 256, values_f32,
-                           static_cast<double *>(workspace));
-    RequantArgs a;
-    a.codes = const_cast<uint32_t *>(W->codes);
-    a.sdup = const_cast<uint32_t *>(W->sdup);
-    a.codes_o = const_cast<uint32_t *>(W->codes_o);
-    a.sd_o = const_cast<uint32_t *>(W->sd_o);
-    a.codes4_o = const_cast<uint32_t *>(W->codes4_o);
-    a.values = values;
-    a.pos = pos;
-    a.src_block = src_block;
+    AbsSumJobs sums{};
+    sums.job[0] = {values, static_cast<double *>(workspace), (int64_t)W->nnz * 256, values_f32};
+    RequantJobs jobs{};
+    RequantArgs &a = jobs.job[0] = requant_args(W, values, values_f32, pos, src_block, transpose, threshold, status, workspace);
     a.scale_in = scale_in;
     a.scale_out = scale_out;
-    a.status = status;
-    a.partial = static_cast<const double *>(workspace);
-    a.nnz = W->nnz;
-    a.f32 = values_f32;
-    a.transpose = transpose;
     a.mode = scale_mode;
-    a.threshold = threshold;
     a.ternary_tol = ternary_tol;
-    const dim3 grid((W->nnz + 15) / 16);
-    if (values_f32) hipLaunchKernelGGL(requant_kernel<true>, grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(requant_kernel<false>, grid, dim3(256), 0, st, a);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "requantize: %s", hipGetErrorString(e));
-    return MORTAR_OK;
+    return launch_requant(sums, scale_mode == 0, jobs, 1, st);
+}
+
+extern "C" int mortar_requantize_pairs(const mortar_repack_t *m, int32_t n, void *stream) {
+    if (!m || n < 1 || 2 * n > MAX_JOBS) return mortar_fail(MORTAR_ERR_ARG, "requantize_pairs: 1 to %d matrices", MAX_JOBS / 2);
+    AbsSumJobs sums{};
+    RequantJobs jobs{};
+    int nj = 0;
+    for (int i = 0; i < n; ++i) {
+        int rc = check_requant(m[i].W, m[i].values, m[i].pos, m[i].threshold);
+        if (rc == MORTAR_OK && m[i].Wt) rc = check_requant(m[i].Wt, m[i].values, m[i].pos_t, m[i].threshold);
+        if (rc) return rc;
+        if (!m[i].workspace || (m[i].Wt && (!m[i].src_t || m[i].Wt->nnz != m[i].W->nnz)))
+            return mortar_fail(MORTAR_ERR_ARG, "requantize_pairs: matrix %d: workspace missing, or W^T does not match W", i);
+        sums.job[i] = {m[i].values, static_cast<double *>(m[i].workspace), (int64_t)m[i].W->nnz * 256, m[i].values_f32};
+        jobs.job[nj] = requant_args(m[i].W, m[i].values, m[i].values_f32, m[i].pos, nullptr, 0, m[i].threshold, m[i].status, m[i].workspace);
+        jobs.job[nj++].scale_out = m[i].scale_out;
+        if (m[i].Wt)
+            jobs.job[nj++] = requant_args(m[i].Wt, m[i].values, m[i].values_f32, m[i].pos_t, m[i].src_t, 1, m[i].threshold, m[i].status_t, m[i].workspace);
+    }
+    return launch_requant(sums, n, jobs, nj, static_cast<hipStream_t>(stream));
 }

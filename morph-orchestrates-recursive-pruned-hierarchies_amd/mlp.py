@@ -66,7 +66,12 @@ class _SwiGLUMortarFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x: Tensor, data_gu: Tensor, data_dn: Tensor, mlp: "_SwiGLUMortar") -> Tensor:
         cg, cd = mlp.gate_up._cms, mlp.down._cms
-        cg.invalidate_pack(); cd.invalidate_pack()     # re-encode: .data writes do not advance the version counter
+        # re-encoded at every step (.data writes do not advance the version counter), with the W^T that the backward will need
+        need_x, need_gu = ctx.needs_input_grad[:2]
+        if cg._mortar_blocking == cd._mortar_blocking == 16 and data_gu.is_cuda and data_gu.device == data_dn.device:
+            cg.repack_for_step([(cg, need_x), (cd, need_x or need_gu)])
+        else:
+            cg.invalidate_pack(); cd.invalidate_pack()
         gu = ops.spmm(x, cg.mortar_pack())
         h = ops.swiglu(gu)
         y = ops.spmm(h, cd.mortar_pack())

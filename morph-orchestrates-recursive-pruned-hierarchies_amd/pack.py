@@ -358,16 +358,8 @@ class MortarPack:
         read the scale on the device) and lets the device status word accumulate: ``poll_status()`` / ``raise_status()`` report it later.
         ``ternary_tol`` > 0 (with a given ``scale``): values that are neither 0 nor +-scale within that relative bound
         are reported as an error (the values are expected to be ternary already)."""
-        if values.device != self.device or values.dtype not in (torch.bfloat16, torch.float32):
-            raise ValueError("requantize: values must be bf16 or fp32 on the pack's device")
-        if tuple(values.shape) != (self.nnz, BLK, BLK) or not values.is_contiguous():
-            raise ValueError(f"requantize: values must be contiguous [{self.nnz}, 16, 16], got {tuple(values.shape)}")
-        self._h_codes, self._h_sdup, self._dview = None, None, {}      # the host copy of the codes is stale from here on
+        self._before_repack(values)
         L = _lib.lib()
-        if self._pos is None:
-            self._pos = torch.from_numpy(octet_positions(self.h_offsets, self.Rb, self.Cb, self.seg_cb, self.h_col)).to(self.device)
-            self._ws = torch.empty(int(L.mortar_requantize_workspace_bytes()) // 8, dtype=torch.float64, device=self.device)
-            self._status = torch.zeros(2, dtype=torch.int32, device=self.device)
         if scale is not None:
             scale = scale.detach().to(device=self.device, dtype=torch.float32).reshape(-1).contiguous()
             if scale.numel() not in (1, self.nnz):
@@ -396,11 +388,50 @@ class MortarPack:
                 us = float(out.to(torch.bfloat16).float().item())
         elif ternary_tol:
             self._post_status()
-        one = int(not sync and mode in (0, 2) and self.scale_after_sum)
-        if us != self.uniform_scale or one != self.one_scale:
-            self.uniform_scale, self.one_scale = us, one
-            self.struct.uniform_scale, self.struct.one_scale = us, one
+        self._set_scale_form(us, int(not sync and mode in (0, 2) and self.scale_after_sum))
         return out
+
+    def _before_repack(self, values: torch.Tensor) -> None:
+        if values.device != self.device or values.dtype not in (torch.bfloat16, torch.float32):
+            raise ValueError("requantize: values must be bf16 or fp32 on the pack's device")
+        if tuple(values.shape) != (self.nnz, BLK, BLK) or not values.is_contiguous():
+            raise ValueError(f"requantize: values must be contiguous [{self.nnz}, 16, 16], got {tuple(values.shape)}")
+        self._h_codes, self._h_sdup, self._dview = None, None, {}      # the host copy of the codes is stale from here on
+        if self._pos is None:
+            self._pos = torch.from_numpy(octet_positions(self.h_offsets, self.Rb, self.Cb, self.seg_cb, self.h_col)).to(self.device)
+            self._ws = torch.empty(int(_lib.lib().mortar_requantize_workspace_bytes()) // 8, dtype=torch.float64, device=self.device)
+            self._status = torch.zeros(2, dtype=torch.int32, device=self.device)
+
+    def _set_scale_form(self, uniform: float, one: int) -> None:
+        if uniform != self.uniform_scale or one != self.one_scale:
+            self.uniform_scale, self.one_scale = uniform, one
+            self.struct.uniform_scale, self.struct.one_scale = uniform, one
+
+    @staticmethod
+    def requantize_pairs(jobs: list) -> list:
+        """``requantize(values, threshold, sync=False)`` of one or two packs and, where asked for, of their transposes with the
+        same scale, in two launches.  jobs: (pack, values, threshold, with transpose) each; returns the scale tensors."""
+        arr = (_lib.RepackStruct * len(jobs))()
+        scales = []
+        for r, (W, values, threshold, with_t) in zip(arr, jobs):
+            W._before_repack(values)
+            s = torch.empty(1, dtype=torch.float32, device=W.device)
+            r.W, r.pos, r.values, r.scale_out = C.addressof(W.struct), W._pos.data_ptr(), values.data_ptr(), s.data_ptr()
+            r.status, r.workspace = W._status.data_ptr(), W._ws.data_ptr()
+            r.values_f32, r.threshold = int(values.dtype == torch.float32), threshold
+            packs = [W]
+            if with_t:
+                T = W.transposed()
+                T._before_repack(values)
+                r.Wt, r.pos_t, r.src_t, r.status_t = C.addressof(T.struct), T._pos.data_ptr(), T.src_block.data_ptr(), T._status.data_ptr()
+                packs.append(T)
+            for p in packs:
+                p.scales_f32 = s
+                p._set_scale_form(0.0, int(p.scale_after_sum))
+            scales.append(s)
+        dev = jobs[0][0].device
+        _lib.check(_lib.lib().mortar_requantize_pairs(C.addressof(arr), len(jobs), torch.cuda.current_stream(dev).cuda_stream), "mortar_requantize_pairs")
+        return scales
 
     # status of asynchronous re-packs: the device words are copied to pinned host memory behind every call; reading them
     # costs no synchronisation once the copy has landed

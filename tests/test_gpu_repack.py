@@ -620,3 +620,33 @@ def test_one_scale_known_on_the_device_only(dev, M, out_b, in_b):
     A.requantize(vt, per_block=True, sync=False)
     H.requantize(vt, per_block=True)
     assert A.one_scale == 0 and torch.equal(ops.spmm(x, A), ops.spmm(x, H))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("with_t", [(False,), (True,), (False, True), (True, False), (True, True)])
+def test_requantize_pairs(dev, dtype, with_t):
+    """One to four matrices in one launch (block counts that are no multiple of a workgroup's sixteen): the arrays, the scales and the
+    status words of one requantize each."""
+    shapes = [(16 * 5, 16 * 11), (16 * 9, 16 * 170)]
+    packs, ref, jobs = [], [], []
+    for i, t in enumerate(with_t):
+        o, k = shapes[i]
+        m = synth.synth_matrix(o, k, 0.3, seed=51 + i)
+        v = _values(m["col_idx"].size, 53 + i, dtype)[0].to(dev)
+        A, B = (MortarPack(None, None, m["col_idx"], m["offsets"], o, k, dev) for _ in range(2))
+        s = B.requantize(v, threshold=0.4 + 0.2 * i, sync=False)
+        if t:
+            B.transposed().requantize(v, threshold=0.4 + 0.2 * i, scale=s, transpose=True, sync=False)
+        packs.append((A, B, t)); ref.append(s); jobs.append((A, v, 0.4 + 0.2 * i, t))
+    for got, want in zip(MortarPack.requantize_pairs(jobs), ref):
+        assert torch.equal(got, want)
+    for A, B, t in packs:
+        for P, Q in ((A, B), (A.transposed(), B.transposed())) if t else ((A, B),):
+            assert P.one_scale == Q.one_scale == 1 and P._status.tolist() == [0, 0]
+            for name in ARRAYS:
+                assert torch.equal(getattr(P, name), getattr(Q, name)), name
+    jobs[0][1].fill_(1e35)                               # mean|w| outside the window: reported, as by a single re-pack
+    MortarPack.requantize_pairs(jobs)
+    for P in (packs[0][0], packs[0][0].transposed()) if with_t[0] else (packs[0][0],):
+        with pytest.raises(ValueError, match="outside"):
+            P.raise_status()
