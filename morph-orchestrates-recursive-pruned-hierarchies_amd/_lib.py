@@ -101,8 +101,15 @@ _SIGS = {
 }
 
 class PackHandle(C.Structure):
-    """One packed matrix for the native call layer: its mortar_bcsr_t and the schedules built so far."""
-    _fields_ = [("w", c_vp), ("sched1", c_vp), ("sched2", c_vp)]
+    """One packed matrix for the native call layer: its mortar_bcsr_t, the schedules built so far and, once it has been re-packed,
+    what a re-pack needs beside the values."""
+    _fields_ = [("w", c_vp), ("sched1", c_vp), ("sched2", c_vp), ("pos", c_vp), ("src", c_vp), ("scale", c_vp), ("status", c_vp),
+                ("workspace", c_vp)]
+
+
+class TopologyHandle(C.Structure):
+    """One pack.BcsrTopology for the native call layer."""
+    _fields_ = [("row_ptr", c_vp), ("col", c_vp), ("seg_ptr", c_vp), ("src", c_vp), ("Rb", c_i32), ("Cb", c_i32), ("nnz", c_i64)]
 
 
 EXPORTS = tuple(_SIGS)

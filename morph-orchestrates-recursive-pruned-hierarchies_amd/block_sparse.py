@@ -262,6 +262,42 @@ class CMSBlockLinear(nn.Module):
             if with_t:
                 m._pack_t_gen = m._pack_gen
 
+    def step_pack(self, with_t: bool) -> MortarPack | None:
+        """The pack for a native training step that re-encodes the values into it (and into its transpose) itself; the state of the
+        layer is that behind ``repack_for_step``.  None where the step has to take the general path."""
+        d = self._parameters.get("mortar_data")
+        if (type(self) is not CMSBlockLinear or d is None or self._mortar_blocking != 16 or not self._values_ternary_mode
+                or "mortar_packed" in self._buffers or not d.is_cuda or d.dtype not in (torch.bfloat16, torch.float32)
+                or not d.is_contiguous() or d.shape[0] == 0):
+            return None
+        W = self._qat_pack()
+        if W.device != d.device or d.shape[0] != W.nnz:
+            return None
+        if W._pos is None:
+            W._before_repack(d.detach())
+        W.before_pair_repack(d, W._scale)
+        W.sched(1)
+        state = self.__dict__
+        if with_t:
+            T = W.transposed()
+            if T._pos is None:
+                T._before_repack(d.detach())
+            T.before_pair_repack(d, W._scale)
+            T.sched(1)
+        state["_pack_scale"], state["_pack_key"] = W._scale, (d.data_ptr(), d._version)
+        state["_pack_gen"] += 1
+        if with_t:
+            state["_pack_t_gen"] = state["_pack_gen"]
+        return W
+
+    def step_pack_fresh(self, with_t: bool) -> MortarPack | None:
+        """The pack that ``step_pack`` handed out, if the values have not changed since and nothing re-packed it otherwise."""
+        d = self._parameters.get("mortar_data")
+        W = self._pack
+        if W is None or d is None or self._pack_key != (d.data_ptr(), d._version) or (with_t and self._pack_t_gen != self._pack_gen):
+            return None
+        return W
+
     def mortar_pack_t(self) -> MortarPack:
         """The pack of W^T for the dX product (QAT layers on the GPU), refreshed like ``mortar_pack``."""
         if "mortar_packed" in self._buffers or not self.mortar_data.is_cuda:

@@ -15,18 +15,28 @@
 #include <c10/core/GradMode.h>
 #include <c10/core/InferenceMode.h>
 #include <c10/hip/HIPStream.h>
+#include <ATen/core/dispatch/Dispatcher.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../include/mortar_hip.h"
 
 namespace {
 
 // One packed matrix as the Python side hands it over (pack.MortarPack.handle): the struct of the C-ABI and the two
-// schedules, null until the Python side has built them.
+// schedules, null until the Python side has built them; then what a re-pack needs (null in a pack that has seen none).
 struct PackHandle {
     const mortar_bcsr_t *w;
     const int32_t *sched1, *sched2;
+    const int32_t *pos, *src;
+    float *scale;
+    int32_t *status;
+    void *workspace;
 };
 
 constexpr int DECODE_MAX_ROWS = 64;
@@ -350,6 +360,336 @@ PyObject *py_gemv_f32(PyObject *, PyObject *const *a, Py_ssize_t na) {
     return THPVariable_Wrap(std::move(y));
 }
 
+// ---- training step of the MLP ------------------------------------------------------------------------------------
+
+// Block values [nnz, 16, 16] of a matrix, bf16 or fp32.
+bool is_values(const at::Tensor &v, const mortar_bcsr_t *w, const at::Tensor &x) {
+    return v.device() == x.device() && (v.scalar_type() == at::kBFloat16 || v.scalar_type() == at::kFloat) && v.dim() == 3 && v.size(0) == w->nnz &&
+           v.size(1) == 16 && v.size(2) == 16 && v.is_contiguous() && aligned16(v.const_data_ptr());
+}
+
+bool repackable(const PackHandle *h) { return h->pos && h->status && h->workspace && h->sched1; }
+
+mortar_repack_t repack_of(const PackHandle *h, const PackHandle *t, const at::Tensor &v, double threshold) {
+    mortar_repack_t r{};
+    r.W = h->w; r.pos = h->pos; r.status = h->status; r.workspace = h->workspace; r.scale_out = h->scale;
+    if (t) { r.Wt = t->w; r.pos_t = t->pos; r.src_t = t->src; r.status_t = t->status; }
+    r.values = v.const_data_ptr();
+    r.values_f32 = v.scalar_type() == at::kFloat;
+    r.threshold = (float)threshold;
+    return r;
+}
+
+// train_forward(x, gate_up values, down values, gate_up, its W^T or 0, down, its W^T or 0, thresholds of the two) -> (y, gu, h): the
+// re-pack of both matrices and the transposes named, then gate_up, SwiGLU and down on the rows of x.  No autograd of its own.
+PyObject *py_train_forward(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 9) {
+        PyErr_SetString(PyExc_TypeError, "train_forward: 9 arguments");
+        return nullptr;
+    }
+    const at::Tensor *xt = tensor_of(a[0]), *vg = tensor_of(a[1]), *vd = tensor_of(a[2]);
+    const PackHandle *gu = handle_of(a[3]), *gut = handle_of(a[4]), *dn = handle_of(a[5]), *dnt = handle_of(a[6]);
+    if (PyErr_Occurred()) return nullptr;
+    const double tg = PyFloat_AsDouble(a[7]), td = PyFloat_AsDouble(a[8]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!xt || !vg || !vd || !gu || !dn || !repackable(gu) || !repackable(dn) || (gut && !(repackable(gut) && gut->src)) ||
+        (dnt && !(repackable(dnt) && dnt->src)))
+        Py_RETURN_NONE;
+    const at::Tensor &x = *xt;
+    const int64_t d = (int64_t)gu->w->Cb * 16, f2 = (int64_t)gu->w->Rb * 16, f = (int64_t)dn->w->Cb * 16, dy = (int64_t)dn->w->Rb * 16;
+    if (x.dim() != 2 || !is_rows(x, d) || f2 != 2 * f || !is_values(*vg, gu->w, x) || !is_values(*vd, dn->w, x)) Py_RETURN_NONE;
+    const int64_t M = x.size(0);
+    const c10::DeviceGuard guard(x.device());
+    void *st = stream_of(x);
+    const mortar_repack_t re[2] = {repack_of(gu, gut, *vg, tg), repack_of(dn, dnt, *vd, td)};
+    at::Tensor g = new_bf16(x, {M, f2}), h = new_bf16(x, {M, f}), y = new_bf16(x, {M, dy});
+    int rc = mortar_requantize_pairs(re, 2, st);
+    if (rc == MORTAR_OK) rc = mortar_spmm_bf16(gu->w, gu->sched1, u16(x), M, d, u16m(g), f2, st);
+    if (rc == MORTAR_OK) rc = mortar_swiglu_bf16(u16(g), f2, M, (int32_t)f, u16m(h), f, st);
+    if (rc == MORTAR_OK) rc = mortar_spmm_bf16(dn->w, dn->sched1, u16(h), M, f, u16m(y), dy, st);
+    if (rc) return raise_rc(rc, "mortar_train_forward");
+    return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(y)), THPVariable_Wrap(std::move(g)), THPVariable_Wrap(std::move(h)));
+}
+
+// A weight gradient's plan as the Python side hands it over: (address, workgroups, blocks per wave), or None / no need.
+struct SddPlan {
+    const int32_t *plan = nullptr;
+    int32_t n_wg = 0, nb = 0;
+};
+bool read_plan(PyObject *o, SddPlan &p) {
+    if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) < 3) return false;
+    p.plan = static_cast<const int32_t *>(PyLong_AsVoidPtr(PyTuple_GET_ITEM(o, 0)));
+    p.n_wg = (int32_t)PyLong_AsLong(PyTuple_GET_ITEM(o, 1));
+    p.nb = (int32_t)PyLong_AsLong(PyTuple_GET_ITEM(o, 2));
+    return !PyErr_Occurred() && p.plan;
+}
+
+// out[j] = a[:, rows of block j]^T b[:, columns of block j] on a topology of Rb x Cb block-rows and -columns.
+int run_sdd(const SddPlan &p, int32_t Rb, int32_t Cb, int64_t nnz, const at::Tensor &a, const at::Tensor &b, at::Tensor &out, void *st) {
+    const int64_t M = a.size(0), ws = mortar_sdd_workspace_bytes(p.n_wg, (int32_t)nnz, p.nb, M);
+    if (ws < 0) return (int)ws;
+    const at::Tensor acc = at::empty({ws}, a.options().dtype(at::kByte).requires_grad(false));
+    out = new_bf16(a, {nnz, 16, 16});
+    return mortar_sdd_bf16(p.plan, p.n_wg, p.nb, Rb, Cb, (int32_t)nnz, u16(a), a.stride(0), u16(b), b.stride(0), M, static_cast<float *>(acc.data_ptr()),
+                           u16m(out), st);
+}
+
+PyObject *wrap_or_none(at::Tensor &t) {
+    if (t.defined()) return THPVariable_Wrap(std::move(t));
+    Py_RETURN_NONE;
+}
+
+// train_backward(dy, x, gu, h, gate_up, its W^T or 0, down, its W^T or 0, plan of d(gate_up) or None, plan of d(down) or None) ->
+// (dx, d gate_up, d down): dx where gate_up's W^T is given, the weight gradients where their plans are; None elsewhere.
+PyObject *py_train_backward(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 10) {
+        PyErr_SetString(PyExc_TypeError, "train_backward: 10 arguments");
+        return nullptr;
+    }
+    const at::Tensor *t[4];
+    for (int i = 0; i < 4; ++i) t[i] = tensor_of(a[i]);
+    const PackHandle *gu = handle_of(a[4]), *gut = handle_of(a[5]), *dn = handle_of(a[6]), *dnt = handle_of(a[7]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!t[0] || !t[1] || !t[2] || !t[3] || !gu || !dn) Py_RETURN_NONE;
+    const at::Tensor &dy = *t[0], &x = *t[1], &g = *t[2], &h = *t[3];
+    const int64_t d = (int64_t)gu->w->Cb * 16, f2 = (int64_t)gu->w->Rb * 16, f = (int64_t)dn->w->Cb * 16, dd = (int64_t)dn->w->Rb * 16;
+    for (int i = 0; i < 4; ++i)
+        if (t[i]->dim() != 2 || !is_rows(*t[i], i == 0 ? dd : i == 1 ? d : i == 2 ? f2 : f) || t[i]->size(0) != x.size(0) || t[i]->device() != x.device())
+            Py_RETURN_NONE;
+    SddPlan pg, pd;
+    const bool need_gu = a[8] != Py_None, need_dn = a[9] != Py_None;
+    if ((need_gu && !read_plan(a[8], pg)) || (need_dn && !read_plan(a[9], pd))) {
+        if (PyErr_Occurred()) return nullptr;
+        Py_RETURN_NONE;
+    }
+    if ((gut && !gut->sched1) || ((gut || need_gu) && (!dnt || !dnt->sched1))) Py_RETURN_NONE;
+    const int64_t M = x.size(0);
+    const c10::DeviceGuard guard(x.device());
+    void *st = stream_of(x);
+    at::Tensor dx, dgu, ddn;
+    int rc = MORTAR_OK;
+    if (need_dn) rc = run_sdd(pd, dn->w->Rb, dn->w->Cb, dn->w->nnz, dy, h, ddn, st);
+    if (rc == MORTAR_OK && (gut || need_gu)) {
+        const at::Tensor dh = new_bf16(x, {M, f}), dg = new_bf16(x, {M, f2});
+        rc = mortar_spmm_bf16(dnt->w, dnt->sched1, u16(dy), M, dd, u16m(dh), f, st);
+        if (rc == MORTAR_OK) rc = mortar_swiglu_backward_bf16(u16(g), f2, u16(dh), f, M, (int32_t)f, u16m(dg), f2, st);
+        if (rc == MORTAR_OK && need_gu) rc = run_sdd(pg, gu->w->Rb, gu->w->Cb, gu->w->nnz, dg, x, dgu, st);
+        if (rc == MORTAR_OK && gut) {
+            dx = new_bf16(x, {M, d});
+            rc = mortar_spmm_bf16(gut->w, gut->sched1, u16(dg), M, f2, u16m(dx), d, st);
+        }
+    }
+    if (rc) return raise_rc(rc, "mortar_train_backward");
+    PyObject *r0 = wrap_or_none(dx), *r1 = wrap_or_none(dgu), *r2 = wrap_or_none(ddn);
+    return Py_BuildValue("(NNN)", r0, r1, r2);
+}
+
+// ---- the product over stored block values as one autograd node ---------------------------------------------------
+
+// pack.BcsrTopology as the Python side hands it over; src: of a transposed topology, the block of W behind each block.
+struct TopologyHandle {
+    const int32_t *row_ptr;
+    const int16_t *col;
+    const int32_t *seg_ptr, *src;
+    int32_t Rb, Cb;
+    int64_t nnz;
+};
+
+// An owned Python reference that may be dropped on a thread that does not hold the interpreter.
+struct PyOwned {
+    PyObject *o = nullptr;
+    explicit PyOwned(PyObject *p) : o(p) {}
+    PyOwned(const PyOwned &) = delete;
+    PyOwned &operator=(const PyOwned &) = delete;
+    ~PyOwned() {
+        if (!o || !Py_IsInitialized()) return;
+        const PyGILState_STATE g = PyGILState_Ensure();
+        Py_DECREF(o);
+        PyGILState_Release(g);
+    }
+};
+
+// Nothing rides on the tensor that a kernel launched on its address would pass by: no subclass, functorch wrapper, lazy view or
+// forward gradient.
+c10::DispatchKeySet riders() {
+    using K = c10::DispatchKey;
+    return c10::DispatchKeySet({K::Python, K::PythonTLSSnapshot, K::FuncTorchGradWrapper, K::FuncTorchBatched, K::FuncTorchDynamicLayerFrontMode,
+                                K::FuncTorchDynamicLayerBackMode, K::Batched, K::Functionalize, K::Conjugate, K::Negative, K::ZeroTensor, K::Tracer});
+}
+bool is_bare(const at::Tensor &t) {
+    return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(riders()) && !t._fw_grad(0).defined();
+}
+// No transform, mode or tracer looks on.
+bool nothing_looks_on() {
+    return !c10::impl::tls_local_dispatch_key_set().included_.has_any(riders()) && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+           !at::impl::torch_function_mode_enabled() && !torch::jit::tracer::isTracing();
+}
+
+struct DdsShape {
+    int64_t s0, s1;
+    bool tb;
+};
+
+// Operands that the native product takes: x [M, s0] bf16 rows and data [nnz, 16, 16] bf16.
+bool dds_covers(const at::Tensor &x, const at::Tensor &data, DdsShape s) {
+    return x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.size(0) > 0 && x.size(0) <= (1 << 30) && x.size(1) == s.s0 && s.s0 > 0 && s.s1 > 0 &&
+           x.stride(1) == 1 && x.stride(0) >= s.s0 && x.stride(0) % 8 == 0 && aligned16(x.const_data_ptr()) && data.scalar_type() == at::kBFloat16 &&
+           data.dim() == 3 && data.size(0) > 0 && data.size(1) == 16 && data.size(2) == 16 && data.is_contiguous() && aligned16(data.const_data_ptr()) &&
+           data.device() == x.device();
+}
+
+// Calls one of the Python side's look-ups; the result holds what the launches read until they are enqueued.  Needs the interpreter.
+PyObject *look_up(PyObject *fn, const at::Tensor &off, const at::Tensor &col, const at::Tensor &data, int64_t out_f, int64_t in_f, PyObject *last) {
+    return PyObject_CallFunction(fn, "NNNLLN", THPVariable_Wrap(off), THPVariable_Wrap(col), THPVariable_Wrap(data), (long long)out_f, (long long)in_f, last);
+}
+
+// y = x W^T (tb) or x W on a looked-up topology; undefined, with nothing launched, where the entry point refuses the call.
+at::Tensor run_dds(const TopologyHandle *t, const at::Tensor &x, const at::Tensor &data) {
+    const c10::DeviceGuard guard(x.device());
+    void *st = stream_of(x);
+    const int64_t M = x.size(0), n = (int64_t)t->Rb * 16;
+    at::Tensor w = data;
+    int rc = MORTAR_OK;
+    if (t->src) {
+        w = new_bf16(data, data.sizes());
+        rc = mortar_transpose_blocks_bf16(u16(data), t->src, t->nnz, u16m(w), st);
+    }
+    at::Tensor y = new_bf16(x, {M, n});
+    if (rc == MORTAR_OK)
+        rc = mortar_dds_values_bf16(t->row_ptr, t->col, t->seg_ptr, u16(w), t->Rb, t->Cb, t->nnz, u16(x), M, x.stride(0), u16m(y), n, st);
+    TORCH_CHECK(rc == MORTAR_OK, "mortar_dds_values_bf16 failed (", rc, "): ", mortar_last_error());
+    return y;
+}
+
+// The look-ups of stk.py, owned by the node that will use them in its backward.
+struct LookUps : torch::CustomClassHolder {
+    PyOwned topology, plan;
+    LookUps(PyObject *t, PyObject *p) : topology(Py_NewRef(t)), plan(Py_NewRef(p)) {}
+};
+struct DdsCall {
+    const TopologyHandle *topo;            // of the forward product: not kept
+    PyObject *find_topology, *find_plan;
+};
+
+at::Tensor call_op(const char *name, std::vector<c10::IValue> args) {
+    const auto op = c10::Dispatcher::singleton().findSchemaOrThrow(name, "");
+    torch::jit::Stack stack(std::move(args));
+    op.callBoxed(&stack);
+    return stack.at(0).toTensor();
+}
+
+struct DdsFn : public torch::autograd::Function<DdsFn> {
+    static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &x, const at::Tensor &data, const at::Tensor &off, const at::Tensor &row,
+                              const at::Tensor &col, const at::Tensor &off_t, const at::Tensor &col_t, const at::Tensor &blk_t, DdsShape s, DdsCall c) {
+        ctx->save_for_backward({x, data, off, row, col, off_t, col_t, blk_t});
+        ctx->saved_data["s0"] = s.s0;
+        ctx->saved_data["s1"] = s.s1;
+        ctx->saved_data["tb"] = s.tb;
+        ctx->saved_data["find"] = c10::IValue::make_capsule(c10::make_intrusive<LookUps>(c.find_topology, c.find_plan));
+        return run_dds(c.topo, x, data);
+    }
+
+    // dx = dy (W if tb else W^T): another dds; ddata = (dy^T x if tb else x^T dy) on the topology (reference: custom_ops.py:99-136).
+    // Gradients of other kinds, and those that autograd records again, go through the operators.
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto v = ctx->get_saved_variables();
+        const at::Tensor &x = v[0], &data = v[1], &off = v[2], &col = v[4];
+        const DdsShape s{ctx->saved_data["s0"].toInt(), ctx->saved_data["s1"].toInt(), ctx->saved_data["tb"].toBool()};
+        const auto look = c10::static_intrusive_pointer_cast<LookUps>(ctx->saved_data["find"].toCapsule());
+        torch::autograd::variable_list out(10);
+        if (!grads[0].defined()) return out;
+        const at::Tensor dy = grads[0].contiguous();
+        const bool native = !c10::GradMode::is_enabled() && nothing_looks_on() && is_bare(dy) && is_bare(x) && is_bare(data) &&
+                            dds_covers(dy, data, {s.s1, s.s0, !s.tb}) && dds_covers(x, data, s) && dy.size(0) == x.size(0) && dy.device() == x.device();
+        if (ctx->needs_input_grad(0)) {
+            if (native) {
+                const PyOwned held(find(look->topology.o, off, col, data, s.tb ? s.s1 : s.s0, s.tb ? s.s0 : s.s1, s.tb ? Py_True : Py_False, -1));
+                out[0] = run_dds(topology_of(held.o), dy, data);
+            } else {
+                out[0] = call_op("mortar_amd::dds", {dy, data, off, v[3], col, v[5], v[6], v[7], s.s1, s.s0, !s.tb});
+            }
+        }
+        if (ctx->needs_input_grad(1)) {
+            const at::Tensor &a = s.tb ? dy : x, &b = s.tb ? x : dy;
+            if (native) {
+                const int64_t out_f = s.tb ? s.s1 : s.s0, in_f = s.tb ? s.s0 : s.s1;
+                const PyOwned held(find(look->plan.o, off, col, data, out_f, in_f, nullptr, dy.size(0)));
+                SddPlan p;
+                {
+                    const PyGILState_STATE g = PyGILState_Ensure();
+                    const bool ok = read_plan(held.o, p);
+                    PyErr_Clear();
+                    PyGILState_Release(g);
+                    TORCH_CHECK(ok, "stk_dds: no plan for the weight gradient");
+                }
+                const c10::DeviceGuard guard(x.device());
+                const int rc = run_sdd(p, (int32_t)(out_f / 16), (int32_t)(in_f / 16), data.size(0), a, b, out[1], stream_of(x));
+                TORCH_CHECK(rc == MORTAR_OK, "mortar_sdd_bf16 failed (", rc, "): ", mortar_last_error());
+            } else {
+                out[1] = call_op("mortar_amd::sdd_at_b", {a, b, data, off, v[3], col});
+                if (out[1].scalar_type() != data.scalar_type()) out[1] = out[1].to(data.scalar_type());
+            }
+        }
+        return out;
+    }
+
+    static const TopologyHandle *topology_of(PyObject *held) {
+        const PyGILState_STATE g = PyGILState_Ensure();
+        const auto *t = static_cast<const TopologyHandle *>(PyLong_AsVoidPtr(PyTuple_GET_ITEM(held, 0)));
+        PyGILState_Release(g);
+        return t;
+    }
+
+    // A look-up from the backward's thread; its Python errors travel with the autograd engine's.
+    static PyObject *find(PyObject *fn, const at::Tensor &off, const at::Tensor &col, const at::Tensor &data, int64_t out_f, int64_t in_f, PyObject *flag,
+                          int64_t number) {
+        const PyGILState_STATE g = PyGILState_Ensure();
+        if (flag) Py_INCREF(flag);
+        PyObject *r = look_up(fn, off, col, data, out_f, in_f, flag ? flag : PyLong_FromLongLong(number));
+        if (!r) {
+            python_error err;
+            err.persist();
+            PyGILState_Release(g);
+            throw err;
+        }
+        PyGILState_Release(g);
+        return r;
+    }
+};
+
+// dds(topology look-up, plan look-up, lhs, data, offsets, row_indices, column_indices, offsets_t, column_indices_t, block_offsets_t, shape0,
+// shape1, transpose_b) -> y with its autograd node, or None: stk_dds on plain bf16 tensors.
+PyObject *py_dds(PyObject *, PyObject *const *a, Py_ssize_t na) {
+    if (na != 13) {
+        PyErr_SetString(PyExc_TypeError, "dds: 13 arguments");
+        return nullptr;
+    }
+    const at::Tensor *t[8];
+    for (int i = 0; i < 8; ++i)
+        if (!(t[i] = tensor_of(a[2 + i]))) Py_RETURN_NONE;
+    if (!PyLong_CheckExact(a[10]) || !PyLong_CheckExact(a[11]) || !PyBool_Check(a[12]) || !nothing_looks_on()) Py_RETURN_NONE;
+    const DdsShape s{PyLong_AsLongLong(a[10]), PyLong_AsLongLong(a[11]), a[12] == Py_True};
+    if (PyErr_Occurred()) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    const at::Tensor &x = *t[0], &data = *t[1];
+    if (!is_bare(x) || !is_bare(data) || !dds_covers(x, data, s) || s.s0 % 16 || s.s1 % 16 || t[2]->scalar_type() != at::kInt ||
+        t[3]->scalar_type() != at::kShort || t[4]->scalar_type() != at::kShort)
+        Py_RETURN_NONE;
+    const bool record = c10::GradMode::is_enabled() && (x.requires_grad() || data.requires_grad());
+    for (int i = 0; i < 8; ++i)
+        if (record && t[i]->is_inference()) Py_RETURN_NONE;
+    PyObject *flag = s.tb ? Py_False : Py_True;
+    Py_INCREF(flag);
+    const PyOwned held(look_up(a[0], *t[2], *t[4], data, s.tb ? s.s1 : s.s0, s.tb ? s.s0 : s.s1, flag));
+    if (!held.o) return nullptr;
+    const TopologyHandle *topo = static_cast<const TopologyHandle *>(PyLong_AsVoidPtr(PyTuple_GET_ITEM(held.o, 0)));
+    if (!topo || topo->Rb >= 1 << 26) Py_RETURN_NONE;
+    at::Tensor y = record ? DdsFn::apply(x, data, *t[2], *t[3], *t[4], *t[5], *t[6], *t[7], s, DdsCall{topo, a[0], a[1]}) : run_dds(topo, x, data);
+    return THPVariable_Wrap(std::move(y));
+}
+
 template <PyObject *(*F)(PyObject *, PyObject *const *, Py_ssize_t)>
 PyObject *guarded(PyObject *self, PyObject *const *a, Py_ssize_t na) {      // torch's C++ exceptions (out of memory) as Python ones
     HANDLE_TH_ERRORS
@@ -363,6 +703,9 @@ PyMethodDef methods[] = {
     MORTAR_METHOD("routed_decode", py_routed_decode, "RMSNorm, router and gated MLP for decode rows, or None."),
     MORTAR_METHOD("route", py_route, "The router of the rows of x and its load statistics, or None."),
     MORTAR_METHOD("gemv_f32", py_gemv_f32, "The fp32 decode product of a one-scale matrix, or None."),
+    MORTAR_METHOD("train_forward", py_train_forward, "Re-pack, gate_up, SwiGLU and down of a training step, or None."),
+    MORTAR_METHOD("train_backward", py_train_backward, "The gradients of a training step, or None."),
+    MORTAR_METHOD("dds", py_dds, "The product over stored block values with its autograd node, or None."),
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_mortar_native", "Native call layer of the MORTAR runtime.", -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -13,6 +13,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from . import _lib, ops
+from .block_sparse import CMSBlockLinear
 from .routing import TileRouter
 from .sparsity import MortarLinear
 
@@ -57,6 +58,36 @@ def _make_swiglu(d_model: int, d_ff: int, dropout: float) -> nn.Module:
     return mlp
 
 
+def _native_step(x: Tensor, cg: CMSBlockLinear, cd: CMSBlockLinear, t_gu: bool, t_dn: bool) -> tuple | None:
+    """Re-pack (with the transposes asked for), gate_up, SwiGLU and down of a training step in one native call: (y, gate_up output, h)."""
+    if type(x) is not Tensor or not x.is_cuda or x.numel() == 0:
+        return None
+    W = cg.step_pack(t_gu)
+    D = cd.step_pack(t_dn) if W is not None else None
+    r = None
+    if D is not None:
+        r = _lib.native().train_forward(x, cg.mortar_data, cd.mortar_data, W.address, W._transposed.address if t_gu else 0,
+                                        D.address, D._transposed.address if t_dn else 0, cg._values_threshold, cd._values_threshold)
+    if r is None:                     # nothing was launched: the general path re-packs
+        cg.invalidate_pack(), cd.invalidate_pack()
+    return r
+
+
+def _native_step_backward(dy: Tensor, x: Tensor, gu: Tensor, h: Tensor, cg, cd, need_x: bool, need_gu: bool, need_dn: bool) -> tuple | None:
+    """The gradients (dx, d gate_up, d down; None where not needed) of a step in one native call, while its packs are still those of
+    the forward."""
+    if type(cg) is not CMSBlockLinear or type(cd) is not CMSBlockLinear or not (need_x or need_gu or need_dn):
+        return None
+    W, D = cg.step_pack_fresh(need_x), cd.step_pack_fresh(need_x or need_gu)
+    if W is None or D is None:
+        return None
+    M = x.shape[0]
+    pg, pd = W.sdd_plan(M) if need_gu else None, D.sdd_plan(M) if need_dn else None
+    return _lib.native().train_backward(dy, x, gu, h, W.address, W._transposed.address if need_x else 0, D.address,
+                                        D._transposed.address if need_x or need_gu else 0,
+                                        pg and (pg[0].data_ptr(), pg[1], pg[2]), pd and (pd[0].data_ptr(), pd[1], pd[2]))
+
+
 class _SwiGLUMortarFn(torch.autograd.Function):
     """The carved MLP as one differentiable op for QAT training: y = down(silu(gate) * up), gate_up kept for the
     backward.  Forward: SpMM, SwiGLU, SpMM.  Backward (reference: torch autograd over transformer.py:411-431 with the
@@ -66,8 +97,17 @@ class _SwiGLUMortarFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x: Tensor, data_gu: Tensor, data_dn: Tensor, mlp: "_SwiGLUMortar") -> Tensor:
         cg, cd = mlp.gate_up._cms, mlp.down._cms
+        ctx.mlp = mlp
+        ctx.dtypes = (data_gu.dtype, data_dn.dtype)
         # re-encoded at every step (.data writes do not advance the version counter), with the W^T that the backward will need
         need_x, need_gu = ctx.needs_input_grad[:2]
+        r = None
+        if type(cg) is type(cd) is CMSBlockLinear and data_gu is cg.mortar_data and data_dn is cd.mortar_data:
+            r = _native_step(x, cg, cd, need_x, need_x or need_gu)
+        if r is not None:
+            y, gu, h = r
+            ctx.save_for_backward(x, gu, h)
+            return y
         if cg._mortar_blocking == cd._mortar_blocking == 16 and data_gu.is_cuda and data_gu.device == data_dn.device:
             cg.repack_for_step([(cg, need_x), (cd, need_x or need_gu)])
         else:
@@ -75,8 +115,6 @@ class _SwiGLUMortarFn(torch.autograd.Function):
         gu = ops.spmm(x, cg.mortar_pack())
         h = ops.swiglu(gu)
         y = ops.spmm(h, cd.mortar_pack())
-        ctx.mlp = mlp
-        ctx.dtypes = (data_gu.dtype, data_dn.dtype)
         ctx.save_for_backward(x, gu, h)
         return y
 
@@ -86,6 +124,11 @@ class _SwiGLUMortarFn(torch.autograd.Function):
         cg, cd = ctx.mlp.gate_up._cms, ctx.mlp.down._cms
         dy = (dy if dy.dtype == torch.bfloat16 else dy.to(torch.bfloat16)).contiguous()
         need_x, need_gu, need_dn = ctx.needs_input_grad[:3]
+        r = _native_step_backward(dy, x, gu, h, cg, cd, need_x, need_gu, need_dn)
+        if r is not None:
+            dx, d_gu, d_dn = r
+            return (dx, d_gu.to(ctx.dtypes[0]) if need_gu and d_gu.dtype != ctx.dtypes[0] else d_gu,
+                    d_dn.to(ctx.dtypes[1]) if need_dn and d_dn.dtype != ctx.dtypes[1] else d_dn, None)
         d_dn = ops.sdd(dy, h, cd.mortar_pack()).to(ctx.dtypes[1]) if need_dn else None
         dx = d_gu = None
         if need_x or need_gu:
@@ -160,6 +203,22 @@ class _SwiGLUMortar(nn.Module):
             p.mate = weakref.ref(q)
         return p, q
 
+    def _train_step(self, x: Tensor) -> Tensor | None:
+        """The training call of plain QAT layers on bf16 activations, found out by looking into the modules' dictionaries (the same
+        conditions as in ``forward``, whose attribute look-ups take 20 us); None: ``forward`` decides."""
+        cg, cd = self._modules["gate_up"]._modules.get("_cms"), self._modules["down"]._modules.get("_cms")
+        if type(cg) is not CMSBlockLinear or type(cd) is not CMSBlockLinear or type(x) is not Tensor or not x.is_cuda or x.dtype != torch.bfloat16:
+            return None
+        dg, dd = cg._parameters.get("mortar_data"), cd._parameters.get("mortar_data")
+        if dg is None or dd is None or not (x.requires_grad or dg.requires_grad or dd.requires_grad):
+            return None
+        for m in (cg, cd):
+            if not m._mortar or not m._values_ternary_mode or "mortar_packed" in m._buffers or m.bias is not None:
+                return None
+        x2 = x if x.dim() == 2 else x.reshape(-1, self.d_model)
+        y = _SwiGLUMortarFn.apply(x2, dg, dd, self)
+        return y if x.dim() == 2 else y.reshape(*x.shape[:-1], self.d_model)
+
     def _routed(self, x: Tensor, iter_idx: int):
         """(gates, auxiliary loss) of the module's router: one native call where calling it is nothing but its forward."""
         rt = self.router
@@ -179,6 +238,8 @@ class _SwiGLUMortar(nn.Module):
                 y = _lib.native().mlp(x, pair[0].address, pair[1].address, False, norm is not None, nw, eps, None)
                 if y is not None:
                     return y
+            elif norm is None and torch.is_grad_enabled() and (y := self._train_step(x)) is not None:
+                return y
         train = self._carved() and self._wants_grad(x)
         if norm is not None:
             fused = (self._carved() and x.is_cuda and not train and (self.router is None or gates is not None)

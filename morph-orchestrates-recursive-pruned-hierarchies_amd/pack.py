@@ -201,13 +201,17 @@ class BcsrTopology:
                        "mortar_segment_ptr_host")
             self.seg_ptr = torch.from_numpy(sp).to(self.device)
         self._t = None
+        self._handle = _lib.TopologyHandle(self.row_ptr.data_ptr(), self.col.data_ptr(), self.seg_ptr.data_ptr() if self.seg_ptr is not None else None,
+                                           None, self.Rb, self.Cb, self.nnz)
+        self.address = C.addressof(self._handle)
 
     def transposed(self):
         """(topology of W^T, src): block j of W^T is block src[j] of W, transposed (int32 device index)."""
         if self._t is None:
             off_t, col_t, src = transpose_topology(self.h_offsets, self.h_col, self.Rb, self.Cb)
-            self._t = (BcsrTopology(off_t, col_t, self.in_features, self.out_features, self.device),
-                       torch.from_numpy(src).to(self.device))
+            t, s = BcsrTopology(off_t, col_t, self.in_features, self.out_features, self.device), torch.from_numpy(src).to(self.device)
+            t._handle.src = s.data_ptr()              # (self._t keeps both alive)
+            self._t = (t, s)
         return self._t
 
 
@@ -288,7 +292,7 @@ class MortarPack:
         self._worklists: dict[tuple, tuple] = {}
         # what decode_view() rebuilds the stream from; dropped once the values are rewritten on the device
         self._h_codes, self._h_sdup, self._dview = (codes, sdup, {}) if packed is not None else (None, None, {})
-        self._pos = self._ws = self._status = self.src_block = self._sdd = None
+        self._pos = self._ws = self._status = self.src_block = self._scale = self._sdd = None
         self._status_host = self._status_event = None
         self._transposed: "MortarPack | None" = None
         self._bind_struct()
@@ -297,11 +301,17 @@ class MortarPack:
         """(Re)builds what the entry points take this matrix by: the C struct, its reference, the native call layer's handle."""
         self.struct = self._make_struct()
         self.ref = C.byref(self.struct)
-        self._handle = _lib.PackHandle(C.addressof(self.struct), None, None)
+        self._handle = _lib.PackHandle(w=C.addressof(self.struct))
         self.address = C.addressof(self._handle)
         for rpu, t in self._scheds.items():
             setattr(self._handle, f"sched{rpu}", t.data_ptr())
+        self._bind_repack()
         self.mate = None      # weak reference to the `down` pack that this gate_up pack was found to chain with (native_pair)
+
+    def _bind_repack(self) -> None:
+        h = self._handle
+        for name, t in (("pos", self._pos), ("src", self.src_block), ("scale", self._scale), ("status", self._status), ("workspace", self._ws)):
+            setattr(h, name, t.data_ptr() if t is not None else None)
 
     @property
     def on_gpu(self) -> bool:
@@ -401,11 +411,21 @@ class MortarPack:
             self._pos = torch.from_numpy(octet_positions(self.h_offsets, self.Rb, self.Cb, self.seg_cb, self.h_col)).to(self.device)
             self._ws = torch.empty(int(_lib.lib().mortar_requantize_workspace_bytes()) // 8, dtype=torch.float64, device=self.device)
             self._status = torch.zeros(2, dtype=torch.int32, device=self.device)
+            self._scale = torch.empty(1, dtype=torch.float32, device=self.device)
+            self._bind_repack()
 
     def _set_scale_form(self, uniform: float, one: int) -> None:
         if uniform != self.uniform_scale or one != self.one_scale:
             self.uniform_scale, self.one_scale = uniform, one
             self.struct.uniform_scale, self.struct.one_scale = uniform, one
+
+    def before_pair_repack(self, values: torch.Tensor, scale: torch.Tensor) -> None:
+        """What ``requantize(values, sync=False)`` does beside the launches, for a re-pack through mortar_requantize_pairs whose scale
+        goes to ``scale`` (fp32 [1])."""
+        if self._pos is None or self._h_codes is not None or self._dview:
+            self._before_repack(values)
+        self.scales_f32 = scale
+        self._set_scale_form(0.0, int(self.scale_after_sum))
 
     @staticmethod
     def requantize_pairs(jobs: list) -> list:
@@ -416,18 +436,15 @@ class MortarPack:
         for r, (W, values, threshold, with_t) in zip(arr, jobs):
             W._before_repack(values)
             s = torch.empty(1, dtype=torch.float32, device=W.device)
+            W.before_pair_repack(values, s)
             r.W, r.pos, r.values, r.scale_out = C.addressof(W.struct), W._pos.data_ptr(), values.data_ptr(), s.data_ptr()
             r.status, r.workspace = W._status.data_ptr(), W._ws.data_ptr()
             r.values_f32, r.threshold = int(values.dtype == torch.float32), threshold
-            packs = [W]
             if with_t:
                 T = W.transposed()
                 T._before_repack(values)
+                T.before_pair_repack(values, s)
                 r.Wt, r.pos_t, r.src_t, r.status_t = C.addressof(T.struct), T._pos.data_ptr(), T.src_block.data_ptr(), T._status.data_ptr()
-                packs.append(T)
-            for p in packs:
-                p.scales_f32 = s
-                p._set_scale_form(0.0, int(p.scale_after_sum))
             scales.append(s)
         dev = jobs[0][0].device
         _lib.check(_lib.lib().mortar_requantize_pairs(C.addressof(arr), len(jobs), torch.cuda.current_stream(dev).cuda_stream), "mortar_requantize_pairs")
@@ -495,6 +512,7 @@ class MortarPack:
                            prefill_stream=self.codes4_o is not None, scale_after_sum=self.scale_after_sum,
                            allow_empty_rows=True)        # a block-column of W without blocks: that slice of dX is 0
             t.src_block = torch.from_numpy(src).to(self.device)
+            t._bind_repack()
             self._transposed = t
         return self._transposed
 

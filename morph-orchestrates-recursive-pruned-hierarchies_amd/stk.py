@@ -10,7 +10,7 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from . import ops
+from . import _lib, ops
 from .pack import BcsrTopology, MortarPack
 
 _cache: dict = {}
@@ -98,6 +98,22 @@ def stk_check() -> None:
                     raise ValueError("stk_dds_ternary: " + str(e).split(": ", 1)[-1]) from None
 
 
+def _dds_topology(offsets: Tensor, column_indices: Tensor, data: Tensor, out_f: int, in_f: int, transposed: bool) -> tuple:
+    """For the native layer: (address of the topology that a dds call multiplies with, what keeps it alive)."""
+    T = _bcsr(offsets, column_indices, data.shape[0], out_f, in_f, data.device)
+    if transposed:
+        t = T.transposed()
+        return t[0].address, t
+    return T.address, T
+
+
+def _sdd_plan(offsets: Tensor, column_indices: Tensor, data: Tensor, out_f: int, in_f: int, M: int) -> tuple:
+    """For the native layer: (address, workgroups, blocks per wave) of the weight gradient's plan, and what keeps it alive."""
+    W = _topology(offsets, column_indices, data.shape[0], out_f, in_f, data.device)
+    plan, n_wg, nb = W.sdd_plan(M)
+    return plan.data_ptr(), n_wg, nb, plan
+
+
 def _check_meta(offsets: Tensor, row_indices: Tensor, column_indices: Tensor) -> None:
     if row_indices.dtype != torch.int16 or column_indices.dtype != torch.int16:
         raise ValueError(f"Expected int16 row/column indices. Got {row_indices.dtype} / {column_indices.dtype}.")
@@ -130,6 +146,24 @@ def stk_dds(lhs: Tensor, data: Tensor, offsets: Tensor, row_indices: Tensor, col
         db = ops.transpose_blocks(db, src)
     y = ops.dds_values(x, db, T)
     return y if y.dtype == lhs.dtype else y.to(lhs.dtype)
+
+
+class _DdsOp(type(stk_dds)):
+    """The custom op, whose plain calls - bf16 tensors of torch's own class on the GPU with no transform, mode, tracer or forward
+    gradient in sight - are assembled in native code, autograd node included.  The op's Python layers (schema, autograd, backend
+    selection) are 30 to 40 us of host work per product; every other call goes through them."""
+
+    def __call__(self, *args, **kwargs):
+        if torch.compiler.is_compiling():                       # traced: the registered operator itself
+            return torch.ops.mortar_amd.dds.default(*args, **kwargs)
+        if len(args) == 11 and not kwargs and type(args[0]) is Tensor and args[0].is_cuda:
+            y = _lib.native().dds(_dds_topology, _sdd_plan, *args)
+            if y is not None:
+                return y
+        return super().__call__(*args, **kwargs)
+
+
+stk_dds.__class__ = _DdsOp
 
 
 @stk_dds.register_fake
