@@ -52,6 +52,7 @@ void fill(SpmmParams &p, const mortar_bcsr_t *W, const int32_t *sched, const uin
     p.sched = reinterpret_cast<const u32x4_t *>(sched);
     p.seg_cb = W->seg_cb < W->Cb ? W->seg_cb : W->Cb; p.nseg = (W->Cb + p.seg_cb - 1) / p.seg_cb; p.Rb = W->Rb;
     p.Cb = W->Cb;
+    p.avg_octets = (int)(((int64_t)W->nnz + 8 * (int64_t)W->Rb * p.nseg - 1) / (8 * (int64_t)W->Rb * p.nseg));
     p.x = x; p.ldx = ldx; p.M = (int)M; p.y = y; p.ldy = ldy;
     p.n_clusters = 1; p.cluster_size = 1 << 30;
     p.uscale = 0.5f * W->uniform_scale;

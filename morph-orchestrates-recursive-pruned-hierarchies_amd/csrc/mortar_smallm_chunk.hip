@@ -1,0 +1,64 @@
+// Decode launches (one matrix, up to 64 rows) that spread few units over the whole chip: the part-split kernel with its row parts cut
+// into chunks, fewer units per workgroup and more waves per unit.
+//
+// A workgroup of four units leaves most CUs idle where a product has few: at one row `down` of d_model 2048 was 32 workgroups, of
+// d_model 768 twelve.  The units per workgroup come down to what one round of the chip (256 workgroups) holds, and every row part is
+// cut into runs of whole octets on waves of their own.
+#include "mortar_spmm_core.h"
+
+namespace {
+
+// Waves per part for a unit of `nparts` parts of about `octets` octets each, UW units per workgroup: 4 or 2 where built, at most one
+// wave per octet (a part of one octet is cut in two all the same: the waves then share the staging); 0: none.
+int chunk_waves(int nparts, int octets, int uw) {
+    for (int cs : {4, 2}) {
+        const int pw = nparts * cs;
+        if (cs > 2 && cs > octets) continue;
+        if (uw == 1 ? pw == 8 || pw == 12 : uw == 2 ? pw == 4 || pw == 6 || pw == 8 : pw == 4) return cs;
+    }
+    return 0;
+}
+
+template <int MT, int NACC, int CODE>
+int launch(int pw, int cs, int uw, SpmmParams &p, hipStream_t st) {
+    switch (uw * 1000 + pw * 10 + cs) {
+        case 1082: return mortar_launch_partsplit<MT, NACC, false, false, 8, 1, CODE, 2>(p, st);
+        case 1084: return mortar_launch_partsplit<MT, NACC, false, false, 8, 1, CODE, 4>(p, st);
+        case 1122: return mortar_launch_partsplit<MT, NACC, false, false, 12, 1, CODE, 2>(p, st);
+        case 1124: return mortar_launch_partsplit<MT, NACC, false, false, 12, 1, CODE, 4>(p, st);
+        case 2042: return mortar_launch_partsplit<MT, NACC, false, false, 4, 2, CODE, 2>(p, st);
+        case 2044: return mortar_launch_partsplit<MT, NACC, false, false, 4, 2, CODE, 4>(p, st);
+        case 2062: return mortar_launch_partsplit<MT, NACC, false, false, 6, 2, CODE, 2>(p, st);
+        case 2082: return mortar_launch_partsplit<MT, NACC, false, false, 8, 2, CODE, 2>(p, st);
+        case 2084: return mortar_launch_partsplit<MT, NACC, false, false, 8, 2, CODE, 4>(p, st);
+        case 4042: return mortar_launch_partsplit<MT, NACC, false, false, 4, 4, CODE, 2>(p, st);
+        case 4044: return mortar_launch_partsplit<MT, NACC, false, false, 4, 4, CODE, 4>(p, st);
+    }
+    return -1;
+}
+
+template <int MT, int CODE>
+int launch_kind(int kind, int cs, int uw, SpmmParams &p, hipStream_t st) {
+    return kind == 0 ? launch<MT, 1, CODE>(p.nseg * cs, cs, uw, p, st) : launch<MT, 2, CODE>(2 * p.nseg * cs, cs, uw, p, st);
+}
+
+}  // namespace
+
+int mortar_chunk_launch(int kind, int mt, SpmmParams &p, hipStream_t st) {
+    // (gated gate_up stays with the form that adds in the order of the token-list kernels: the two give the same bits)
+    if ((kind != 0 && kind != 1) || (kind == 1 && p.gates)) return -1;
+    const int nacc = kind + 1, nparts = p.nseg * nacc;
+    const int64_t tiles = (p.M + mt - 1) / mt;
+    for (int uw : {1, 2, 4}) {
+        // gate_up in workgroups of four units has two waves per unit to begin with: without chunks it is as fast or up to a tenth
+        // faster (d_model 768, 64 rows: 3.6 against 4.0 us), but where wide rows are normalised twice the waves share that work
+        // (16 rows with the norm, d_model 1024 4.9 against 5.0, 1536 5.7 against 5.7, 2048 6.0 against 5.8)
+        if (uw == 4 && kind == 1 && !(p.norm && p.Cb >= 96)) continue;
+        if (tiles * ((p.n_units + uw - 1) / uw) > 256) continue;
+        const int cs = chunk_waves(nparts, p.avg_octets, uw);
+        if (cs == 0 || tile_bytes(mt, p.Cb) + cs * nparts * uw * nacc * 1024 > 160 * 1024) continue;
+        if (p.uscale != 0.f) return mt == 4 ? launch_kind<4, CODE_UNIFORM>(kind, cs, uw, p, st) : launch_kind<8, CODE_UNIFORM>(kind, cs, uw, p, st);
+        return mt == 4 ? launch_kind<4, CODE_2BIT>(kind, cs, uw, p, st) : launch_kind<8, CODE_2BIT>(kind, cs, uw, p, st);
+    }
+    return -1;
+}

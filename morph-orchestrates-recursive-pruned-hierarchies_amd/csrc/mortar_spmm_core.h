@@ -54,6 +54,8 @@ struct SpmmParams {
     // into LDS.  y_tiled: the SwiGLU epilogue stores so; x_tiled: the 32-token prefill tiles are staged from it.
     int x_tiled, y_tiled;
     const uint32_t *scale_dev;   // CODE_UNIFORM kernels: the scale's pattern in device memory (mortar_bcsr_t.one_scale), or null
+    int avg_octets;              // host only: octets of a row part on average, rounded up (mortar_chunk_launch)
+    int pad_[3];
 };
 
 // Device-side view of the launch parameters: the pointers carry the global address space in their type, so
@@ -368,6 +370,70 @@ __device__ __forceinline__ void mortar_stage_tile_norm(const SpmmView &p, uint4 
     mortar_stage_quads<MT, WAVES, false, true>(p, reinterpret_cast<unsigned char *>(lx), m0, 0, ncb, tid, rs);
 }
 
+// The same staging for the decode tiles of one launch, in two halves: begin() requests everything at the start of the kernel - whole
+// rows for the sums, and the tile's pieces in staging order - and finish() forms the row factors, scales the pieces and stores them.
+// Read one after the other, descriptor, row and piece were three round trips (0.2 us of gate_up at 1 and at 13 rows, d_model 2048); the
+// registers are there, the kernel holds one weight batch otherwise.  Same order of additions, same bits.
+template <int MT, int WAVES>
+struct NormStage {
+    static constexpr int RPI = MT >= 16 ? 16 : 4, LPR = 64 / RPI, RG = (MT + RPI - 1) / RPI;
+    static constexpr int RW = (MT + WAVES - 1) / WAVES, CU = NORM_MAX_CB * 2 / 64, KQ = (NORM_MAX_CB * 2 / LPR + WAVES - 1) / WAVES;
+    u32x4_t row[RW][CU], piece[KQ][RG], w[KQ];
+
+    __device__ __forceinline__ void begin(const SpmmView &p, int m0, int ncb, int tid) {
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, nch = 2 * ncb;
+        const int rlast = (p.M - m0 < MT ? p.M - m0 : MT) - 1;
+        const MORTAR_GLOBAL char *xt = p.x + (int64_t)m0 * p.ldx * 2;
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+            const int rr = wave + r * WAVES < rlast ? wave + r * WAVES : rlast;
+#pragma unroll
+            for (int b = 0; b < CU; ++b) {
+                const int ch = b * 64 + lane < nch ? b * 64 + lane : nch - 1;
+                row[r][b] = *(const MORTAR_GLOBAL u32x4_t *)(xt + (int64_t)rr * p.ldx * 2 + (uint32_t)ch * 16u);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < KQ; ++k) {
+            int u = (wave + k * WAVES) * LPR + lane % LPR;
+            u = u < nch ? u : nch - 1;
+            w[k] = p.norm_w != nullptr ? p.norm_w[u] : u32x4_t{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int rg = 0; rg < RG; ++rg) {
+                int rr = rg * RPI + lane / LPR;
+                rr = rr < rlast ? rr : rlast;
+                piece[k][rg] = *(const MORTAR_GLOBAL u32x4_t *)(xt + (int64_t)rr * p.ldx * 2 + (uint32_t)u * 16u);
+            }
+        }
+    }
+    __device__ __forceinline__ void finish(const SpmmView &p, unsigned char *lb, int m0, int ncb, int tid, float *rs) {
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, nch = 2 * ncb;
+        const int rlast = (p.M - m0 < MT ? p.M - m0 : MT) - 1;
+#pragma unroll
+        for (int r = 0; r < RW; ++r) {
+            if (wave + r * WAVES > rlast) break;
+            float ss = 0.f;
+#pragma unroll
+            for (int b = 0; b < CU; ++b)
+                if (b * 64 + lane < nch) ss = rms_sumsq8(row[r][b], ss);
+            const float f = rms_scale(rms_wave_sum(ss), 8 * nch, p.norm_eps);
+            if (lane == 0) rs[wave + r * WAVES] = f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < KQ; ++k) {
+            const int u = (wave + k * WAVES) * LPR + lane % LPR;
+#pragma unroll
+            for (int rg = 0; rg < RG; ++rg) {
+                const int rr = rg * RPI + lane / LPR;
+                if (rr <= rlast && u < nch)
+                    *reinterpret_cast<u32x4_t *>(lb + (uint32_t)(u >> 1) * (uint32_t)(MT * 32) + rr * 32 + (u & 1) * 16) =
+                        rms_apply8(piece[k][rg], rs[rr], w[k], p.norm_w != nullptr);
+            }
+        }
+    }
+};
+
 // Four consecutive values of a carrier stream (bf16 or fp32 storage) as floats, and back.
 __device__ __forceinline__ f32x4_t mortar_load4(const MORTAR_GLOBAL char *base, int64_t elem, bool f32) {
     if (f32) return *(const MORTAR_GLOBAL f32x4_t *)(base + elem * 4);
@@ -483,6 +549,19 @@ __device__ __forceinline__ u32x4_t mortar_part_desc(const SpmmView &p, int pos, 
                             : (uint32_t)(sg * p.Rb + pos + a * p.n_units);
     u32x4_t d = base[idx];
     d[3] = sc ? d[3] : (uint32_t)pos;
+    return d;
+}
+
+// The same through the scalar cache, for a wave-uniform position: the start of a decode kernel waits for this load before anything
+// else can be requested.  (Not in the product loops: a scalar load in flight turns their counted LDS waits into full ones.)
+template <int NACC>
+__device__ __forceinline__ u32x4_t mortar_part_desc_scalar(const SpmmView &p, int pos, int q) {
+    typedef const __attribute__((address_space(4))) u32x4_t *cptr;
+    const bool sc = p.sched != nullptr;
+    const uint32_t idx = sc ? (uint32_t)pos * (uint32_t)(p.nseg * NACC) + (uint32_t)q
+                            : (uint32_t)(q / NACC * p.Rb + pos + q % NACC * p.n_units);
+    u32x4_t d = ((cptr)(uintptr_t)(sc ? p.sched : p.row_desc))[idx];
+    if (!sc) d[3] = (uint32_t)pos;
     return d;
 }
 
@@ -719,8 +798,13 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
 // their partial accumulators meet in LDS and the unit's first wave applies the epilogue.  A workgroup holds UW
 // units (PW * UW waves) and one resident token tile.  Every wave fetches its first descriptor and weight batch
 // before the tile is staged, so the only serial global round trips are descriptor -> batch.
+// CS > 0: the launches that would leave half the chip idle otherwise.  PW is CS times the number of parts, every part is cut into
+// CS runs of whole octets, one per wave, and a workgroup holds fewer units (down to one): the products and what the slowest
+// wave keeps the others waiting for shrink with the run.  At d_model 2048 and one row `down` has 128 workgroups instead of 32 and takes
+// 3.7 us instead of 5.1, at 16 rows 4.3 instead of 5.3; at d_model 768 3.0 and 3.2 instead of 3.8 and 5.7.  (Nothing here divides by a value that is not known at compile
+// time: such a division is forty instructions, and these kernels live 3 to 5 us.)
 // ---------------------------------------------------------------------------------------------------------
-template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE>
+template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE, int CS = 0>
 __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const SpmmParams p0) {
     constexpr int MSUB = (MT + 15) / 16, WAVES = PW * UW;
     SpmmView p = mortar_view(p0);
@@ -730,7 +814,7 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4, bsel = g >> 1, hsel = g & 1;
-    const int mt = blockIdx.x / p.n_split, sp = blockIdx.x % p.n_split;
+    const int mt = blockIdx.y, sp = blockIdx.x;
     const int m0 = mt * MT;
     const uint32_t lane_xo = (uint32_t)(hsel * 16 + (ROUTED ? 0 : n * 32));
     const bool has_gates = p.gates != nullptr;
@@ -738,16 +822,29 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
     const int pos = sp * UW + ug;
     const bool valid = pos < p.n_units;
     const int nparts = p.nseg * NACC;
+    constexpr int CW = CS > 0 ? CS : 1;                  // waves per part
+    static_assert(PW % CW == 0 && !(CS > 0 && ROUTED), "whole parts; token lists have no chunked form");
 
-    // first part of this wave: q = wq  (q = segment * NACC + a)
+    constexpr bool NS = MT < 16;           // (a 16-token tile's rows and pieces together are more than the waves can hold in flight: 8.5 against 8.7 us)
+    NormStage<NS ? MT : 4, WAVES> ns;
+    const bool fused_norm = NACC == 2 && !MASKED && p.norm;
+    if (NS && fused_norm) ns.begin(p, m0, p.Cb, tid);
+
+    // first part of this wave: q = segment * NACC + a (every part's descriptor names the unit)
     MortarBatch first;
-    u32x4_t d = u32x4_t{0u, 0u, 0u, 0u};
-    if (valid && wq < nparts) {
-        d = mortar_part_desc<NACC>(p, pos, wq / NACC, wq % NACC);
-        const int g0 = __builtin_amdgcn_readfirstlane((int)d[0]), g1 = __builtin_amdgcn_readfirstlane((int)d[1]);
-        if (g0 < g1) mortar_load_batch<CODE>(p, first, g0, g1, n, bsel, hsel);
+    const int q0 = wq / CW;
+    int d0 = 0, d1 = 0, dnb = 0, unit = 0;
+    if (valid) {
+        const u32x4_t d = mortar_part_desc_scalar<NACC>(p, pos, q0 < nparts ? q0 : 0);
+        unit = (int)d[3];
+        if (q0 < nparts) { d0 = (int)d[0]; d1 = (int)d[1]; dnb = (int)d[2]; }
+        if (CS > 0) {
+            const int no = d1 - d0, c = wq % CW, lo = no * c / CW, hi = no * (c + 1) / CW;
+            dnb = dnb - 8 * lo < 8 * (hi - lo) ? dnb - 8 * lo : 8 * (hi - lo);
+            d1 = d0 + hi; d0 += lo;
+        }
+        if (d0 < d1) mortar_load_batch<CODE>(p, first, d0, d1, n, bsel, hsel);
     }
-    const int unit = valid ? __builtin_amdgcn_readfirstlane((int)mortar_part_desc<NACC>(p, pos, 0, 0)[3]) : 0;
 
     int cnt = MT;
     uint32_t tk[MSUB];
@@ -774,7 +871,8 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
     if (GATE_SKIP && valid && has_gates && p.cluster_size % 16 == 0 && n < MT && m0 + n < p.M)
         gsk = p.gates[(int64_t)(m0 + n) * p.n_clusters + (unit * 16) / p.cluster_size];
 
-    if (NACC == 2 && !MASKED && p.norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(red));
+    if (NS && fused_norm) ns.finish(p, smem, m0, p.Cb, tid, reinterpret_cast<float *>(red));
+    else if (fused_norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(red));
     else mortar_stage_tile<MT, WAVES, MASKED>(p, lx, m0, 0, p.Cb, tid);
     __syncthreads();
     mortar_resolve_scale<CODE>(p);
@@ -786,6 +884,26 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
     for (int a = 0; a < NACC; ++a)
 #pragma unroll
         for (int ms = 0; ms < MSUB; ++ms) acc[a][ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if constexpr (CS > 0) {
+        if (!idle && d0 < d1)
+            mortar_row_part<MSUB, MT, false, CODE>(p, lx, first, d0, d1, dnb, lane_xo + (uint32_t)(q0 / NACC * p.seg_cb) * (uint32_t)(MT * 32), tk, nsub,
+                                                   n, bsel, hsel, acc[0]);
+#pragma unroll
+        for (int ms = 0; ms < MSUB; ++ms) red[(wave * MSUB + ms) * 64 + lane] = acc[0][ms];
+        __syncthreads();
+        if (wq != 0 || skip) return;
+#pragma unroll
+        for (int ms = 0; ms < MSUB; ++ms) acc[0][ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < PW; ++w)
+#pragma unroll
+            for (int ms = 0; ms < MSUB; ++ms) {
+                const f32x4_t v = red[((wave + w) * MSUB + ms) * 64 + lane];
+                acc[w / CW % NACC][ms] += v;
+            }
+        mortar_store_tile<MSUB, NACC, CODE, (MT <= 16 && NACC == 1)>(p, unit, m0, tk, MT, n, g, has_gates, acc[0], acc[NACC - 1]);
+        return;
+    }
     if (!idle) {
         for (int sg = 0; sg < p.nseg; ++sg) {
             const uint32_t xo_base = lane_xo + (uint32_t)(sg * p.seg_cb) * (uint32_t)(MT * 32);
@@ -794,9 +912,12 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
                 const int q = sg * NACC + a;
                 if (q % PW != wq) continue;
                 const bool is_first = q == wq;
-                const u32x4_t dq = is_first ? d : mortar_part_desc<NACC>(p, pos, sg, a);
-                const int g0 = __builtin_amdgcn_readfirstlane((int)dq[0]), g1 = __builtin_amdgcn_readfirstlane((int)dq[1]);
-                const int nb = __builtin_amdgcn_readfirstlane((int)dq[2]);
+                int g0 = d0, g1 = d1, nb = dnb;
+                if (!is_first) {
+                    const u32x4_t dq = mortar_part_desc<NACC>(p, pos, sg, a);
+                    g0 = __builtin_amdgcn_readfirstlane((int)dq[0]); g1 = __builtin_amdgcn_readfirstlane((int)dq[1]);
+                    nb = __builtin_amdgcn_readfirstlane((int)dq[2]);
+                }
                 if (g0 >= g1) continue;
                 if (!is_first) mortar_load_batch<CODE>(p, first, g0, g1, n, bsel, hsel);
                 mortar_row_part<MSUB, MT, ROUTED, CODE>(p, lx, first, g0, g1, nb, xo_base, tk, nsub, n, bsel, hsel, acc[a]);
@@ -926,21 +1047,21 @@ int mortar_launch_segmented(SpmmParams &p, const SpmmParams *table, int layers, 
     return MORTAR_OK;
 }
 
-template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE = 0>
+template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE = 0, int CS = 0>
 int mortar_launch_partsplit(SpmmParams &p, hipStream_t st) {
     constexpr int WAVES = PW * UW;
+    if (CS > 0 && PW != CS * p.nseg * NACC) return mortar_fail(MORTAR_ERR_ARG, "chunked launch: %d waves for %d parts", PW, p.nseg * NACC);
     const int smem = tile_bytes(MT, p.Cb) + WAVES * NACC * ((MT + 15) / 16) * 64 * 16;
     if (smem > 160 * 1024) return mortar_fail(MORTAR_ERR_LIMIT, "part-split tile of %d bytes does not fit LDS", smem);
     static bool attr_done = false;
-    auto kern = mortar_partsplit_kernel<MT, NACC, ROUTED, MASKED, PW, UW, CODE>;
+    auto kern = mortar_partsplit_kernel<MT, NACC, ROUTED, MASKED, PW, UW, CODE, CS>;
     int rc = mortar_allow_big_lds(kern, attr_done);
     if (rc) return rc;
     p.n_mtiles = (p.M + MT - 1) / MT;
     p.n_split = (p.n_units + UW - 1) / UW;
     p.xcd_map = 0;
-    const int64_t grid = (int64_t)p.n_mtiles * p.n_split;
-    if ((rc = mortar_launch_check(grid, 1))) return rc;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(WAVES * 64), smem, st, p);
+    if ((rc = mortar_launch_check(p.n_split, p.n_mtiles))) return rc;
+    hipLaunchKernelGGL(kern, dim3((unsigned)p.n_split, (unsigned)p.n_mtiles), dim3(WAVES * 64), smem, st, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "spmm launch: %s", hipGetErrorString(e));
     return MORTAR_OK;
@@ -951,6 +1072,9 @@ int mortar_launch_partsplit(SpmmParams &p, hipStream_t st) {
 __attribute__((visibility("hidden"))) int mortar_smallm_launch(int kind, SpmmParams &p, const SpmmParams *table,
                                                                int layers, hipStream_t st);
 __attribute__((visibility("hidden"))) int mortar_smallm_tile(int Cb, int seg_cb, int64_t M, int kind);
+// Decode launches whose workgroups would leave half the chip idle: the part-split kernel with parts cut into chunks
+// (mortar_smallm_chunk.hip).  kind 0 or 1, 4- or 8-token tiles; -1 when it has no form for the shape, or none that is better.
+__attribute__((visibility("hidden"))) int mortar_chunk_launch(int kind, int mt, SpmmParams &p, hipStream_t st);
 // Fills the launch-shape fields (n_mtiles, n_split) of a table entry exactly as mortar_smallm_launch would.
 __attribute__((visibility("hidden"))) int mortar_smallm_shape(int kind, SpmmParams &p, int layers);
 

@@ -134,3 +134,47 @@ def test_fp32_decode_product_on_either_side_of_the_one_launch_form(dev, out_b, K
     f = 8 * out_b
     want = torch.nn.functional.silu(on[:, :f]) * on[:, f:] * gates.double().repeat_interleave(f // 16, 1)
     close(mortar_amd.mortar_gemv(x, W, swiglu_out=True, gates=gates, row_act=ra, col_act=ca), want)
+
+
+@pytest.mark.parametrize("units,in_b,density,zipf", [(1, 2, 1.0, None), (5, 9, 0.3, None), (37, 128, 0.25, None), (37, 128, 0.2, 1.3), (130, 200, 0.05, None),
+                                                     (9, 352, 0.25, 1.2), (64, 352, 0.02, None), (3, 620, 0.25, None)])
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 33])
+@pytest.mark.parametrize("one_scale", [False, True])
+def test_decode_products_of_few_units(dev, units, in_b, density, zipf, M, one_scale):
+    """Row parts cut into chunks over many waves: one to four K segments, parts of less than an octet and ragged ones, odd numbers of
+    units, rows past the tile, both scale forms, clusters that are off, against float64."""
+    K = 16 * in_b
+    x = synth.synth_x(M, K, 61)
+    xd = torch.from_numpy(x).to(torch.bfloat16).to(dev)
+    xf = xd.double().cpu()
+
+    def product(m):
+        w = np.zeros((m["shape"][0], K))
+        s = m["scales"].astype(np.float64) if m["scales"].size > 1 else np.full(m["col_idx"].size, float(m["scales"][0]))
+        s = torch.from_numpy(s).to(torch.bfloat16).double().numpy()
+        for j, (r, c) in enumerate(zip(m["row_idx"], m["col_idx"])):
+            w[16 * r:16 * r + 16, 16 * c:16 * c + 16] = m["codes"][j] * s[j]
+        return xf @ torch.from_numpy(w).t()
+    for rows in (units, 2 * units):
+        m = synth.synth_matrix(16 * rows, K, density, seed=62, zipf_s=zipf)
+        if one_scale:
+            m["scales"] = m["scales"][:1]
+        W = synth.to_pack(m, dev)
+        want = product(m)
+        # fp32 sums of K products, rounded once: half a bf16 ulp, and a few ulps of fp32 of the row's largest
+        tol = 2.0 ** -8 * want.abs() + 2.0 ** -18 * want.abs().max()
+        assert ((ops.spmm(xd, W).double().cpu() - want).abs() <= tol).all()
+        if rows == 2 * units:
+            gates = torch.rand(M, units, device=dev) * (torch.rand(M, units, device=dev) < 0.4)
+            gates[:, 0] = 0
+            for g in (None, gates):
+                h = ops.gateup_swiglu(xd, W, gates=g)
+                gu = ops.spmm(xd, W)
+                ref = ops.swiglu(gu).float()
+                if g is not None:
+                    ref = (ref * g.to(torch.bfloat16).float().repeat_interleave(16, 1)).to(torch.bfloat16).float()
+                assert torch.allclose(h.float(), ref, rtol=2.0 ** -6, atol=2.0 ** -7 * float(ref.abs().max()))      # gate, up one ulp apart
+            if ops.norm_fusable(W):
+                nw = (1 + 0.1 * torch.randn(K, device=dev)).to(torch.bfloat16)
+                for w in (nw, None):
+                    assert torch.equal(ops.gateup_swiglu(xd, W, norm=(w, 1e-6)), ops.gateup_swiglu(ops.rmsnorm(xd, w, 1e-6), W))
