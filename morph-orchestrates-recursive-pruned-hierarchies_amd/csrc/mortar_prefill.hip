@@ -175,11 +175,14 @@ int dispatch(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
     }
     if (W->codes4_o) {
         p.codes_o = reinterpret_cast<const u32x4_t *>(W->codes4_o);
+        const int rc = mortar_mid_launch(kind, p.uscale != 0.f ? CODE_4BIT | CODE_UNIFORM : CODE_4BIT, p, st);
+        if (rc >= 0) return rc;
         if (p.uscale != 0.f) return dispatch_prefill<CODE_4BIT | CODE_UNIFORM>(kind, p, st);
         return dispatch_prefill<CODE_4BIT>(kind, p, st);
     }
     p.uscale = 0.f; p.scale_dev = nullptr;      // per-block path: the 2-bit prefill kernels multiply every block by its own pattern
-    return dispatch_prefill<CODE_2BIT>(kind, p, st);
+    const int rc = mortar_mid_launch(kind, CODE_2BIT, p, st);
+    return rc >= 0 ? rc : dispatch_prefill<CODE_2BIT>(kind, p, st);
 }
 
 }  // namespace
@@ -336,7 +339,7 @@ int gateup_common(const mortar_bcsr_t *W, const int32_t *sched, const uint16_t *
 namespace {
 // Rows from which both launches of the MLP certainly run the 32-token prefill tiles (below, products over several K
 // segments have small-tile forms): the hidden activations then travel in tile order.
-constexpr int64_t MLP_TILED_MIN_ROWS = 513;
+constexpr int64_t MLP_TILED_MIN_ROWS = MLP_SEPARATE_MAX_ROWS + 1;
 
 bool mlp_tiled(const mortar_bcsr_t *Wgu, const mortar_bcsr_t *Wdn, int64_t M) {
     if (M < MLP_TILED_MIN_ROWS || !Wgu->codes4_o || !Wdn->codes4_o) return false;
@@ -393,7 +396,8 @@ extern "C" int mortar_mlp_bf16(const mortar_bcsr_t *Wgu, const int32_t *sched_gu
         }
         p.y_tiled = 1;
         p.codes_o = reinterpret_cast<const u32x4_t *>(Wgu->codes4_o);
-        rc = p.uscale != 0.f ? dispatch_gateup_tiled<CODE_4BIT | CODE_UNIFORM>(p, st) : dispatch_gateup_tiled<CODE_4BIT>(p, st);
+        rc = mortar_mid_launch(1, p.uscale != 0.f ? CODE_4BIT | CODE_UNIFORM : CODE_4BIT, p, st);
+        if (rc < 0) rc = p.uscale != 0.f ? dispatch_gateup_tiled<CODE_4BIT | CODE_UNIFORM>(p, st) : dispatch_gateup_tiled<CODE_4BIT>(p, st);
         if (rc) return rc;
     }
     if (phase != 1) {

@@ -130,6 +130,7 @@ __device__ __forceinline__ void mortar_resolve_scale(SpmmView &p) {
 
 constexpr int MORTAR_SMALLM_MAX = 64;    // rows up to which the small-tile (decode) instantiations are used
 constexpr int MORTAR_PARTSPLIT_MAX = 128; // rows up to which a plain product over several K segments runs 8-token tiles of all K
+constexpr int MLP_SEPARATE_MAX_ROWS = 512; // rows up to which the MLP runs the two products' own entry points (row-major hidden activations)
 constexpr int RES_GROUPS = 4;            // octets (4 block pairs each) loaded per batch
 constexpr int LDS_BUDGET = 156 * 1024;   // bytes of LDS a token tile may take
 constexpr int LDS_PAD = 32;              // 16-byte units past the tile that idle lanes of a narrow tile may read
@@ -804,13 +805,14 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
 // 3.7 us instead of 5.1, at 16 rows 4.3 instead of 5.3; at d_model 768 3.0 and 3.2 instead of 3.8 and 5.7.  (Nothing here divides by a value that is not known at compile
 // time: such a division is forty instructions, and these kernels live 3 to 5 us.)
 // ---------------------------------------------------------------------------------------------------------
-template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE, int CS = 0>
+template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE, int CS = 0, bool YT = false>
 __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const SpmmParams p0) {
     constexpr int MSUB = (MT + 15) / 16, WAVES = PW * UW;
     SpmmView p = mortar_view(p0);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint4 *lx = reinterpret_cast<uint4 *>(smem);
-    f32x4_t *red = reinterpret_cast<f32x4_t *>(smem + tile_bytes(MT, p.Cb));   // [WAVES][NACC][MSUB][64]
+    constexpr bool ALIAS = MT >= 32;      // the partial sums of the prefill-sized tile take its place once everybody has multiplied
+    f32x4_t *red = reinterpret_cast<f32x4_t *>(smem + (ALIAS ? 0 : tile_bytes(MT, p.Cb)));   // [WAVES][NACC][MSUB][64]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4, bsel = g >> 1, hsel = g & 1;
@@ -872,7 +874,7 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
         gsk = p.gates[(int64_t)(m0 + n) * p.n_clusters + (unit * 16) / p.cluster_size];
 
     if (NS && fused_norm) ns.finish(p, smem, m0, p.Cb, tid, reinterpret_cast<float *>(red));
-    else if (fused_norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(red));
+    else if (fused_norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(smem + tile_bytes(MT, p.Cb)));
     else mortar_stage_tile<MT, WAVES, MASKED>(p, lx, m0, 0, p.Cb, tid);
     __syncthreads();
     mortar_resolve_scale<CODE>(p);
@@ -888,6 +890,7 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
         if (!idle && d0 < d1)
             mortar_row_part<MSUB, MT, false, CODE>(p, lx, first, d0, d1, dnb, lane_xo + (uint32_t)(q0 / NACC * p.seg_cb) * (uint32_t)(MT * 32), tk, nsub,
                                                    n, bsel, hsel, acc[0]);
+        if (ALIAS) __syncthreads();
 #pragma unroll
         for (int ms = 0; ms < MSUB; ++ms) red[(wave * MSUB + ms) * 64 + lane] = acc[0][ms];
         __syncthreads();
@@ -926,6 +929,7 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
     }
     // partial sums of the unit's waves meet in LDS; its first wave finishes the unit
     if (PW > 1) {
+        if (ALIAS) __syncthreads();
 #pragma unroll
         for (int a = 0; a < NACC; ++a)
 #pragma unroll
@@ -940,8 +944,8 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
                 for (int ms = 0; ms < MSUB; ++ms) acc[a][ms] += red[(((wave + w) * NACC + a) * MSUB + ms) * 64 + lane];
     }
     if (skip) return;
-    mortar_store_tile<MSUB, NACC, CODE, (MT <= 16 && NACC == 1)>(p, unit, m0, tk, ROUTED ? cnt : MT, n, g, has_gates, acc[0],
-                                                                 acc[NACC - 1]);
+    mortar_store_tile<MSUB, NACC, CODE, (MT <= 16 && NACC == 1), YT>(p, unit, m0, tk, ROUTED ? cnt : MT, n, g, has_gates, acc[0],
+                                                                     acc[NACC - 1]);
 }
 
 // ---- launchers -------------------------------------------------------------------------------------------
@@ -1047,14 +1051,17 @@ int mortar_launch_segmented(SpmmParams &p, const SpmmParams *table, int layers, 
     return MORTAR_OK;
 }
 
-template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE = 0, int CS = 0>
+template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE = 0, int CS = 0, bool YT = false>
 int mortar_launch_partsplit(SpmmParams &p, hipStream_t st) {
     constexpr int WAVES = PW * UW;
+    static_assert(!YT || (MT == 32 && NACC == 2 && CS == 0), "tile order is that of 32-token tiles");
+    if (YT != (p.y_tiled != 0)) return mortar_fail(MORTAR_ERR_ARG, "spmm launch: activation layout mismatch");
     if (CS > 0 && PW != CS * p.nseg * NACC) return mortar_fail(MORTAR_ERR_ARG, "chunked launch: %d waves for %d parts", PW, p.nseg * NACC);
-    const int smem = tile_bytes(MT, p.Cb) + WAVES * NACC * ((MT + 15) / 16) * 64 * 16;
+    const int tile = tile_bytes(MT, p.Cb) + (MT >= 32 ? LDS_EXTRA : 0), sums = WAVES * (CS > 0 ? 1 : NACC) * ((MT + 15) / 16) * 64 * 16;
+    const int smem = MT >= 32 ? (tile > sums ? tile : sums) : tile + sums;
     if (smem > 160 * 1024) return mortar_fail(MORTAR_ERR_LIMIT, "part-split tile of %d bytes does not fit LDS", smem);
     static bool attr_done = false;
-    auto kern = mortar_partsplit_kernel<MT, NACC, ROUTED, MASKED, PW, UW, CODE, CS>;
+    auto kern = mortar_partsplit_kernel<MT, NACC, ROUTED, MASKED, PW, UW, CODE, CS, YT>;
     int rc = mortar_allow_big_lds(kern, attr_done);
     if (rc) return rc;
     p.n_mtiles = (p.M + MT - 1) / MT;
@@ -1075,6 +1082,8 @@ __attribute__((visibility("hidden"))) int mortar_smallm_tile(int Cb, int seg_cb,
 // Decode launches whose workgroups would leave half the chip idle: the part-split kernel with parts cut into chunks
 // (mortar_smallm_chunk.hip).  kind 0 or 1, 4- or 8-token tiles; -1 when it has no form for the shape, or none that is better.
 __attribute__((visibility("hidden"))) int mortar_chunk_launch(int kind, int mt, SpmmParams &p, hipStream_t st);
+// The same for more rows than that in 32-token tiles: matrices of one K segment, not kind 2; code: how p.codes_o is read.
+__attribute__((visibility("hidden"))) int mortar_mid_launch(int kind, int code, SpmmParams &p, hipStream_t st);
 // Fills the launch-shape fields (n_mtiles, n_split) of a table entry exactly as mortar_smallm_launch would.
 __attribute__((visibility("hidden"))) int mortar_smallm_shape(int kind, SpmmParams &p, int layers);
 

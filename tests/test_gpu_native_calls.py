@@ -178,3 +178,36 @@ def test_decode_products_of_few_units(dev, units, in_b, density, zipf, M, one_sc
                 nw = (1 + 0.1 * torch.randn(K, device=dev)).to(torch.bfloat16)
                 for w in (nw, None):
                     assert torch.equal(ops.gateup_swiglu(xd, W, norm=(w, 1e-6)), ops.gateup_swiglu(ops.rmsnorm(xd, w, 1e-6), W))
+
+
+@pytest.mark.parametrize("units,in_b,density", [(1, 3, 1.0), (5, 48, 0.25), (37, 128, 0.25), (48, 128, 0.05), (130, 155, 0.1)])
+@pytest.mark.parametrize("M", [65, 96, 97, 250, 700])
+@pytest.mark.parametrize("one_scale", [False, True])
+def test_mid_sized_products(dev, units, in_b, density, M, one_scale):
+    """32-token tiles with a unit on one, two or four waves (65 rows up to one round of the chip): remainders of tiles and of units, parts of
+    less than an octet, the widest tile, both scale forms, gates and the norm, against float64."""
+    K = 16 * in_b
+    xd = torch.from_numpy(synth.synth_x(M, K, 71)).to(torch.bfloat16).to(dev)
+    for rows in (units, 2 * units):
+        m = synth.synth_matrix(16 * rows, K, density, seed=72, zipf_s=1.1)
+        if one_scale:
+            m["scales"] = m["scales"][:1]
+        W = synth.to_pack(m, dev)
+        w = torch.zeros(16 * rows, K, dtype=torch.float64)
+        s = torch.from_numpy(np.broadcast_to(m["scales"], m["col_idx"].shape).copy()).to(torch.bfloat16).double()
+        for j, (r, c) in enumerate(zip(m["row_idx"], m["col_idx"])):
+            w[16 * r:16 * r + 16, 16 * c:16 * c + 16] = torch.from_numpy(m["codes"][j]).double() * s[j]
+        want = (xd.double() @ w.to(dev).t())
+        tol = 2.0 ** -8 * want.abs() + 2.0 ** -18 * want.abs().max()       # one bf16 rounding of an fp32 sum
+        assert ((ops.spmm(xd, W).double() - want).abs() <= tol).all()
+        if rows == 2 * units:
+            gates = torch.rand(M, units, device=dev) * (torch.rand(M, units, device=dev) < 0.4)
+            gu = want.float().to(torch.bfloat16).float()
+            ref = (torch.nn.functional.silu(gu[:, :16 * units]) * gu[:, 16 * units:])
+            for g in (None, gates):
+                r = ref if g is None else ref * g.repeat_interleave(16, 1)
+                # four bf16 roundings (gate_up, silu, product, gated product) of 2^-9 each, silu's slope up to 1.1
+                assert torch.allclose(ops.gateup_swiglu(xd, W, gates=g).float(), r, rtol=2.0 ** -6, atol=2.0 ** -9 * float(r.abs().max()))
+            if ops.norm_fusable(W):
+                nw = (1 + 0.1 * torch.randn(K, device=dev)).to(torch.bfloat16)
+                assert torch.equal(ops.gateup_swiglu(xd, W, norm=(nw, 1e-6)), ops.gateup_swiglu(ops.rmsnorm(xd, nw, 1e-6), W))
