@@ -11,7 +11,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB = os.path.join(_HERE, "libmortar_hip.so")
 NATIVE = os.path.join(_HERE, "_mortar_native.so")
-SOURCES = ["mortar_host.cpp", "mortar_prefill.hip", "mortar_smallm.hip", "mortar_smallm_chunk.hip", "mortar_mid.hip", "mortar_decode.hip", "mortar_gemv_f32.hip", "mortar_route.hip", "mortar_router_gemm.hip",
+SOURCES = ["mortar_host.cpp", "mortar_prefill.hip", "mortar_smallm.hip", "mortar_smallm_chunk.hip", "mortar_mid.hip", "mortar_pipe.hip", "mortar_decode.hip", "mortar_gemv_f32.hip", "mortar_route.hip", "mortar_router_gemm.hip",
            "mortar_pack.hip", "mortar_sdd.hip", "mortar_swiglu.hip", "mortar_values.hip"]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

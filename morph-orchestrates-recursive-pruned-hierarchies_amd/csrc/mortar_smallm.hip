@@ -159,6 +159,10 @@ static int smallm_launch_code(int kind, SpmmParams &p, const SpmmParams *table, 
             const int rc = launch_partsplit<8, CODE>(kind, p, st);
             if (rc >= 0) return rc;
         }
+        if (mortar_wide_tile_better(kind, p) && fits(16, p.Cb)) {
+            const int rc = launch_partsplit<16, CODE>(kind, p, st);
+            if (rc >= 0) return rc;
+        }
         const int64_t tiles = (p.M + 15) / 16;
         if (tiles * ((p.n_units + 7) / 8) <= 256) return launch_kind<16, 8, CODE>(kind, false, p, nullptr, 1, st);
         if (tiles * ((p.n_units + 15) / 16) <= 256) return launch_kind<16, 16, CODE>(kind, false, p, nullptr, 1, st);

@@ -1084,6 +1084,13 @@ __attribute__((visibility("hidden"))) int mortar_smallm_tile(int Cb, int seg_cb,
 __attribute__((visibility("hidden"))) int mortar_chunk_launch(int kind, int mt, SpmmParams &p, hipStream_t st);
 // The same for more rows than that in 32-token tiles: matrices of one K segment, not kind 2; code: how p.codes_o is read.
 __attribute__((visibility("hidden"))) int mortar_mid_launch(int kind, int code, SpmmParams &p, hipStream_t st);
+// A plain product over two K segments, 65 rows and more, that 16-token tiles of all K serve best: the tile is small enough for the sums
+// beside it, and the workgroups of eight units are one round of the chip.
+inline bool mortar_wide_tile_better(int kind, const SpmmParams &p) {
+    return (kind == 0 || kind == 3) && p.nseg == 2 && p.Cb <= 192 && (p.M + 15) / 16 * (int64_t)((p.n_units + 7) / 8) <= 256;
+}
+// The same for matrices of several K segments (mortar_pipe.hip).
+__attribute__((visibility("hidden"))) int mortar_pipe_launch(int kind, int code, SpmmParams &p, hipStream_t st);
 // Fills the launch-shape fields (n_mtiles, n_split) of a table entry exactly as mortar_smallm_launch would.
 __attribute__((visibility("hidden"))) int mortar_smallm_shape(int kind, SpmmParams &p, int layers);
 

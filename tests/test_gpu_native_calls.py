@@ -137,7 +137,8 @@ def test_fp32_decode_product_on_either_side_of_the_one_launch_form(dev, out_b, K
 
 
 @pytest.mark.parametrize("units,in_b,density,zipf", [(1, 2, 1.0, None), (5, 9, 0.3, None), (37, 128, 0.25, None), (37, 128, 0.2, 1.3), (130, 200, 0.05, None),
-                                                     (9, 352, 0.25, 1.2), (64, 352, 0.02, None), (3, 620, 0.25, None)])
+                                                     (9, 352, 0.25, 1.2), (64, 352, 0.02, None), (3, 620, 0.25, None),
+                                                     (350, 100, 0.04, None)])
 @pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 33])
 @pytest.mark.parametrize("one_scale", [False, True])
 def test_decode_products_of_few_units(dev, units, in_b, density, zipf, M, one_scale):
@@ -180,12 +181,14 @@ def test_decode_products_of_few_units(dev, units, in_b, density, zipf, M, one_sc
                     assert torch.equal(ops.gateup_swiglu(xd, W, norm=(w, 1e-6)), ops.gateup_swiglu(ops.rmsnorm(xd, w, 1e-6), W))
 
 
-@pytest.mark.parametrize("units,in_b,density", [(1, 3, 1.0), (5, 48, 0.25), (37, 128, 0.25), (48, 128, 0.05), (130, 155, 0.1)])
-@pytest.mark.parametrize("M", [65, 96, 97, 250, 700])
+@pytest.mark.parametrize("units,in_b,density", [(1, 3, 1.0), (5, 48, 0.25), (37, 128, 0.25), (48, 128, 0.05), (130, 155, 0.1),
+                                                (1, 156, 1.0), (70, 180, 0.2), (37, 352, 0.25), (130, 311, 0.03), (9, 700, 0.1)])
+@pytest.mark.parametrize("M", [65, 96, 97, 250, 512, 700])
 @pytest.mark.parametrize("one_scale", [False, True])
 def test_mid_sized_products(dev, units, in_b, density, M, one_scale):
-    """32-token tiles with a unit on one, two or four waves (65 rows up to one round of the chip): remainders of tiles and of units, parts of
-    less than an octet, the widest tile, both scale forms, gates and the norm, against float64."""
+    """Up to 155 block-columns: 32-token tiles with a unit on one, two or four waves (65 rows up to one round of the chip); beyond: several K
+    segments through two buffers (up to 512 rows).  Remainders of tiles, segments and units, parts of less than an octet, the widest tile
+    and segment, both scale forms, gates, input mask and norm, against float64."""
     K = 16 * in_b
     xd = torch.from_numpy(synth.synth_x(M, K, 71)).to(torch.bfloat16).to(dev)
     for rows in (units, 2 * units):
@@ -200,6 +203,8 @@ def test_mid_sized_products(dev, units, in_b, density, M, one_scale):
         want = (xd.double() @ w.to(dev).t())
         tol = 2.0 ** -8 * want.abs() + 2.0 ** -18 * want.abs().max()       # one bf16 rounding of an fp32 sum
         assert ((ops.spmm(xd, W).double() - want).abs() <= tol).all()
+        act = torch.randint(0, 2, (M, in_b), dtype=torch.uint8, device=dev)
+        assert torch.equal(ops.spmm(xd, W, active=act), ops.spmm(xd * act.repeat_interleave(16, 1).to(xd.dtype), W))
         if rows == 2 * units:
             gates = torch.rand(M, units, device=dev) * (torch.rand(M, units, device=dev) < 0.4)
             gu = want.float().to(torch.bfloat16).float()
