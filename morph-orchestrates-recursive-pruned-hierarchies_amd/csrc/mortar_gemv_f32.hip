@@ -22,10 +22,14 @@ struct GemvOneArgs {
 
 __device__ __forceinline__ float sigmoid_f32(float g) { return 1.0f / (1.0f + __expf(-g)); }
 
-// T tokens per tile (3 T rows of 16 MFMA columns), PW waves share the parts of a unit, 4 units per workgroup.
-template <int T, int NACC, int PW>
-__global__ void __launch_bounds__(PW * 4 * 64) gemv_f32_one_kernel(const SpmmParams p0, const GemvOneArgs a) {
-    constexpr int MT = 3 * T, UW = 4, WAVES = PW * UW, THREADS = WAVES * 64;
+// T tokens per tile (3 T rows of 16 MFMA columns), PW waves share the parts of a unit, UW units per workgroup.  CS > 0: PW is CS times
+// the number of parts and each wave takes a run of a part's octets, for launches that would leave half of the chip idle: latency bounds
+// these, a wave's chain of batches first, so it is cut.  At d_model 2048, density 0.25, us, the whole parts against the cut ones: SwiGLU
+// form 1 row 5.01 -> 4.32, 8 rows 5.32 -> 5.18; plain product over 5632 inputs 4.86 -> 3.91, 8 rows 6.85 -> 6.13.  A third of that is the
+// grid of two dimensions and the staging without integer divisions, which the launches with whole parts share.
+template <int T, int NACC, int PW, int UW, int CS>
+__global__ void __launch_bounds__(PW * UW * 64) gemv_f32_one_kernel(const SpmmParams p0, const GemvOneArgs a) {
+    constexpr int MT = 3 * T, WAVES = PW * UW, THREADS = WAVES * 64, CW = CS > 0 ? CS : 1;
     const SpmmView p = mortar_view(p0);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint4 *lx = reinterpret_cast<uint4 *>(smem);
@@ -33,17 +37,23 @@ __global__ void __launch_bounds__(PW * 4 * 64) gemv_f32_one_kernel(const SpmmPar
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4, bsel = g >> 1, hsel = g & 1;
-    const int mt = blockIdx.x / p.n_split, sp = blockIdx.x % p.n_split;
+    const int mt = blockIdx.y, sp = blockIdx.x;
     const int t0 = mt * T, nt = p.M - t0 < T ? p.M - t0 : T;                           // p.M counts tokens here
     const int ug = wave / PW, wq = wave % PW, pos = sp * UW + ug;
     const bool valid = pos < p.n_units;
     const int nparts = p.nseg * NACC;
     MortarBatch first;
-    u32x4_t d = u32x4_t{0u, 0u, 0u, 0u};
-    if (valid && wq < nparts) {          // the first weights are on their way before the tile is staged
-        d = mortar_part_desc<NACC>(p, pos, wq / NACC, wq % NACC);
-        const int g0 = __builtin_amdgcn_readfirstlane((int)d[0]), g1 = __builtin_amdgcn_readfirstlane((int)d[1]);
-        if (g0 < g1) mortar_load_batch<CODE_UNIFORM>(p, first, g0, g1, n, bsel, hsel);
+    const int q0 = wq / CW;
+    int d0 = 0, d1 = 0, dnb = 0;
+    if (valid && q0 < nparts) {          // the first weights are on their way before the tile is staged
+        const u32x4_t d = mortar_part_desc_scalar<NACC>(p, pos, q0);
+        d0 = (int)d[0]; d1 = (int)d[1]; dnb = (int)d[2];
+        if (CS > 0) {
+            const int no = d1 - d0, c = wq % CW, lo = no * c / CW, hi = no * (c + 1) / CW;
+            dnb = dnb - 8 * lo < 8 * (hi - lo) ? dnb - 8 * lo : 8 * (hi - lo);
+            d1 = d0 + hi; d0 += lo;
+        }
+        if (d0 < d1) mortar_load_batch<CODE_UNIFORM>(p, first, d0, d1, n, bsel, hsel);
     }
     // what the epilogue reads besides the sums, requested early: the lane's gate and row flags (token n)
     const int tok = t0 + n;
@@ -68,7 +78,10 @@ __global__ void __launch_bounds__(PW * 4 * 64) gemv_f32_one_kernel(const SpmmPar
         for (int u = 0; u < 4; ++u) {
             const int i = i0 + u * THREADS;
             if (i >= nt * nch) break;
-            const int t = i / nch, c = i - t * nch;
+            int t = 0;
+#pragma unroll
+            for (int k = 1; k < T; ++k) t += i >= k * nch;               // i / nch without the forty instructions of a division
+            const int c = i - t * nch;
             const float4 *src = reinterpret_cast<const float4 *>(a.x + (int64_t)(t0 + t) * a.ldx + c * 8);
             q[u][0] = src[0];
             q[u][1] = src[1];
@@ -106,23 +119,36 @@ __global__ void __launch_bounds__(PW * 4 * 64) gemv_f32_one_kernel(const SpmmPar
 #pragma unroll
     for (int b = 0; b < NACC; ++b) acc[b][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const uint32_t tk[1] = {(uint32_t)n};
-    if (work) {
+    if constexpr (CS > 0) {
+        if (work && d0 < d1)
+            mortar_row_part<1, MT, false, CODE_UNIFORM>(p, lx, first, d0, d1, dnb, (uint32_t)(hsel * 16 + n * 32) + (uint32_t)(q0 / NACC * p.seg_cb) * (uint32_t)(MT * 32),
+                                                        tk, 1, n, bsel, hsel, acc[0]);
+        red[wave * 64 + lane] = acc[0][0];
+        __syncthreads();
+        if (wq != 0) return;
+        acc[0][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < PW; ++w) acc[w / CW % NACC][0] += red[(wave + w) * 64 + lane];
+    } else if (work) {
         for (int sg = 0; sg < p.nseg; ++sg) {
             const uint32_t xo = (uint32_t)(hsel * 16 + n * 32) + (uint32_t)(sg * p.seg_cb) * (uint32_t)(MT * 32);
 #pragma unroll
             for (int b = 0; b < NACC; ++b) {
                 const int q = sg * NACC + b;
                 if (q % PW != wq) continue;
-                const u32x4_t dq = q == wq ? d : mortar_part_desc<NACC>(p, pos, sg, b);
-                const int g0 = __builtin_amdgcn_readfirstlane((int)dq[0]), g1 = __builtin_amdgcn_readfirstlane((int)dq[1]);
+                int g0 = d0, g1 = d1, nb = dnb;
+                if (q != wq) {
+                    const u32x4_t dq = mortar_part_desc<NACC>(p, pos, sg, b);
+                    g0 = __builtin_amdgcn_readfirstlane((int)dq[0]); g1 = __builtin_amdgcn_readfirstlane((int)dq[1]);
+                    nb = __builtin_amdgcn_readfirstlane((int)dq[2]);
+                }
                 if (g0 >= g1) continue;
                 if (q != wq) mortar_load_batch<CODE_UNIFORM>(p, first, g0, g1, n, bsel, hsel);
-                mortar_row_part<1, MT, false, CODE_UNIFORM>(p, lx, first, g0, g1, __builtin_amdgcn_readfirstlane((int)dq[2]), xo, tk, 1, n, bsel,
-                                                            hsel, acc[b]);
+                mortar_row_part<1, MT, false, CODE_UNIFORM>(p, lx, first, g0, g1, nb, xo, tk, 1, n, bsel, hsel, acc[b]);
             }
         }
     }
-    if (PW > 1) {
+    if (PW > 1 && CS == 0) {
 #pragma unroll
         for (int b = 0; b < NACC; ++b) red[(wave * NACC + b) * 64 + lane] = acc[b][0];
         __syncthreads();
@@ -170,29 +196,57 @@ OneShape one_shape(const mortar_bcsr_t *W, int mode, int B) {
     return {t, pw};
 }
 
-template <int T, int NACC, int PW>
+template <int T, int NACC, int PW, int UW, int CS>
 int launch_one(SpmmParams &p, const GemvOneArgs &a, hipStream_t st) {
-    const int smem = one_lds(T, NACC, PW, p.Cb);
+    const int smem = tile_bytes(3 * T, p.Cb) + (PW > 1 ? PW * UW * (CS > 0 ? 1 : NACC) * 1024 : 0);
     static bool done = false;
-    int rc = mortar_allow_big_lds(gemv_f32_one_kernel<T, NACC, PW>, done);
+    int rc = mortar_allow_big_lds(gemv_f32_one_kernel<T, NACC, PW, UW, CS>, done);
     if (rc) return rc;
     p.n_mtiles = (p.M + T - 1) / T;
-    p.n_split = (p.n_units + 3) / 4;
-    if ((rc = mortar_launch_check((int64_t)p.n_mtiles * p.n_split, 1))) return rc;
-    hipLaunchKernelGGL((gemv_f32_one_kernel<T, NACC, PW>), dim3((unsigned)(p.n_mtiles * p.n_split)), dim3(PW * 256), smem, st, p, a);
+    p.n_split = (p.n_units + UW - 1) / UW;
+    if ((rc = mortar_launch_check(p.n_split, p.n_mtiles))) return rc;
+    hipLaunchKernelGGL((gemv_f32_one_kernel<T, NACC, PW, UW, CS>), dim3((unsigned)p.n_split, (unsigned)p.n_mtiles), dim3(PW * UW * 64), smem, st, p, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "gemv_f32 launch: %s", hipGetErrorString(e));
     return MORTAR_OK;
 }
 
+// Few units: as many waves per unit as the part-split launches of mortar_smallm_chunk.hip take, in workgroups of one or two units while
+// they are one round of the chip.  -1: no such form, or no need of one.
+template <int T, int NACC>
+int launch_chunk(SpmmParams &p, const GemvOneArgs &a, hipStream_t st) {
+    const int nparts = p.nseg * NACC;
+    for (int uw : {1, 2}) {
+        if ((int64_t)((p.M + T - 1) / T) * ((p.n_units + uw - 1) / uw) > 256) continue;
+        for (int cs : {4, 2}) {
+            const int pw = nparts * cs;
+            if ((cs == 4 && p.avg_octets < 4) || tile_bytes(3 * T, p.Cb) + pw * uw * 1024 > 160 * 1024) continue;
+            switch (uw * 1000 + pw * 10 + cs) {
+                case 1082: return launch_one<T, NACC, 8, 1, 2>(p, a, st);
+                case 1084: return launch_one<T, NACC, 8, 1, 4>(p, a, st);
+                case 1122: return launch_one<T, NACC, 12, 1, 2>(p, a, st);
+                case 1124: return launch_one<T, NACC, 12, 1, 4>(p, a, st);
+                case 2042: return launch_one<T, NACC, 4, 2, 2>(p, a, st);
+                case 2044: return launch_one<T, NACC, 4, 2, 4>(p, a, st);
+                case 2062: return launch_one<T, NACC, 6, 2, 2>(p, a, st);
+                case 2082: return launch_one<T, NACC, 8, 2, 2>(p, a, st);
+                case 2084: return launch_one<T, NACC, 8, 2, 4>(p, a, st);
+            }
+        }
+    }
+    return -1;
+}
+
 template <int T, int NACC>
 int launch_pw(int pw, SpmmParams &p, const GemvOneArgs &a, hipStream_t st) {
+    const int rc = launch_chunk<T, NACC>(p, a, st);
+    if (rc >= 0) return rc;
     switch (pw) {
-        case 1: return launch_one<T, NACC, 1>(p, a, st);
-        case 2: return launch_one<T, NACC, 2>(p, a, st);
-        case 3: return launch_one<T, NACC, 3>(p, a, st);
+        case 1: return launch_one<T, NACC, 1, 4, 0>(p, a, st);
+        case 2: return launch_one<T, NACC, 2, 4, 0>(p, a, st);
+        case 3: return launch_one<T, NACC, 3, 4, 0>(p, a, st);
     }
-    return launch_one<T, NACC, 4>(p, a, st);
+    return launch_one<T, NACC, 4, 4, 0>(p, a, st);
 }
 
 template <int NACC>
@@ -245,6 +299,7 @@ extern "C" int mortar_gemv_f32_one(const mortar_bcsr_t *W, const float *scale, i
     p.seg_cb = W->seg_cb < W->Cb ? W->seg_cb : W->Cb;
     p.nseg = (W->Cb + p.seg_cb - 1) / p.seg_cb;
     p.Rb = W->Rb; p.Cb = W->Cb; p.M = B;
+    p.avg_octets = (int)(((int64_t)W->nnz + 8 * (int64_t)W->Rb * p.nseg - 1) / (8 * (int64_t)W->Rb * p.nseg));
     p.n_units = mode == 0 ? W->Rb : W->Rb / 2;
     p.n_clusters = 1; p.cluster_size = gates ? (int)(nout / n_clusters) : 1 << 30;
     const OneShape sh = one_shape(W, mode, B);

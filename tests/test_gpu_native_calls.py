@@ -136,6 +136,25 @@ def test_fp32_decode_product_on_either_side_of_the_one_launch_form(dev, out_b, K
     close(mortar_amd.mortar_gemv(x, W, swiglu_out=True, gates=gates, row_act=ra, col_act=ca), want)
 
 
+@pytest.mark.parametrize("units,in_b,density", [(37, 128, 0.3), (257, 128, 0.3), (511, 128, 0.05), (513, 128, 0.3),     # one, two, two, four units a workgroup
+                                                (37, 352, 0.3), (259, 352, 0.03)])
+@pytest.mark.parametrize("B", [1, 5, 9])
+def test_fp32_decode_products_of_few_units(dev, units, in_b, density, B):
+    """Row parts cut over many waves, odd numbers of units, parts of less than an octet: plain and SwiGLU forms against float64."""
+    x = torch.randn(B, 16 * in_b, device=dev, generator=torch.Generator(device=dev).manual_seed(B))
+    for rows in (units, 2 * units):
+        m = synth.synth_matrix(16 * rows, 16 * in_b, density, seed=63, per_tensor_scale=True)
+        W = synth.to_pack(m, dev)
+        dense = torch.zeros(rows, in_b, 16, 16, dtype=torch.float64, device=dev)
+        dense[torch.from_numpy(m["row_idx"]).long(), torch.from_numpy(m["col_idx"]).long()] = torch.from_numpy(m["codes"]).to(dev).double()
+        want = x.double() @ (dense.permute(0, 2, 1, 3).reshape(16 * rows, -1) * float(m["scales"][0])).t()
+        assert (mortar_amd.mortar_gemv(x, W).double() - want).abs().max() <= 3e-6 * want.abs().max()      # fp32 sums of up to 1700 exact terms
+        if rows == 2 * units:
+            f = 16 * units
+            h = torch.nn.functional.silu(want[:, :f]) * want[:, f:]
+            assert torch.allclose(mortar_amd.mortar_gemv(x, W, swiglu_out=True).double(), h, rtol=1e-4, atol=1e-5 * h.abs().max().item())
+
+
 @pytest.mark.parametrize("units,in_b,density,zipf", [(1, 2, 1.0, None), (5, 9, 0.3, None), (37, 128, 0.25, None), (37, 128, 0.2, 1.3), (130, 200, 0.05, None),
                                                      (9, 352, 0.25, 1.2), (64, 352, 0.02, None), (3, 620, 0.25, None),
                                                      (350, 100, 0.04, None)])
