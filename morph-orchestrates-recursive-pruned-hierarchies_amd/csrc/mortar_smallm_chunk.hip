@@ -55,6 +55,7 @@ int mortar_chunk_launch(int kind, int mt, SpmmParams &p, hipStream_t st) {
         // (16 rows with the norm, d_model 1024 4.9 against 5.0, 1536 5.7 against 5.7, 2048 6.0 against 5.8; without it 4.5 against 4.7 - by the
         // width alone, not by the norm, so that the fused norm gives the bits of the separate one).
         if (uw == 4 && kind == 1 && p.Cb < 96) continue;
+        if (tiles * ((p.n_units + uw - 1) / uw) > 256) continue;
         const int cs = chunk_waves(nparts, p.avg_octets, uw);
         if (cs == 0 || tile_bytes(mt, p.Cb) + cs * nparts * uw * nacc * 1024 > 160 * 1024) continue;
         if (p.uscale != 0.f) return mt == 4 ? launch_kind<4, CODE_UNIFORM>(kind, cs, uw, p, st) : launch_kind<8, CODE_UNIFORM>(kind, cs, uw, p, st);
