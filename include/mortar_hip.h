@@ -272,6 +272,13 @@ int mortar_router_bf16(const void *x, int32_t x_is_f32, int64_t B, int32_t d, in
                        const float *kb, int32_t nsk, const float *bias, int32_t n, int32_t k, float *qv,
                        float *logits_out, float *gates, uint8_t *active, void *stream);
 
+/* mortar_rmsnorm_bf16(x) -> xn (bf16 [B, d], rows contiguous, 16-byte aligned), then mortar_router_bf16 on the normalised rows: same bits,
+ * with the norm inside the projection's launch up to d = 2048.  norm_w bf16 [d] or NULL. */
+int mortar_norm_router_bf16(const uint16_t *x, int64_t B, int32_t d, int64_t ldx, const uint16_t *norm_w, float norm_eps, uint16_t *xn,
+                            const float *wq, const float *iter_vec, const float *ln_w, const float *ln_b, float ln_eps,
+                            const float *ka, const float *kb, int32_t nsk, const float *bias, int32_t n, int32_t k, float *qv,
+                            float *logits_out, float *gates, uint8_t *active, void *stream);
+
 /* The router's dense query projection for prefill-sized calls (routing.py:181-186): qv[m, o] = sum_i x[m, i] wq[o, i] for
  * bf16 x [M, d_in] (row stride ldx, a multiple of 8) and fp32 wq [d_out, d_in], qv fp32 [M, d_out] (row stride ldq, a
  * multiple of 4); d_in a multiple of 8, d_out of 4, everything 16-byte aligned.  Exact products (the weights enter the

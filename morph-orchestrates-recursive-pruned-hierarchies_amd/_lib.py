@@ -76,6 +76,8 @@ _SIGS = {
     "mortar_remoe_route": (C.c_int, [c_vp, c_i64, c_i32, c_i32, c_vp, c_vp, c_vp]),
     "mortar_router_bf16": (C.c_int, [c_vp, c_i32, c_i64, c_i32, c_i64, c_vp, c_vp, c_vp, c_vp, c_f32, c_vp, c_vp, c_i32,
                                      c_vp, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp, c_vp]),
+    "mortar_norm_router_bf16": (C.c_int, [c_vp, c_i64, c_i32, c_i64, c_vp, c_f32, c_vp, c_vp, c_vp, c_vp, c_vp, c_f32, c_vp, c_vp, c_i32,
+                                          c_vp, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "mortar_router_tail_f32": (C.c_int, [c_vp, c_i64, c_i32, c_i64, c_vp, c_vp, c_vp, c_f32, c_vp, c_vp, c_i32, c_vp, c_i32,
                                          c_i32, c_vp, c_vp, c_vp, c_vp]),
     "mortar_router_project_bf16": (C.c_int, [c_vp, c_i64, c_i32, c_i64, c_vp, c_i32, c_vp, c_i64, c_vp]),

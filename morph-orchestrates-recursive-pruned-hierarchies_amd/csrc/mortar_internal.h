@@ -19,8 +19,10 @@ __attribute__((visibility("hidden"))) int mortar_spmm_codes_f32(const mortar_bcs
                                                                  int64_t M, int64_t ldx, float *y32, int64_t ldy, void *stream);
 
 // qv[m, :] = x[m, :] W^T + bias for few tokens (bias may be null): K shared by the waves of a workgroup.  The caller has checked
-// the shapes: d_in % 8 == 0, d_out % 4 == 0, all pointers and rows 16-byte aligned.
+// the shapes: d_in % 8 == 0, d_in <= 2048, d_out % 4 == 0, all pointers and rows 16-byte aligned.  xn [M, d_in], M <= 16: the rows of x
+// are RMS-normalised first (norm_w may be null) and written there as well.
 __attribute__((visibility("hidden"))) int mortar_router_project_skinny(const uint16_t *x, int64_t M, int32_t d_in, int64_t ldx, const float *wq,
-                                                                       int32_t d_out, const float *bias, float *qv, int64_t ldq, void *stream);
+                                                                       int32_t d_out, const float *bias, float *qv, int64_t ldq, void *stream,
+                                                                       const uint16_t *norm_w = nullptr, float eps = 0.f, uint16_t *xn = nullptr);
 
 #endif

@@ -186,6 +186,69 @@ __global__ void __launch_bounds__(256) router_project_kernel(const void *xv, int
     }
 }
 
+// The projection of 1 to TB <= 4 bf16 rows with the RMSNorm before it, d <= 2048: wave w of every workgroup normalises row w into LDS
+// (rms_* of mortar_device.h: the bits of rmsnorm_rows_kernel) while the weight rows are on their way, the first workgroup also writes
+// the rows to xn for the products.  A launch of its own for the norm is a chain of 3.4 us with one wave per row.  Same products and
+// order of sums as router_project_kernel.  (Figures: launch_router.)
+template <int TB>
+__global__ void __launch_bounds__(256) router_norm_project_kernel(const uint16_t *x, int B, int d, int64_t ldx, const uint16_t *nw, float eps, uint16_t *xn,
+                                                                  const float *wq, const float *iter_vec, float *qv) {
+    extern __shared__ __attribute__((aligned(16))) float sm[];       // bf16 [TB][d]
+    u32x4_t *xs = reinterpret_cast<u32x4_t *>(sm);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int o = blockIdx.x * 4 + wave, n4 = d / 4, nch = d / 8;       // d % 8 == 0: every wave has an output
+    const bool norm = wave < B && wave < TB;
+    u32x4_t u[4], w8[4];
+    if (norm) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int ch = lane + 64 * j < nch ? lane + 64 * j : nch - 1;
+            u[j] = reinterpret_cast<const u32x4_t *>(x + wave * ldx)[ch];
+            w8[j] = nw ? reinterpret_cast<const u32x4_t *>(nw)[ch] : u32x4_t{0u, 0u, 0u, 0u};
+        }
+    }
+    float4 w[8];
+    const float4 *wr = reinterpret_cast<const float4 *>(wq + (int64_t)o * d);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[j] = lane + 64 * j < n4 ? wr[lane + 64 * j] : float4{0.f, 0.f, 0.f, 0.f};
+    const float bias = iter_vec ? iter_vec[o] : 0.f;
+    if (norm) {
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (lane + 64 * j < nch) ss = rms_sumsq8(u[j], ss);
+        const float r = rms_scale(rms_wave_sum(ss), d, eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int ch = lane + 64 * j;
+            if (ch < nch) {
+                const u32x4_t v = rms_apply8(u[j], r, w8[j], nw != nullptr);
+                xs[wave * nch + ch] = v;
+                if (blockIdx.x == 0) reinterpret_cast<u32x4_t *>(xn + (int64_t)wave * d)[ch] = v;
+            }
+        }
+    }
+    __syncthreads();
+    float acc[TB];
+#pragma unroll
+    for (int t = 0; t < TB; ++t) acc[t] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int i4 = lane + 64 * j < n4 ? lane + 64 * j : n4 - 1;
+#pragma unroll
+        for (int t = 0; t < TB; ++t) {
+            const uint2 xx = reinterpret_cast<const uint2 *>(xs)[(t < B ? t : B - 1) * n4 + i4];
+            acc[t] = __builtin_fmaf(__builtin_bit_cast(float, xx.y & 0xffff0000u), w[j].w, __builtin_fmaf(__builtin_bit_cast(float, xx.y << 16), w[j].z,
+                     __builtin_fmaf(__builtin_bit_cast(float, xx.x & 0xffff0000u), w[j].y, __builtin_fmaf(__builtin_bit_cast(float, xx.x << 16), w[j].x, acc[t]))));
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+        const float s = wave_sum(acc[t]);
+        if (lane == 0 && t < B) qv[(int64_t)t * d + o] = s + bias;
+    }
+}
+
 __device__ __forceinline__ float block_sum256(float v, float *red) {      // red: 4 floats of LDS; all 256 threads call
     v = wave_sum(v);
     __syncthreads();
@@ -910,11 +973,10 @@ static int launch_tail(const float *qv, int64_t N, int32_t d, int64_t ldq, const
     return check_launch("router tail");
 }
 
-extern "C" int mortar_router_bf16(const void *x, int32_t x_is_f32, int64_t B, int32_t d, int64_t ldx, const float *wq,
-                                  const float *iter_vec, const float *ln_w, const float *ln_b, float ln_eps,
-                                  const float *ka, const float *kb, int32_t nsk, const float *bias, int32_t n,
-                                  int32_t k, float *qv, float *logits_out, float *gates, uint8_t *active,
-                                  void *stream) {
+// xn: the rows of x (bf16) are RMS-normalised on the way in and written there; null: they are taken as they are.
+static int launch_router(const void *x, bool x_is_f32, int64_t B, int32_t d, int64_t ldx, const uint16_t *norm_w, float norm_eps, uint16_t *xn,
+                         const float *wq, const float *iter_vec, const float *ln_w, const float *ln_b, float ln_eps, const float *ka, const float *kb,
+                         int32_t nsk, const float *bias, int32_t n, int32_t k, float *qv, float *logits_out, float *gates, uint8_t *active, void *stream) {
     if (!x || !wq || !ln_w || !ln_b || !ka || !kb || !bias || !qv || !gates)
         return mortar_fail(MORTAR_ERR_ARG, "router: null pointer");
     if (B <= 0 || B > 64) return mortar_fail(MORTAR_ERR_LIMIT, "router: the fused front end serves 1..64 tokens (got %lld)", (long long)B);
@@ -931,9 +993,22 @@ extern "C" int mortar_router_bf16(const void *x, int32_t x_is_f32, int64_t B, in
     // From 5 bf16 tokens up the projection runs on the matrix cores (2048 x 2048, with the tail: 5 tokens 13.6 -> 12.0 us, 16 19.5 -> 12.4,
     // 64 46 -> 15.6; 4 tokens 11.0 against 11.8); fp32 activations, wider rows and fewer tokens take one wave per output.
     const bool aligned = ((reinterpret_cast<uintptr_t>(qv) | reinterpret_cast<uintptr_t>(iter_vec)) & 15) == 0;
+    const uint16_t *xb = static_cast<const uint16_t *>(x);
     int rc;
+    // The norm inside the projection, whole routed step with a launch of its own against it, d_model 2048: 4 rows 25.7 -> 22.5 us, 8 26.2 -> 25.5,
+    // 16 28.1 -> 27.1; 1024, 16 rows 20.8 -> 20.2.  A second tile of tokens loses: 24 rows 31.4 -> 33.0, 1024 21.4 -> 22.0.
+    if (xn && (d > 2048 || B > 16 || (B > 4 && !aligned) || ((reinterpret_cast<uintptr_t>(xn) | reinterpret_cast<uintptr_t>(norm_w)) & 15))) {
+        if ((rc = mortar_rmsnorm_bf16(xb, B, d, ldx, norm_w, norm_eps, xn, d, stream))) return rc;
+        x = xb = xn; ldx = d; xn = nullptr;
+        if (reinterpret_cast<uintptr_t>(x) & 15) return mortar_fail(MORTAR_ERR_ARG, "router: xn must be 16-byte aligned");
+    }
     if (!x_is_f32 && B > 4 && d <= 2048 && aligned) {
-        rc = mortar_router_project_skinny(static_cast<const uint16_t *>(x), B, d, ldx, wq, d, iter_vec, qv, d, stream);
+        rc = mortar_router_project_skinny(xb, B, d, ldx, wq, d, iter_vec, qv, d, stream, norm_w, norm_eps, xn);
+    } else if (xn) {
+        const int smem = (B == 1 ? 1 : 4) * d * 2;
+        if (B == 1) hipLaunchKernelGGL(router_norm_project_kernel<1>, pg, blk, smem, st, xb, (int)B, d, ldx, norm_w, norm_eps, xn, wq, iter_vec, qv);
+        else hipLaunchKernelGGL(router_norm_project_kernel<4>, pg, blk, smem, st, xb, (int)B, d, ldx, norm_w, norm_eps, xn, wq, iter_vec, qv);
+        rc = check_launch("router projection");
     } else {
 #define MORTAR_PROJ(TB, F) hipLaunchKernelGGL((router_project_kernel<TB, F>), pg, blk, 0, st, x, (int)B, d, ldx, wq, iter_vec, qv)
         if (x_is_f32) { if (B == 1) MORTAR_PROJ(1, true); else if (B <= 4) MORTAR_PROJ(4, true); else if (B <= 8) MORTAR_PROJ(8, true); else MORTAR_PROJ(16, true); }
@@ -943,6 +1018,24 @@ extern "C" int mortar_router_bf16(const void *x, int32_t x_is_f32, int64_t B, in
     }
     if (rc) return rc;
     return launch_tail(qv, B, d, d, nullptr, ln_w, ln_b, ln_eps, ka, kb, nsk, bias, n, k, logits_out, gates, active, st);
+}
+
+extern "C" int mortar_router_bf16(const void *x, int32_t x_is_f32, int64_t B, int32_t d, int64_t ldx, const float *wq,
+                                  const float *iter_vec, const float *ln_w, const float *ln_b, float ln_eps,
+                                  const float *ka, const float *kb, int32_t nsk, const float *bias, int32_t n,
+                                  int32_t k, float *qv, float *logits_out, float *gates, uint8_t *active,
+                                  void *stream) {
+    return launch_router(x, x_is_f32 != 0, B, d, ldx, nullptr, 0.f, nullptr, wq, iter_vec, ln_w, ln_b, ln_eps, ka, kb, nsk, bias, n, k, qv, logits_out,
+                         gates, active, stream);
+}
+
+extern "C" int mortar_norm_router_bf16(const uint16_t *x, int64_t B, int32_t d, int64_t ldx, const uint16_t *norm_w, float norm_eps, uint16_t *xn,
+                                       const float *wq, const float *iter_vec, const float *ln_w, const float *ln_b, float ln_eps,
+                                       const float *ka, const float *kb, int32_t nsk, const float *bias, int32_t n, int32_t k, float *qv,
+                                       float *logits_out, float *gates, uint8_t *active, void *stream) {
+    if (!xn) return mortar_fail(MORTAR_ERR_ARG, "norm_router: null pointer");
+    return launch_router(x, false, B, d, ldx, norm_w, norm_eps, xn, wq, iter_vec, ln_w, ln_b, ln_eps, ka, kb, nsk, bias, n, k, qv, logits_out, gates,
+                         active, stream);
 }
 
 extern "C" int mortar_router_tail_f32(const float *qv, int64_t N, int32_t d, int64_t ldq, const float *iter_vec,

@@ -172,11 +172,14 @@ int launch_gemm(const uint16_t *x, int M, int K, int64_t ldx, const float *W, in
 // pieces: operand loads straight from L2 (16 rows of 64 bytes at a power-of-two stride) took 2 us per tile.  The eight partial sums
 // of a group of 64 tokens meet in LDS.  The high terms have accumulators of their own, four chains per tile: the error stays that
 // of the wave-wide fp32 sums that this replaces.
+// NORM (M <= 16, one tile): the rows are RMS-normalised on the way into the products.  The waves share the rows' scales (rms_* of
+// mortar_device.h, the bits of rmsnorm_rows_kernel) while the weights are on their way, and the workgroups of the first outputs also
+// write the rows to xn, for the products that follow the router.  (Figures: launch_router.)
 constexpr int RS_TG = 4;                  // token tiles of 16 per group
 
-template <int CH>
+template <int CH, bool NORM>
 __global__ void __launch_bounds__(512) router_skinny_kernel(const uint16_t *x, int M, int K, int64_t ldx, const float *W, int N, const float *bias,
-                                                            float *qv, int64_t ldq) {
+                                                            float *qv, int64_t ldq, const uint16_t *nw, float eps, uint16_t *xn) {
     constexpr int WU = 8 * CH, XU = 4 * CH, XT = 16 * XU * 16;      // 16-byte units of a row piece (weights, activations); bytes of a tile
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];       // 8 waves x 2 tiles (first the weights) | partial sums
     const int tid = threadIdx.x, lane = tid & 63;
@@ -208,6 +211,33 @@ __global__ void __launch_bounds__(512) router_skinny_kernel(const uint16_t *x, i
     u32x4_t x0[CH];                        // the first tile waits in registers: its LDS holds the weights
 #pragma unroll
     for (int i = 0; i < CH; ++i) x0[i] = *reinterpret_cast<const u32x4_t *>(x_src(0, i));
+    u32x4_t w8[NORM ? CH : 1];             // norm weights of this lane's operand pieces
+    if constexpr (NORM) {
+        const int nch = K / 8;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const int k = kw + 32 * c + 8 * g;
+            w8[c] = nw ? *reinterpret_cast<const u32x4_t *>(nw + (k < K ? k : 0)) : u32x4_t{0u, 0u, 0u, 0u};
+        }
+        float *scale = reinterpret_cast<float *>(part);
+        if (wave < M) {                                             // rows wave, wave + 8
+            u32x4_t u[2][CH / 2];
+            const int m = wave, m1 = m + 8 < M ? m + 8 : m;
+#pragma unroll
+            for (int j = 0; j < CH / 2; ++j) {
+                const int ch = lane + 64 * j < nch ? lane + 64 * j : nch - 1;
+                u[0][j] = reinterpret_cast<const u32x4_t *>(x + (int64_t)m * ldx)[ch];
+                u[1][j] = reinterpret_cast<const u32x4_t *>(x + (int64_t)m1 * ldx)[ch];
+            }
+            float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+            for (int j = 0; j < CH / 2; ++j)
+                if (lane + 64 * j < nch) { s0 = rms_sumsq8(u[0][j], s0); s1 = rms_sumsq8(u[1][j], s1); }
+            s0 = rms_scale(rms_wave_sum(s0), K, eps);
+            s1 = rms_scale(rms_wave_sum(s1), K, eps);
+            if (lane == 0) { scale[m] = s0; scale[m1] = s1; }
+        }
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     u32x4_t p[CH][3];
 #pragma unroll
@@ -225,6 +255,12 @@ __global__ void __launch_bounds__(512) router_skinny_kernel(const uint16_t *x, i
 #pragma unroll
     for (int i = 0; i < CH; ++i) *reinterpret_cast<u32x4_t *>(own + i * 1024 + lane * 16) = x0[i];
     if (tile_row(1) < M) x_copy(1);
+    float rms = 0.f;
+    if constexpr (NORM) {
+        __syncthreads();
+        rms = reinterpret_cast<const float *>(part)[n < M ? n : 0];
+        __syncthreads();                   // the partial sums go where the scales were
+    }
     for (int t0 = 0; tile_row(t0) < M; t0 += RS_TG) {
         f32x4_t acc[RS_TG];
 #pragma unroll
@@ -242,6 +278,15 @@ __global__ void __launch_bounds__(512) router_skinny_kernel(const uint16_t *x, i
                 for (int c = 0; c < CH; ++c) b[c] = *reinterpret_cast<const u32x4_t *>(own + (t & 1) * XT + (n * XU + ((4 * c + g) ^ n)) * 16);
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 if (tile_row(t + 2) < M) x_copy(t + 2);
+                if constexpr (NORM) {
+                    const int m = tile_row(t) + n;
+#pragma unroll
+                    for (int c = 0; c < CH; ++c) {
+                        const int k = kw + 32 * c + 8 * g;
+                        b[c] = rms_apply8(b[c], rms, w8[c], nw != nullptr);
+                        if (blockIdx.x == 0 && m < M && k < K) *reinterpret_cast<u32x4_t *>(xn + (int64_t)m * K + k) = b[c];
+                    }
+                }
 #pragma unroll
                 for (int c = 0; c < CH; ++c) {
                     if (kw + 32 * c + 8 * g >= K) b[c] = u32x4_t{0u, 0u, 0u, 0u};
@@ -349,17 +394,18 @@ int check_launch(const char *what) {
 }  // namespace
 
 namespace {
-template <int CH>
-int launch_skinny(dim3 grid, const uint16_t *x, int M, int K, int64_t ldx, const float *W, int N, const float *bias, float *qv, int64_t ldq, hipStream_t st) {
+template <int CH, bool NORM>
+int launch_skinny(dim3 grid, const uint16_t *x, int M, int K, int64_t ldx, const float *W, int N, const float *bias, float *qv, int64_t ldq,
+                  const uint16_t *nw, float eps, uint16_t *xn, hipStream_t st) {
     constexpr int smem = 16 * (16 * 4 * CH * 16) + 8 * RS_TG * 1024;
     static_assert(smem <= 160 * 1024, "LDS of a CU");
     static bool done = false;
     if (!done) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(router_skinny_kernel<CH>), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(router_skinny_kernel<CH, NORM>), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "router projection: %s", hipGetErrorString(e));
         done = true;
     }
-    hipLaunchKernelGGL(router_skinny_kernel<CH>, grid, dim3(512), smem, st, x, M, K, ldx, W, N, bias, qv, ldq);
+    hipLaunchKernelGGL((router_skinny_kernel<CH, NORM>), grid, dim3(512), smem, st, x, M, K, ldx, W, N, bias, qv, ldq, nw, eps, xn);
     return check_launch("router projection");
 }
 }  // namespace
@@ -371,14 +417,17 @@ static int64_t skinny_rounds(int64_t M, int32_t d_out) {
 }
 
 int mortar_router_project_skinny(const uint16_t *x, int64_t M, int32_t d_in, int64_t ldx, const float *wq, int32_t d_out, const float *bias,
-                                 float *qv, int64_t ldq, void *stream) {
+                                 float *qv, int64_t ldq, void *stream, const uint16_t *norm_w, float eps, uint16_t *xn) {
     const int nt = (d_out + 15) / 16;
     const int64_t groups = (M + 16 * RS_TG - 1) / (16 * RS_TG), rounds = skinny_rounds(M, d_out);
     const int64_t gy = (groups + rounds - 1) / rounds;
     const dim3 grid((unsigned)nt, (unsigned)gy);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (d_in <= 1024) return launch_skinny<4>(grid, x, (int)M, d_in, ldx, wq, d_out, bias, qv, ldq, st);
-    return launch_skinny<8>(grid, x, (int)M, d_in, ldx, wq, d_out, bias, qv, ldq, st);
+    if (d_in <= 1024)
+        return xn ? launch_skinny<4, true>(grid, x, (int)M, d_in, ldx, wq, d_out, bias, qv, ldq, norm_w, eps, xn, st)
+                  : launch_skinny<4, false>(grid, x, (int)M, d_in, ldx, wq, d_out, bias, qv, ldq, nullptr, 0.f, nullptr, st);
+    return xn ? launch_skinny<8, true>(grid, x, (int)M, d_in, ldx, wq, d_out, bias, qv, ldq, norm_w, eps, xn, st)
+              : launch_skinny<8, false>(grid, x, (int)M, d_in, ldx, wq, d_out, bias, qv, ldq, nullptr, 0.f, nullptr, st);
 }
 
 extern "C" int mortar_router_project_bf16(const uint16_t *x, int64_t M, int32_t d_in, int64_t ldx, const float *wq, int32_t d_out, float *qv,

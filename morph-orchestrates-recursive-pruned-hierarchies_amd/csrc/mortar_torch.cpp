@@ -234,10 +234,8 @@ PyObject *py_routed_decode(PyObject *, PyObject *const *a, Py_ssize_t na) {
     const at::Tensor ws = at::empty({M * (d + n)}, x.options().dtype(at::kFloat).requires_grad(false));
     float *qv = static_cast<float *>(ws.data_ptr()), *gates = qv + M * d;
     at::Tensor y = new_bf16(x, {M, 1, (int64_t)dn->w->Rb * 16});
-    int rc = mortar_rmsnorm_bf16(u16(x), M, (int32_t)d, d, nm.w, nm.eps, u16m(xn), d, st);
-    if (rc == MORTAR_OK)
-        rc = mortar_router_bf16(u16(xn), 0, M, (int32_t)d, d, r.wq, r.iter_vec, r.ln_w, r.ln_b, (float)ln_eps, r.ka, r.kb, r.nsk, r.bias,
-                                r.n, (int32_t)sh[3], qv, nullptr, gates, nullptr, st);
+    int rc = mortar_norm_router_bf16(u16(x), M, (int32_t)d, d, nm.w, nm.eps, u16m(xn), r.wq, r.iter_vec, r.ln_w, r.ln_b, (float)ln_eps, r.ka, r.kb,
+                                     r.nsk, r.bias, r.n, (int32_t)sh[3], qv, nullptr, gates, nullptr, st);
     if (rc == MORTAR_OK) rc = run_mlp(gu, dn, xn, M, Norm{}, gates, (int)n, u16m(y), st);
     if (rc) return raise_rc(rc, "mortar_routed_decode");
     return THPVariable_Wrap(std::move(y));

@@ -235,3 +235,30 @@ def test_mid_sized_products(dev, units, in_b, density, M, one_scale):
             if ops.norm_fusable(W):
                 nw = (1 + 0.1 * torch.randn(K, device=dev)).to(torch.bfloat16)
                 assert torch.equal(ops.gateup_swiglu(xd, W, norm=(nw, 1e-6)), ops.gateup_swiglu(ops.rmsnorm(xd, nw, 1e-6), W))
+
+
+@pytest.mark.parametrize("d,nsk,n", [(8, 2, 4), (264, 4, 16), (1024, 4, 16), (1032, 19, 352), (2048, 4, 16), (2056, 4, 16)])      # one wave's piece, ragged, both widths, too wide
+@pytest.mark.parametrize("B", [1, 2, 4, 5, 16, 17, 33, 64])
+@pytest.mark.parametrize("weight", [True, False])
+def test_router_with_the_norm_inside_gives_the_bits_of_both_launches(dev, d, nsk, n, B, weight):
+    g = torch.Generator(device=dev).manual_seed(B)
+    rand = lambda *s: torch.randn(*s, device=dev, generator=g)
+    x = (3 * rand(B, d)).to(torch.bfloat16)
+    nw = (1 + 0.1 * rand(d)).to(torch.bfloat16) if weight else None
+    wq, it, lnw, lnb, bias = rand(d, d) / d ** 0.5, rand(d), rand(d), rand(d), rand(n)
+    ka, kb = rand(nsk, d // 2), rand(nsk, d // 2)
+    want_x = ops.rmsnorm(x, nw, 1e-5)
+    outs = []
+    for fused in (False, True):
+        xn = torch.full((B + 1, d), 7.0, dtype=torch.bfloat16, device=dev)
+        qv, gates = torch.empty(B, d, device=dev), torch.empty(B, n, device=dev)
+        p = lambda t: None if t is None else t.data_ptr()
+        tail = (p(wq), p(it), p(lnw), p(lnb), 1e-5, p(ka), p(kb), nsk, p(bias), n, max(1, n // 4), p(qv), None, p(gates), None,
+                torch.cuda.current_stream().cuda_stream)
+        if fused:
+            _lib.check(_lib.lib().mortar_norm_router_bf16(p(x), B, d, d, p(nw), 1e-5, p(xn), *tail), "norm_router")
+            assert torch.equal(xn[:B], want_x) and (xn[B] == 7).all()
+        else:
+            _lib.check(_lib.lib().mortar_router_bf16(p(want_x), 0, B, d, d, *tail), "router")
+        outs.append((qv, gates))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
