@@ -8,17 +8,14 @@
 // dwords into `codes`, the octet stream and its 4-bit copy.
 #include <hip/hip_runtime.h>
 
+#include "mortar_device.h"
 #include "mortar_internal.h"
+
+#include <type_traits>
 
 namespace {
 
 constexpr int PARTIALS = 256;           // workgroups of the |w| reduction; the workspace holds one double each
-
-__device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    return x;
-}
 
 // sum |w| over all values -> partial[blockIdx] (fixed order: the result does not depend on timing).  n is a multiple
 // of 256 (whole blocks) and the array is 16-byte aligned, so every thread reads 16-byte pieces.
@@ -59,7 +56,7 @@ __device__ __forceinline__ void abs_sum(const void *values, int64_t n, int f32, 
         for (int u = 0; u < 8; ++u)
             if (i + u * STEP < m) add(q[u]);
     }
-    s = wave_sum(s);
+    s = mortar_wave_sum(s);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) partial[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
@@ -133,15 +130,17 @@ __device__ __forceinline__ void requant(const RequantArgs &a, int block) {
     }
     float s;
     if (a.mode == 0) {
-        const double t = wave_sum((a.partial[lane] + a.partial[lane + 64]) + (a.partial[lane + 128] + a.partial[lane + 192]));
+        const double t = mortar_wave_sum((a.partial[lane] + a.partial[lane + 64]) + (a.partial[lane + 128] + a.partial[lane + 192]));
         s = fmaxf((float)(t / ((double)a.nnz * 256.0)), 1e-8f);
     } else if (a.mode == 1) {
         double t[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             t[q] = ((double)fabsf(w[4 * q]) + (double)fabsf(w[4 * q + 1])) + ((double)fabsf(w[4 * q + 2]) + (double)fabsf(w[4 * q + 3]));
-#pragma unroll
-            for (int o = 8; o > 0; o >>= 1) t[q] += __shfl_xor(t[q], o);
+            t[q] += mortar_row_xor<8>(t[q]);
+            t[q] += mortar_row_xor<4>(t[q]);
+            t[q] += mortar_row_xor<2>(t[q]);
+            t[q] += mortar_row_xor<1>(t[q]);
         }
         s = fmaxf((float)(((t[0] + t[2]) + (t[1] + t[3])) * (1.0 / 256.0)), 1e-6f);
     } else {
@@ -189,14 +188,15 @@ __device__ __forceinline__ void requant(const RequantArgs &a, int block) {
     }
     if (sd == 0) row = 0;
     if (a.transpose) {                                  // 16 x 16 codes across the 16 lanes of the block
-        auto turn = [&](int o, int bits, uint32_t low) {        // swaps the off-diagonal halves of every 2 o x 2 o square
-            const uint32_t other = (uint32_t)__shfl_xor((int)row, o);
+        auto turn = [&](auto distance, int bits, uint32_t low) {        // swaps the off-diagonal halves of every 2 o x 2 o square
+            constexpr int o = decltype(distance)::value;
+            const uint32_t other = mortar_row_xor<o>(row);
             row = (n & o) ? (row & ~low) | ((other & ~low) >> bits) : (row & low) | ((other & low) << bits);
         };
-        turn(8, 16, 0x0000ffffu);
-        turn(4, 8, 0x00ff00ffu);
-        turn(2, 4, 0x0f0f0f0fu);
-        turn(1, 2, 0x33333333u);
+        turn(std::integral_constant<int, 8>{}, 16, 0x0000ffffu);
+        turn(std::integral_constant<int, 4>{}, 8, 0x00ff00ffu);
+        turn(std::integral_constant<int, 2>{}, 4, 0x0f0f0f0fu);
+        turn(std::integral_constant<int, 1>{}, 2, 0x33333333u);
     }
     // device order of a row: column c < 8 in field 2 c + 1, column c >= 8 in field 2 (c - 8)
     auto spread = [](uint32_t x) {

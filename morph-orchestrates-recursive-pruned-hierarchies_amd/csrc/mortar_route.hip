@@ -23,11 +23,7 @@ __device__ __forceinline__ float key_to_float(uint32_t k) {
     return __builtin_bit_cast(float, u);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
+__device__ __forceinline__ float wave_sum(float v) { return mortar_wave_sum(v); }
 
 // Sum over the wavefront with DPP adds only (no LDS crossbar): quads, half rows, rows, then the row broadcasts; the total
 // arrives in the last row and is read from lane 63.  Adds in another order than wave_sum, so not for results that have
@@ -93,12 +89,7 @@ __device__ __forceinline__ void remoe_gates_wave(const float *lp, int n, int k, 
             uint32_t m = 0;
 #pragma unroll
             for (int i = 0; i < MAXPL; ++i) m = (key[i] >> (bit + 1)) == (prefix >> (bit + 1)) && key[i] > m ? key[i] : m;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const uint32_t t = (uint32_t)__shfl_xor((int)m, o, 64);
-                m = t > m ? t : m;
-            }
-            prefix = m;
+            prefix = mortar_wave_reduce(m, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
         }
         kth = key_to_float(prefix);
     }
@@ -690,6 +681,13 @@ __global__ void __launch_bounds__(256, J == 8 ? 2 : 3) router_tail_group_kernel(
 //                          of one token per chunk in registers from the one read of the row to the products.
 //   router_rank_kernel     one wave per token: logits (ranked when there are more products than groups), gating tail.
 // The scores travel in the token's own row of `gates` (2 nsk <= n), which the second kernel reads before it writes it.
+__device__ __forceinline__ float rows_sum(float v) {             // over the four 16-lane rows: lanes ^ 16, then ^ 32
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 template <int KT, int CH>     // key tiles of 16 per half, chunks of 16 values per wave
 __global__ void __launch_bounds__(512) router_scores_kernel(const float *qv, int64_t N, int d, int64_t ldq, const float *iter_vec,
                                                              const float *ln_w, const float *ln_b, float ln_eps, const float *ka,
@@ -744,8 +742,7 @@ __global__ void __launch_bounds__(512) router_scores_kernel(const float *qv, int
         if (at(j) >= d2) v[j] = zero4;
         s += (v[j].x + v[j].y) + (v[j].z + v[j].w);
     }
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
+    s = rows_sum(s);
     if (g == 0) red[0][wave][tok] = s;
     __syncthreads();
     float mean = 0.f;
@@ -760,8 +757,7 @@ __global__ void __launch_bounds__(512) router_scores_kernel(const float *qv, int
             s = __builtin_fmaf(e, e, __builtin_fmaf(c, c, __builtin_fmaf(b, b, __builtin_fmaf(a, a, s))));
         }
     }
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
+    s = rows_sum(s);
     if (g == 0) red[1][wave][tok] = s;
     __syncthreads();
     float var = 0.f;

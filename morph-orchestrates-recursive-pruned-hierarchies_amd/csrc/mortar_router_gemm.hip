@@ -346,8 +346,7 @@ __global__ void __launch_bounds__(1024) router_stats_part_kernel(const float *ga
 }
 
 __device__ __forceinline__ double block_sum_f64(double v, double *red) {      // 1024 threads
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    v = mortar_wave_sum(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
