@@ -42,20 +42,9 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
-// Sum of a per-lane count over the wavefront with DPP adds only (quads, half rows, rows, then the row broadcasts): the
-// total arrives in the lanes of the last row and is read from lane 63.
-__device__ __forceinline__ int wave_count_total(uint32_t v) {
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false);    // quad_perm [1,0,3,2]
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false);    // quad_perm [2,3,0,1]
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false);   // row_half_mirror
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false);   // row_mirror
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
-    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
-    return __builtin_amdgcn_readlane((int)v, 63);
-}
-
 // Gating tail of one token on one wavefront.  The k-th largest logit is found exactly by an MSB-first radix
-// select on order-preserving keys: for each bit the wave counts the keys >= the candidate prefix.  Ties need no special care: the result is a VALUE, and the gate rule is `logit > kth`.
+// select on order-preserving keys: for each bit the wave counts the keys >= the candidate prefix (ballots and scalar
+// counts: with four waves to a SIMD the vector ALU is what is short; 17.6 -> 12.9 us with the sort below, 4096 tokens x 352 groups).  Ties need no special care: the result is a VALUE, and the gate rule is `logit > kth`.
 // `lp` may point to global memory or LDS; gates / active are this token's output rows.
 template <int MAXPL>      // logits per lane this instantiation holds: n <= 64 * MAXPL
 __device__ __forceinline__ void remoe_gates_wave(const float *lp, int n, int k, float *gates, uint8_t *active, int lane) {
@@ -69,7 +58,17 @@ __device__ __forceinline__ void remoe_gates_wave(const float *lp, int n, int k, 
     }
     float kth = 0.f;
     const bool thresh = k < n;
-    if (thresh) {
+    if (thresh && MAXPL == 1 && n <= 32) {
+        // few groups: every lane counts the keys above its own and those not below it; the k-th largest is where k lies between
+        int above = 0, from = 0;
+        for (int j = 0; j < n; ++j) {
+            const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)key[0], j);
+            above += o > key[0] ? 1 : 0;
+            from += o >= key[0] ? 1 : 0;
+        }
+        const uint64_t at = __ballot(lane < n && above < k && k <= from);
+        kth = key_to_float((uint32_t)__builtin_amdgcn_readlane((int)key[0], __builtin_ctzll(at)));
+    } else if (thresh) {
         // [prefix, prefix + 2^(bit+1)) is the bucket that holds the k-th largest key: c_lo keys are >= its lower end, c_hi keys
         // >= its upper end.  Once the bucket holds ONE key that key is the answer and the remaining bits need no counting
         // (distinct logits get there after about log2(n) + the exponent bits they share; exact ties walk all 32 bits).
@@ -77,12 +76,9 @@ __device__ __forceinline__ void remoe_gates_wave(const float *lp, int n, int k, 
         int c_lo = 64 * MAXPL, c_hi = 0, bit = 31;
         for (; bit >= 0 && c_lo - c_hi > 1; --bit) {
             const uint32_t cand = prefix | (1u << bit);
-            // counted on the vector ALU: a ballot + scalar popcount per key would queue on the one scalar ALU that the
-            // sixteen waves of a CU share
-            uint32_t own = 0;
+            int c = 0;
 #pragma unroll
-            for (int i = 0; i < MAXPL; ++i) own += key[i] >= cand ? 1u : 0u;             // padding keys are 0 < cand
-            const int c = wave_count_total(own);
+            for (int i = 0; i < MAXPL; ++i) c += (int)__popcll(__ballot(key[i] >= cand));            // padding keys are 0 < cand
             if (c >= k) { prefix = cand; c_lo = c; } else { c_hi = c; }
         }
         if (bit >= 0) {                       // left early: the bucket's one key (bits 0..bit of it were never looked at)
@@ -248,61 +244,93 @@ __device__ __forceinline__ float block_sum256(float v, float *red) {      // red
     return red[0] + red[1] + red[2] + red[3];
 }
 
-// The value of lane (lane ^ X), X a power of two: DPP within quads and 16-lane rows, the LDS crossbar for 4, half-wave and
-// row swaps of gfx950 for 16 and 32.
-template <int X>
-__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
-    if constexpr (X == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true);          // quad_perm [1,0,3,2]
-    else if constexpr (X == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true);     // quad_perm [2,3,0,1]
-    else if constexpr (X == 4) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, 0x101F);                // xor 4
-    else if constexpr (X == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true);    // row_ror:8
-    else return (uint32_t)__shfl_xor((int)v, X, 64);
+// Descending sort of 64 * KPL keys held KPL per lane (element lane * KPL + r in register r), KPL a power of two or three times one: a
+// bitonic sort whose runs start at KPL keys instead of one.  Every lane sorts its own; then runs of L lanes alternate in direction and are
+// merged, by exchanges between lanes (half-wave and row swaps, DPP: no LDS) and a merge inside the lane.  A bitonic sequence of any even
+// length falls into two bitonic halves, so a lane's KPL need not be a power of two.  Lanes of ascending runs hold inverted keys, so that
+// no comparison inside a lane needs a select.  What counts is the number of instructions, with four waves to a SIMD: 361 keys in 6 per lane
+// 520 of them, where 512 padded ones in 8 per lane took 1000: router_rank_kernel at 4096
+// tokens 17.6 -> 14.2 us, a routed decode step of one row with 128 clusters (144 keys, 4 per lane) 21.7 -> 19.0.
+__device__ __forceinline__ void sort_cx(uint32_t &a, uint32_t &b) {
+    const uint32_t hi = a > b ? a : b, lo = a > b ? b : a;
+    a = hi;
+    b = lo;
 }
-
-// Descending bitonic sort of 64 * KPL keys held KPL per lane (element lane * KPL + r in register r): steps between
-// elements of one lane are register compare-exchanges, steps between lanes one exchange per register.  No LDS memory, no
-// barrier.  Fully unrolled: every exchange distance is a constant (lane_xor), which a loop over shuffles cannot have.
-template <int KPL, int LJ>
-__device__ __forceinline__ void sort_lane_step(uint32_t (&key)[KPL], bool keep_max) {
+template <int N, int O, int KPL>
+__device__ __forceinline__ void sort_three(uint32_t (&key)[KPL]) {
+    sort_cx(key[O], key[O + 1]);
+    sort_cx(key[O + 1], key[O + 2]);
+    sort_cx(key[O], key[O + 1]);
+}
+template <int N, int O, int KPL>
+__device__ __forceinline__ void sort_merge(uint32_t (&key)[KPL]) {          // key[O .. O + N) bitonic
+    if constexpr (N == 3) sort_three<N, O>(key);
+    else if constexpr (N > 1) {
 #pragma unroll
-    for (int r = 0; r < KPL; ++r) {
-        const uint32_t a = key[r], o = lane_xor<LJ>(a);
-        const uint32_t hi = a > o ? a : o, lo = a > o ? o : a;
-        key[r] = keep_max ? hi : lo;
+        for (int i = 0; i < N / 2; ++i) sort_cx(key[O + i], key[O + N / 2 + i]);
+        sort_merge<N / 2, O>(key);
+        sort_merge<N / 2, O + N / 2>(key);
     }
 }
-template <int KPL, int K2>
-__device__ __forceinline__ void sort_stage(uint32_t (&key)[KPL], int lane) {
-    const bool lane_desc = ((lane * KPL) & K2) == 0;           // direction of this lane's elements once K2 >= KPL
-    auto step = [&](auto lj) {
-        constexpr int LJ = decltype(lj)::value;
-        if constexpr (LJ * KPL * 2 <= K2) sort_lane_step<KPL, LJ>(key, ((lane & LJ) == 0) == lane_desc);
-    };
-    step(std::integral_constant<int, 32>{});
-    step(std::integral_constant<int, 16>{});
-    step(std::integral_constant<int, 8>{});
-    step(std::integral_constant<int, 4>{});
-    step(std::integral_constant<int, 2>{});
-    step(std::integral_constant<int, 1>{});
+template <int N, int O, int KPL>
+__device__ __forceinline__ void sort_lane(uint32_t (&key)[KPL]) {
+    if constexpr (N == 3) sort_three<N, O>(key);
+    else if constexpr (N > 1) {
+        sort_lane<N / 2, O>(key);
+        sort_lane<N / 2, O + N / 2>(key);
 #pragma unroll
-    for (int j = KPL / 2; j > 0; j >>= 1) {                      // partners in this lane's registers (distance j < K2)
-        if (j < K2) {
+        for (int i = 0; i < N / 2; ++i) sort_cx(key[O + i], key[O + N - 1 - i]);
+        sort_merge<N / 2, O>(key);
+        sort_merge<N / 2, O + N / 2>(key);
+    }
+}
+template <int LJ, int KPL>
+__device__ __forceinline__ void sort_exchange(uint32_t (&key)[KPL], int lane) {      // the larger key to the lane with bit LJ clear
+    if constexpr (LJ >= 16) {
+        // the swap brings two keys' partners to the same lane, a second one takes the results back
 #pragma unroll
-            for (int r = 0; r < KPL; ++r) {
-                if ((r & j) == 0) {
-                    const bool desc = K2 < KPL ? (r & K2) == 0 : lane_desc;
-                    const uint32_t a = key[r], c = key[r | j];
-                    const uint32_t hi = a > c ? a : c, lo = a > c ? c : a;
-                    key[r] = desc ? hi : lo;
-                    key[r | j] = desc ? lo : hi;
-                }
-            }
+        for (int r = 0; r < KPL; r += 2) {
+            const auto s = LJ == 32 ? __builtin_amdgcn_permlane32_swap(key[r], key[r + 1], false, false)
+                                    : __builtin_amdgcn_permlane16_swap(key[r], key[r + 1], false, false);
+            uint32_t hi = s[0], lo = s[1];
+            sort_cx(hi, lo);
+            const auto t = LJ == 32 ? __builtin_amdgcn_permlane32_swap(hi, lo, false, false) : __builtin_amdgcn_permlane16_swap(hi, lo, false, false);
+            key[r] = t[0];
+            key[r + 1] = t[1];
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < KPL; ++r) {
+            const uint32_t a = key[r], o = mortar_row_xor<LJ>(a);
+            const uint32_t hi = a > o ? a : o, lo = a > o ? o : a;
+            key[r] = (lane & LJ) == 0 ? hi : lo;
         }
     }
-    if constexpr (K2 < 64 * KPL) sort_stage<KPL, K2 * 2>(key, lane);
+}
+template <int L, int KPL>
+__device__ __forceinline__ void sort_runs(uint32_t (&key)[KPL], int lane) {          // runs of L lanes from runs of L / 2
+    const bool was_up = (lane & (L / 2)) != 0, up = L < 64 && (lane & L) != 0;
+    const uint32_t flip = was_up != up ? ~0u : 0u;
+#pragma unroll
+    for (int r = 0; r < KPL; ++r) key[r] ^= flip;
+    if constexpr (L >= 64) sort_exchange<32>(key, lane);
+    if constexpr (L >= 32) sort_exchange<16>(key, lane);
+    if constexpr (L >= 16) sort_exchange<8>(key, lane);
+    if constexpr (L >= 8) sort_exchange<4>(key, lane);
+    if constexpr (L >= 4) sort_exchange<2>(key, lane);
+    sort_exchange<1>(key, lane);
+    sort_merge<KPL, 0>(key);
+    if constexpr (L < 64) sort_runs<L * 2>(key, lane);
 }
 template <int KPL>
-__device__ __forceinline__ void wave_sort_desc(uint32_t (&key)[KPL], int lane) { sort_stage<KPL, 2>(key, lane); }
+__device__ __forceinline__ void wave_sort_desc(uint32_t (&key)[KPL], int lane) {
+    static_assert(KPL % 2 == 0, "exchanges of two keys");
+    const uint32_t flip = (lane & 1) ? ~0u : 0u;
+#pragma unroll
+    for (int r = 0; r < KPL; ++r) key[r] ^= flip;
+    sort_lane<KPL, 0>(key);
+    sort_runs<2>(key, lane);
+}
 
 // The n largest of the P = nsk * nsk product scores of one token in descending order (+ bias) -> lgt[0 .. n), on one wave.
 template <int KPL>
@@ -331,6 +359,14 @@ __device__ __attribute__((noinline)) void ranked_logits(const float *sct, int ns
             if (logits_row) logits_row[g] = l;
         }
     }
+}
+
+__device__ __forceinline__ void rank_products(const float *sct, int nsk, int P, const float *bias, int n, float *lgt, float *logits_row, int lane) {
+    if (P <= 128) ranked_logits<2>(sct, nsk, P, bias, n, lgt, logits_row, lane);
+    else if (P <= 256) ranked_logits<4>(sct, nsk, P, bias, n, lgt, logits_row, lane);
+    else if (P <= 384) ranked_logits<6>(sct, nsk, P, bias, n, lgt, logits_row, lane);
+    else if (P <= 512) ranked_logits<8>(sct, nsk, P, bias, n, lgt, logits_row, lane);
+    else ranked_logits<16>(sct, nsk, P, bias, n, lgt, logits_row, lane);           // P <= 1024
 }
 
 // Launch 2, one workgroup per token: LayerNorm(qv) -> sub-key scores of the two query halves -> product-key logits
@@ -444,10 +480,7 @@ __global__ void __launch_bounds__(256) router_tail_kernel(const float *qv, int d
         // up to 1024 products, through LDS by the whole workgroup beyond.
         if (P <= 1024) {           // one wave ranks them in its registers (no LDS traffic, no barrier per step)
             float *lrow = logits_out ? logits_out + (int64_t)b * n : nullptr;
-            if (wave == 0) {
-                if (P <= 512) ranked_logits<8>(sc, nsk, P, bias, n, lg, lrow, lane);
-                else ranked_logits<16>(sc, nsk, P, bias, n, lg, lrow, lane);
-            }
+            if (wave == 0) rank_products(sc, nsk, P, bias, n, lg, lrow, lane);
         } else {
             uint32_t *sk = reinterpret_cast<uint32_t *>(red + 4);
             int P2 = 1;
@@ -650,8 +683,7 @@ __global__ void __launch_bounds__(256, J == 8 ? 2 : 3) router_tail_group_kernel(
             float *lrow = logits_out ? logits_out + (g0 + t) * n : nullptr;
             if (P > n) {
                 // more product keys than groups: the n largest product scores in descending order (routing.py:212-222)
-                if (P <= 512) ranked_logits<8>(sct, nsk, P, bias, n, lgt, lrow, lane);
-                else ranked_logits<16>(sct, nsk, P, bias, n, lgt, lrow, lane);        // the host admits P <= 1024
+                rank_products(sct, nsk, P, bias, n, lgt, lrow, lane);        // the host admits P <= 1024
             } else {
                 for (int g = lane; g < n; g += 64) {
                     const int pr = g % P;
@@ -818,8 +850,7 @@ __global__ void __launch_bounds__(256) router_rank_kernel(int64_t N, int nsk, co
     };
     wave_fence();
     if (P > n) {
-        if (P <= 512) ranked_logits<8>(sct, nsk, P, bias, n, lgt, lrow, lane);
-        else ranked_logits<16>(sct, nsk, P, bias, n, lgt, lrow, lane);
+        rank_products(sct, nsk, P, bias, n, lgt, lrow, lane);
     } else {
         for (int g = lane; g < n; g += 64) {
             const int pr = g % P;
@@ -1068,7 +1099,9 @@ extern "C" int mortar_router_tail_f32(const float *qv, int64_t N, int32_t d, int
         const size_t rs = (size_t)4 * (2 * nsk + n) * sizeof(float);
         const int pl = (n + 63) / 64;
 #define MORTAR_RANK(PL) hipLaunchKernelGGL((router_rank_kernel<PL>), rg, dim3(256), rs, st, N, nsk, bias, n, k, logits_out, gates, active)
-        if (pl <= 2) MORTAR_RANK(2);
+        if (pl <= 1) MORTAR_RANK(1);
+        else if (pl <= 2) MORTAR_RANK(2);
+        else if (pl <= 4) MORTAR_RANK(4);
         else if (pl <= 6) MORTAR_RANK(6);
         else MORTAR_RANK(16);
 #undef MORTAR_RANK

@@ -153,3 +153,37 @@ def test_projection_keeps_non_finite_values_to_their_row_and_output(dev, M, d_in
     x[:, d_in - 1] = 2.0 ** -8
     w = torch.full((d_out, d_in), torch.finfo(torch.float32).max, device=dev)
     assert torch.equal(_project(x, w), (w[:, -1] * 2.0 ** -8).expand(M, -1))
+
+
+@pytest.mark.parametrize("nsk", [2, 11, 12, 16, 17, 19, 20, 22, 23, 32])       # 2, 4, 6, 8 and 16 keys per lane, the smallest and largest of each
+@pytest.mark.parametrize("N", [3, 530])                                      # a workgroup per token, a wave per token
+def test_ranked_products_are_the_sorted_direct_ones(dev, nsk, N):
+    """The logits of P - 1 groups under P = nsk^2 product keys against those of P groups, sorted: the same sums, bit for bit."""
+    d, P = 64, nsk * nsk
+    g = torch.Generator(device=dev).manual_seed(nsk)
+    qv = torch.randn(N, d, device=dev, generator=g)
+    qv[0] = 0                                                                # exact ties
+    ka, kb = (torch.randn(nsk, d // 2, device=dev, generator=g) for _ in range(2))
+    one, zero = torch.ones(d, device=dev), torch.zeros(max(d, P), device=dev)
+
+    def logits(n):
+        out, gates = torch.empty(N, n, device=dev), torch.empty(N, n, device=dev)
+        _lib.check(_lib.lib().mortar_router_tail_f32(qv.data_ptr(), N, d, d, None, one.data_ptr(), zero.data_ptr(), 1e-5, ka.data_ptr(), kb.data_ptr(), nsk,
+                                                     zero.data_ptr(), n, 1, out.data_ptr(), gates.data_ptr(), None,
+                                                     torch.cuda.current_stream().cuda_stream), "tail")
+        return out
+    assert torch.equal(logits(P - 1), logits(P).sort(-1, descending=True).values[:, :P - 1])
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 16, 31, 32, 33, 64])
+def test_gates_of_few_groups_with_ties(dev, n):
+    g = torch.Generator(device=dev).manual_seed(n)
+    logits = torch.randint(-3, 4, (67, n), device=dev, generator=g).float()
+    logits[1] = torch.randn(n, device=dev, generator=g)
+    for k in range(1, n + 1):
+        gates = torch.empty(67, n, device=dev)
+        _lib.check(_lib.lib().mortar_remoe_gates(logits.data_ptr(), 67, n, k, gates.data_ptr(), None, torch.cuda.current_stream().cuda_stream), "gates")
+        kth = logits.topk(k, -1).values[:, -1:] if k < n else torch.zeros(67, 1, device=dev)
+        r = torch.relu(logits - kth).double()
+        want = r * k / r.sum(-1, keepdim=True).clamp(min=1e-6)
+        assert torch.equal(gates > 0, want > 0) and torch.allclose(gates.double(), want, rtol=64 * 2.0 ** -24)      # a sum of up to 64, a quotient, a product
