@@ -251,6 +251,15 @@ int launch_pw(int pw, SpmmParams &p, const GemvOneArgs &a, hipStream_t st) {
 
 template <int NACC>
 int launch_t(int t, int pw, SpmmParams &p, const GemvOneArgs &a, hipStream_t st) {
+    // The plain product takes the smallest tile that still is one round of the chip: a workgroup stages its tokens' fp32 values of all K,
+    // which costs more than the weights read by another tile (5632 inputs, 2048 outputs, 4 rows in tiles of 4 / 2 / 1 tokens 5.8 / 4.3 / - us,
+    // 8 rows 6.1 / 4.7 / -; 4096 inputs, 1536 outputs, 4 rows 5.1 / 4.1).  The SwiGLU form reads twice the weights of a narrower tile:
+    // d_model 1536, 4 rows 4.6 -> 4.2 at density 0.25, but 2 rows at 0.5 4.1 -> 4.7.
+    if (NACC == 1) {
+        int rc = t > 1 ? launch_chunk<1, NACC>(p, a, st) : -1;
+        if (rc < 0 && t > 2) rc = launch_chunk<2, NACC>(p, a, st);
+        if (rc >= 0) return rc;
+    }
     switch (t) {
         case 1: return launch_pw<1, NACC>(pw, p, a, st);
         case 2: return launch_pw<2, NACC>(pw, p, a, st);
