@@ -169,11 +169,17 @@ static int smallm_launch_code(int kind, SpmmParams &p, const SpmmParams *table, 
         return -1;
     }
     if (!table && layers == 1 && kind <= 1) {
-        // Few units: chunks of the row parts over the whole chip.  4-token tiles where a product has them (gate_up: up to 4 rows); 8-token
+        // Few units: chunks of the row parts over the whole chip.  4-token tiles where a product has them (gate_up: up to 4 rows, and see below); 8-token
         // ones only where 4-token ones are more than a round of the chip, whose smaller tiles are staged faster (`down` of d_model
         // 3072, 9..16 rows: 5.0 against 5.4 us in chunks of 8-token tiles).
         int rc = -1;
-        const bool four = fits(4, p.Cb) && (kind == 0 ? (p.M + 3) / 4 * (int64_t)((p.n_units + 3) / 4) <= 256 : p.M <= 4);
+        // gate_up with the norm in it: a workgroup normalises its whole tile, so half the tile is worth twice the workgroups where the chunked
+        // form keeps its two units and two waves per part (us, 8 rows, density 0.25: d_model 768 4.3 -> 3.9, 1024 4.4 -> 4.0, 1536 5.0 -> 4.4; 16
+        // rows, 768 4.4 -> 4.0), and the bits are those of the 8-token tile.  Without the norm 3 % slower, and parts of four octets and more
+        // have the one-unit form of the 8-token tile (1536 at density 0.5, 8 rows: 5.05 against 5.12).
+        const int64_t tiles4 = (p.M + 3) / 4;
+        const bool narrow = p.norm && p.nseg == 1 && p.avg_octets < 4 && tiles4 * ((p.n_units + 1) / 2) <= 256;
+        const bool four = fits(4, p.Cb) && (kind == 0 ? tiles4 * ((p.n_units + 3) / 4) <= 256 : p.M <= 4 || (!p.gates && narrow));
         if (four) rc = mortar_chunk_launch(kind, 4, p, st);
         else if (p.M > 4 && fits(8, p.Cb)) rc = mortar_chunk_launch(kind, 8, p, st);
         if (rc >= 0) return rc;

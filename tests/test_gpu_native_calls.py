@@ -157,7 +157,7 @@ def test_fp32_decode_products_of_few_units(dev, units, in_b, density, B):
 
 @pytest.mark.parametrize("units,in_b,density,zipf", [(1, 2, 1.0, None), (5, 9, 0.3, None), (37, 128, 0.25, None), (37, 128, 0.2, 1.3), (130, 200, 0.05, None),
                                                      (9, 352, 0.25, 1.2), (64, 352, 0.02, None), (3, 620, 0.25, None),
-                                                     (350, 100, 0.04, None)])
+                                                     (350, 100, 0.04, None), (128, 48, 0.25, None)])
 @pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 33])
 @pytest.mark.parametrize("one_scale", [False, True])
 def test_decode_products_of_few_units(dev, units, in_b, density, zipf, M, one_scale):
