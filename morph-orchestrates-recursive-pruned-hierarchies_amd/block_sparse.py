@@ -256,6 +256,8 @@ class CMSBlockLinear(nn.Module):
         """Re-encodes the values of up to two QAT layers (layer, whether its W^T is needed too) for a training step, in two
         launches; mortar_pack() and mortar_pack_t() then find them fresh until the values change again."""
         jobs = [(m._qat_pack(), m._values(), m._values_threshold, with_t) for m, with_t in layers]
+        for m, _ in layers:
+            m.invalidate_pack()               # fresh once the launches are enqueued, not if they fail
         for (m, with_t), scale in zip(layers, MortarPack.requantize_pairs(jobs)):
             m._pack_scale, m._pack_key = scale, (m.mortar_data.data_ptr(), m.mortar_data._version)
             m._pack_gen += 1
@@ -263,8 +265,8 @@ class CMSBlockLinear(nn.Module):
                 m._pack_t_gen = m._pack_gen
 
     def step_pack(self, with_t: bool) -> MortarPack | None:
-        """The pack for a native training step that re-encodes the values into it (and into its transpose) itself; the state of the
-        layer is that behind ``repack_for_step``.  None where the step has to take the general path."""
+        """The pack for a native training step that re-encodes the values into it (and into its transpose) itself.  It counts as stale
+        until ``step_packed`` says that the step has done so.  None where the step has to take the general path."""
         d = self._parameters.get("mortar_data")
         if (type(self) is not CMSBlockLinear or d is None or self._mortar_blocking != 16 or not self._values_ternary_mode
                 or "mortar_packed" in self._buffers or not d.is_cuda or d.dtype not in (torch.bfloat16, torch.float32)
@@ -273,25 +275,37 @@ class CMSBlockLinear(nn.Module):
         W = self._qat_pack()
         if W.device != d.device or d.shape[0] != W.nnz:
             return None
-        if W._pos is None:
-            W._before_repack(d.detach())
-        W.before_pair_repack(d, W._scale)
-        W.sched(1)
         state = self.__dict__
-        if with_t:
-            T = W.transposed()
-            if T._pos is None:
-                T._before_repack(d.detach())
-            T.before_pair_repack(d, W._scale)
-            T.sched(1)
-        state["_pack_scale"], state["_pack_key"] = W._scale, (d.data_ptr(), d._version)
+        state["_pack_key"], state["_step_key"] = None, (d.data_ptr(), d._version)
+        for P in (W, W.transposed()) if with_t else (W,):
+            if P._pos is None or P._h_codes is not None or P._dview:
+                P._before_repack(d.detach())
+            P._set_scale_form(0.0, int(P.scale_after_sum))          # the form that the step's own products read
+            P.sched(1)
+        return W
+
+    def step_packed(self, with_t: bool) -> None:
+        """The native step has enqueued the re-pack that ``step_pack`` prepared: the state of the layer is now that behind
+        ``repack_for_step``."""
+        W, state = self._pack, self.__dict__
+        for P in (W, W._transposed) if with_t else (W,):
+            P.after_pair_repack(W._scale)
+        state["_pack_scale"], state["_pack_key"] = W._scale, state.pop("_step_key")
         state["_pack_gen"] += 1
         if with_t:
             state["_pack_t_gen"] = state["_pack_gen"]
-        return W
+
+    def step_failed(self) -> None:
+        """The step was declined, or ended in an error of which nobody knows whether it came before the re-pack: the next use
+        re-encodes, and a pack that someone still holds runs in the form that is right for old and new values alike."""
+        self.invalidate_pack()
+        if self.__dict__.pop("_step_key", None) is not None:         # step_pack had set the form
+            for P in (self._pack, self._pack._transposed):
+                if P is not None:
+                    P._set_scale_form(0.0, 0)
 
     def step_pack_fresh(self, with_t: bool) -> MortarPack | None:
-        """The pack that ``step_pack`` handed out, if the values have not changed since and nothing re-packed it otherwise."""
+        """The pack that ``step_packed`` declared fresh, if the values have not changed since and nothing re-packed it otherwise."""
         d = self._parameters.get("mortar_data")
         W = self._pack
         if W is None or d is None or self._pack_key != (d.data_ptr(), d._version) or (with_t and self._pack_t_gen != self._pack_gen):

@@ -62,14 +62,18 @@ def _native_step(x: Tensor, cg: CMSBlockLinear, cd: CMSBlockLinear, t_gu: bool, 
     """Re-pack (with the transposes asked for), gate_up, SwiGLU and down of a training step in one native call: (y, gate_up output, h)."""
     if type(x) is not Tensor or not x.is_cuda or x.numel() == 0:
         return None
-    W = cg.step_pack(t_gu)
-    D = cd.step_pack(t_dn) if W is not None else None
     r = None
-    if D is not None:
-        r = _lib.native().train_forward(x, cg.mortar_data, cd.mortar_data, W.address, W._transposed.address if t_gu else 0,
-                                        D.address, D._transposed.address if t_dn else 0, cg._values_threshold, cd._values_threshold)
-    if r is None:                     # nothing was launched: the general path re-packs
-        cg.invalidate_pack(), cd.invalidate_pack()
+    try:
+        W = cg.step_pack(t_gu)
+        D = cd.step_pack(t_dn) if W is not None else None
+        if D is not None:
+            r = _lib.native().train_forward(x, cg.mortar_data, cd.mortar_data, W.address, W._transposed.address if t_gu else 0,
+                                            D.address, D._transposed.address if t_dn else 0, cg._values_threshold, cd._values_threshold)
+    finally:
+        if r is None:                 # nothing was launched (the general path re-packs), or an exception is on its way
+            cg.step_failed(), cd.step_failed()
+    if r is not None:
+        cg.step_packed(t_gu), cd.step_packed(t_dn)
     return r
 
 

@@ -419,11 +419,9 @@ class MortarPack:
             self.uniform_scale, self.one_scale = uniform, one
             self.struct.uniform_scale, self.struct.one_scale = uniform, one
 
-    def before_pair_repack(self, values: torch.Tensor, scale: torch.Tensor) -> None:
-        """What ``requantize(values, sync=False)`` does beside the launches, for a re-pack through mortar_requantize_pairs whose scale
-        goes to ``scale`` (fp32 [1])."""
-        if self._pos is None or self._h_codes is not None or self._dview:
-            self._before_repack(values)
+    def after_pair_repack(self, scale: torch.Tensor) -> None:
+        """What ``requantize(values, sync=False)`` leaves in the pack beside its arrays, once mortar_requantize_pairs has enqueued the
+        launches that write those and ``scale`` (fp32 [1])."""
         self.scales_f32 = scale
         self._set_scale_form(0.0, int(self.scale_after_sum))
 
@@ -436,18 +434,19 @@ class MortarPack:
         for r, (W, values, threshold, with_t) in zip(arr, jobs):
             W._before_repack(values)
             s = torch.empty(1, dtype=torch.float32, device=W.device)
-            W.before_pair_repack(values, s)
             r.W, r.pos, r.values, r.scale_out = C.addressof(W.struct), W._pos.data_ptr(), values.data_ptr(), s.data_ptr()
             r.status, r.workspace = W._status.data_ptr(), W._ws.data_ptr()
             r.values_f32, r.threshold = int(values.dtype == torch.float32), threshold
             if with_t:
                 T = W.transposed()
                 T._before_repack(values)
-                T.before_pair_repack(values, s)
                 r.Wt, r.pos_t, r.src_t, r.status_t = C.addressof(T.struct), T._pos.data_ptr(), T.src_block.data_ptr(), T._status.data_ptr()
             scales.append(s)
         dev = jobs[0][0].device
         _lib.check(_lib.lib().mortar_requantize_pairs(C.addressof(arr), len(jobs), torch.cuda.current_stream(dev).cuda_stream), "mortar_requantize_pairs")
+        for (W, _, _, with_t), s in zip(jobs, scales):
+            for P in (W, W._transposed) if with_t else (W,):
+                P.after_pair_repack(s)
         return scales
 
     # status of asynchronous re-packs: the device words are copied to pinned host memory behind every call; reading them

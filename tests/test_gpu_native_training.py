@@ -200,3 +200,30 @@ def test_train_step_after_the_values_have_changed(dev, took):
     assert took == ["train_forward"]
     want = mlp(x.detach().requires_grad_())
     assert torch.equal(want, -y) and x.grad is not None
+
+
+def test_train_step_that_failed_leaves_no_stale_weights(dev, took):
+    """The re-pack refuses a negative threshold, behind the point where the step's packs were handed out: the next inference call
+    multiplies the values as they are, not those of the last pack, and the next step is a native one again."""
+    mlp = synth.qat_mlp_module(synth.synth_mlp(64, 176, 0.3, seed=3), dev, seed=5)
+    x = torch.randn(70, 64, device=dev).to(torch.bfloat16)
+    layers = [mlp.gate_up._cms, mlp.down._cms]
+    mlp(x.requires_grad_()).sum().backward()
+    for m in layers:
+        m._values_threshold = -1.0
+    with torch.no_grad():
+        mlp.down._cms.mortar_data.neg_()
+    with pytest.raises(ValueError, match="threshold"):
+        mlp(x)
+    for m in layers:
+        m._values_threshold = 0.5
+        m.mortar_data.requires_grad_(False)           # an inference call re-packs by the key alone
+    with torch.no_grad():
+        y = mlp(x)
+    for m in layers:
+        m.invalidate_pack()
+    with torch.no_grad():
+        assert torch.equal(y, mlp(x))
+    for m in layers:
+        m.mortar_data.requires_grad_(True)
+    assert mlp(x).requires_grad and took.count("train_forward") == 2

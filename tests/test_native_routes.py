@@ -268,3 +268,71 @@ def test_iteration_index_and_k_are_taken_as_integers(native, monkeypatch):
     mlp.router._native_route(X, 1.0, False)
     args = native.calls[-1][1]
     assert type(args[6]) is int and all(type(v) is int for v in args[4])
+
+
+@pytest.mark.parametrize("fails", ["forward", "step_pack", "declined", None])
+def test_packs_are_fresh_only_behind_a_training_forward_that_ended(native, monkeypatch, fails):
+    """A native training forward that raises (out of memory before its re-pack, an error code) or declines leaves both layers to
+    re-encode at their next use, whatever key they had before; one that returns leaves them fresh."""
+    from mortar_amd import mlp as M
+    from mortar_amd.pack import MortarPack
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    encoded = []
+    monkeypatch.setattr(MortarPack, "requantize", lambda self, v, **kw: (encoded.append(self), torch.ones(1))[1])
+    mlp = synth.qat_mlp_module(synth.synth_mlp(64, 128, 0.5, seed=1), torch.device("cpu"), seed=2)
+    layers = [mlp.gate_up._cms, mlp.down._cms]
+    packs = [m.mortar_pack() for m in layers]
+    assert encoded == packs and [m.mortar_pack() for m in layers] == packs and len(encoded) == 2
+    if fails == "forward":
+        def train_forward(*a):
+            raise RuntimeError("out of memory")
+    else:
+        def train_forward(*a):
+            return None if fails == "declined" else (1, 2, 3)
+    native.train_forward = train_forward
+    if fails == "step_pack":
+        monkeypatch.setattr(packs[1], "sched", lambda n: (_ for _ in ()).throw(RuntimeError("out of memory")))
+    x = torch.zeros(2, 64, dtype=torch.bfloat16)
+    if fails in ("forward", "step_pack"):
+        with pytest.raises(RuntimeError, match="out of memory"):
+            M._native_step(x, *layers, True, True)
+    else:
+        assert M._native_step(x, *layers, True, True) == (None if fails else (1, 2, 3))
+    encoded.clear()
+    assert [m.mortar_pack() for m in layers] == packs
+    assert encoded == ([] if fails is None else packs)
+    forms = [(P.uniform_scale, P.one_scale) for W in packs for P in (W, W._transposed) if P is not None]
+    assert forms == [(0.0, 1 if fails is None else 0)] * len(forms)
+    assert [W.scales_f32 is W._scale for W in packs] == [fails is None] * 2
+
+
+def test_packs_are_stale_behind_a_re_pack_that_failed(monkeypatch):
+    from mortar_amd.block_sparse import CMSBlockLinear
+    from mortar_amd.pack import MortarPack
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    mlp = synth.qat_mlp_module(synth.synth_mlp(64, 128, 0.5, seed=1), torch.device("cpu"), seed=2)
+    encoded = []
+    monkeypatch.setattr(MortarPack, "requantize", lambda self, v, **kw: (encoded.append(self), torch.ones(1))[1])
+    cms = mlp.gate_up._cms
+    W = cms.mortar_pack()
+
+    def failing(jobs):
+        raise RuntimeError("launch failed")
+    monkeypatch.setattr(MortarPack, "requantize_pairs", staticmethod(failing))
+    with pytest.raises(RuntimeError, match="launch failed"):
+        CMSBlockLinear.repack_for_step([(cms, True)])
+    assert cms.mortar_pack() is W and encoded == [W, W]
+
+
+def test_a_declined_training_step_leaves_deployed_packs_alone(monkeypatch):
+    """One matrix deployed, the other trainable: the deployed pack keeps the form it was built with."""
+    from mortar_amd import mlp as M
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    spec = dict(synth.synth_mlp(64, 128, 0.5, seed=1), gate_up=synth.synth_matrix(256, 64, 0.5, seed=3, per_tensor_scale=True))
+    mlp = synth.mlp_module(spec, torch.device("cpu"))
+    cms = mlp.gate_up._cms
+    W = cms.mortar_pack()
+    assert W.uniform_scale != 0
+    form = W.uniform_scale
+    assert M._native_step(torch.zeros(2, 64, dtype=torch.bfloat16), cms, mlp.down._cms, True, True) is None
+    assert cms.mortar_pack() is W and (W.uniform_scale, W.struct.uniform_scale, W.one_scale) == (form, form, 0)
