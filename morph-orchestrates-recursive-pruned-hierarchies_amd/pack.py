@@ -201,9 +201,21 @@ class BcsrTopology:
                        "mortar_segment_ptr_host")
             self.seg_ptr = torch.from_numpy(sp).to(self.device)
         self._t = None
+        self._bind_handle()
+
+    def _bind_handle(self) -> None:
+        """What the native call layer takes this topology by.  It holds device addresses: every copy binds its own."""
         self._handle = _lib.TopologyHandle(self.row_ptr.data_ptr(), self.col.data_ptr(), self.seg_ptr.data_ptr() if self.seg_ptr is not None else None,
                                            None, self.Rb, self.Cb, self.nnz)
         self.address = C.addressof(self._handle)
+
+    def __getstate__(self) -> dict:
+        return {k: v for k, v in self.__dict__.items() if k not in ("_handle", "address", "_t")}
+
+    def __setstate__(self, state: dict) -> None:
+        self.__dict__.update(state)
+        self._t = None                                # (a copy derives its transposed topology when it is asked for it)
+        self._bind_handle()
 
     def transposed(self):
         """(topology of W^T, src): block j of W^T is block src[j] of W, transposed (int32 device index)."""

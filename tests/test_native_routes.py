@@ -336,3 +336,25 @@ def test_a_declined_training_step_leaves_deployed_packs_alone(monkeypatch):
     form = W.uniform_scale
     assert M._native_step(torch.zeros(2, 64, dtype=torch.bfloat16), cms, mlp.down._cms, True, True) is None
     assert cms.mortar_pack() is W and (W.uniform_scale, W.struct.uniform_scale, W.one_scale) == (form, form, 0)
+
+
+def test_a_topology_copies_and_pickles():
+    """By copy, deepcopy, pickle and torch.save, before and after its transposed form was made; every copy hands out the addresses of
+    its own arrays."""
+    from mortar_amd.pack import BcsrTopology
+    m = synth.synth_matrix(16 * 5, 16 * 400, 0.2, seed=1)              # wide enough for per-segment row pointers
+    T = BcsrTopology(m["offsets"], m["col_idx"], 16 * 5, 16 * 400, "cpu")
+    assert T.seg_ptr is not None
+
+    def saved(t):
+        f = io.BytesIO()
+        torch.save(t, f)
+        return torch.load(io.BytesIO(f.getvalue()), weights_only=False)
+    for _ in range(2):
+        for make in (copy.copy, copy.deepcopy, lambda t: pickle.loads(pickle.dumps(t)), saved):
+            t = make(T)
+            assert t.address != T.address and (t.Rb, t.Cb, t.nnz, t.nseg, t.seg_cb) == (T.Rb, T.Cb, T.nnz, T.nseg, T.seg_cb)
+            for name in ("row_ptr", "col", "seg_ptr"):
+                assert torch.equal(getattr(t, name), getattr(T, name)) and getattr(t._handle, name) == getattr(t, name).data_ptr()
+            (a, src), (b, want) = t.transposed(), T.transposed()
+            assert torch.equal(src, want) and a._handle.src == src.data_ptr() != want.data_ptr() and torch.equal(a.col, b.col)
