@@ -77,7 +77,11 @@ typedef struct {
                               0: per-block scales (always valid, also for a uniform matrix). */
     int32_t one_scale;     /* 1, with uniform_scale == 0: every block has the same scale, but its value is known on the
                               device only (sdup[0], written by mortar_requantize in modes 0 / 2 with no host wait): the
-                              products run in the same form and read it there.  0 otherwise. */
+                              products run in the same form and read it there.  That holds for a launch made now: work
+                              recorded to run later (a stream under capture, mortar_stack_prepare) takes the per-block
+                              form, since the matrix may be re-packed with a scale per block by then.  2: as 1, and also
+                              under capture, for a caller whose captured work re-packs the matrix in mode 0 itself.
+                              0 otherwise. */
 } mortar_bcsr_t;
 
 const char *mortar_last_error(void);

@@ -42,8 +42,19 @@ int check_common(const mortar_bcsr_t *W, const uint16_t *x, int64_t M, int64_t l
     return MORTAR_OK;
 }
 
+// Whether work enqueued on `st` is recorded to run again later.
+bool recorded(hipStream_t st) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();        // the null stream while another one records: nothing launched there is recorded
+    return false;
+}
+
+// The scale of a matrix that only the device knows (one_scale) is one at the launch, by what the host enqueued so far.  Work that runs
+// again later (a captured graph, the table of a layer stack, `live` false) may find the matrix re-packed with a scale per block
+// by then: it takes the per-block form, which is right for both.  one_scale = 2 says that the recorded work re-packs itself.
 void fill(SpmmParams &p, const mortar_bcsr_t *W, const int32_t *sched, const uint16_t *x, int64_t M, int64_t ldx,
-          uint16_t *y, int64_t ldy) {
+          uint16_t *y, int64_t ldy, hipStream_t st, bool live = true) {
     p = SpmmParams{};
     p.row_desc = reinterpret_cast<const u32x4_t *>(W->row_desc);
     p.codes_o = reinterpret_cast<const u32x4_t *>(W->codes_o);
@@ -56,7 +67,7 @@ void fill(SpmmParams &p, const mortar_bcsr_t *W, const int32_t *sched, const uin
     p.x = x; p.ldx = ldx; p.M = (int)M; p.y = y; p.ldy = ldy;
     p.n_clusters = 1; p.cluster_size = 1 << 30;
     p.uscale = 0.5f * W->uniform_scale;
-    if (W->uniform_scale == 0.f && W->one_scale && W->sdup) { p.uscale = 1.f; p.scale_dev = W->sdup; }
+    if (W->uniform_scale == 0.f && W->one_scale && W->sdup && live && (W->one_scale == 2 || !recorded(st))) { p.uscale = 1.f; p.scale_dev = W->sdup; }
 }
 
 // Token tile of the resident prefill kernel for a matrix with Cb block-columns (0 = does not fit).
@@ -164,7 +175,7 @@ int dispatch_prefill(int kind, SpmmParams &p, hipStream_t st) {
 // kind: 0 spmm, 1 gate_up + SwiGLU, 2 routed gate_up + SwiGLU, 3 spmm with an input mask.
 // Prefill-sized launches read the 4-bit code stream when the matrix carries one (cheaper unpack: one conversion
 // per register instead of shift + mask); decode-sized launches always stream the 2-bit codes (half the bytes).
-// A matrix with one scale (uniform_scale != 0, or one_scale) runs the kernels that multiply +-2 / 0 blocks and scale the
+// A matrix with one scale (uniform_scale != 0, or one_scale: fill) runs the kernels that multiply +-2 / 0 blocks and scale the
 // accumulators once (decode-sized launches always, prefill-sized ones through the 4-bit stream).
 int dispatch(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
     // products over several K segments have small-tile forms beyond the decode sizes as well (the launcher returns -1
@@ -212,7 +223,7 @@ extern "C" int mortar_spmm_bf16(const mortar_bcsr_t *W, const int32_t *sched, co
     int rc = check_common(W, x, M, ldx, y, ldy, W ? (int64_t)W->Rb * 16 : 0);
     if (rc) return rc;
     SpmmParams p;
-    fill(p, W, sched, x, M, ldx, y, ldy);
+    fill(p, W, sched, x, M, ldx, y, ldy, static_cast<hipStream_t>(stream));
     p.n_units = W->Rb;
     return dispatch(0, p, W, static_cast<hipStream_t>(stream));
 }
@@ -223,7 +234,7 @@ int mortar_spmm_codes_f32(const mortar_bcsr_t *W, const int32_t *sched, const ui
     if (rc) return rc;
     if (reinterpret_cast<uintptr_t>(y32) & 15) return mortar_fail(MORTAR_ERR_ARG, "spmm: the fp32 output must be 16-byte aligned");
     SpmmParams p;
-    fill(p, W, sched, x, M, ldx, nullptr, ldy);
+    fill(p, W, sched, x, M, ldx, nullptr, ldy, static_cast<hipStream_t>(stream));
     p.n_units = W->Rb;
     p.y32 = y32;
     p.uscale = 0.5f; p.scale_dev = nullptr;      // the kernels multiply the blocks as +-2 / 0
@@ -245,7 +256,7 @@ extern "C" int mortar_spmm_bf16_masked(const mortar_bcsr_t *W, const int32_t *sc
     if (!active || n_clusters <= 0 || (W->Cb * 16) % n_clusters || ((W->Cb * 16) / n_clusters) % 8)
         return mortar_fail(MORTAR_ERR_ARG, "spmm_masked: in_features/n_clusters must be a multiple of 8");
     SpmmParams p;
-    fill(p, W, sched, x, M, ldx, y, ldy);
+    fill(p, W, sched, x, M, ldx, y, ldy, static_cast<hipStream_t>(stream));
     p.n_units = W->Rb;
     p.active = active; p.n_clusters = n_clusters; p.cluster_size = (W->Cb * 16) / n_clusters;
     return dispatch(3, p, W, static_cast<hipStream_t>(stream));
@@ -267,7 +278,7 @@ extern "C" int mortar_spmm_hc_post(const mortar_bcsr_t *W, const int32_t *sched,
     if ((reinterpret_cast<uintptr_t>(carrier) & al) || (reinterpret_cast<uintptr_t>(out) & al) || (reinterpret_cast<uintptr_t>(term) & al))
         return mortar_fail(MORTAR_ERR_ARG, "spmm_hc_post: carrier, term and out must be %d-byte aligned", (int)al + 1);
     SpmmParams p;
-    fill(p, W, sched, x, M, ldx, reinterpret_cast<uint16_t *>(out), (int64_t)W->Rb * 16);
+    fill(p, W, sched, x, M, ldx, reinterpret_cast<uint16_t *>(out), (int64_t)W->Rb * 16, static_cast<hipStream_t>(stream));
     p.n_units = W->Rb;
     p.hc_h = carrier; p.hc_out = out; p.hc_res = hres; p.hc_post = hpost; p.hc_term = term; p.hc_n = n_streams; p.hc_f32 = carrier_f32 != 0;
     int kind = 0;
@@ -313,7 +324,7 @@ int gateup_common(const mortar_bcsr_t *W, const int32_t *sched, const uint16_t *
     int rc = check_common(W, x, M, ldx, h, ldh, d_ff);
     if (rc) return rc;
     SpmmParams p;
-    fill(p, W, sched, x, M, ldx, h, ldh);
+    fill(p, W, sched, x, M, ldx, h, ldh, static_cast<hipStream_t>(stream));
     p.n_units = W->Rb / 2;
     if (norm) {
         if (!mortar_norm_fusable(W->Cb) || p.nseg != 1)
@@ -386,7 +397,7 @@ extern "C" int mortar_mlp_bf16(const mortar_bcsr_t *Wgu, const int32_t *sched_gu
         int rc = check_common(Wgu, x, M, ldx, h, d_ff, d_ff);
         if (rc) return rc;
         SpmmParams p;
-        fill(p, Wgu, sched_gu, x, M, ldx, h, d_ff);
+        fill(p, Wgu, sched_gu, x, M, ldx, h, d_ff, st);
         p.n_units = Wgu->Rb / 2;
         if (norm) {
             if (!mortar_norm_fusable(Wgu->Cb) || p.nseg != 1)
@@ -411,7 +422,7 @@ extern "C" int mortar_mlp_bf16(const mortar_bcsr_t *Wgu, const int32_t *sched_gu
         int rc = check_common(Wdn, h, M, d_ff, y, ldy, (int64_t)Wdn->Rb * 16);
         if (rc) return rc;
         SpmmParams p;
-        fill(p, Wdn, sched_dn, h, M, d_ff, y, ldy);
+        fill(p, Wdn, sched_dn, h, M, d_ff, y, ldy, st);
         p.n_units = Wdn->Rb;
         p.x_tiled = 1;
         p.codes_o = reinterpret_cast<const u32x4_t *>(Wdn->codes4_o);
@@ -433,24 +444,24 @@ extern "C" int mortar_stack_prepare(int32_t swiglu, int32_t n_layers, const mort
     if (n_layers <= 0 || n_layers > 65535 || !W || !x || !y || !table_dev)
         return mortar_fail(MORTAR_ERR_ARG, "stack_prepare: bad arguments");
     if (M > 64) return mortar_fail(MORTAR_ERR_LIMIT, "stack_prepare: layer-batched launches serve M <= 64 (got %lld)", (long long)M);
+    hipStream_t st = static_cast<hipStream_t>(stream);
     std::vector<SpmmParams> tab((size_t)n_layers);
     for (int l = 0; l < n_layers; ++l) {
         if (W[l].Rb != W[0].Rb || W[l].Cb != W[0].Cb || W[l].seg_cb != W[0].seg_cb)
             return mortar_fail(MORTAR_ERR_ARG, "stack_prepare: layer %d differs in shape from layer 0", l);
         if (swiglu && (W[l].Rb & 1)) return mortar_fail(MORTAR_ERR_ARG, "stack_prepare: odd number of block-rows");
-        if ((W[l].uniform_scale != 0.f || W[l].one_scale) != (W[0].uniform_scale != 0.f || W[0].one_scale))
+        if ((W[l].uniform_scale != 0.f) != (W[0].uniform_scale != 0.f))
             return mortar_fail(MORTAR_ERR_ARG, "stack_prepare: layer %d and layer 0 differ in having a uniform scale "
-                               "(set uniform_scale = 0 and one_scale = 0 on all layers to run them together)", l);
+                               "(set uniform_scale = 0 on all layers to run them together)", l);
         const int64_t out_cols = swiglu ? (int64_t)W[l].Rb * 8 : (int64_t)W[l].Rb * 16;
         int rc = check_common(&W[l], x[l], M, ldx, y[l], ldy, out_cols);
         if (rc) return rc;
         SpmmParams &p = tab[(size_t)l];
-        fill(p, &W[l], sched ? sched[l] : nullptr, x[l], M, ldx, y[l], ldy);
+        fill(p, &W[l], sched ? sched[l] : nullptr, x[l], M, ldx, y[l], ldy, st, false);
         p.n_units = swiglu ? W[l].Rb / 2 : W[l].Rb;
         rc = mortar_smallm_shape(swiglu ? 1 : 0, p, n_layers);
         if (rc) return rc;
     }
-    hipStream_t st = static_cast<hipStream_t>(stream);
     hipError_t e = hipMemcpyAsync(table_dev, tab.data(), tab.size() * sizeof(SpmmParams), hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "stack_prepare: %s", hipGetErrorString(e));
@@ -462,7 +473,7 @@ extern "C" int mortar_stack_run(int32_t swiglu, int32_t n_layers, const mortar_b
     if (n_layers <= 0 || n_layers > 65535 || !W0 || !table_dev || M <= 0 || M > 64)
         return mortar_fail(MORTAR_ERR_ARG, "stack_run: bad arguments");
     SpmmParams p;
-    fill(p, W0, nullptr, nullptr, M, 0, nullptr, 0);
+    fill(p, W0, nullptr, nullptr, M, 0, nullptr, 0, static_cast<hipStream_t>(stream), false);
     p.n_units = swiglu ? W0->Rb / 2 : W0->Rb;
     const int rc = mortar_smallm_launch(swiglu ? 1 : 0, p, static_cast<const SpmmParams *>(table_dev), n_layers,
                                         static_cast<hipStream_t>(stream));

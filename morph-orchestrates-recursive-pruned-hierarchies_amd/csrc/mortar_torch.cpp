@@ -366,6 +366,14 @@ bool is_values(const at::Tensor &v, const mortar_bcsr_t *w, const at::Tensor &x)
            v.size(1) == 16 && v.size(2) == 16 && v.is_contiguous() && aligned16(v.const_data_ptr());
 }
 
+// A matrix as the products of a training step take it: the step re-packs it, so that its scale is one at every replay of a captured
+// step as well.
+mortar_bcsr_t step_form(const PackHandle *h) {
+    mortar_bcsr_t w = *h->w;
+    if (w.one_scale) w.one_scale = 2;
+    return w;
+}
+
 bool repackable(const PackHandle *h) { return h->pos && h->status && h->workspace && h->sched1; }
 
 mortar_repack_t repack_of(const PackHandle *h, const PackHandle *t, const at::Tensor &v, double threshold) {
@@ -401,10 +409,11 @@ PyObject *py_train_forward(PyObject *, PyObject *const *a, Py_ssize_t na) {
     void *st = stream_of(x);
     const mortar_repack_t re[2] = {repack_of(gu, gut, *vg, tg), repack_of(dn, dnt, *vd, td)};
     at::Tensor g = new_bf16(x, {M, f2}), h = new_bf16(x, {M, f}), y = new_bf16(x, {M, dy});
+    const mortar_bcsr_t wg = step_form(gu), wd = step_form(dn);
     int rc = mortar_requantize_pairs(re, 2, st);
-    if (rc == MORTAR_OK) rc = mortar_spmm_bf16(gu->w, gu->sched1, u16(x), M, d, u16m(g), f2, st);
+    if (rc == MORTAR_OK) rc = mortar_spmm_bf16(&wg, gu->sched1, u16(x), M, d, u16m(g), f2, st);
     if (rc == MORTAR_OK) rc = mortar_swiglu_bf16(u16(g), f2, M, (int32_t)f, u16m(h), f, st);
-    if (rc == MORTAR_OK) rc = mortar_spmm_bf16(dn->w, dn->sched1, u16(h), M, f, u16m(y), dy, st);
+    if (rc == MORTAR_OK) rc = mortar_spmm_bf16(&wd, dn->sched1, u16(h), M, f, u16m(y), dy, st);
     if (rc) return raise_rc(rc, "mortar_train_forward");
     return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(y)), THPVariable_Wrap(std::move(g)), THPVariable_Wrap(std::move(h)));
 }
@@ -469,12 +478,14 @@ PyObject *py_train_backward(PyObject *, PyObject *const *a, Py_ssize_t na) {
     if (need_dn) rc = run_sdd(pd, dn->w->Rb, dn->w->Cb, dn->w->nnz, dy, h, ddn, st);
     if (rc == MORTAR_OK && (gut || need_gu)) {
         const at::Tensor dh = new_bf16(x, {M, f}), dg = new_bf16(x, {M, f2});
-        rc = mortar_spmm_bf16(dnt->w, dnt->sched1, u16(dy), M, dd, u16m(dh), f, st);
+        const mortar_bcsr_t wdt = step_form(dnt);
+        rc = mortar_spmm_bf16(&wdt, dnt->sched1, u16(dy), M, dd, u16m(dh), f, st);
         if (rc == MORTAR_OK) rc = mortar_swiglu_backward_bf16(u16(g), f2, u16(dh), f, M, (int32_t)f, u16m(dg), f2, st);
         if (rc == MORTAR_OK && need_gu) rc = run_sdd(pg, gu->w->Rb, gu->w->Cb, gu->w->nnz, dg, x, dgu, st);
         if (rc == MORTAR_OK && gut) {
             dx = new_bf16(x, {M, d});
-            rc = mortar_spmm_bf16(gut->w, gut->sched1, u16(dg), M, f2, u16m(dx), d, st);
+            const mortar_bcsr_t wgt = step_form(gut);
+            rc = mortar_spmm_bf16(&wgt, gut->sched1, u16(dg), M, f2, u16m(dx), d, st);
         }
     }
     if (rc) return raise_rc(rc, "mortar_train_backward");

@@ -650,3 +650,77 @@ def test_requantize_pairs(dev, dtype, with_t):
     for P in (packs[0][0], packs[0][0].transposed()) if with_t[0] else (packs[0][0],):
         with pytest.raises(ValueError, match="outside"):
             P.raise_status()
+
+
+@pytest.mark.parametrize("M,out_b,in_b", [(3, 12, 48), (70, 20, 128), (40, 24, 400)])
+def test_recorded_products_follow_a_re_pack_with_a_scale_per_block(dev, M, out_b, in_b):
+    """Work recorded while the pack had one scale and run after it was re-packed with one per block, without a host wait: a layer
+    stack (which takes such a pack together with a per-block one) and a captured graph, replayed several times with eager work in
+    between, give what the per-block pack gives."""
+    m = synth.synth_matrix(16 * out_b, 16 * in_b, 0.25, seed=61)
+    vt = (_values(m["col_idx"].size, 62, torch.bfloat16)[0] * torch.linspace(0.5, 2.0, m["col_idx"].size).view(-1, 1, 1)).to(torch.bfloat16).to(dev)
+    A, B, P = (MortarPack(None, None, m["col_idx"], m["offsets"], 16 * out_b, 16 * in_b, dev) for _ in range(3))
+    A.requantize(vt, sync=False)
+    B.requantize(vt)                                                      # the scale of A, known on the host
+    P.requantize(vt, per_block=True, sync=False)
+    assert (A.one_scale, P.one_scale) == (1, 0)
+    x = to_dev(synth.synth_x(M, 16 * in_b, 63), dev)
+    one, per = ops.spmm(x, B), ops.spmm(x, P)
+    stack = None
+    if M <= 64:
+        ys = [torch.empty(M, 16 * out_b, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+        stack = ops.LayerStack([P, A], [x, x], ys)
+        stack.run()
+        assert_close_bf16(to_np(ys[1]), to_np(one), "stack before")
+        want = [y.clone() for y in ys]
+    y = torch.empty(M, 16 * out_b, dtype=torch.bfloat16, device=dev)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ops.spmm(x, A, out=y)
+    torch.cuda.current_stream().wait_stream(side)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ops.spmm(x, A, out=y)
+    g.replay()
+    assert_close_bf16(to_np(y), to_np(one), "graph before")
+    A.requantize(vt, per_block=True, sync=False)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        assert torch.equal(y, per)
+        if stack is not None:
+            stack.run()
+            assert torch.equal(ys[0], want[0]) and torch.equal(ys[1], ys[0])
+    A.requantize(vt, sync=False)                                          # and back
+    g.replay()
+    assert_close_bf16(to_np(y), to_np(one), "graph after")
+
+
+def test_a_captured_training_step_re_packs_itself(dev):
+    """The step keeps the one-scale kernels under capture: replays on new values give the bits of the eager step, whatever the packs
+    held in between."""
+    mlp = synth.qat_mlp_module(synth.synth_mlp(64, 176, 0.3, seed=3), dev, seed=5)
+    layers = [mlp.gate_up._cms, mlp.down._cms]
+    data = [m.mortar_data for m in layers]
+    x = torch.randn(70, 64, device=dev).to(torch.bfloat16).requires_grad_()
+    dy = torch.randn(70, 64, device=dev).to(torch.bfloat16)
+    grads = lambda: torch.autograd.grad(mlp(x), [x] + data, dy)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        grads()
+    torch.cuda.current_stream().wait_stream(side)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = grads()
+    for step in range(3):
+        with torch.no_grad():
+            for p in data:
+                p.mul_(-1.25).add_(0.001)
+        for m in layers:
+            m._pack.requantize(m.mortar_data.detach(), per_block=True, sync=False)
+        g.replay()
+        got = [t.clone() for t in out]
+        for a, b in zip(got, grads()):
+            assert torch.equal(a, b)
