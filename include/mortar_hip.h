@@ -277,7 +277,8 @@ int mortar_router_bf16(const void *x, int32_t x_is_f32, int64_t B, int32_t d, in
                        float *logits_out, float *gates, uint8_t *active, void *stream);
 
 /* mortar_rmsnorm_bf16(x) -> xn (bf16 [B, d], rows contiguous, 16-byte aligned), then mortar_router_bf16 on the normalised rows: same bits,
- * with the norm inside the projection's launch up to d = 2048.  norm_w bf16 [d] or NULL. */
+ * with the norm inside the projection's launch up to d = 2048.  norm_w bf16 [d] or NULL.  xn is a buffer of its own: one that overlaps the
+ * rows of x or norm_w is refused. */
 int mortar_norm_router_bf16(const uint16_t *x, int64_t B, int32_t d, int64_t ldx, const uint16_t *norm_w, float norm_eps, uint16_t *xn,
                             const float *wq, const float *iter_vec, const float *ln_w, const float *ln_b, float ln_eps,
                             const float *ka, const float *kb, int32_t nsk, const float *bias, int32_t n, int32_t k, float *qv,

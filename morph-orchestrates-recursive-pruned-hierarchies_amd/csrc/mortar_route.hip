@@ -1015,6 +1015,11 @@ static int launch_router(const void *x, bool x_is_f32, int64_t B, int32_t d, int
     if (n > 64 * MAXPL_LIMIT) return mortar_fail(MORTAR_ERR_LIMIT, "router: n=%d exceeds %d clusters", n, 64 * MAXPL_LIMIT);
     if ((int64_t)nsk * nsk > 2048)
         return mortar_fail(MORTAR_ERR_LIMIT, "router: %d x %d product keys exceed the 2048 the fused front end ranks", nsk, nsk);
+    if (xn) {       // one workgroup writes xn while the others still read the rows and the norm's weights
+        const auto apart = [xn, B, d](const uint16_t *p, int64_t values) { return !p || p + values <= xn || xn + B * d <= p; };
+        if (!apart(static_cast<const uint16_t *>(x), (B - 1) * ldx + d) || !apart(norm_w, d))
+            return mortar_fail(MORTAR_ERR_ARG, "norm_router: xn overlaps x or norm_w");
+    }
     hipStream_t st = static_cast<hipStream_t>(stream);
     const dim3 pg((unsigned)((d + 3) / 4)), blk(256);
     // From 5 bf16 tokens up the projection runs on the matrix cores (2048 x 2048, with the tail: 5 tokens 13.6 -> 12.0 us, 16 19.5 -> 12.4,

@@ -565,3 +565,37 @@ def test_fp32_decode_product_refuses_streams_beyond_32_bit_offsets():
     W = _lib.BcsrStruct(*[4096] * 9, 1 << 15, 1024, 1 << 25, 128, 1.0, 0)       # never read: refused before any launch
     rc = _lib.lib().mortar_gemv_f32_one(C.byref(W), 4096, 0, 0, 4096, 1, 16 * 1024, 4096, 16 << 15, None, 0, 0, None, 0, None, 0, None)
     assert rc == -4 and b"octet stream" in _lib.lib().mortar_last_error()
+
+
+@pytest.fixture
+def no_launch():
+    """For entry points called with host addresses: an argument check answers, or (without a GPU) the launch fails."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("host addresses: only where nothing can be launched")
+
+
+@pytest.mark.parametrize("B,d,gap", [(1, 64, 0), (4, 2048, 0), (16, 1024, 8), (17, 64, 0), (3, 2056, 0)])
+def test_norm_router_refuses_a_result_over_its_operands(no_launch, B, d, gap):
+    """xn is written by one workgroup while others read x and the norm's weight: every overlap is an argument error, in the form with
+    the norm inside and in that with two launches; buffers that only touch are accepted."""
+    L, ld = _lib.lib(), d + gap
+    buf = np.zeros(4 * B * ld + 4 * d + 64, np.uint16)
+    base = buf.ctypes.data + (-buf.ctypes.data) % 16
+    par = np.zeros(d * d + 64, np.float32)
+    p = par.ctypes.data + (-par.ctypes.data) % 16
+    out = np.zeros(B * d + 64, np.float32).ctypes
+
+    def call(x, nw, xn):
+        return L.mortar_norm_router_bf16(x, B, d, ld, nw, 1e-5, xn, p, None, p, p, 1e-5, p, p, 2, p, 4, 1, out.data, None, out.data, None, None)
+    x = base + 2 * B * ld
+    rows = (B - 1) * ld + d
+    free = base + 6 * B * ld                               # behind everything else
+    for nw in (None, free + 2 * d):
+        for xn in (x, x + 2 * (rows - 8), x - 2 * (B * d - 8)):
+            assert call(x, nw, xn) == -1 and b"overlaps" in L.mortar_last_error()
+    for nw in (free, free + 2 * (B * d - 8) // 16 * 16):
+        assert call(x, nw, free) == -1 and b"overlaps" in L.mortar_last_error()
+    for xn in (x + 2 * rows, x - 2 * B * d):
+        if xn % 16 == 0:
+            assert call(x, None, xn) == -3
