@@ -511,7 +511,7 @@ int mortar_requantize(const mortar_bcsr_t *W, const void *values, int32_t values
 
 /* The re-pack of up to two matrices and of their transposes in two launches: what mortar_requantize does for each in mode 0 (flags 1),
  * the transpose with the scale of its matrix.  Wt NULL leaves a transpose out; scale_out / status / status_t may be NULL.  The
- * workspaces of the matrices are different buffers. */
+ * workspaces of the matrices are different buffers (refused otherwise). */
 typedef struct {
     const mortar_bcsr_t *W, *Wt;
     const int32_t *pos, *pos_t, *src_t;   /* octet positions of W and Wt; block j of Wt is block src_t[j] of W, transposed */

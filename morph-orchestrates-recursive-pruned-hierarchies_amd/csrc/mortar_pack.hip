@@ -337,6 +337,11 @@ extern "C" int mortar_requantize_pairs(const mortar_repack_t *m, int32_t n, void
         if (rc) return rc;
         if (!m[i].workspace || (m[i].Wt && (!m[i].src_t || m[i].Wt->nnz != m[i].W->nnz)))
             return mortar_fail(MORTAR_ERR_ARG, "requantize_pairs: matrix %d: workspace missing, or W^T does not match W", i);
+        for (int k = 0; k < i; ++k) {        // both sums are under way at once
+            const int64_t apart = static_cast<const char *>(m[i].workspace) - static_cast<const char *>(m[k].workspace);
+            if (apart < mortar_requantize_workspace_bytes() && -apart < mortar_requantize_workspace_bytes())
+                return mortar_fail(MORTAR_ERR_ARG, "requantize_pairs: matrices %d and %d share a workspace", k, i);
+        }
         sums.job[i] = {m[i].values, static_cast<double *>(m[i].workspace), (int64_t)m[i].W->nnz * 256, m[i].values_f32};
         jobs.job[nj] = requant_args(m[i].W, m[i].values, m[i].values_f32, m[i].pos, nullptr, 0, m[i].threshold, m[i].status, m[i].workspace);
         jobs.job[nj++].scale_out = m[i].scale_out;

@@ -577,11 +577,13 @@ class MortarPack:
         """A second resident copy (own device buffers and schedules) of the same matrix."""
         import copy
         c = copy.copy(self)
-        for name in ("codes", "sdup", "col", "row_ptr", "row_desc", "codes_o", "sd_o", "col_o", "codes4_o", "scales_f32"):
+        for name in ("codes", "sdup", "col", "row_ptr", "row_desc", "codes_o", "sd_o", "col_o", "codes4_o", "scales_f32", "_ws", "_status",
+                     "_scale"):
             if getattr(self, name) is not None:
                 setattr(c, name, getattr(self, name).clone())
         c._scheds = {k: v.clone() for k, v in self._scheds.items()}
         c._worklists = {k: (v[0].clone(), v[1], v[2].clone(), v[3]) for k, v in self._worklists.items()}
         c._transposed, c._dview = None, {}      # the clone builds its own views
+        c._status_host = c._status_event = None
         c._bind_struct()
         return c

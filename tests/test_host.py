@@ -570,7 +570,6 @@ def test_fp32_decode_product_refuses_streams_beyond_32_bit_offsets():
 @pytest.fixture
 def no_launch():
     """For entry points called with host addresses: an argument check answers, or (without a GPU) the launch fails."""
-    import torch
     if torch.cuda.is_available():
         pytest.skip("host addresses: only where nothing can be launched")
 
@@ -599,3 +598,33 @@ def test_norm_router_refuses_a_result_over_its_operands(no_launch, B, d, gap):
     for xn in (x + 2 * rows, x - 2 * B * d):
         if xn % 16 == 0:
             assert call(x, None, xn) == -3
+
+
+def test_requantize_pairs_refuses_one_workspace_for_two_matrices(no_launch):
+    """Both |w| sums are formed in one launch: the same workspace twice, or two that overlap, is an argument error; two that only touch
+    are accepted."""
+    L = _lib.lib()
+    a = np.zeros(1 << 16, np.float64)
+    p, ws = a.ctypes.data + (-a.ctypes.data) % 16, L.mortar_requantize_workspace_bytes()
+    W = _lib.BcsrStruct(p, p, p, p, p, p, p, p, p, 2, 2, 4, 2, 0.0, 0)
+    arr = (_lib.RepackStruct * 2)()
+    for off, want in ((0, -1), (8, -1), (ws - 8, -1), (ws, -3)):
+        for first, second in ((p + 1024, p + 1024 + off), (p + 1024 + off, p + 1024)):
+            for r, w in zip(arr, (first, second)):
+                r.W, r.pos, r.values, r.workspace, r.threshold = C.addressof(W), p, p, w, 0.5
+            assert L.mortar_requantize_pairs(C.addressof(arr), 2, None) == want
+            assert want == -3 or b"workspace" in L.mortar_last_error()
+
+
+def test_a_cloned_pack_re_packs_through_buffers_of_its_own():
+    m = synth.synth_matrix(16 * 5, 16 * 11, 0.3, seed=5)
+    W = P.MortarPack(None, None, m["col_idx"], m["offsets"], 16 * 5, 16 * 11, "cpu")
+    W._before_repack(torch.zeros(W.nnz, 16, 16))
+    W._status[0] = 1
+    c = W.clone_weights()
+    for name in ("workspace", "status"):
+        assert getattr(c._handle, name) != getattr(W._handle, name)
+    assert c._status.tolist() == [1, 0] and c._scale.data_ptr() != W._scale.data_ptr()
+    W._status.zero_()
+    with pytest.raises(ValueError, match="outside"):
+        c.raise_status()
