@@ -105,8 +105,7 @@ _SIGS = {
 class PackHandle(C.Structure):
     """One packed matrix for the native call layer: its mortar_bcsr_t, the schedules built so far and, once it has been re-packed,
     what a re-pack needs beside the values."""
-    _fields_ = [("w", c_vp), ("sched1", c_vp), ("sched2", c_vp), ("pos", c_vp), ("src", c_vp), ("scale", c_vp), ("status", c_vp),
-                ("workspace", c_vp)]
+    _fields_ = [("w", c_vp), ("sched1", c_vp), ("sched2", c_vp), ("pos", c_vp), ("src", c_vp), ("status", c_vp), ("workspace", c_vp)]
 
 
 class TopologyHandle(C.Structure):

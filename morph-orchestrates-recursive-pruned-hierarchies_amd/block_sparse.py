@@ -284,13 +284,13 @@ class CMSBlockLinear(nn.Module):
             P.sched(1)
         return W
 
-    def step_packed(self, with_t: bool) -> None:
-        """The native step has enqueued the re-pack that ``step_pack`` prepared: the state of the layer is now that behind
-        ``repack_for_step``."""
+    def step_packed(self, scale: Tensor, with_t: bool) -> None:
+        """The native step has enqueued the re-pack that ``step_pack`` prepared, which writes ``scale``: the state of the layer is now
+        that behind ``repack_for_step``."""
         W, state = self._pack, self.__dict__
         for P in (W, W._transposed) if with_t else (W,):
-            P.after_pair_repack(W._scale)
-        state["_pack_scale"], state["_pack_key"] = W._scale, state.pop("_step_key")
+            P.after_pair_repack(scale)
+        state["_pack_scale"], state["_pack_key"] = scale, state.pop("_step_key")
         state["_pack_gen"] += 1
         if with_t:
             state["_pack_t_gen"] = state["_pack_gen"]

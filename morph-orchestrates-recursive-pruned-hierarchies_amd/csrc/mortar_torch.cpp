@@ -34,7 +34,6 @@ struct PackHandle {
     const mortar_bcsr_t *w;
     const int32_t *sched1, *sched2;
     const int32_t *pos, *src;
-    float *scale;
     int32_t *status;
     void *workspace;
 };
@@ -376,9 +375,9 @@ mortar_bcsr_t step_form(const PackHandle *h) {
 
 bool repackable(const PackHandle *h) { return h->pos && h->status && h->workspace && h->sched1; }
 
-mortar_repack_t repack_of(const PackHandle *h, const PackHandle *t, const at::Tensor &v, double threshold) {
+mortar_repack_t repack_of(const PackHandle *h, const PackHandle *t, const at::Tensor &v, double threshold, const at::Tensor &scale) {
     mortar_repack_t r{};
-    r.W = h->w; r.pos = h->pos; r.status = h->status; r.workspace = h->workspace; r.scale_out = h->scale;
+    r.W = h->w; r.pos = h->pos; r.status = h->status; r.workspace = h->workspace; r.scale_out = static_cast<float *>(scale.data_ptr());
     if (t) { r.Wt = t->w; r.pos_t = t->pos; r.src_t = t->src; r.status_t = t->status; }
     r.values = v.const_data_ptr();
     r.values_f32 = v.scalar_type() == at::kFloat;
@@ -386,8 +385,9 @@ mortar_repack_t repack_of(const PackHandle *h, const PackHandle *t, const at::Te
     return r;
 }
 
-// train_forward(x, gate_up values, down values, gate_up, its W^T or 0, down, its W^T or 0, thresholds of the two) -> (y, gu, h): the
-// re-pack of both matrices and the transposes named, then gate_up, SwiGLU and down on the rows of x.  No autograd of its own.
+// train_forward(x, gate_up values, down values, gate_up, its W^T or 0, down, its W^T or 0, thresholds of the two) -> (y, gu, h,
+// scale of gate_up, of down): the re-pack of both matrices and the transposes named, then gate_up, SwiGLU and down on the rows of x.  No
+// autograd of its own.
 PyObject *py_train_forward(PyObject *, PyObject *const *a, Py_ssize_t na) {
     if (na != 9) {
         PyErr_SetString(PyExc_TypeError, "train_forward: 9 arguments");
@@ -407,7 +407,9 @@ PyObject *py_train_forward(PyObject *, PyObject *const *a, Py_ssize_t na) {
     const int64_t M = x.size(0);
     const c10::DeviceGuard guard(x.device());
     void *st = stream_of(x);
-    const mortar_repack_t re[2] = {repack_of(gu, gut, *vg, tg), repack_of(dn, dnt, *vd, td)};
+    const auto f32 = x.options().dtype(at::kFloat).requires_grad(false);
+    at::Tensor sg = at::empty({1}, f32), sd = at::empty({1}, f32);
+    const mortar_repack_t re[2] = {repack_of(gu, gut, *vg, tg, sg), repack_of(dn, dnt, *vd, td, sd)};
     at::Tensor g = new_bf16(x, {M, f2}), h = new_bf16(x, {M, f}), y = new_bf16(x, {M, dy});
     const mortar_bcsr_t wg = step_form(gu), wd = step_form(dn);
     int rc = mortar_requantize_pairs(re, 2, st);
@@ -415,7 +417,8 @@ PyObject *py_train_forward(PyObject *, PyObject *const *a, Py_ssize_t na) {
     if (rc == MORTAR_OK) rc = mortar_swiglu_bf16(u16(g), f2, M, (int32_t)f, u16m(h), f, st);
     if (rc == MORTAR_OK) rc = mortar_spmm_bf16(&wd, dn->sched1, u16(h), M, f, u16m(y), dy, st);
     if (rc) return raise_rc(rc, "mortar_train_forward");
-    return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(y)), THPVariable_Wrap(std::move(g)), THPVariable_Wrap(std::move(h)));
+    return Py_BuildValue("(NNNNN)", THPVariable_Wrap(std::move(y)), THPVariable_Wrap(std::move(g)), THPVariable_Wrap(std::move(h)),
+                         THPVariable_Wrap(std::move(sg)), THPVariable_Wrap(std::move(sd)));
 }
 
 // A weight gradient's plan as the Python side hands it over: (address, workgroups, blocks per wave), or None / no need.

@@ -73,7 +73,8 @@ def _native_step(x: Tensor, cg: CMSBlockLinear, cd: CMSBlockLinear, t_gu: bool, 
         if r is None:                 # nothing was launched (the general path re-packs), or an exception is on its way
             cg.step_failed(), cd.step_failed()
     if r is not None:
-        cg.step_packed(t_gu), cd.step_packed(t_dn)
+        cg.step_packed(r[3], t_gu), cd.step_packed(r[4], t_dn)
+        r = r[:3]
     return r
 
 

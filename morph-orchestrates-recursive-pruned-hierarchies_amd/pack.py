@@ -304,7 +304,7 @@ class MortarPack:
         self._worklists: dict[tuple, tuple] = {}
         # what decode_view() rebuilds the stream from; dropped once the values are rewritten on the device
         self._h_codes, self._h_sdup, self._dview = (codes, sdup, {}) if packed is not None else (None, None, {})
-        self._pos = self._ws = self._status = self.src_block = self._scale = self._sdd = None
+        self._pos = self._ws = self._status = self.src_block = self._sdd = None
         self._status_host = self._status_event = None
         self._transposed: "MortarPack | None" = None
         self._bind_struct()
@@ -322,7 +322,7 @@ class MortarPack:
 
     def _bind_repack(self) -> None:
         h = self._handle
-        for name, t in (("pos", self._pos), ("src", self.src_block), ("scale", self._scale), ("status", self._status), ("workspace", self._ws)):
+        for name, t in (("pos", self._pos), ("src", self.src_block), ("status", self._status), ("workspace", self._ws)):
             setattr(h, name, t.data_ptr() if t is not None else None)
 
     @property
@@ -423,7 +423,6 @@ class MortarPack:
             self._pos = torch.from_numpy(octet_positions(self.h_offsets, self.Rb, self.Cb, self.seg_cb, self.h_col)).to(self.device)
             self._ws = torch.empty(int(_lib.lib().mortar_requantize_workspace_bytes()) // 8, dtype=torch.float64, device=self.device)
             self._status = torch.zeros(2, dtype=torch.int32, device=self.device)
-            self._scale = torch.empty(1, dtype=torch.float32, device=self.device)
             self._bind_repack()
 
     def _set_scale_form(self, uniform: float, one: int) -> None:
@@ -577,8 +576,7 @@ class MortarPack:
         """A second resident copy (own device buffers and schedules) of the same matrix."""
         import copy
         c = copy.copy(self)
-        for name in ("codes", "sdup", "col", "row_ptr", "row_desc", "codes_o", "sd_o", "col_o", "codes4_o", "scales_f32", "_ws", "_status",
-                     "_scale"):
+        for name in ("codes", "sdup", "col", "row_ptr", "row_desc", "codes_o", "sd_o", "col_o", "codes4_o", "scales_f32", "_ws", "_status"):
             if getattr(self, name) is not None:
                 setattr(c, name, getattr(self, name).clone())
         c._scheds = {k: v.clone() for k, v in self._scheds.items()}

@@ -227,3 +227,21 @@ def test_train_step_that_failed_leaves_no_stale_weights(dev, took):
     for m in layers:
         m.mortar_data.requires_grad_(True)
     assert mlp(x).requires_grad and took.count("train_forward") == 2
+
+
+def test_the_scales_of_a_step_stay_as_they_were(dev, took):
+    """Every step hands out scale tensors of its own: what a caller kept of step N does not change in step N + 1."""
+    mlp = synth.qat_mlp_module(synth.synth_mlp(64, 176, 0.3, seed=3), dev, seed=5)
+    layers = [mlp.gate_up._cms, mlp.down._cms]
+    x = torch.randn(70, 64, device=dev).to(torch.bfloat16).requires_grad_()
+    kept = []
+    for step in range(3):
+        mlp(x)
+        kept.append([m._pack.scales_f32 for m in layers])
+        for m, s in zip(layers, kept[-1]):
+            assert m._pack_scale is s is m._pack._transposed.scales_f32
+            m.mortar_data.data.mul_(2)
+    assert took == ["train_forward"] * 3
+    for step in (1, 2):
+        for first, s in zip(kept[0], kept[step]):
+            assert torch.equal(s, first * 2 ** step)           # a power of two scales every sum exactly

@@ -283,12 +283,13 @@ def test_packs_are_fresh_only_behind_a_training_forward_that_ended(native, monke
     layers = [mlp.gate_up._cms, mlp.down._cms]
     packs = [m.mortar_pack() for m in layers]
     assert encoded == packs and [m.mortar_pack() for m in layers] == packs and len(encoded) == 2
+    scales = torch.ones(1), torch.ones(1)
     if fails == "forward":
         def train_forward(*a):
             raise RuntimeError("out of memory")
     else:
         def train_forward(*a):
-            return None if fails == "declined" else (1, 2, 3)
+            return None if fails == "declined" else (1, 2, 3, *scales)
     native.train_forward = train_forward
     if fails == "step_pack":
         monkeypatch.setattr(packs[1], "sched", lambda n: (_ for _ in ()).throw(RuntimeError("out of memory")))
@@ -303,7 +304,7 @@ def test_packs_are_fresh_only_behind_a_training_forward_that_ended(native, monke
     assert encoded == ([] if fails is None else packs)
     forms = [(P.uniform_scale, P.one_scale) for W in packs for P in (W, W._transposed) if P is not None]
     assert forms == [(0.0, 1 if fails is None else 0)] * len(forms)
-    assert [W.scales_f32 is W._scale for W in packs] == [fails is None] * 2
+    assert [W.scales_f32 is s for W, s in zip(packs, scales)] == [fails is None] * 2
 
 
 def test_packs_are_stale_behind_a_re_pack_that_failed(monkeypatch):
