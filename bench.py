@@ -429,7 +429,7 @@ def main() -> None:
                                    "decode_stack_b1_us_per_mlp": t_s * 1e3 / n_sets,
                                    "decode_stack_b1_GBps": b_s / (t_s * 1e-3) / 1e9,
                                    "decode_stack_b1_frac_hbm": b_s / (t_s * 1e-3) / 1e9 / PEAK_HBM_GBS,
-                                   "note": "blocks multiplied as +-2 / 0, fp32 sums scaled once (scale-after-sum, as the "
+                                   "note": "blocks multiplied as a power of two / 0, fp32 sums scaled once (scale-after-sum, as the "
                                            "reference's decode kernel); the headline uses per-block scales"}
         # the reference engine's own decode arithmetic on that format: fp32 activations in and out, exact products,
         # fp32 scale after the sums (mortar_gemv with fp32 x); 8 MLPs (gate_up + SwiGLU, then down) per graph replay

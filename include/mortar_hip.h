@@ -72,8 +72,9 @@ typedef struct {
     int32_t seg_cb;   /* block-columns per K segment of the octet stream (>= Cb: one segment) */
     float uniform_scale;   /* != 0: every block has this (bf16-representable) scale, the reference's per-tensor
                               mortar_scale (deploy_quant.py:344-374); from mortar_uniform_scale_host.  The kernels then
-                              multiply +-2 / 0 blocks and scale the fp32 sums once, as the reference's decode kernel
-                              does (fused_decode_step.py:1441-1443), instead of scaling every block's weights.
+                              multiply the blocks as the power of two below the scale and apply the rest to the fp32 sums
+                              once, as the reference's decode kernel does with all of it (fused_decode_step.py:1441-1443),
+                              instead of scaling every block's weights.
                               0: per-block scales (always valid, also for a uniform matrix). */
     int32_t one_scale;     /* 1, with uniform_scale == 0: every block has the same scale, but its value is known on the
                               device only (sdup[0], written by mortar_requantize in modes 0 / 2 with no host wait): the

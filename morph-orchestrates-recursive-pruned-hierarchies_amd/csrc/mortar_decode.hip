@@ -475,7 +475,7 @@ int launch_gemv_f32(const GemvF32Params &p, hipStream_t st) {
 
 // ---- one scale for the whole matrix: the product runs on the bandwidth-bound SpMM kernels ----------------
 // The three bf16 terms of every activation row become three rows of a bf16 matrix [3B, in_features] (hi rows, then
-// mid, then lo); the SpMM kernels for matrices with one scale contract them with the +-2 / 0 blocks (every product
+// mid, then lo); the SpMM kernels for matrices with one scale contract them with the +-1 / 0 blocks (every product
 // exact, fp32 sums in the matrix pipe) and store the sums unrounded; a last kernel adds the three sums of a row, applies
 // the fp32 scale once (the reference's scale-after-sum) and the SwiGLU / gate epilogue.  Same arithmetic as the
 // work-list kernel above up to the order of the fp32 additions.

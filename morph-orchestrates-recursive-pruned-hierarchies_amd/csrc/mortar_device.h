@@ -39,13 +39,13 @@ __device__ __forceinline__ u32x4_t mortar_scale4(uint32_t nib, uint32_t sd) {
 __device__ __forceinline__ u32x4_t mortar_unpack8(uint32_t t, uint32_t sd) {
     return mortar_scale4(t & 0xCCCCCCCCu, sd);
 }
-// The conversions alone: bf16 +-2 / 0 for the eight nibbles (matrices with one scale, applied after the sums).
-__device__ __forceinline__ u32x4_t mortar_nib4(uint32_t nib) {
+// The conversions alone: bf16 +-2 cs / 0 for the eight nibbles, cs a power of two (matrices with one scale, applied after the sums).
+__device__ __forceinline__ u32x4_t mortar_nib4(uint32_t nib, float cs = 1.0f) {
     u32x4_t r;
-    r[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, 1.0f, 0));
-    r[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, 1.0f, 1));
-    r[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, 1.0f, 2));
-    r[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, 1.0f, 3));
+    r[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, cs, 0));
+    r[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, cs, 1));
+    r[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, cs, 2));
+    r[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(nib, cs, 3));
     return r;
 }
 

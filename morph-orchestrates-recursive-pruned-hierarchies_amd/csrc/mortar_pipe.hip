@@ -75,6 +75,7 @@ __global__ void __launch_bounds__(PIPE_WAVES * 64) mortar_pipe_kernel(const Spmm
     };
     descriptors(0);
     fetch(0, width(0));
+    mortar_resolve_scale<CODE>(p);
 
     auto segment = [&](int sg, auto last) {
         constexpr bool LAST = decltype(last)::value;
@@ -104,7 +105,6 @@ __global__ void __launch_bounds__(PIPE_WAVES * 64) mortar_pipe_kernel(const Spmm
         if (!LAST) descriptors(sg + 1);
         put(lb, width(sg));
         __syncthreads();
-        if (sg == 0) mortar_resolve_scale<CODE>(p);
         if (!LAST) fetch((sg + 1) * p.seg_cb, width(sg + 1));
 #pragma unroll
         for (int a = 0; a < RW; ++a) {

@@ -66,7 +66,7 @@ void fill(SpmmParams &p, const mortar_bcsr_t *W, const int32_t *sched, const uin
     p.avg_octets = (int)(((int64_t)W->nnz + 8 * (int64_t)W->Rb * p.nseg - 1) / (8 * (int64_t)W->Rb * p.nseg));
     p.x = x; p.ldx = ldx; p.M = (int)M; p.y = y; p.ldy = ldy;
     p.n_clusters = 1; p.cluster_size = 1 << 30;
-    p.uscale = 0.5f * W->uniform_scale;
+    mortar_set_scale(p, W->uniform_scale);
     if (W->uniform_scale == 0.f && W->one_scale && W->sdup && live && (W->one_scale == 2 || !recorded(st))) { p.uscale = 1.f; p.scale_dev = W->sdup; }
 }
 
@@ -175,8 +175,8 @@ int dispatch_prefill(int kind, SpmmParams &p, hipStream_t st) {
 // kind: 0 spmm, 1 gate_up + SwiGLU, 2 routed gate_up + SwiGLU, 3 spmm with an input mask.
 // Prefill-sized launches read the 4-bit code stream when the matrix carries one (cheaper unpack: one conversion
 // per register instead of shift + mask); decode-sized launches always stream the 2-bit codes (half the bytes).
-// A matrix with one scale (uniform_scale != 0, or one_scale: fill) runs the kernels that multiply +-2 / 0 blocks and scale the
-// accumulators once (decode-sized launches always, prefill-sized ones through the 4-bit stream).
+// A matrix with one scale (uniform_scale != 0, or one_scale: fill) runs the kernels that multiply the blocks as one power of two
+// (mortar_set_scale) and scale the accumulators once (decode-sized launches always, prefill-sized ones through the 4-bit stream).
 int dispatch(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
     // products over several K segments have small-tile forms beyond the decode sizes as well (the launcher returns -1
     // once they would need more than one round of workgroups)
@@ -237,13 +237,14 @@ int mortar_spmm_codes_f32(const mortar_bcsr_t *W, const int32_t *sched, const ui
     fill(p, W, sched, x, M, ldx, nullptr, ldy, static_cast<hipStream_t>(stream));
     p.n_units = W->Rb;
     p.y32 = y32;
-    p.uscale = 0.5f; p.scale_dev = nullptr;      // the kernels multiply the blocks as +-2 / 0
+    mortar_set_scale(p, 1.f);
+    p.scale_dev = nullptr;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (M <= MORTAR_SMALLM_MAX) {
         rc = mortar_smallm_launch(0, p, nullptr, 1, st);
         if (rc >= 0) return rc;
     }
-    if (!W->codes4_o) return MORTAR_NO_KERNEL;      // prefill-sized tiles multiply +-2 / 0 blocks only from the 4-bit stream
+    if (!W->codes4_o) return MORTAR_NO_KERNEL;      // prefill-sized tiles multiply blocks without scales only from the 4-bit stream
     p.codes_o = reinterpret_cast<const u32x4_t *>(W->codes4_o);
     return dispatch_prefill<CODE_4BIT | CODE_UNIFORM>(0, p, st);
 }

@@ -36,7 +36,7 @@ struct SpmmParams {
     int xcd_map;              // 1: workgroup ids are renumbered per XCD (grid padded to a multiple of 8)
     int norm;                 // 1: rows of x are RMS-normalised while they are staged (single-segment tiles only)
     float norm_eps;
-    float uscale;             // CODE_UNIFORM kernels: half the matrix's (bf16-rounded) scale (any value but 0 with scale_dev)
+    float uscale;             // CODE_UNIFORM kernels: what the sums are multiplied by (mortar_set_scale; any value but 0 with scale_dev)
     float *y32;               // plain products: unrounded fp32 output [M, ldy] in place of the bf16 store, or null
     const uint16_t *norm_w;   // bf16 [in_features] weight of that norm, or null for none
     // hyper-connection POST write in place of the plain store (small tiles, plain products): out[t, i, :] =
@@ -55,7 +55,8 @@ struct SpmmParams {
     int x_tiled, y_tiled;
     const uint32_t *scale_dev;   // CODE_UNIFORM kernels: the scale's pattern in device memory (mortar_bcsr_t.one_scale), or null
     int avg_octets;              // host only: octets of a row part on average, rounded up (mortar_chunk_launch)
-    int pad_[3];
+    float cscale;                // CODE_UNIFORM kernels: half the power of two that the codes stand for (mortar_set_scale)
+    int pad_[2];
 };
 
 // Device-side view of the launch parameters: the pointers carry the global address space in their type, so
@@ -74,6 +75,7 @@ struct SpmmView {
     int64_t ldx, ldy;
     int n_units, Cb, M, n_clusters, cluster_size, n_mtiles, n_split, seg_cb, nseg, Rb, xcd_map, norm;
     float norm_eps, uscale;
+    float cscale, cscale_host;                        // CODE_UNIFORM kernels: the blocks are multiplied as +-2 cscale / 0
     uint32_t scale_pat;                               // pattern behind SpmmParams::scale_dev, 0 without (mortar_resolve_scale)
     bool scale_on_dev;
     const MORTAR_GLOBAL u32x4_t *norm_w;
@@ -107,25 +109,38 @@ __device__ __forceinline__ SpmmView mortar_view(const SpmmParams &q) {
     v.hc_out = (MORTAR_GLOBAL char *)q.hc_out; v.hc_res = (const MORTAR_GLOBAL float *)q.hc_res;
     v.hc_post = (const MORTAR_GLOBAL float *)q.hc_post; v.hc_n = q.hc_n; v.hc_f32 = q.hc_f32;
     v.x_tiled = q.x_tiled; v.y_tiled = q.y_tiled;
+    v.cscale = 1.f; v.cscale_host = q.cscale;
     v.scale_on_dev = q.scale_dev != nullptr;
     v.scale_pat = v.scale_on_dev ? *(const MORTAR_GLOBAL uint32_t *)q.scale_dev : 0u;
     return v;
 }
 
 // How a kernel reads the code stream (template parameter CODE): bit 0 = the 4-bit stream, bit 1 = one scale for the
-// whole matrix (the reference's per-tensor mortar_scale): the blocks are multiplied as +-2 / 0 and the accumulators
-// are scaled once in the epilogue, which saves the packed multiplies and the scale broadcast of every pair.
+// whole matrix (the reference's per-tensor mortar_scale): the blocks are multiplied as one power of two and the
+// accumulators are scaled once in the epilogue (mortar_set_scale), which saves the packed multiplies and the scale broadcast of every pair.
 constexpr int CODE_2BIT = 0, CODE_4BIT = 1, CODE_UNIFORM = 2;
 
-// Half the scale from its pattern in device memory, for the CODE_UNIFORM kernels of a matrix whose scale the host does not
-// know.  The pattern is requested with the parameters and taken up here, behind the barrier that ends the staging: a load
-// still in flight in the product loop would make its counted waits full ones.  (Trainable matrices: five of the ten vector
-// instructions of a block pair fall away; the training step of 4096 tokens at 2048 x 5632 went 482 -> 462 us.)
+// The scale of the CODE_UNIFORM kernels in two factors: its power of two goes into the conversions of the codes, which take one for
+// nothing, and the mantissa (1 to 2, with the sign) to the epilogue.  A sum is then never larger than that of the scaled weights and
+// overflows only where that does (as +-2 / 0 the blocks overflowed at activations of 2^127, whatever the scale); everything short of
+// that has the same bits, a power of two being exact.
+inline void mortar_set_scale(SpmmParams &p, float scale) {
+    int e = 0;
+    p.uscale = 2.f * frexpf(scale, &e);            // 0 without a scale: not a CODE_UNIFORM launch
+    p.cscale = ldexpf(0.5f, e - 1);                // the conversions make +-2 of it
+}
+// Both factors of a matrix whose scale the host does not know, from its pattern in device memory (one fp16 exponent step below the bf16
+// scale).  The pattern is requested with the parameters and taken up where the staging ends (in front of the loop over K segments): a
+// load still in flight in the product loop would make its counted waits full ones.  (Trainable matrices: five of the ten vector instructions of a block pair fall
+// away; the training step of 4096 tokens at 2048 x 5632 went 482 -> 462 us.)
 template <int CODE>
 __device__ __forceinline__ void mortar_resolve_scale(SpmmView &p) {
-    if (!(CODE & CODE_UNIFORM) || !p.scale_on_dev) return;
-    const uint32_t pat = (uint32_t)__builtin_amdgcn_readfirstlane((int)p.scale_pat) & 0xffffu;
-    p.uscale = pat ? 0.5f * bf16_to_f32(pat + 0x0400u) : 0.f;      // the pattern is one fp16 exponent step below the bf16 scale
+    if (!(CODE & CODE_UNIFORM)) return;
+    p.cscale = p.cscale_host;
+    if (!p.scale_on_dev) return;
+    const uint32_t half = ((uint32_t)__builtin_amdgcn_readfirstlane((int)p.scale_pat) << 16) + 0x04000000u - 0x00800000u;
+    p.cscale = __builtin_bit_cast(float, half & 0x7f800000u);      // (a scale of 0 gives some other one: all its codes are 0)
+    p.uscale = __builtin_bit_cast(float, (half & 0x807fffffu) | 0x3f800000u);
 }
 
 constexpr int MORTAR_SMALLM_MAX = 64;    // rows up to which the small-tile (decode) instantiations are used
@@ -238,7 +253,7 @@ __device__ __forceinline__ void mortar_row_part(const SpmmView &p, const uint4 *
                     const int u = 4 * k + t;
                     if (t == 2 && u >= pairs) break;                  // the padded half of the last octet
                     const uint32_t nib = (CODE & CODE_4BIT) ? b.cw[k][t] : ((b.cw[k][t] << (2 * hsel)) & 0xCCCCCCCCu);
-                    const u32x4_t A = (CODE & CODE_UNIFORM) ? mortar_nib4(nib) : mortar_scale4(nib, mortar_row_bcast(b.sdv, u));
+                    const u32x4_t A = (CODE & CODE_UNIFORM) ? mortar_nib4(nib, p.cscale) : mortar_scale4(nib, mortar_row_bcast(b.sdv, u));
                     if (u + PD < NP) {
                         const uint32_t xo = mortar_row_bcast(ccs, u + PD) + xo_base;
 #pragma unroll
@@ -481,7 +496,7 @@ __device__ __forceinline__ void mortar_hc_post(const SpmmView &p, int tok, int f
 template <int NACC, int CODE = 0, bool HC = false, bool YT = false>
 __device__ __forceinline__ void mortar_store_unit(const SpmmView &p, int unit, int tok, int g, bool has_gates, float gv,
                                                   f32x4_t a0, f32x4_t a1) {
-    if (CODE & CODE_UNIFORM) {      // the blocks were multiplied as +-2: p.uscale is half the matrix's scale
+    if (CODE & CODE_UNIFORM) {      // the blocks were multiplied as a power of two: p.uscale is the rest of the scale (mortar_set_scale)
         a0 *= p.uscale;
         if (NACC == 2) a1 *= p.uscale;
     }
@@ -608,8 +623,8 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
 
     if (NACC == 2 && p.norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(next_unit + 4));      // gate_up may carry the norm
     else mortar_stage_tile<MT, WAVES, false, XT>(p, lx, m0, 0, p.Cb, tid);
-    __syncthreads();
     mortar_resolve_scale<CODE>(p);
+    __syncthreads();
 
     while (pos < u_end) {
         uint32_t drawn = 0;
@@ -714,6 +729,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
 #pragma unroll
     for (int q = 0; q < NP; ++q) dn[q] = mortar_part_desc<NACC>(p, pos0 + WAVES * (q / NACC), 0, q % NACC);
     int units[UPW];
+    mortar_resolve_scale<CODE>(p);
 
     for (int sg = 0; sg < p.nseg; ++sg) {
         const int c0 = sg * p.seg_cb;
@@ -746,7 +762,6 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
         if (sg > 0) __syncthreads();
         mortar_stage_tile<MT, WAVES, MASKED, XT>(p, lx, m0, c0, ncb, tid);
         __syncthreads();
-        if (sg == 0) mortar_resolve_scale<CODE>(p);
         if (!BATCH_AHEAD) {
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
@@ -876,8 +891,8 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
     if (NS && fused_norm) ns.finish(p, smem, m0, p.Cb, tid, reinterpret_cast<float *>(red));
     else if (fused_norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(smem + tile_bytes(MT, p.Cb)));
     else mortar_stage_tile<MT, WAVES, MASKED>(p, lx, m0, 0, p.Cb, tid);
-    __syncthreads();
     mortar_resolve_scale<CODE>(p);
+    __syncthreads();
     bool idle = skip;
     if (GATE_SKIP && valid && has_gates && p.cluster_size % 16 == 0) idle = __ballot(gsk != 0.f) == 0ull;      // NaN and negative gates multiply like any other
 

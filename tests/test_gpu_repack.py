@@ -724,3 +724,37 @@ def test_a_captured_training_step_re_packs_itself(dev):
         got = [t.clone() for t in out]
         for a, b in zip(got, grads()):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("M", [1, 5, 40, 70, 300, 600])
+@pytest.mark.parametrize("out_b,in_b", [(12, 48), (24, 160)])
+@pytest.mark.parametrize("scale", [0.021, -0.75, 2.0 ** -80, 1.0])
+def test_one_scale_products_of_large_activations(dev, M, out_b, in_b, scale):
+    """Activations near the largest bf16: a product with one scale overflows only where the scaled weights do, also with the scale on
+    the device, for W and W^T (values 0.9 to 1 of the largest that keep every result finite)."""
+    m = synth.synth_matrix(16 * out_b, 16 * in_b, 0.25, seed=31)
+    nnz = m["col_idx"].size
+    vt = torch.from_numpy(np.random.default_rng(3).choice(np.array([-1, 0, 1], np.float32), (nnz, 16, 16), p=[0.3, 0.4, 0.3]) * np.float32(abs(scale)))
+    packs = [MortarPack(None, None, m["col_idx"], m["offsets"], 16 * out_b, 16 * in_b, dev) for _ in range(2)]
+    s = torch.tensor([scale])
+    dense = np.zeros((out_b, in_b, 16, 16))
+    rows = np.repeat(np.arange(out_b), np.diff(m["offsets"]))
+    dense[rows, m["col_idx"]] = np.sign(vt.numpy()) * np.float64(O.bf16_round(np.array([abs(scale)], np.float32))[0])
+    dense = dense.transpose(0, 2, 1, 3).reshape(16 * out_b, 16 * in_b)
+    for t in (False, True):
+        w = dense.T if t else dense
+        top = min(3.3e38, 3.3e38 / np.abs(w).sum(axis=1).max())
+        rng = np.random.default_rng(M)
+        x = O.bf16_round((rng.uniform(0.9, 1.0, (M, w.shape[1])) * rng.choice([-1, 1], (M, w.shape[1])) * top).astype(np.float32))
+        want = x.astype(np.float64) @ w.T
+        for W, sync in zip(packs, (False, True)):
+            W.requantize(vt.to(dev), scale=s, sync=sync)
+            P = W
+            if t:
+                P = W.transposed()
+                P.requantize(vt.to(dev), scale=s, transpose=True, sync=sync)
+            got = to_np(ops.spmm(to_dev(x, dev), P)).astype(np.float64)
+            assert np.isfinite(got).all()
+            # fp32 sums of the terms |w x| of a row in any order, then one bf16 rounding
+            bound = np.abs(x).astype(np.float64) @ np.abs(w).T * 2.0 ** -20 + np.abs(want) * 2.0 ** -8
+            assert (np.abs(got - want) <= bound).all()
