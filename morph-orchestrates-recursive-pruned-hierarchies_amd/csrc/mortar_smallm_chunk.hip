@@ -50,10 +50,12 @@ int mortar_chunk_launch(int kind, int mt, SpmmParams &p, hipStream_t st) {
     const int nacc = kind + 1, nparts = p.nseg * nacc;
     const int64_t tiles = (p.M + mt - 1) / mt;
     for (int uw : {1, 2, 4}) {
-        // gate_up in workgroups of four units has two waves per unit to begin with: without chunks it is as fast or up to a tenth
-        // faster (d_model 768, 64 rows: 3.6 against 4.0 us), but where wide rows are normalised twice the waves share that work
-        // (16 rows with the norm, d_model 1024 4.9 against 5.0, 1536 5.7 against 5.7, 2048 6.0 against 5.8; without it 4.5 against 4.7 - by the
-        // width alone, not by the norm, so that the fused norm gives the bits of the separate one).
+        // gate_up in workgroups of four units has two waves per unit to begin with.  Four share the normalising of the rows, which is
+        // longer the wider they are, and cost an exchange more.  Two against four, us, 13 to 64 rows wherever this form is
+        // taken: with the norm 48 block-columns 4.7 against 4.9, 64 4.8 against 4.9, 72 to 88 5.2 to 5.5 either way, 96 5.46 against 5.43,
+        // 104 and 112 equal, 128 5.8 against 5.7; without it two are faster at every width (48 3.6 against 3.9, 88 4.1 against
+        // 4.4, 96 4.1 against 4.5, 128 4.4 against 4.6).  So the line lies where the norm's side turns: by the width alone,
+        // not by the norm, so that the fused norm gives the bits of the separate one.
         if (uw == 4 && kind == 1 && p.Cb < 96) continue;
         if (tiles * ((p.n_units + uw - 1) / uw) > 256) continue;
         const int cs = chunk_waves(nparts, p.avg_octets, uw);

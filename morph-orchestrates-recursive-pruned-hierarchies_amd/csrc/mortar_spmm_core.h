@@ -1099,8 +1099,12 @@ __attribute__((visibility("hidden"))) int mortar_smallm_tile(int Cb, int seg_cb,
 __attribute__((visibility("hidden"))) int mortar_chunk_launch(int kind, int mt, SpmmParams &p, hipStream_t st);
 // The same for more rows than that in 32-token tiles: matrices of one K segment, not kind 2; code: how p.codes_o is read.
 __attribute__((visibility("hidden"))) int mortar_mid_launch(int kind, int code, SpmmParams &p, hipStream_t st);
-// A plain product over two K segments, 65 rows and more, that 16-token tiles of all K serve best: the tile is small enough for the sums
-// beside it, and the workgroups of eight units are one round of the chip.
+// A plain product over two K segments, 65 rows and more, that 16-token tiles of all K serve best: the workgroups of eight units are one
+// round of the chip, and the tile (512 bytes per block-column) is staged faster in one go than two half tiles behind a barrier each.
+// Against the two buffers of mortar_pipe.hip, 48 to 128 units, 65 to 512 rows, 25 %: 160 block-columns 1.15 to 1.27 times as fast, 176
+// 1.13 to 1.23, 192 1.09 to 1.20, 208 1.04 to 1.17, 224 1.00 to 1.10, 240 0.92 to 1.07, 256 0.83 to 1.07, and half as fast at 288, where
+// the sums of eight units no longer fit beside the tile.  The line keeps a distance from 224, where the last row counts break even; no matrix of the
+// repository's configurations lies between 176 and 256.
 inline bool mortar_wide_tile_better(int kind, const SpmmParams &p) {
     return (kind == 0 || kind == 3) && p.nseg == 2 && p.Cb <= 192 && (p.M + 15) / 16 * (int64_t)((p.n_units + 7) / 8) <= 256;
 }
