@@ -75,7 +75,7 @@ class CMSBlockLinear(nn.Module):
         self._dense_mode, self._mortar, self._mortar_blocking = True, False, 0
         self._values_ternary_mode, self._values_threshold = False, 0.5
         self._pack: MortarPack | None = None
-        self._pack_key = None
+        self._pack_key = self._step_key = None       # _step_key: of the values that a step under way is encoding (step_pack)
         self._pack_gen, self._pack_t_gen = 0, -1
 
     # ------------------------------------------------------------------ masks / carve
@@ -288,18 +288,18 @@ class CMSBlockLinear(nn.Module):
         """The native step has enqueued the re-pack that ``step_pack`` prepared, which writes ``scale``: the state of the layer is now
         that behind ``repack_for_step``."""
         W, state = self._pack, self.__dict__
-        for P in (W, W._transposed) if with_t else (W,):
-            P.after_pair_repack(scale)
-        state["_pack_scale"], state["_pack_key"] = scale, state.pop("_step_key")
-        state["_pack_gen"] += 1
+        W.scales_f32 = state["_pack_scale"] = scale                 # (step_pack has set the form)
+        state["_pack_key"], state["_step_key"] = state["_step_key"], None
+        gen = state["_pack_gen"] = state["_pack_gen"] + 1
         if with_t:
-            state["_pack_t_gen"] = state["_pack_gen"]
+            W._transposed.scales_f32, state["_pack_t_gen"] = scale, gen
 
     def step_failed(self) -> None:
         """The step was declined, or ended in an error of which nobody knows whether it came before the re-pack: the next use
         re-encodes, and a pack that someone still holds runs in the form that is right for old and new values alike."""
         self.invalidate_pack()
-        if self.__dict__.pop("_step_key", None) is not None:         # step_pack had set the form
+        if self._step_key is not None:                               # step_pack had set the form
+            self._step_key = None
             for P in (self._pack, self._pack._transposed):
                 if P is not None:
                     P._set_scale_form(0.0, 0)

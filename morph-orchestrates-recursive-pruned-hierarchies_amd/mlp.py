@@ -67,7 +67,7 @@ def _native_step(x: Tensor, cg: CMSBlockLinear, cd: CMSBlockLinear, t_gu: bool, 
         W = cg.step_pack(t_gu)
         D = cd.step_pack(t_dn) if W is not None else None
         if D is not None:
-            r = _lib.native().train_forward(x, cg.mortar_data, cd.mortar_data, W.address, W._transposed.address if t_gu else 0,
+            r = _lib.native().train_forward(x, cg._parameters["mortar_data"], cd._parameters["mortar_data"], W.address, W._transposed.address if t_gu else 0,
                                             D.address, D._transposed.address if t_dn else 0, cg._values_threshold, cd._values_threshold)
     finally:
         if r is None:                 # nothing was launched (the general path re-packs), or an exception is on its way
@@ -107,7 +107,7 @@ class _SwiGLUMortarFn(torch.autograd.Function):
         # re-encoded at every step (.data writes do not advance the version counter), with the W^T that the backward will need
         need_x, need_gu = ctx.needs_input_grad[:2]
         r = None
-        if type(cg) is type(cd) is CMSBlockLinear and data_gu is cg.mortar_data and data_dn is cd.mortar_data:
+        if type(cg) is type(cd) is CMSBlockLinear and data_gu is cg._parameters.get("mortar_data") and data_dn is cd._parameters.get("mortar_data"):
             r = _native_step(x, cg, cd, need_x, need_x or need_gu)
         if r is not None:
             y, gu, h = r
