@@ -59,6 +59,8 @@ class _MortarLinearFn(torch.autograd.Function):
 
 
 class CMSBlockLinear(nn.Module):
+    _step_key = None          # of the values that a native step under way is encoding (step_pack); modules saved before it have none
+
     def __init__(self, in_features: int, out_features: int, tile_size: int = 16, density: float = 1.0,
                  bias: bool = True, score_ema_alpha: float = 0.95, device=None, dtype=None) -> None:
         super().__init__()
@@ -75,7 +77,7 @@ class CMSBlockLinear(nn.Module):
         self._dense_mode, self._mortar, self._mortar_blocking = True, False, 0
         self._values_ternary_mode, self._values_threshold = False, 0.5
         self._pack: MortarPack | None = None
-        self._pack_key = self._step_key = None       # _step_key: of the values that a step under way is encoding (step_pack)
+        self._pack_key = None
         self._pack_gen, self._pack_t_gen = 0, -1
 
     # ------------------------------------------------------------------ masks / carve
