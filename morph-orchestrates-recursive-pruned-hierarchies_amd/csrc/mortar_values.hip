@@ -131,7 +131,10 @@ struct ValOut {
                 v[h] = s[0];
                 v[2 + h] = s[1];
             }
-            __builtin_amdgcn_raw_buffer_store_b128(v, r, both || !odd ? off[ms] : 0xfffffff0u, row * 32, 0);
+            // The row goes into the vector offset: behind a 16-byte store with a scalar offset the compiler may overwrite the data
+            // registers in the next instruction, and gfx950 then stores the new values in the last lanes of a row (seen with
+            // `v_mov_b32` there; with a scalar offset the compiler assumes that no wait state is needed).
+            __builtin_amdgcn_raw_buffer_store_b128(v, r, (both || !odd) && off[ms] != 0xfffffff0u ? off[ms] + (uint32_t)row * 32 : 0xfffffff0u, 0, 0);
         }
     }
 };
