@@ -29,7 +29,6 @@ struct ValArgs {
     int seg_cb, nfine;          // fine K segments of seg_cb block-columns
     int sub;                    // fine segments that one LDS segment holds
     int n_split, per;           // workgroups that share a token tile; block-rows of one of them
-    int unit;                   // all of K in one tile: block-rows that a wave draws at a time (1 or 2)
 };
 
 // Tile layout in LDS: [pair of block-columns][token][64 bytes].  A wave instruction copies 16 tokens x 64 bytes straight from
@@ -40,22 +39,24 @@ struct ValArgs {
 template <int MT>
 __device__ __forceinline__ int val_enc(int c) { return (c >> 1) * (MT * 64) + (c & 1) * 32; }
 
-// Copies block-columns [c0, c0 + ncb) of the tile at token m0 into `dst`, as loader `w` of `nw`.  Tokens past M repeat the last
+// Copies block-columns [c0, c0 + ncb) of the tile at token m0 into `dst`, as loader `w` of NW.  Tokens past M repeat the last
 // one, a missing second column of the last pair repeats the first: both feed results that are never stored or never read.
-template <int MT>
-__device__ __forceinline__ void val_copy(const ValArgs &a, unsigned char *dst, int m0, int c0, int ncb, int i, int lane) {
-    constexpr int TG = MT / 16;
-    const int t = lane >> 2, u = (lane & 3) ^ mortar_unit_swz(t);
-    const int tg = i % TG, pr = i / TG;
-    const int tok = m0 + tg * 16 + t;
-    int c = 2 * pr + (u >> 1);
-    c = c < ncb ? c : ncb - 1;
-    const uint16_t *src = a.x + (int64_t)(tok < a.M ? tok : a.M - 1) * a.ldx + (int64_t)(c0 + c) * 16 + (u & 1) * 8;
-    mortar_load_to_lds((const MORTAR_GLOBAL char *)src, __builtin_amdgcn_readfirstlane(mortar_lds_addr(dst + (pr * MT + tg * 16) * 64)));
-}
-template <int MT>
-__device__ __forceinline__ void val_stage(const ValArgs &a, unsigned char *dst, int m0, int c0, int ncb, int w, int nw, int lane) {
-    for (int i = w; i < (ncb + 1) / 2 * (MT / 16); i += nw) val_copy<MT>(a, dst, m0, c0, ncb, i, lane);
+template <int MT, int NW>
+__device__ __forceinline__ void val_stage(const ValArgs &a, unsigned char *dst, int m0, int c0, int ncb, int w, int lane) {
+    constexpr int TG = MT / 16, PS = NW / TG;              // a loader keeps its 16 tokens and walks over the pairs
+    static_assert(NW % TG == 0, "loaders x token groups");
+    const int t = lane >> 2, u = (lane & 3) ^ mortar_unit_swz(t), tg = w % TG;
+    int tok = m0 + tg * 16 + t;
+    tok = tok < a.M ? tok : a.M - 1;
+    int pr = w / TG;
+    const MORTAR_GLOBAL char *src = (const MORTAR_GLOBAL char *)(a.x + (int64_t)tok * a.ldx + (int64_t)c0 * 16 + u * 8) + pr * 64;
+    uint32_t d = __builtin_amdgcn_readfirstlane(mortar_lds_addr(dst + (pr * MT + tg * 16) * 64));
+    for (; 2 * pr + 1 < ncb; pr += PS) {
+        mortar_load_to_lds(src, d);
+        src += PS * 64;
+        d += PS * MT * 64;
+    }
+    if (2 * pr < ncb) mortar_load_to_lds(src - (u >> 1) * 32, d);
 }
 
 // Four block pairs of one block-row part in registers: values as MFMA operands, the columns on lanes 0..3 of every 16-lane row.
@@ -63,6 +64,7 @@ struct ValBatch {
     u32x4_t A[4];
     int col;
 };
+constexpr int VAL_LOADS = 5;                          // load instructions of a batch
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t val_rsrc(const void *base, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
@@ -88,68 +90,93 @@ __device__ __forceinline__ void val_multiply(const unsigned char *lb, const ValB
     constexpr int MSUB = MT / 16;
     if (cnt <= 0) return;
     const uint32_t enc = (uint32_t)val_enc<MT>(b.col - c0);
-    u32x4_t B[2][MSUB];
-    auto operands = [&](int u) {
-        const unsigned char *p = lb + (mortar_row_bcast(enc, u) ^ lane_x);
+    u32x4_t B[MSUB];
+    auto operand = [&](int u, int ms) { return *reinterpret_cast<const u32x4_t *>(lb + (mortar_row_bcast(enc, u) ^ lane_x) + ms * 1024); };
 #pragma unroll
-        for (int ms = 0; ms < MSUB; ++ms) B[u & 1][ms] = *reinterpret_cast<const u32x4_t *>(p + ms * 1024);
-    };
-    operands(0);
+    for (int ms = 0; ms < MSUB; ++ms) B[ms] = operand(0, ms);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         if (2 * u >= cnt) break;
-        if (u < 3) operands(u + 1);
 #pragma unroll
-        for (int ms = 0; ms < MSUB; ++ms) acc[ms] = mortar_mfma(b.A[u], B[u & 1][ms], acc[ms]);
+        for (int ms = 0; ms < MSUB; ++ms) {
+            acc[ms] = mortar_mfma(b.A[u], B[ms], acc[ms]);
+            if (u < 3) B[ms] = operand(u + 1, ms);
+        }
     }
 }
 
-// Results of two consecutive block-rows, stored together: the lane groups exchange halves, so that a lane holds 8 consecutive
-// features of one row and a token's 32 features are one 64-byte piece (one row at a time, 32-byte pieces, the stores alone
-// bound the wide products).  Bounded buffer stores drop the tokens past M and, for the last row of an odd count, row b.
-template <int MT>
+// Results of RU = 2 or 4 consecutive block-rows in bf16 pairs, as a lane holds them ([row][sub-tile]: features 4 g .. + 3 of token n),
+// stored together.  Two rows: the lane groups exchange halves, so that a lane holds 8 consecutive features of one row and a token's
+// 32 features are one 64-byte piece.  Four: the halves of a 16-lane row then trade their second and first pair of rows, so that an
+// instruction stores 128-byte pieces of eight tokens.  Pieces matter where the rows of y lie a power of two apart, which puts the pieces
+// of a wave on few memory channels (64 tokens x 8 KB per workgroup: 32-byte pieces 71..117 us for 134 MB, 64-byte ones 34..42, 128-byte
+// ones 24, a fill 21).  Bounded buffer stores drop the tokens past M and the rows past the end (`rows` of the RU exist).  No scalar
+// offset: behind a 16-byte store that has one the compiler may overwrite the data registers in the next instruction, and gfx950 then
+// stores the new values in the last lanes of a row.
+// NT: non-temporal, the values and the tiles stay in the L2 (16384 x 768 x 4096: 53 -> 46 us); not for pieces below 64 bytes, which the
+// L2 then passes on unmerged (three times as slow).
+template <int MT, int RU, bool NT>
 struct ValOut {
+    static constexpr int TPI = RU == 4 ? 8 : 16;          // tokens per instruction
     __amdgpu_buffer_rsrc_t r;
-    uint32_t off[MT / 16], odd;
+    uint32_t off, ld;
+    int slot, nt;                                         // row of the unit that this lane stores; tokens from its first one on
     __device__ __forceinline__ ValOut(const ValArgs &a, int m0, int n, int g) {
-        const int nt = a.M - m0 < MT ? a.M - m0 : MT;
-        r = val_rsrc(a.y + (int64_t)m0 * a.ldy, (int)((nt - 1) * a.ldy * 2 + a.Rb * 32));
-        odd = g & 1;
-#pragma unroll
-        for (int ms = 0; ms < MT / 16; ++ms) {
-            const int t = ms * 16 + n;
-            off[ms] = t < nt ? (uint32_t)(t * a.ldy * 2) + odd * 32 + (g >> 1) * 16 : 0xfffffff0u;
-        }
+        const int tokens = a.M - m0 < MT ? a.M - m0 : MT, t = RU == 4 ? n & 7 : n;
+        r = val_rsrc(a.y + (int64_t)m0 * a.ldy, (int)((tokens - 1) * a.ldy * 2 + a.Rb * 32));
+        slot = (RU == 4 ? (n >> 3) * 2 : 0) + (g & 1);
+        nt = tokens - t;
+        ld = (uint32_t)(a.ldy * 2);
+        off = (uint32_t)t * ld + slot * 32 + (g >> 1) * 16;
     }
-    __device__ __forceinline__ void store(int row, bool both, const f32x4_t (&a0)[MT / 16], const f32x4_t (&a1)[MT / 16]) const {
+    __device__ __forceinline__ void store(int row, int rows, const u32x2_t (&p)[RU][MT / 16]) const {
+        const bool mine = slot < rows;
 #pragma unroll
         for (int ms = 0; ms < MT / 16; ++ms) {
-            u32x4_t v;
+            u32x4_t v[RU / 2];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const auto s = __builtin_amdgcn_permlane16_swap(bf16_pack2(a0[ms][2 * h], a0[ms][2 * h + 1]), bf16_pack2(a1[ms][2 * h], a1[ms][2 * h + 1]), false, false);
-                v[h] = s[0];
-                v[2 + h] = s[1];
+            for (int q = 0; q < RU / 2; ++q)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const auto s = __builtin_amdgcn_permlane16_swap(p[2 * q][ms][h], p[2 * q + 1][ms][h], false, false);
+                    v[q][h] = s[0];
+                    v[q][2 + h] = s[1];
+                }
+            if constexpr (RU == 4) {
+                const bool up = slot >= 2;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t got = __builtin_amdgcn_mov_dpp(up ? v[0][i] : v[1][i], 0x128, 0xf, 0xf, true);        // row_ror:8
+                    const uint32_t lo = up ? got : v[0][i], hi = up ? v[1][i] : got;
+                    v[0][i] = lo;
+                    v[1][i] = hi;
+                }
             }
-            // The row goes into the vector offset: behind a 16-byte store with a scalar offset the compiler may overwrite the data
-            // registers in the next instruction, and gfx950 then stores the new values in the last lanes of a row (seen with
-            // `v_mov_b32` there; with a scalar offset the compiler assumes that no wait state is needed).
-            __builtin_amdgcn_raw_buffer_store_b128(v, r, (both || !odd) && off[ms] != 0xfffffff0u ? off[ms] + (uint32_t)row * 32 : 0xfffffff0u, 0, 0);
+#pragma unroll
+            for (int h = 0; h < RU / 2; ++h) {
+                const int t0 = ms * 16 + h * TPI;
+                __builtin_amdgcn_raw_buffer_store_b128(v[h], r, mine && t0 < nt ? off + (uint32_t)t0 * ld + (uint32_t)row * 32 : 0xfffffff0u, 0, NT ? 2 : 0);
+            }
         }
     }
 };
+template <int MSUB>
+__device__ __forceinline__ void val_pack(const f32x4_t (&acc)[MSUB], u32x2_t (&p)[MSUB]) {
+#pragma unroll
+    for (int ms = 0; ms < MSUB; ++ms) p[ms] = u32x2_t{bf16_pack2(acc[ms][0], acc[ms][1]), bf16_pack2(acc[ms][2], acc[ms][3])};
+}
 
 // A uniform index array as scalar loads.
 __device__ __forceinline__ int val_idx(const int32_t *p, int i) {
     return ((const __attribute__((address_space(4))) int32_t *)p)[__builtin_amdgcn_readfirstlane(i)];
 }
 
-// All of K in one tile.  The waves draw block-rows (a.unit = 2: pairs of them) from a counter, so that rows of any length keep
-// all of them busy; a wave's batches form one stream across rows, requested two ahead of their products.  Narrow K is bound by
-// the results and the values together (16384 x 768 x 4096 at 25 %, 134 MB of results, a fill of which takes 21 us: 84 -> 51 us in a
-// loop over the same buffers, 57 over six sets of them, 65..69 in the trace of a training step, 153 MB written there; rows one at a
-// time took a quarter longer), wide K by the values from the L2, once per 32 tokens (4096 x 2048 x 11264: 102 -> 83 us, 18 TB/s of values).
-template <int MT>
+// All of K in one tile.  The waves draw units of RU consecutive block-rows from a counter, so that rows of any length keep all of them
+// busy; a wave's batches form one stream across rows, requested two ahead of their products, the first two before the tile is waited
+// for.  Narrow K is bound by the results and the values together: 16384 x 768 x 4096 at 25 % (134 MB of results, a fill of which takes
+// 21 us) takes 50 us over rotating buffers, of which stage and store alone are 33, the values alone 21, the products alone 25 (before
+// the non-temporal 128-byte pieces: 59 us).  Wide K is bound by the values from the L2, once per 32 tokens (4096 x 2048 x 11264: 82 us).
+template <int MT, int RU>
 __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const ValArgs a) {
     constexpr int MSUB = MT / 16;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -163,73 +190,79 @@ __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const V
     const uint32_t lane_x = (uint32_t)(n * 64 + (hsel ^ mortar_unit_swz(n)) * 16);
     const uint32_t lane_o = (uint32_t)(bsel * 512 + n * 32 + hsel * 16);
     const int lane_k = 2 * (n & 3) + bsel;
-    const ValOut<MT> out(a, m0, n, g);
-    struct Unit { int r, p0, p1, p2; };                   // rows r and r + 1 (unit == 1: r alone): blocks p0 .. p1 and p1 .. p2
+    struct Unit { int r, p0, p1, p2, p3, p4; };           // rows r .. r + 3: blocks p0 .. p1, p1 .. p2, ... (none past the range's end)
     auto load_unit = [&](int r) {
-        Unit q{r, 0, 0, 0};
+        Unit q{r, 0, 0, 0, 0, 0};
         if (r < r1) {
             q.p0 = val_idx(a.row_ptr, r);
             q.p1 = val_idx(a.row_ptr, r + 1);
-            q.p2 = a.unit == 2 && r + 1 < r1 ? val_idx(a.row_ptr, r + 2) : q.p1;
+            q.p2 = val_idx(a.row_ptr, r + 2 < r1 ? r + 2 : r1);
+            if (RU > 2) q.p3 = val_idx(a.row_ptr, r + 3 < r1 ? r + 3 : r1);
+            if (RU > 2) q.p4 = val_idx(a.row_ptr, r + 4 < r1 ? r + 4 : r1);
         }
         return q;
     };
-    Unit u = load_unit(r0 + a.unit * wave), v{r1, 0, 0, 0};
-    // request cursor: part f of the sequence u row 0, u row 1, v row 0, v row 1; blocks fj .. fje
+    Unit u = load_unit(r0 + RU * wave), v{r1, 0, 0, 0, 0, 0};
+    // request cursor: part f of the sequence u row 0, ..., v row 0, ...; blocks fj .. fje
     int f = 0, fj = u.p0, fje = u.p1;
+    auto part_end = [&](int i) {
+        if (RU == 2) return i < 2 ? (i < 1 ? u.p1 : u.p2) : (i < 3 ? v.p1 : v.p2);
+        return i < 4 ? (i < 2 ? (i < 1 ? u.p1 : u.p2) : (i < 3 ? u.p3 : u.p4)) : (i < 6 ? (i < 5 ? v.p1 : v.p2) : (i < 7 ? v.p3 : v.p4));
+    };
     auto request = [&](ValBatch &b) {
         val_fetch(a, b, fj, fje - fj, lane_o, lane_k);
         fj += 8;
         if (fj >= fje) {
             ++f;
-            const int up1 = u.p1, up2 = u.p2, vp0 = v.p0, vp1 = v.p1, vp2 = v.p2;
-            fj = f == 1 ? up1 : f == 2 ? vp0 : vp1;
-            fje = f == 1 ? up2 : f == 2 ? vp1 : vp2;
+            fj = f == RU ? v.p0 : fje;                    // the rows of a unit follow each other
+            fje = part_end(f);
         }
     };
-    if (tid == 0) *next_row = r0 + a.unit * VAL_WAVES;
-    val_stage<MT>(a, smem, m0, 0, a.Cb, wave, VAL_WAVES, lane);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (tid == 0) *next_row = r0 + RU * VAL_WAVES;
+    val_stage<MT, VAL_WAVES>(a, smem, m0, 0, a.Cb, wave, lane);
+    ValBatch b0, b1, b2;
+    request(b0);                                          // within the first unit
+    request(b1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * VAL_LOADS) : "memory");      // the tile has landed, the batches are on their way
     __syncthreads();
     auto draw = [&]() {
         int d = 0;
-        if (lane == 0) d = atomicAdd(next_row, a.unit);
+        if (lane == 0) d = atomicAdd(next_row, RU);
         return d;
     };
     if (u.r >= r1) return;
     v = load_unit(__builtin_amdgcn_readfirstlane(draw()));
     int drawn = draw();
-    ValBatch b0, b1, b2;
-    request(b0);
-    request(b1);
-    f32x4_t acc[MSUB], first[MSUB];
+    if (f == RU) { fj = v.p0; fje = v.p1; }
+    f32x4_t acc[MSUB];
+    u32x2_t done[RU][MSUB];                               // finished rows of the unit
 #pragma unroll
-    for (int ms = 0; ms < MSUB; ++ms) acc[ms] = first[ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    int k = 0, j = u.p0, je = u.p1;                       // part of u that is being multiplied
+    for (int ms = 0; ms < MSUB; ++ms) acc[ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    int k = 0, j = u.p0, je = u.p1;                       // row of u that is being multiplied
+    const ValOut<MT, RU, true> out(a, m0, n, g);
     // one batch; false when the wave's rows are done
     auto step = [&](const ValBatch &c, ValBatch &nx) {
         request(nx);
         val_multiply<MT>(smem, c, je - j, 0, lane_x, acc);
         j += 8;
         if (j < je) return true;
-        if (k == 0) {
 #pragma unroll
-            for (int ms = 0; ms < MSUB; ++ms) {
-                first[ms] = acc[ms];
-                acc[ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            }
-            k = 1; j = u.p1; je = u.p2;
-            return true;
-        }
-        out.store(u.r, a.unit == 2 && u.r + 1 < r1, first, acc);
+        for (int q = 0; q < RU; ++q)
+            if (q == k) val_pack<MSUB>(acc, done[q]);
 #pragma unroll
         for (int ms = 0; ms < MSUB; ++ms) acc[ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (++k < RU) {
+            j = je;
+            je = part_end(k);
+            return true;
+        }
+        out.store(u.r, r1 - u.r, done);
         u = v;
         if (u.r >= r1) return false;
-        f -= 2;
+        f -= RU;
         k = 0; j = u.p0; je = u.p1;
         v = load_unit(__builtin_amdgcn_readfirstlane(drawn));
-        if (f == 2) { fj = v.p0; fje = v.p1; }            // the cursor stands at the first part of a unit that was not known yet
+        if (f == RU) { fj = v.p0; fje = v.p1; }           // the cursor stands at the first part of a unit that was not known yet
         drawn = draw();
         return true;
     };
@@ -239,8 +272,8 @@ __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const V
 // Wider K: segments through two LDS buffers, one barrier each.  Four loader waves copy the next segment while twelve multiply the
 // current one: a wave's loads complete in order, so a wave that did both would wait for the copies (from beyond the L2) at its
 // next weights.  A consumer keeps the accumulators of its UPW block-rows in registers over the segments.  The values (once per
-// 64 tokens from the L2) and the operand reads from LDS bound it.  16384 x 4096 x 768 at 25 %: 91 -> 50 us in a loop over the same
-// buffers, 62 over six sets of them, 61..72 in the trace of a training step.  Segments of 24 columns in three buffers took 6 % longer
+// 64 tokens from the L2) and the operand reads from LDS bound it.  16384 x 4096 x 768 at 25 %: 58 us over rotating buffers (62 before its
+// results left in 128-byte non-temporal pieces), of which the copies alone are 28, the values alone 28, the products alone 32.  Segments of 24 columns in three buffers took 6 % longer
 // (short parts leave a batch half empty), batches requested two ahead 18 % (registers, moves).
 template <int MT, int UPW>
 __global__ void __launch_bounds__((VAL_CW + VAL_LOADERS) * 64) values_segmented_kernel(const ValArgs a) {
@@ -256,7 +289,7 @@ __global__ void __launch_bounds__((VAL_CW + VAL_LOADERS) * 64) values_segmented_
         // segment sg is in its buffer at barrier sg; the other buffer was multiplied before that barrier
         for (int sg = 0; sg <= nseg; ++sg) {
             const int c0 = sg * seg, ncb = a.Cb - c0 < seg ? a.Cb - c0 : seg;
-            if (sg < nseg) val_stage<MT>(a, smem + (sg & 1) * buf_bytes, m0, c0, ncb, wave - VAL_CW, VAL_LOADERS, lane);
+            if (sg < nseg) val_stage<MT, VAL_LOADERS>(a, smem + (sg & 1) * buf_bytes, m0, c0, ncb, wave - VAL_CW, lane);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
         }
@@ -310,10 +343,16 @@ __global__ void __launch_bounds__((VAL_CW + VAL_LOADERS) * 64) values_segmented_
         for (int k = 1; k <= UPW; ++k) range(sg + 1 + k / UPW, k % UPW, lo[k], hi[k]);
         __syncthreads();
     }
-    const ValOut<MT> out(a, m0, n, g);
+    constexpr int RU = UPW < 4 ? 2 : 4;
+    const ValOut<MT, RU, (UPW > 1)> out(a, m0, n, g);
 #pragma unroll
-    for (int k = 0; k < UPW; k += 2)
-        if (row0 + k < a.Rb) out.store(row0 + k, k + 1 < UPW && row0 + k + 1 < a.Rb, acc[k], acc[k + 1 < UPW ? k + 1 : k]);
+    for (int k = 0; k < UPW; k += RU) {
+        u32x2_t p[RU][MSUB];
+#pragma unroll
+        for (int q = 0; q < RU; ++q) val_pack<MSUB>(acc[k + q < UPW ? k + q : k], p[q]);
+        const int rows = a.Rb - row0 - k;
+        if (rows > 0) out.store(row0 + k, UPW < RU && rows > UPW ? UPW : rows, p);
+    }
 }
 
 __global__ void __launch_bounds__(256) values_zero_kernel(uint16_t *y, int64_t M, int n4, int64_t ldy) {      // a matrix without blocks
@@ -353,14 +392,18 @@ int val_launch(K kern, bool &done, const ValArgs &a, int64_t grid, int threads, 
 
 template <int MT>
 int launch_resident(ValArgs &a, hipStream_t st) {
-    static bool done = false;
+    static bool done4 = false, done2 = false;
     const int tiles = (a.M + MT - 1) / MT, max_split = (a.Rb + VAL_WAVES - 1) / VAL_WAVES;
     int split = 256 / tiles;                 // about one workgroup per CU and round; every workgroup stages the whole tile
     split = split < 1 ? 1 : (split > max_split ? max_split : split);
     a.n_split = split;
-    a.per = ((a.Rb + split - 1) / split + 1) & ~1;
-    a.unit = a.per >= 4 * VAL_WAVES ? 2 : 1;              // pairs of rows (64-byte stores) while every wave has two of them
-    return val_launch(values_resident_kernel<MT>, done, a, (int64_t)tiles * split, VAL_WAVES * 64, (a.Cb + 1) / 2 * (MT * 64) + 16, st);
+    a.per = ((a.Rb + split - 1) / split + 3) & ~3;
+    const int smem = (a.Cb + 1) / 2 * (MT * 64) + 16;
+    // Four rows per unit while every wave has two such units, else two.  16384 x 768 x 4096 at 12.5 / 25 %: 37 / 51 us against 47 / 51 with
+    // two rows, 8192 tokens 23 / 31 against 27 / 31; 4099 tokens (1.4 units of four per wave) 17.2 / 21.3 against 15.3 / 20.1, 300 tokens
+    // 7.0 / 8.8 against 5.7 / 6.7.
+    if (a.per >= 8 * VAL_WAVES) return val_launch(values_resident_kernel<MT, 4>, done4, a, (int64_t)tiles * split, VAL_WAVES * 64, smem, st);
+    return val_launch(values_resident_kernel<MT, 2>, done2, a, (int64_t)tiles * split, VAL_WAVES * 64, smem, st);
 }
 
 template <int MT, int UPW>

@@ -38,6 +38,12 @@ def test_values_product_edges(dev, Rb, Cb, M, density):
         assert torch.equal(ops.transpose_blocks(data, src), data[src.long()].transpose(1, 2))
 
 
+@pytest.mark.parametrize("Rb,Cb,M", [(131, 5, 16400), (129, 80, 8161), (256, 3, 8137)])      # units of four rows: 64- and 32-token tiles, rows and tokens left over
+@pytest.mark.parametrize("density", [0.04, 0.5])
+def test_values_product_four_rows_at_a_time(dev, Rb, Cb, M, density):
+    test_values_product_edges(dev, Rb, Cb, M, density)
+
+
 @pytest.mark.parametrize("Rb,Cb", [(5, 3), (33, 170)])                 # all of K in one tile, K segments
 @pytest.mark.parametrize("ld,M", [(2 ** 23 + 8, 70), (2 ** 26, 19), (2 ** 30, 3)])      # 64 rows of y in 31 bits; 16 of them; one
 def test_values_product_into_rows_far_apart(dev, Rb, Cb, ld, M):
