@@ -88,48 +88,84 @@ int launch_resident_any(SpmmParams &p, hipStream_t st) {
     }
 }
 
-constexpr int SEG_WAVES = 16, SEG_UPW = 4;
+constexpr int SEG_WAVES = 16;
 
-// Row units per wave of the K-segmented plain product: 4, 2 or 1.  Fewer units per wave mean more workgroups per token
-// tile (64 units per workgroup left 8 workgroups for 128 tokens) but every workgroup stages the tile's segments again,
-// and workgroups beyond the 256 CUs wait for a second round: take the choice with the least rounds x (staging + units),
-// staging weighing about three units.
-int segmented_upw(const SpmmParams &p) {
-    const int64_t tiles = (p.M + 31) / 32;
-    int best = SEG_UPW;
-    int64_t best_cost = 0;
-    for (int upw = SEG_UPW; upw >= 1; upw >>= 1) {
-        const int64_t wgs = tiles * ((p.n_units + SEG_WAVES * upw - 1) / (SEG_WAVES * upw));
-        const int64_t cost = ((wgs + 255) / 256) * (3 + upw);
-        if (upw == SEG_UPW || cost < best_cost) { best = upw; best_cost = cost; }
+// Shape of a K-segmented launch: row units per wave that share one staging of the tile's segments, and the length of the runs over the
+// rows of units of all tiles that the workgroups take (SpmmParams::span, 0: one group of units each).
+struct SegShape { int upw, span; };
+
+// Fewer units per wave mean more workgroups per token tile (64 units per workgroup left 8 workgroups for 128 tokens), but every
+// workgroup stages the tile's segments again, and workgroups beyond the 256 CUs wait for a second round: the choice with the least
+// rounds x (staging + units).  In between, runs of equal length for 256 workgroups (up to run_upw units per wave, mortar_seg_runs):
+// the slowest one's units and stagings.  `down` of d_model 2048: 4500 rows (282 workgroups of four units per wave) 65 -> 52 us, 9000 112 ->
+// 101, 2500 (three units per wave, new with the runs) 33.5 -> 28; [2048, 11264] at 5000 rows 133 -> 104; 4096 and 8192 rows, whole
+// rounds as they were, unchanged.
+template <int N>
+SegShape seg_shape(const SpmmParams &p, const int (&upws)[N], int stage, int unit, int run_upw) {
+    const int64_t tiles = (p.M + 31) / 32, rows = (p.n_units + SEG_WAVES - 1) / SEG_WAVES, all = tiles * rows;
+    SegShape best{upws[0], 0};
+    int64_t best_cost = INT64_MAX;
+    for (int upw : upws) {
+        const int64_t wgs = tiles * ((rows + upw - 1) / upw), cost = (wgs + 255) / 256 * (stage + unit * upw);
+        if (cost < best_cost) { best = SegShape{upw, 0}; best_cost = cost; }
+    }
+    if (all >= 0x7fffffff) return best;
+    const int64_t span = (all + 255) / 256;
+    for (int upw : upws) {
+        if (upw > run_upw) continue;
+        int64_t groups = 0;                                           // of the workgroup that has most of them
+        for (int64_t w = 0; w < rows && w * span < all; ++w) {        // where the runs start repeats after at most `rows` of them
+            int64_t at = w * span % rows, left = span, n = 0;
+            while (left > 0) {
+                const int64_t len = rows - at < left ? rows - at : left;
+                n += (len + upw - 1) / upw;
+                left -= len;
+                at = 0;
+            }
+            groups = n > groups ? n : groups;
+        }
+        const int64_t cost = unit * span + stage * groups;
+        if (cost * 21 < best_cost * 20) { best = SegShape{upw, (int)span}; best_cost = cost; }
     }
     return best;
 }
 
-// Gate/up unit pairs per wave of the K-segmented gate_up: 1, 2 or 3 (four spill), the choice with the least rounds of 256
-// workgroups x (staging + units).  A unit pair takes about 6.7 us and staging the segments 5 us (d_model 3072 and 4096), so a round
-// weighs 3 + 4 upw.  With two units per wave throughout, 400 rows of d_model 4096 were 286 workgroups: 83 -> 70 us for the MLP; 150
-// rows 52 -> 44, 1999 rows (1386 workgroups, 5.4 rounds) 236 -> 227; d_model 3072 at 200 rows 40.9 -> 34.6, at 600 64 -> 52.5.
-int gateup_upw(const SpmmParams &p) {
-    const int64_t tiles = (p.M + 31) / 32;
-    int best = 2;
-    int64_t best_cost = INT64_MAX;
-    for (int upw : {2, 3, 1}) {
-        const int64_t wgs = tiles * ((p.n_units + SEG_WAVES * upw - 1) / (SEG_WAVES * upw));
-        const int64_t cost = (wgs + 255) / 256 * (3 + 4 * upw);
-        if (cost < best_cost) { best = upw; best_cost = cost; }
+// The plain product: staging weighs about three units.
+template <bool MASKED, bool TL>
+SegShape segmented_shape(const SpmmParams &p) { return seg_shape(p, {4, 3, 2, 1}, 3, 1, MASKED ? 0 : TL ? 4 : 3); }
+
+// gate_up: 1, 2 or 3 unit pairs per wave (four spill).  A unit pair takes about 6.7 us and staging the segments 5 us (d_model 3072 and
+// 4096).  With two units per wave throughout, 400 rows of d_model 4096 were 286 workgroups: 83 -> 70 us for the MLP; 150
+// rows 52 -> 44; d_model 3072 at 200 rows 40.9 -> 34.6, at 600 64 -> 52.5.
+SegShape gateup_shape(const SpmmParams &p) { return seg_shape(p, {2, 3, 1}, 3, 4, 0); }
+
+template <bool MASKED, int CODE, bool TL = false>
+int launch_segmented_plain(SpmmParams &p, hipStream_t st) {
+    const SegShape s = segmented_shape<MASKED, TL>(p);
+    p.span = s.span;
+    switch (s.upw) {
+        case 1: return mortar_launch_segmented<32, 1, MASKED, SEG_WAVES, 1, false, CODE, TL>(p, nullptr, 1, st);
+        case 2: return mortar_launch_segmented<32, 1, MASKED, SEG_WAVES, 2, false, CODE, TL>(p, nullptr, 1, st);
+        case 3: return mortar_launch_segmented<32, 1, MASKED, SEG_WAVES, 3, false, CODE, TL>(p, nullptr, 1, st);
     }
-    return best;
+    return mortar_launch_segmented<32, 1, MASKED, SEG_WAVES, 4, false, CODE, TL>(p, nullptr, 1, st);
+}
+
+template <int CODE, bool TL = false>
+int launch_segmented_gateup(SpmmParams &p, hipStream_t st) {
+    const SegShape s = gateup_shape(p);
+    p.span = s.span;
+    switch (s.upw) {
+        case 2: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 2, false, CODE, TL>(p, nullptr, 1, st);
+        case 3: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 3, false, CODE, TL>(p, nullptr, 1, st);
+    }
+    return mortar_launch_segmented<32, 2, false, SEG_WAVES, 1, false, CODE, TL>(p, nullptr, 1, st);
 }
 
 template <int CODE>
 int dispatch_gateup_tiled(SpmmParams &p, hipStream_t st) {     // gate_up + SwiGLU storing tile-ordered hidden activations
     if (p.nseg == 1) return launch_resident_any<2, false, CODE, true>(p, st);
-    switch (gateup_upw(p)) {
-        case 2: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 2, false, CODE, true>(p, nullptr, 1, st);
-        case 3: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 3, false, CODE, true>(p, nullptr, 1, st);
-    }
-    return mortar_launch_segmented<32, 2, false, SEG_WAVES, 1, false, CODE, true>(p, nullptr, 1, st);
+    return launch_segmented_gateup<CODE, true>(p, st);
 }
 
 // Plain product of a `down` whose input is stored in tile order (mortar_mlp_bf16): the instantiations that copy their
@@ -137,38 +173,16 @@ int dispatch_gateup_tiled(SpmmParams &p, hipStream_t st) {     // gate_up + SwiG
 template <int CODE>
 int dispatch_prefill_tiled(SpmmParams &p, hipStream_t st) {
     if (p.nseg == 1) return mortar_launch_resident<32, 1, false, 16, false, CODE, true>(p, nullptr, 1, st);
-    switch (segmented_upw(p)) {
-        case 1: return mortar_launch_segmented<32, 1, false, SEG_WAVES, 1, false, CODE, true>(p, nullptr, 1, st);
-        case 2: return mortar_launch_segmented<32, 1, false, SEG_WAVES, 2, false, CODE, true>(p, nullptr, 1, st);
-    }
-    return mortar_launch_segmented<32, 1, false, SEG_WAVES, SEG_UPW, false, CODE, true>(p, nullptr, 1, st);
+    return launch_segmented_plain<false, CODE, true>(p, st);
 }
 
 template <int CODE>
 int dispatch_prefill(int kind, SpmmParams &p, hipStream_t st) {
     switch (kind) {
-        case 0:
-            if (p.nseg == 1) return launch_resident_any<1, false, CODE>(p, st);
-            switch (segmented_upw(p)) {
-                case 1: return mortar_launch_segmented<32, 1, false, SEG_WAVES, 1, false, CODE>(p, nullptr, 1, st);
-                case 2: return mortar_launch_segmented<32, 1, false, SEG_WAVES, 2, false, CODE>(p, nullptr, 1, st);
-            }
-            return mortar_launch_segmented<32, 1, false, SEG_WAVES, SEG_UPW, false, CODE>(p, nullptr, 1, st);
-        case 1:
-            if (p.nseg == 1) return launch_resident_any<2, false, CODE>(p, st);
-            switch (gateup_upw(p)) {
-                case 2: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 2, false, CODE>(p, nullptr, 1, st);
-                case 3: return mortar_launch_segmented<32, 2, false, SEG_WAVES, 3, false, CODE>(p, nullptr, 1, st);
-            }
-            return mortar_launch_segmented<32, 2, false, SEG_WAVES, 1, false, CODE>(p, nullptr, 1, st);
-        case 2:
-            return launch_resident_any<2, true, CODE>(p, st);
-        default:
-            switch (segmented_upw(p)) {
-                case 1: return mortar_launch_segmented<32, 1, true, SEG_WAVES, 1, false, CODE>(p, nullptr, 1, st);
-                case 2: return mortar_launch_segmented<32, 1, true, SEG_WAVES, 2, false, CODE>(p, nullptr, 1, st);
-            }
-            return mortar_launch_segmented<32, 1, true, SEG_WAVES, SEG_UPW, false, CODE>(p, nullptr, 1, st);
+        case 0: return p.nseg == 1 ? launch_resident_any<1, false, CODE>(p, st) : launch_segmented_plain<false, CODE>(p, st);
+        case 1: return p.nseg == 1 ? launch_resident_any<2, false, CODE>(p, st) : launch_segmented_gateup<CODE>(p, st);
+        case 2: return launch_resident_any<2, true, CODE>(p, st);
+        default: return launch_segmented_plain<true, CODE>(p, st);
     }
 }
 

@@ -56,7 +56,9 @@ struct SpmmParams {
     const uint32_t *scale_dev;   // CODE_UNIFORM kernels: the scale's pattern in device memory (mortar_bcsr_t.one_scale), or null
     int avg_octets;              // host only: octets of a row part on average, rounded up (mortar_chunk_launch)
     float cscale;                // CODE_UNIFORM kernels: half the power of two that the codes stand for (mortar_set_scale)
-    int pad_[2];
+    int span;                    // prefill tiles: > 0: workgroups take runs of this length over the units of all tiles (mortar_span_resident,
+                                 // mortar_span_segmented), 0: n_split workgroups per tile
+    int pad_[1];
 };
 
 // Device-side view of the launch parameters: the pointers carry the global address space in their type, so
@@ -82,7 +84,7 @@ struct SpmmView {
     const MORTAR_GLOBAL char *hc_h, *hc_term;
     MORTAR_GLOBAL char *hc_out;
     const MORTAR_GLOBAL float *hc_res, *hc_post;
-    int hc_n, hc_f32, x_tiled, y_tiled;
+    int hc_n, hc_f32, x_tiled, y_tiled, span;
 };
 static_assert(sizeof(SpmmParams) % 16 == 0, "table entries are copied in 16-byte words");
 // Entry i of a parameter table in device memory (uniform address: scalar loads).
@@ -108,7 +110,7 @@ __device__ __forceinline__ SpmmView mortar_view(const SpmmParams &q) {
     v.hc_h = (const MORTAR_GLOBAL char *)q.hc_h; v.hc_term = (const MORTAR_GLOBAL char *)q.hc_term;
     v.hc_out = (MORTAR_GLOBAL char *)q.hc_out; v.hc_res = (const MORTAR_GLOBAL float *)q.hc_res;
     v.hc_post = (const MORTAR_GLOBAL float *)q.hc_post; v.hc_n = q.hc_n; v.hc_f32 = q.hc_f32;
-    v.x_tiled = q.x_tiled; v.y_tiled = q.y_tiled;
+    v.x_tiled = q.x_tiled; v.y_tiled = q.y_tiled; v.span = q.span;
     v.cscale = 1.f; v.cscale_host = q.cscale;
     v.scale_on_dev = q.scale_dev != nullptr;
     v.scale_pat = v.scale_on_dev ? *(const MORTAR_GLOBAL uint32_t *)q.scale_dev : 0u;
@@ -581,107 +583,133 @@ __device__ __forceinline__ u32x4_t mortar_part_desc_scalar(const SpmmView &p, in
     return d;
 }
 
+// The thread's index, unknown to the compiler but for its range: what is computed from it inside a loop stays there.  (The addresses of
+// the staging and of the stores, kept in registers across the products instead, made the prefill kernels spill.  Without the range the
+// addresses take 64 bits.)
+__device__ __forceinline__ int mortar_opaque_tid(int tid) {
+    asm volatile("" : "+v"(tid));
+    return tid & 1023;
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // Resident kernel.  The workgroup stages x[MT, K] once; then every wave walks whole row units on its own,
 // streaming the unit's block pairs straight from global memory in batches (a row's blocks are contiguous).
 // No barrier after the first one.  A wave's work is a chain of row parts (unit, segment, row of the unit) whose
 // descriptors come from the schedule table one part ahead; latency is hidden by the waves that share a SIMD.
 // ---------------------------------------------------------------------------------------------------------
+// RUNS: the workgroups take runs of SpmmParams::span units (a kernel of its own: the loop costs the other launches 0.4 us).
 // TL: the hidden activations of the two-launch MLP are in tile order: a plain product (NACC = 1) stages its input from
 // them (SpmmParams::x_tiled), a gate_up (NACC = 2) stores its result so (SpmmParams::y_tiled).
-template <int MT, int NACC, bool ROUTED, int WAVES, bool TABLE, int CODE, bool TL = false>
+template <int MT, int NACC, bool ROUTED, int WAVES, bool TABLE, int CODE, bool TL = false, bool RUNS = false>
 __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmParams p0, const SpmmParams *table) {
     constexpr int MSUB = (MT + 15) / 16;
     constexpr bool XT = TL && NACC == 1, YT = TL && NACC == 2;
     SpmmView p = mortar_view(TABLE ? mortar_table_entry(table, blockIdx.y) : p0);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint4 *lx = reinterpret_cast<uint4 *>(smem);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n = lane & 15, g = lane >> 4, bsel = g >> 1, hsel = g & 1;
+    const int tid0 = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
     // Workgroups are dealt round-robin over the 8 XCDs (each with its own L2): renumber them so that the
     // n_split workgroups that stage the same token tile run on one XCD and share its copy of the tile.
     const int wg = p.xcd_map ? (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
-    if (wg >= p.n_mtiles * p.n_split) return;
-    const int mt = wg / p.n_split, sp = wg % p.n_split;
-    const int m0 = mt * MT;
-    const uint32_t lane_xo = (uint32_t)(hsel * 16 + (ROUTED ? 0 : n * 32));
     const bool has_gates = p.gates != nullptr;
-
-    const int per = (p.n_units + p.n_split - 1) / p.n_split;
-    const int u_end = (sp + 1) * per < p.n_units ? (sp + 1) * per : p.n_units;
-    // Units are handed out dynamically: a wave starts with position `wave` of the workgroup's window and draws
-    // its next position from a counter in LDS when it begins a unit (one unit ahead, so that the descriptor of the
-    // next unit's first part can still be fetched early).  The SIMD arbiter favours the oldest wave, so with a
-    // fixed assignment the waves of a SIMD would finish one after another and leave it with one or two waves;
-    // drawing positions keeps all waves busy until the window is empty.
     uint32_t *next_unit = reinterpret_cast<uint32_t *>(smem + tile_bytes(MT, p.Cb));
-    if (tid == 0) *next_unit = WAVES;
-    const int base = sp * per;
-    int pos = base + wave;
-    u32x4_t d0 = mortar_part_desc<NACC>(p, pos, 0, 0);
 
-    if (NACC == 2 && p.norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(next_unit + 4));      // gate_up may carry the norm
-    else mortar_stage_tile<MT, WAVES, false, XT>(p, lx, m0, 0, p.Cb, tid);
-    mortar_resolve_scale<CODE>(p);
-    __syncthreads();
+    // The workgroup's units: a run of one tile's or, with a span, a run over the units of all tiles, cut where a tile ends.
+    int mt, base, left;
+    if (RUNS) {
+        const int first = wg * p.span, all = p.n_mtiles * p.n_units;
+        if (first >= all) return;
+        mt = first / p.n_units;
+        base = first - mt * p.n_units;
+        left = all - first < p.span ? all - first : p.span;
+    } else {
+        if (wg >= p.n_mtiles * p.n_split) return;
+        const int per = (p.n_units + p.n_split - 1) / p.n_split;
+        mt = wg / p.n_split;
+        base = wg % p.n_split * per;
+        left = p.n_units - base < per ? p.n_units - base : per;
+    }
+    for (bool again = false;; again = true) {
+        const int m0 = mt * MT;
+        const int tid = RUNS ? mortar_opaque_tid(tid0) : tid0, lane = tid & 63, n = lane & 15, g = lane >> 4, bsel = g >> 1, hsel = g & 1;
+        const uint32_t lane_xo = (uint32_t)(hsel * 16 + (ROUTED ? 0 : n * 32));
+        const int u_end = base + left < p.n_units ? base + left : p.n_units;
+        if (RUNS && again) __syncthreads();           // the tile before has been multiplied
+        // Units are handed out dynamically: a wave starts with position `wave` of the workgroup's window and draws
+        // its next position from a counter in LDS when it begins a unit (one unit ahead, so that the descriptor of the
+        // next unit's first part can still be fetched early).  The SIMD arbiter favours the oldest wave, so with a
+        // fixed assignment the waves of a SIMD would finish one after another and leave it with one or two waves;
+        // drawing positions keeps all waves busy until the window is empty.
+        if (tid == 0) *next_unit = WAVES;
+        int pos = base + wave;
+        u32x4_t d0 = mortar_part_desc<NACC>(p, pos, 0, 0);
 
-    while (pos < u_end) {
-        uint32_t drawn = 0;
-        if (lane == 0) drawn = atomicAdd(next_unit, 1u);
-        // coordinates of the part after the current one; its descriptor is fetched while the current part runs
-        int p1 = pos, s1 = 0, a1 = 0;
-        int npos = -1;       // position of this wave's next unit, known from the second part on
-        auto advance = [&](int &ps, int &s, int &a_) {
-            if (++a_ == NACC) { a_ = 0; if (++s == p.nseg) { s = 0; ps = npos; } }
-        };
-        const int unit = __builtin_amdgcn_readfirstlane((int)d0[3]);
-        int cnt = MT;
-        uint32_t tk[MSUB];
-#pragma unroll
-        for (int ms = 0; ms < MSUB; ++ms) tk[ms] = ms * 16 + n;
-        bool skip = false;
-        if (ROUTED) {
-            const int cl = (unit * 16) / p.cluster_size;
-            const int64_t e = (int64_t)mt * p.n_clusters + cl;
-            cnt = __builtin_amdgcn_readfirstlane(p.tok_cnt[e]);
-            skip = cnt == 0;
-#pragma unroll
-            for (int ms = 0; ms < MSUB; ++ms) {
-                const int i = ms * 16 + n;
-                tk[ms] = i < cnt ? p.tok_list[e * MT + i] : 0;
-            }
-        }
-        const int nsub = ROUTED ? (cnt + 15) >> 4 : MSUB;
-        f32x4_t acc[NACC][MSUB];
-#pragma unroll
-        for (int a = 0; a < NACC; ++a)
-#pragma unroll
-            for (int ms = 0; ms < MSUB; ++ms) acc[a][ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (NACC == 2 && p.norm) mortar_stage_tile_norm<MT, WAVES>(p, lx, m0, p.Cb, tid, reinterpret_cast<float *>(next_unit + 4));      // gate_up may carry the norm
+        else mortar_stage_tile<MT, WAVES, false, XT>(p, lx, m0, 0, p.Cb, tid);
+        if (!again) mortar_resolve_scale<CODE>(p);
+        __syncthreads();
 
-        for (int sg = 0; sg < p.nseg; ++sg) {
-            const uint32_t xo_base = lane_xo + (uint32_t)(sg * p.seg_cb) * (uint32_t)(MT * 32);
-#pragma unroll
-            for (int a = 0; a < NACC; ++a) {
-                const bool last_part = sg + 1 == p.nseg && a + 1 == NACC;
-                if (last_part) npos = base + (int)__builtin_amdgcn_readfirstlane(drawn);
-                advance(p1, s1, a1);
-                const u32x4_t d1 = mortar_part_desc<NACC>(p, p1, s1, a1);
-                const int g0 = __builtin_amdgcn_readfirstlane((int)d0[0]), g1 = __builtin_amdgcn_readfirstlane((int)d0[1]);
-                const int nb = __builtin_amdgcn_readfirstlane((int)d0[2]);
-                if (!skip && g0 < g1) {
-                    MortarBatch b;
-                    mortar_load_batch<CODE>(p, b, g0, g1, n, bsel, hsel);
-                    mortar_row_part<MSUB, MT, ROUTED, CODE>(p, lx, b, g0, g1, nb, xo_base, tk, nsub, n, bsel, hsel, acc[a]);
+        while (pos < u_end) {
+            uint32_t drawn = 0;
+            if (lane == 0) drawn = atomicAdd(next_unit, 1u);
+            // coordinates of the part after the current one; its descriptor is fetched while the current part runs
+            int p1 = pos, s1 = 0, a1 = 0;
+            int npos = -1;       // position of this wave's next unit, known from the second part on
+            auto advance = [&](int &ps, int &s, int &a_) {
+                if (++a_ == NACC) { a_ = 0; if (++s == p.nseg) { s = 0; ps = npos; } }
+            };
+            const int unit = __builtin_amdgcn_readfirstlane((int)d0[3]);
+            int cnt = MT;
+            uint32_t tk[MSUB];
+    #pragma unroll
+            for (int ms = 0; ms < MSUB; ++ms) tk[ms] = ms * 16 + n;
+            bool skip = false;
+            if (ROUTED) {
+                const int cl = (unit * 16) / p.cluster_size;
+                const int64_t e = (int64_t)mt * p.n_clusters + cl;
+                cnt = __builtin_amdgcn_readfirstlane(p.tok_cnt[e]);
+                skip = cnt == 0;
+    #pragma unroll
+                for (int ms = 0; ms < MSUB; ++ms) {
+                    const int i = ms * 16 + n;
+                    tk[ms] = i < cnt ? p.tok_list[e * MT + i] : 0;
                 }
-                d0 = d1;
             }
-        }
-        pos = npos;
-        if (skip) continue;
+            const int nsub = ROUTED ? (cnt + 15) >> 4 : MSUB;
+            f32x4_t acc[NACC][MSUB];
+    #pragma unroll
+            for (int a = 0; a < NACC; ++a)
+    #pragma unroll
+                for (int ms = 0; ms < MSUB; ++ms) acc[a][ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-        mortar_store_tile<MSUB, NACC, CODE, (MT <= 16 && NACC == 1 && !TABLE), YT>(p, unit, m0, tk, ROUTED ? cnt : MT, n, g, has_gates,
-                                                                                   acc[0], acc[NACC - 1]);
+            for (int sg = 0; sg < p.nseg; ++sg) {
+                const uint32_t xo_base = lane_xo + (uint32_t)(sg * p.seg_cb) * (uint32_t)(MT * 32);
+    #pragma unroll
+                for (int a = 0; a < NACC; ++a) {
+                    const bool last_part = sg + 1 == p.nseg && a + 1 == NACC;
+                    if (last_part) npos = base + (int)__builtin_amdgcn_readfirstlane(drawn);
+                    advance(p1, s1, a1);
+                    const u32x4_t d1 = mortar_part_desc<NACC>(p, p1, s1, a1);
+                    const int g0 = __builtin_amdgcn_readfirstlane((int)d0[0]), g1 = __builtin_amdgcn_readfirstlane((int)d0[1]);
+                    const int nb = __builtin_amdgcn_readfirstlane((int)d0[2]);
+                    if (!skip && g0 < g1) {
+                        MortarBatch b;
+                        mortar_load_batch<CODE>(p, b, g0, g1, n, bsel, hsel);
+                        mortar_row_part<MSUB, MT, ROUTED, CODE>(p, lx, b, g0, g1, nb, xo_base, tk, nsub, n, bsel, hsel, acc[a]);
+                    }
+                    d0 = d1;
+                }
+            }
+            pos = npos;
+            if (skip) continue;
+
+            mortar_store_tile<MSUB, NACC, CODE, (MT <= 16 && NACC == 1 && !TABLE), YT>(p, unit, m0, tk, ROUTED ? cnt : MT, n, g, has_gates,
+                                                                                       acc[0], acc[NACC - 1]);
+        }        left -= u_end - base;
+        if (!RUNS || left <= 0) break;
+        ++mt;
+        base = 0;
     }
 }
 
@@ -692,119 +720,143 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
 // The descriptors of the next segment are fetched before the barrier pair, so their latency hides behind the
 // staging.
 // ---------------------------------------------------------------------------------------------------------
-template <int MT, int NACC, bool MASKED, int WAVES, int UPW, bool TABLE, int CODE, bool TL = false>
+// Whether the kernel below has a form that walks runs (RUNS, SpmmParams::span): where the loop around the sums does not spill.  (gate_up with three units per wave:
+// 40 registers, 162 -> 221 us; four units per wave staged through registers: 12 registers, 36 -> 43 us.)
+template <int MT, int NACC, bool MASKED, int UPW, bool TABLE, bool XT>
+constexpr bool mortar_seg_runs() { return MT >= 32 && !TABLE && NACC == 1 && !MASKED && (XT || UPW <= 3); }
+
+template <int MT, int NACC, bool MASKED, int WAVES, int UPW, bool TABLE, int CODE, bool TL = false, bool RUNS = false>
 __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const SpmmParams p0, const SpmmParams *table) {
     constexpr int MSUB = (MT + 15) / 16, NP = UPW * NACC;
     constexpr bool XT = TL && NACC == 1, YT = TL && NACC == 2;
     SpmmView p = mortar_view(TABLE ? mortar_table_entry(table, blockIdx.y) : p0);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint4 *lx = reinterpret_cast<uint4 *>(smem);
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n = lane & 15, g = lane >> 4, bsel = g >> 1, hsel = g & 1;
+    const int tid0 = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
     // Workgroups are dealt round-robin over the 8 XCDs (each with its own L2): renumber them so that the
     // n_split workgroups that stage the same token tile run on one XCD and share its copy of the tile.
     const int wg = p.xcd_map ? (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
-    if (wg >= p.n_mtiles * p.n_split) return;
-    const int mt = wg / p.n_split, sp = wg % p.n_split;
-    const int m0 = mt * MT;
-    const uint32_t lane_xo = (uint32_t)(hsel * 16 + n * 32);
     const bool has_gates = p.gates != nullptr;
 
-    // this wave's units: schedule positions sp*per + wave + WAVES*k
-    constexpr int per = WAVES * UPW;
-    const int pos0 = sp * per + wave;
-    f32x4_t acc[UPW][NACC][MSUB];
-    uint32_t tk[MSUB];
+    // The workgroup's units in rows of one per wave (schedule positions WAVES * slot + wave): UPW rows of one tile or, with a span, a
+    // run over the rows of all tiles, in groups of up to UPW rows of one tile.
+    int mt, slot0, left = UPW, tile_slots = 1 << 30;
+    if (RUNS) {
+        tile_slots = (p.n_units + WAVES - 1) / WAVES;
+        const int first = wg * p.span, all = p.n_mtiles * tile_slots;
+        if (first >= all) return;
+        mt = first / tile_slots;
+        slot0 = first - mt * tile_slots;
+        left = all - first < p.span ? all - first : p.span;
+    } else {
+        if (wg >= p.n_mtiles * p.n_split) return;
+        mt = wg / p.n_split;
+        slot0 = wg % p.n_split * UPW;
+    }
+    for (bool again = false;; again = true) {
+        const int m0 = mt * MT, pos0 = slot0 * WAVES + wave;
+        const int tid = RUNS ? mortar_opaque_tid(tid0) : tid0, lane = tid & 63, n = lane & 15, g = lane >> 4, bsel = g >> 1, hsel = g & 1;
+        const uint32_t lane_xo = (uint32_t)(hsel * 16 + n * 32);
+        int slots = left < UPW ? left : UPW;
+        if (RUNS && tile_slots - slot0 < slots) slots = tile_slots - slot0;
+        f32x4_t acc[UPW][NACC][MSUB];
+        uint32_t tk[MSUB];
 #pragma unroll
-    for (int ms = 0; ms < MSUB; ++ms) tk[ms] = ms * 16;
+        for (int ms = 0; ms < MSUB; ++ms) tk[ms] = ms * 16;
 #pragma unroll
-    for (int k = 0; k < UPW; ++k)
+        for (int k = 0; k < UPW; ++k)
 #pragma unroll
-        for (int a = 0; a < NACC; ++a)
+            for (int a = 0; a < NACC; ++a)
 #pragma unroll
-            for (int ms = 0; ms < MSUB; ++ms) acc[k][a][ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                for (int ms = 0; ms < MSUB; ++ms) acc[k][a][ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    u32x4_t dn[NP];     // descriptors of the coming segment, part q = k * NACC + a
+        u32x4_t dn[NP];     // descriptors of the coming segment, part q = k * NACC + a
 #pragma unroll
-    for (int q = 0; q < NP; ++q) dn[q] = mortar_part_desc<NACC>(p, pos0 + WAVES * (q / NACC), 0, q % NACC);
-    int units[UPW];
-    mortar_resolve_scale<CODE>(p);
+        for (int q = 0; q < NP; ++q) dn[q] = mortar_part_desc<NACC>(p, pos0 + WAVES * (q / NACC), 0, q % NACC);
+        int units[UPW];
+        if (!again) mortar_resolve_scale<CODE>(p);
 
-    for (int sg = 0; sg < p.nseg; ++sg) {
-        const int c0 = sg * p.seg_cb;
-        const int ncb = p.Cb - c0 < p.seg_cb ? p.Cb - c0 : p.seg_cb;
-        int g0[NP], g1[NP], nb[NP];
-#pragma unroll
-        for (int q = 0; q < NP; ++q) {
-            const bool on = pos0 + WAVES * (q / NACC) < p.n_units;
-            g0[q] = on ? __builtin_amdgcn_readfirstlane((int)dn[q][0]) : 0;
-            g1[q] = on ? __builtin_amdgcn_readfirstlane((int)dn[q][1]) : 0;
-            nb[q] = __builtin_amdgcn_readfirstlane((int)dn[q][2]);
-            if (q % NACC == 0) units[q / NACC] = on ? __builtin_amdgcn_readfirstlane((int)dn[q][3]) : -1;
-        }
-        if (sg + 1 < p.nseg) {
-#pragma unroll
-            for (int q = 0; q < NP; ++q) dn[q] = mortar_part_desc<NACC>(p, pos0 + WAVES * (q / NACC), sg + 1, q % NACC);
-        }
-        // The first batch of every part is requested one part ahead (the first part's before the tile is staged), always
-        // and in a fixed order (an empty part reads octet 0), and a part's first batch is multiplied without a load in
-        // between: the wait for it then counts the loads issued since and never includes the newest ones.
-        // (Prefill tiles only: the decode tiles of this kernel run many waves per SIMD on few registers.)
-        constexpr int FIRST = 8 * RES_GROUPS;                      // blocks of a part's first batch
-        constexpr bool BATCH_AHEAD = MT >= 32;
-        auto first_batch = [&](MortarBatch &bb, int q) {
-            const bool any = g0[q] < g1[q];
-            mortar_load_batch<CODE>(p, bb, any ? g0[q] : 0, any ? g1[q] : 1, n, bsel, hsel);
-        };
-        MortarBatch bq;
-        if (BATCH_AHEAD) first_batch(bq, 0);
-        if (sg > 0) __syncthreads();
-        mortar_stage_tile<MT, WAVES, MASKED, XT>(p, lx, m0, c0, ncb, tid);
-        __syncthreads();
-        if (!BATCH_AHEAD) {
+        for (int sg = 0; sg < p.nseg; ++sg) {
+            const int c0 = sg * p.seg_cb;
+            const int ncb = p.Cb - c0 < p.seg_cb ? p.Cb - c0 : p.seg_cb;
+            int g0[NP], g1[NP], nb[NP];
 #pragma unroll
             for (int q = 0; q < NP; ++q) {
-                if (g0[q] < g1[q]) {
-                    MortarBatch b;
-                    mortar_load_batch<CODE>(p, b, g0[q], g1[q], n, bsel, hsel);
-                    mortar_row_part<MSUB, MT, false, CODE>(p, lx, b, g0[q], g1[q], nb[q], lane_xo, tk, MSUB, n, bsel, hsel,
-                                                           acc[q / NACC][q % NACC]);
+                const bool on = (!RUNS || q / NACC < slots) && pos0 + WAVES * (q / NACC) < p.n_units;
+                g0[q] = on ? __builtin_amdgcn_readfirstlane((int)dn[q][0]) : 0;
+                g1[q] = on ? __builtin_amdgcn_readfirstlane((int)dn[q][1]) : 0;
+                nb[q] = __builtin_amdgcn_readfirstlane((int)dn[q][2]);
+                if (q % NACC == 0) units[q / NACC] = on ? __builtin_amdgcn_readfirstlane((int)dn[q][3]) : -1;
+            }
+            if (sg + 1 < p.nseg) {
+#pragma unroll
+                for (int q = 0; q < NP; ++q) dn[q] = mortar_part_desc<NACC>(p, pos0 + WAVES * (q / NACC), sg + 1, q % NACC);
+            }
+            // The first batch of every part is requested one part ahead (the first part's before the tile is staged), always
+            // and in a fixed order (an empty part reads octet 0), and a part's first batch is multiplied without a load in
+            // between: the wait for it then counts the loads issued since and never includes the newest ones.
+            // (Prefill tiles only: the decode tiles of this kernel run many waves per SIMD on few registers.)
+            constexpr int FIRST = 8 * RES_GROUPS;                      // blocks of a part's first batch
+            constexpr bool BATCH_AHEAD = MT >= 32;
+            auto first_batch = [&](MortarBatch &bb, int q) {
+                const bool any = g0[q] < g1[q];
+                mortar_load_batch<CODE>(p, bb, any ? g0[q] : 0, any ? g1[q] : 1, n, bsel, hsel);
+            };
+            MortarBatch bq;
+            if (BATCH_AHEAD) first_batch(bq, 0);
+            if (sg > 0 || (RUNS && again)) __syncthreads();
+            mortar_stage_tile<MT, WAVES, MASKED, XT>(p, lx, m0, c0, ncb, tid);
+            __syncthreads();
+            if (!BATCH_AHEAD) {
+#pragma unroll
+                for (int q = 0; q < NP; ++q) {
+                    if (g0[q] < g1[q]) {
+                        MortarBatch b;
+                        mortar_load_batch<CODE>(p, b, g0[q], g1[q], n, bsel, hsel);
+                        mortar_row_part<MSUB, MT, false, CODE>(p, lx, b, g0[q], g1[q], nb[q], lane_xo, tk, MSUB, n, bsel, hsel,
+                                                               acc[q / NACC][q % NACC]);
+                    }
                 }
+                continue;
             }
-            continue;
-        }
 #pragma unroll
-        for (int q = 0; q < NP; ++q) {
-            // A wave lowers its priority with every part of the segment it has finished: the arbiter serves the oldest wave of
-            // a SIMD first, so without this the four waves finish a segment one after another (4.8 / 6.3 / 8.0 / 9.4 us measured)
-            // and the SIMD runs the end of it on one or two waves.  Tile-ordered form only: with the register-staged forms the
-            // same priorities cost time (the staging of the next segment then starts from uneven waves).
-            if constexpr (XT) mortar_setprio(NP - 1 - q);
-            MortarBatch bn;
-            if (q + 1 < NP) first_batch(bn, q + 1);
-            const int nbq = g0[q] < g1[q] ? nb[q] : 0;
-            mortar_row_part<MSUB, MT, false, CODE, true>(p, lx, bq, g0[q], g1[q], nbq < FIRST ? nbq : FIRST, lane_xo, tk, MSUB,
-                                                         n, bsel, hsel, acc[q / NACC][q % NACC]);
-            if (nbq > FIRST) {                                      // the rest of a long part
-                MortarBatch bt;
-                mortar_load_batch<CODE>(p, bt, g0[q] + RES_GROUPS, g1[q], n, bsel, hsel);
-                mortar_row_part<MSUB, MT, false, CODE>(p, lx, bt, g0[q] + RES_GROUPS, g1[q], nbq - FIRST, lane_xo, tk, MSUB,
-                                                       n, bsel, hsel, acc[q / NACC][q % NACC]);
+            for (int q = 0; q < NP; ++q) {
+                // A wave lowers its priority with every part of the segment it has finished: the arbiter serves the oldest wave of
+                // a SIMD first, so without this the four waves finish a segment one after another (4.8 / 6.3 / 8.0 / 9.4 us measured)
+                // and the SIMD runs the end of it on one or two waves.  Tile-ordered form only: with the register-staged forms the
+                // same priorities cost time (the staging of the next segment then starts from uneven waves).
+                if constexpr (XT) mortar_setprio(NP - 1 - q);
+                MortarBatch bn;
+                if (q + 1 < NP) first_batch(bn, q + 1);
+                const int nbq = g0[q] < g1[q] ? nb[q] : 0;
+                mortar_row_part<MSUB, MT, false, CODE, true>(p, lx, bq, g0[q], g1[q], nbq < FIRST ? nbq : FIRST, lane_xo, tk, MSUB,
+                                                             n, bsel, hsel, acc[q / NACC][q % NACC]);
+                if (nbq > FIRST) {                                      // the rest of a long part
+                    MortarBatch bt;
+                    mortar_load_batch<CODE>(p, bt, g0[q] + RES_GROUPS, g1[q], n, bsel, hsel);
+                    mortar_row_part<MSUB, MT, false, CODE>(p, lx, bt, g0[q] + RES_GROUPS, g1[q], nbq - FIRST, lane_xo, tk, MSUB,
+                                                           n, bsel, hsel, acc[q / NACC][q % NACC]);
+                }
+                if (q + 1 < NP) bq = bn;
             }
-            if (q + 1 < NP) bq = bn;
+            if constexpr (XT) mortar_setprio(0);
         }
-        if constexpr (XT) mortar_setprio(0);
-    }
 
-    uint32_t tl[MSUB];
+        uint32_t tl[MSUB];
 #pragma unroll
-    for (int ms = 0; ms < MSUB; ++ms) tl[ms] = ms * 16 + n;
+        for (int ms = 0; ms < MSUB; ++ms) tl[ms] = ms * 16 + n;
 #pragma unroll
-    for (int k = 0; k < UPW; ++k) {
-        if (units[k] < 0) continue;
-        mortar_store_tile<MSUB, NACC, CODE, (MT <= 16 && NACC == 1 && !TABLE), YT>(p, units[k], m0, tl, MT, n, g, has_gates, acc[k][0],
-                                                                                   acc[k][NACC - 1]);
+        for (int k = 0; k < UPW; ++k) {
+            if (units[k] < 0) continue;
+            mortar_store_tile<MSUB, NACC, CODE, (MT <= 16 && NACC == 1 && !TABLE), YT>(p, units[k], m0, tl, MT, n, g, has_gates, acc[k][0],
+                                                                                       acc[k][NACC - 1]);
+        }
+        if (!RUNS) break;
+        left -= slots;
+        slot0 += slots;
+        if (left <= 0) break;
+        if (slot0 == tile_slots) { slot0 = 0; ++mt; }
     }
 }
 
@@ -992,9 +1044,16 @@ inline int64_t mortar_grid_width(SpmmParams &p, int layers) {
     return p.xcd_map ? (n + 7) / 8 * 8 : n;
 }
 
+// One round of workgroups of `span` consecutive units (or rows of units) out of `all`, neighbours on one XCD.
+inline int64_t mortar_span_grid(SpmmParams &p, int64_t all, int span) {
+    p.span = span;
+    p.xcd_map = 1;
+    return ((all + span - 1) / span + 7) / 8 * 8;
+}
+
 // Fills the launch-shape fields of `p` for the resident kernel and returns the grid width.
 template <int MT, int WAVES>
-inline int64_t mortar_resident_shape(SpmmParams &p, int layers) {
+inline int64_t mortar_resident_shape(SpmmParams &p, int layers, bool runs = false) {
     p.n_mtiles = (p.M + MT - 1) / MT;
     // Prefill tiles: one workgroup per CU (every workgroup stages a whole tile and the last units of its window
     // leave waves idle, so few large ones: one round measured faster than two).  Decode tiles stage little: many
@@ -1020,6 +1079,18 @@ inline int64_t mortar_resident_shape(SpmmParams &p, int layers) {
     const int max_split = (p.n_units + WAVES * upw - 1) / (WAVES * upw);
     split = split < 1 ? 1 : (split > max_split ? max_split : split);
     p.n_split = split;
+    p.span = 0;
+    // Or runs of equal length over the units of all tiles, for 256 workgroups: row counts that leave whole tiles per workgroup with a
+    // nearly empty round.  A workgroup costs its units and about twelve more, every further tile of a run (staged and multiplied by
+    // itself) eighteen.  gate_up of d_model 2048: 4500 rows (141 workgroups of a whole tile each) 101 -> 72 us, 5000 101 -> 77, 6000
+    // 102 -> 91, 9000 (282 tiles, two rounds) 211 -> 146, 3000 (188 half tiles) 55 -> 50; 2500 rows, where the rule keeps 237 workgroups
+    // of a third of a tile, 41.5 against 44; d_model 768, 9000 rows 35 -> 27.5, 5000 17.5 against 19.3.
+    if (runs && layers == 1) {
+        const int64_t all = (int64_t)p.n_mtiles * p.n_units, span = (all + 255) / 256;
+        const int64_t rounds = ((int64_t)p.n_mtiles * split + 255) / 256, per = (p.n_units + split - 1) / split;
+        const int64_t cost = span + 12 + 18 * ((span + p.n_units - 2) / p.n_units);
+        if (all < 0x7fffffff && cost * 21 < rounds * (per + 12) * 20) return mortar_span_grid(p, all, (int)span);
+    }
     return mortar_grid_width(p, layers);
 }
 
@@ -1030,11 +1101,22 @@ int mortar_launch_resident(SpmmParams &p, const SpmmParams *table, int layers, h
     if (smem > LDS_BUDGET + LDS_PAD * 16 + LDS_EXTRA) return mortar_fail(MORTAR_ERR_LIMIT, "resident tile of %d bytes does not fit LDS", smem);
     static bool attr_done = false;
     if (TL != ((NACC == 1 ? p.x_tiled : p.y_tiled) != 0)) return mortar_fail(MORTAR_ERR_ARG, "spmm launch: activation layout mismatch");
-    auto kern = mortar_resident_kernel<MT, NACC, ROUTED, WAVES, TABLE, CODE, TL>;
-    int rc = mortar_allow_big_lds(kern, attr_done);
-    if (rc) return rc;
-    const int64_t grid = mortar_resident_shape<MT, WAVES>(p, layers);
+    constexpr bool RUNS = MT >= 32 && !TABLE && !ROUTED;
+    int rc;
+    const int64_t grid = mortar_resident_shape<MT, WAVES>(p, layers, RUNS);
     if ((rc = mortar_launch_check(grid, layers))) return rc;
+    if constexpr (RUNS) {
+        if (p.span > 0) {
+            static bool runs_done = false;
+            auto runs = mortar_resident_kernel<MT, NACC, ROUTED, WAVES, TABLE, CODE, TL, true>;
+            if ((rc = mortar_allow_big_lds(runs, runs_done))) return rc;
+            hipLaunchKernelGGL(runs, dim3((unsigned)grid), dim3(WAVES * 64), smem, st, p, table);
+            const hipError_t e = hipGetLastError();
+            return e == hipSuccess ? MORTAR_OK : mortar_fail(MORTAR_ERR_HIP, "spmm launch: %s", hipGetErrorString(e));
+        }
+    }
+    auto kern = mortar_resident_kernel<MT, NACC, ROUTED, WAVES, TABLE, CODE, TL>;
+    if ((rc = mortar_allow_big_lds(kern, attr_done))) return rc;
     hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)layers), dim3(WAVES * 64), smem, st, p, table);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "spmm launch: %s", hipGetErrorString(e));
@@ -1045,6 +1127,7 @@ template <int MT, int WAVES, int UPW>
 inline int64_t mortar_segmented_shape(SpmmParams &p, int layers) {
     p.n_mtiles = (p.M + MT - 1) / MT;
     p.n_split = (p.n_units + WAVES * UPW - 1) / (WAVES * UPW);
+    if (p.span > 0) return mortar_span_grid(p, (int64_t)p.n_mtiles * ((p.n_units + WAVES - 1) / WAVES), p.span);
     return mortar_grid_width(p, layers);
 }
 
@@ -1055,12 +1138,23 @@ int mortar_launch_segmented(SpmmParams &p, const SpmmParams *table, int layers, 
     if (smem > LDS_BUDGET + LDS_PAD * 16) return mortar_fail(MORTAR_ERR_LIMIT, "segment tile of %d bytes does not fit LDS", smem);
     static bool attr_done = false;
     if (TL != ((NACC == 1 ? p.x_tiled : p.y_tiled) != 0)) return mortar_fail(MORTAR_ERR_ARG, "spmm launch: activation layout mismatch");
-    auto kern = mortar_segmented_kernel<MT, NACC, MASKED, WAVES, UPW, TABLE, CODE, TL>;
-    int rc = mortar_allow_big_lds(kern, attr_done);
-    if (rc) return rc;
+    int rc;
     const int64_t grid = mortar_segmented_shape<MT, WAVES, UPW>(p, layers);
     if ((rc = mortar_launch_check(grid, layers))) return rc;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)layers), dim3(WAVES * 64), smem, st, p, table);
+    if (p.span > 0) {
+        if constexpr (mortar_seg_runs<MT, NACC, MASKED, UPW, TABLE, TL && NACC == 1>()) {
+            static bool runs_done = false;
+            auto runs = mortar_segmented_kernel<MT, NACC, MASKED, WAVES, UPW, TABLE, CODE, TL, true>;
+            if ((rc = mortar_allow_big_lds(runs, runs_done))) return rc;
+            hipLaunchKernelGGL(runs, dim3((unsigned)grid), dim3(WAVES * 64), smem, st, p, table);
+        } else {
+            return mortar_fail(MORTAR_ERR_ARG, "spmm launch: this form walks no runs");
+        }
+    } else {
+        auto kern = mortar_segmented_kernel<MT, NACC, MASKED, WAVES, UPW, TABLE, CODE, TL>;
+        if ((rc = mortar_allow_big_lds(kern, attr_done))) return rc;
+        hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)layers), dim3(WAVES * 64), smem, st, p, table);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "spmm launch: %s", hipGetErrorString(e));
     return MORTAR_OK;
