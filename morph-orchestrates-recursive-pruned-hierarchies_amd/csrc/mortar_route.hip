@@ -912,16 +912,35 @@ __global__ void __launch_bounds__(256) route_flags_kernel(const float *gates, in
 
 // One wavefront per row, in 16-byte units, with the summation order and rounding steps of the fused form in
 // the gate_up staging (rms_* in mortar_device.h): both give the same bits.
+// A call of few rows is a chain of latencies.  CU > 0: rows of at most 64 CU units stay in registers, everything requested at once; the loops
+// below are a round trip per 64 units, twice.  us (graph replay), the loops -> this: 16 rows of 2048 / 4096 / 8192 values 3.6 -> 2.7, 5.2 -> 3.4, 8.9 ->
+// 5.0; 16384 rows, which run at the rate of memory, 28 -> 21, 58 -> 41, 145 -> 100 (4096 rows of 2048 values: 6.5 -> 6.7).
+template <int CU>
 __global__ void __launch_bounds__(256) rmsnorm_rows_kernel(const uint16_t *x, int64_t M, int d, int64_t ldx,
                                                             const uint16_t *w, float eps, uint16_t *y, int64_t ldy) {
     const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (row >= M) return;
     const u32x4_t *xp = reinterpret_cast<const u32x4_t *>(x + row * ldx);
     const u32x4_t *wp = reinterpret_cast<const u32x4_t *>(w);
     u32x4_t *yp = reinterpret_cast<u32x4_t *>(y + row * ldy);
     const int nch = d / 8;
     float ss = 0.f;
+    if constexpr (CU > 0) {
+        u32x4_t u[CU], w8[CU];
+#pragma unroll
+        for (int j = 0; j < CU; ++j) u[j] = xp[lane + 64 * j < nch ? lane + 64 * j : nch - 1];
+#pragma unroll
+        for (int j = 0; j < CU; ++j) w8[j] = w ? wp[lane + 64 * j < nch ? lane + 64 * j : nch - 1] : u32x4_t{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < CU; ++j)
+            if (lane + 64 * j < nch) ss = rms_sumsq8(u[j], ss);
+        const float r = rms_scale(rms_wave_sum(ss), d, eps);
+#pragma unroll
+        for (int j = 0; j < CU; ++j)
+            if (lane + 64 * j < nch) yp[lane + 64 * j] = rms_apply8(u[j], r, w8[j], w != nullptr);
+        return;
+    }
     for (int ch = lane; ch < nch; ch += 64) ss = rms_sumsq8(xp[ch], ss);
     const float r = rms_scale(rms_wave_sum(ss), d, eps);
     for (int ch = lane; ch < nch; ch += 64)
@@ -1161,8 +1180,14 @@ extern "C" int mortar_rmsnorm_bf16(const uint16_t *x, int64_t M, int32_t d, int6
     const bool units = d % 8 == 0 && ldx % 8 == 0 && ldy % 8 == 0 &&
                        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
     if (units)
-        hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)((M + 3) / 4)), dim3(256), 0, static_cast<hipStream_t>(stream),
+    {
+        // few rows: a workgroup each
+        const int rpw = M <= 1024 ? 1 : 4;
+        const auto kern = d <= 1024 ? rmsnorm_rows_kernel<2> : d <= 2048 ? rmsnorm_rows_kernel<4> : d <= 4096 ? rmsnorm_rows_kernel<8>
+                        : d <= 8192 ? rmsnorm_rows_kernel<16> : rmsnorm_rows_kernel<0>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)((M + rpw - 1) / rpw)), dim3(64 * rpw), 0, static_cast<hipStream_t>(stream),
                            x, M, d, ldx, w, eps, y, ldy);
+    }
     else
         hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)M), dim3(256), 0, static_cast<hipStream_t>(stream), x, M, d,
                            ldx, w, eps, y, ldy);
