@@ -448,6 +448,10 @@ int mortar_norm_gateup_swiglu_bf16(const mortar_bcsr_t *W, const int32_t *sched,
                                    const float *gates, int32_t n_clusters, const int32_t *tok_cnt,
                                    const uint8_t *tok_list, void *stream);
 int mortar_norm_fusable(int32_t Cb);
+/* The same product (no gates) for up to 64 rows of matrices that mortar_norm_fusable refuses: same arguments and bits.  Returns
+ * MORTAR_NO_KERNEL (nothing launched) where the call has no such kernel: call mortar_rmsnorm_bf16 first. */
+int mortar_norm_gateup_decode_bf16(const mortar_bcsr_t *W, const int32_t *sched, const uint16_t *x, int64_t M, int64_t ldx,
+                                   const uint16_t *norm_w, float norm_eps, uint16_t *h, int64_t ldh, void *stream);
 
 /* The carved SwiGLU MLP as one call: y = down(silu(gate) * up [* gates per cluster]) with gate_up applied to x or to
  * RMSNorm(x) -- _SwiGLUMortar.forward, morph/model/transformer.py:402-431 (called as mlp(norm_mlp(x)),

@@ -328,6 +328,19 @@ extern "C" int mortar_norm_gateup_swiglu_bf16(const mortar_bcsr_t *W, const int3
     return gateup_common(W, sched, x, M, ldx, true, norm_w, norm_eps, h, ldh, gates, n_clusters, tok_cnt, tok_list, stream);
 }
 
+extern "C" int mortar_norm_gateup_decode_bf16(const mortar_bcsr_t *W, const int32_t *sched, const uint16_t *x, int64_t M, int64_t ldx,
+                                              const uint16_t *norm_w, float norm_eps, uint16_t *h, int64_t ldh, void *stream) {
+    if (!W || M <= 0 || M > MORTAR_SMALLM_MAX || !(norm_eps >= 0.f) || (reinterpret_cast<uintptr_t>(norm_w) & 15)) return MORTAR_NO_KERNEL;
+    if (W->Rb & 1) return mortar_fail(MORTAR_ERR_ARG, "gateup: odd number of block-rows");
+    const int rc = check_common(W, x, M, ldx, h, ldh, (int64_t)W->Rb * 8);
+    if (rc) return rc;
+    SpmmParams p;
+    fill(p, W, sched, x, M, ldx, h, ldh, static_cast<hipStream_t>(stream));
+    p.n_units = W->Rb / 2;
+    p.norm = NORM_WIDE; p.norm_eps = norm_eps; p.norm_w = norm_w;
+    return mortar_smallm_norm_wide(p, static_cast<hipStream_t>(stream));
+}
+
 extern "C" int mortar_norm_fusable(int32_t Cb) { return Cb > 0 && Cb <= NORM_MAX_CB && resident_mt(Cb) != 0; }
 
 namespace {

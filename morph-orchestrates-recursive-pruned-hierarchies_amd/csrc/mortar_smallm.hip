@@ -83,15 +83,27 @@ static bool partsplit_fits(int mt, int nacc, const SpmmParams &p) {
     return pw != 0 && tile_bytes(mt, p.Cb) + pw * 4 * nacc * ((mt + 15) / 16) * 1024 <= 160 * 1024;
 }
 
+template <int MT>
+static bool partsplit_eight(int kind, const SpmmParams &p) {
+    const int nacc = (kind == 0 || kind == 3) ? 1 : 2;
+    return kind != 2 && p.nseg * nacc >= 2 && (p.M + MT - 1) / MT * (int64_t)((p.n_units + 3) / 4) > 256 &&
+           tile_bytes(MT, p.Cb) + 16 * nacc * ((MT + 15) / 16) * 1024 <= 160 * 1024;
+}
+
 // Part-split launch for one matrix.
 template <int MT, int CODE>
 static int launch_partsplit(int kind, SpmmParams &p, hipStream_t st) {
     const int nacc = (kind == 0 || kind == 3) ? 1 : 2, nparts = p.nseg * nacc, pw = partsplit_waves(nparts);
     if (!partsplit_fits(MT, nacc, p)) return -1;
+    if constexpr (MT == 4 || MT == 8) {
+        if (p.norm == NORM_WIDE) {       // kind 1, two K segments: the forms below with the norm in them
+            if (partsplit_eight<MT>(kind, p)) return mortar_launch_partsplit<MT, 2, false, false, 2, 8, CODE, 0, false, NORM_WIDE_MAX_CB>(p, st);
+            return mortar_launch_partsplit<MT, 2, false, false, 4, 4, CODE, 0, false, NORM_WIDE_MAX_CB>(p, st);
+        }
+    }
     // more tiles x 4-unit workgroups than one round holds (one workgroup fills a CU): 8 units per workgroup, two waves
     // each (gate_up of d_model 2048 at 33..64 rows: 8.3 -> 6.1 us)
-    if (kind != 2 && nparts >= 2 && (p.M + MT - 1) / MT * (int64_t)((p.n_units + 3) / 4) > 256 &&
-        tile_bytes(MT, p.Cb) + 16 * nacc * ((MT + 15) / 16) * 1024 <= 160 * 1024) {
+    if (partsplit_eight<MT>(kind, p)) {
         switch (kind) {
             case 0: return mortar_launch_partsplit<MT, 1, false, false, 2, 8, CODE>(p, st);
             case 1: return mortar_launch_partsplit<MT, 2, false, false, 2, 8, CODE>(p, st);
@@ -249,7 +261,7 @@ static int smallm_launch_code(int kind, SpmmParams &p, const SpmmParams *table, 
             // otherwise (d_model 2048 without the norm, 17..32 rows: 4.7 against 5.6..5.8; 3072 6.4 against 7.2), and in a second
             // round never (d_model 2048, 48 rows: 8.3 against 12.0).
             const int64_t w8 = (p.M + 7) / 8 * (int64_t)((p.n_units + 3) / 4);
-            const bool eight = kind == 1 && t == 16 && w8 <= (p.norm || !partsplit_fits(16, 2, p) ? 512 : 256);
+            const bool eight = kind == 1 && t == 16 && w8 <= (p.norm == 1 || !partsplit_fits(16, 2, p) ? 512 : 256);
             rc = t == 4 ? launch_partsplit<4, CODE>(kind, p, st) : eight ? launch_partsplit<8, CODE>(kind, p, st) : -1;
             if (rc < 0 && t != 4) rc = launch_partsplit<16, CODE>(kind, p, st);
             if (rc < 0 && t == 16 && kind == 1) rc = wide_gate_up();
@@ -283,6 +295,25 @@ int mortar_smallm_launch(int kind, SpmmParams &p, const SpmmParams *table, int l
                            : smallm_launch_code<CODE_2BIT>(kind, p, table, layers, st);
 }
 
+template <int CODE>
+static int smallm_norm_wide(SpmmParams &p, hipStream_t st) {
+    int rc = -1;
+    if (p.M <= 4 && fits(4, p.Cb)) rc = mortar_chunk_launch(1, 4, p, st);
+    else if (p.M > 4 && fits(8, p.Cb)) rc = mortar_chunk_launch(1, 8, p, st);
+    if (rc >= 0) return rc;
+    if (mortar_smallm_tile(p.Cb, p.seg_cb, p.M, 1) == 4) return launch_partsplit<4, CODE>(1, p, st);
+    const int64_t w8 = (p.M + 7) / 8 * (int64_t)((p.n_units + 3) / 4);
+    return w8 <= (partsplit_fits(16, 2, p) ? 256 : 512) ? launch_partsplit<8, CODE>(1, p, st) : -1;
+}
+
+// The norm in front of a wide gate_up, up to 64 rows.  A launch of its own for it is a chain of round trips as long as half of gate_up; inside, the
+// rows and the pieces of the tile arrive while the first descriptors and weights do.  MLP with its norm, us (graph replay), own launch -> inside: d_model
+// 3072 at 1 / 8 / 16 rows 12.9 -> 10.3, 14.2 -> 11.8, 16.9 -> 14.3, d_model 4096 18.6 -> 15.5, 20.0 -> 16.9, 22.9 -> 19.3.
+int mortar_smallm_norm_wide(SpmmParams &p, hipStream_t st) {
+    if (p.nseg != 2 || p.Cb > NORM_WIDE_MAX_CB || p.M > MORTAR_SMALLM_MAX || p.gates || pick_waves(16, p, 1) != 2) return MORTAR_NO_KERNEL;
+    const int rc = p.uscale != 0.f ? smallm_norm_wide<CODE_UNIFORM>(p, st) : smallm_norm_wide<CODE_2BIT>(p, st);
+    return rc == -1 ? MORTAR_NO_KERNEL : rc;
+}
 
 int mortar_smallm_shape(int kind, SpmmParams &p, int layers) {
     switch (stack_tile32(kind, p)) {       // table launches only: the choice of smallm_launch_code

@@ -37,8 +37,18 @@ int launch(int pw, int cs, int uw, SpmmParams &p, hipStream_t st) {
     return -1;
 }
 
+// gate_up over two K segments with the norm of wide rows in it
+template <int MT, int CODE>
+int launch_norm_wide(int cs, int uw, SpmmParams &p, hipStream_t st) {
+    if (cs != 2 || p.nseg != 2) return -1;
+    if (uw == 1) return mortar_launch_partsplit<MT, 2, false, false, 8, 1, CODE, 2, false, NORM_WIDE_MAX_CB>(p, st);
+    if (uw == 2) return mortar_launch_partsplit<MT, 2, false, false, 8, 2, CODE, 2, false, NORM_WIDE_MAX_CB>(p, st);
+    return -1;
+}
+
 template <int MT, int CODE>
 int launch_kind(int kind, int cs, int uw, SpmmParams &p, hipStream_t st) {
+    if (p.norm == NORM_WIDE) return launch_norm_wide<MT, CODE>(cs, uw, p, st);
     return kind == 0 ? launch<MT, 1, CODE>(p.nseg * cs, cs, uw, p, st) : launch<MT, 2, CODE>(2 * p.nseg * cs, cs, uw, p, st);
 }
 

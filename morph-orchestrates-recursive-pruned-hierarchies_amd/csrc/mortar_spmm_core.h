@@ -34,7 +34,7 @@ struct SpmmParams {
     int n_mtiles, n_split;    // token tiles; workgroups that share one token tile
     int seg_cb, nseg;         // K segments of the octet stream
     int xcd_map;              // 1: workgroup ids are renumbered per XCD (grid padded to a multiple of 8)
-    int norm;                 // 1: rows of x are RMS-normalised while they are staged (single-segment tiles only)
+    int norm;                 // 1: rows of x are RMS-normalised while they are staged (single-segment tiles only), NORM_WIDE: by the kernels for wide rows
     float norm_eps;
     float uscale;             // CODE_UNIFORM kernels: what the sums are multiplied by (mortar_set_scale; any value but 0 with scale_dev)
     float *y32;               // plain products: unrounded fp32 output [M, ldy] in place of the bf16 store, or null
@@ -159,6 +159,9 @@ constexpr int LDS_PAD = 32;              // 16-byte units past the tile that idl
 constexpr int tile_bytes(int mt, int ncb) { return ncb * mt * 32 + LDS_PAD * 16; }
 constexpr int LDS_EXTRA = 16 + 256;      // bytes after the tile: the resident kernel's unit counter, per-row norm factors
 constexpr int NORM_MAX_CB = 128;         // block-columns up to which a row fits the registers of the staging wave
+// SpmmParams::norm of decode launches whose rows are wider: 4- or 8-token tiles of up to NORM_WIDE_MAX_CB block-columns in two K segments,
+// in instantiations of their own (mortar_partsplit_kernel, NCB), since the registers of a staging wave grow with the row.
+constexpr int NORM_WIDE = 2, NORM_WIDE_MAX_CB = 256;
 
 // Lane k of every 16-lane row broadcast to the whole row (DPP row_newbcast); K must fold to a constant.
 template <int K>
@@ -391,11 +394,11 @@ __device__ __forceinline__ void mortar_stage_tile_norm(const SpmmView &p, uint4 
 // The same staging for the decode tiles of one launch, in two halves: begin() requests everything at the start of the kernel - whole
 // rows for the sums, and the tile's pieces in staging order - and finish() forms the row factors, scales the pieces and stores them.
 // Read one after the other, descriptor, row and piece were three round trips (0.2 us of gate_up at 1 and at 13 rows, d_model 2048); the
-// registers are there, the kernel holds one weight batch otherwise.  Same order of additions, same bits.
-template <int MT, int WAVES>
+// registers are there, the kernel holds one weight batch otherwise.  Same order of additions, same bits.  NCB: block-columns at most.
+template <int MT, int WAVES, int NCB>
 struct NormStage {
     static constexpr int RPI = MT >= 16 ? 16 : 4, LPR = 64 / RPI, RG = (MT + RPI - 1) / RPI;
-    static constexpr int RW = (MT + WAVES - 1) / WAVES, CU = NORM_MAX_CB * 2 / 64, KQ = (NORM_MAX_CB * 2 / LPR + WAVES - 1) / WAVES;
+    static constexpr int RW = (MT + WAVES - 1) / WAVES, CU = NCB * 2 / 64, KQ = (NCB * 2 / LPR + WAVES - 1) / WAVES;
     u32x4_t row[RW][CU], piece[KQ][RG], w[KQ];
 
     __device__ __forceinline__ void begin(const SpmmView &p, int m0, int ncb, int tid) {
@@ -872,7 +875,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
 // 3.7 us instead of 5.1, at 16 rows 4.3 instead of 5.3; at d_model 768 3.0 and 3.2 instead of 3.8 and 5.7.  (Nothing here divides by a value that is not known at compile
 // time: such a division is forty instructions, and these kernels live 3 to 5 us.)
 // ---------------------------------------------------------------------------------------------------------
-template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE, int CS = 0, bool YT = false>
+template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE, int CS = 0, bool YT = false, int NCB = NORM_MAX_CB>
 __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const SpmmParams p0) {
     constexpr int MSUB = (MT + 15) / 16, WAVES = PW * UW;
     SpmmView p = mortar_view(p0);
@@ -895,7 +898,7 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
     static_assert(PW % CW == 0 && !(CS > 0 && ROUTED), "whole parts; token lists have no chunked form");
 
     constexpr bool NS = MT < 16;           // (a 16-token tile's rows and pieces together are more than the waves can hold in flight: 8.5 against 8.7 us)
-    NormStage<NS ? MT : 4, WAVES> ns;
+    NormStage<NS ? MT : 4, WAVES, NCB> ns;
     const bool fused_norm = NACC == 2 && !MASKED && p.norm;
     if (NS && fused_norm) ns.begin(p, m0, p.Cb, tid);
 
@@ -1160,17 +1163,18 @@ int mortar_launch_segmented(SpmmParams &p, const SpmmParams *table, int layers, 
     return MORTAR_OK;
 }
 
-template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE = 0, int CS = 0, bool YT = false>
+template <int MT, int NACC, bool ROUTED, bool MASKED, int PW, int UW, int CODE = 0, int CS = 0, bool YT = false, int NCB = NORM_MAX_CB>
 int mortar_launch_partsplit(SpmmParams &p, hipStream_t st) {
     constexpr int WAVES = PW * UW;
     static_assert(!YT || (MT == 32 && NACC == 2 && CS == 0), "tile order is that of 32-token tiles");
     if (YT != (p.y_tiled != 0)) return mortar_fail(MORTAR_ERR_ARG, "spmm launch: activation layout mismatch");
+    if (p.norm && p.Cb > NCB) return mortar_fail(MORTAR_ERR_ARG, "spmm launch: rows too wide for the norm");
     if (CS > 0 && PW != CS * p.nseg * NACC) return mortar_fail(MORTAR_ERR_ARG, "chunked launch: %d waves for %d parts", PW, p.nseg * NACC);
     const int tile = tile_bytes(MT, p.Cb) + (MT >= 32 ? LDS_EXTRA : 0), sums = WAVES * (CS > 0 ? 1 : NACC) * ((MT + 15) / 16) * 64 * 16;
     const int smem = MT >= 32 ? (tile > sums ? tile : sums) : tile + sums;
     if (smem > 160 * 1024) return mortar_fail(MORTAR_ERR_LIMIT, "part-split tile of %d bytes does not fit LDS", smem);
     static bool attr_done = false;
-    auto kern = mortar_partsplit_kernel<MT, NACC, ROUTED, MASKED, PW, UW, CODE, CS, YT>;
+    auto kern = mortar_partsplit_kernel<MT, NACC, ROUTED, MASKED, PW, UW, CODE, CS, YT, NCB>;
     int rc = mortar_allow_big_lds(kern, attr_done);
     if (rc) return rc;
     p.n_mtiles = (p.M + MT - 1) / MT;
@@ -1187,6 +1191,9 @@ int mortar_launch_partsplit(SpmmParams &p, hipStream_t st) {
 // 2 gate_up + SwiGLU routed, 3 spmm with an input mask.  Returns -1 when the shape has no small-M variant.
 __attribute__((visibility("hidden"))) int mortar_smallm_launch(int kind, SpmmParams &p, const SpmmParams *table,
                                                                int layers, hipStream_t st);
+// gate_up with p.norm == NORM_WIDE: the launch that mortar_smallm_launch makes for the same call without the norm, where that is a 4- or 8-token
+// tile of all K (the fused norm then gives the bits of the separate one), MORTAR_NO_KERNEL otherwise.
+__attribute__((visibility("hidden"))) int mortar_smallm_norm_wide(SpmmParams &p, hipStream_t st);
 __attribute__((visibility("hidden"))) int mortar_smallm_tile(int Cb, int seg_cb, int64_t M, int kind);
 // Decode launches whose workgroups would leave half the chip idle: the part-split kernel with parts cut into chunks
 // (mortar_smallm_chunk.hip).  kind 0 or 1, 4- or 8-token tiles; -1 when it has no form for the shape, or none that is better.

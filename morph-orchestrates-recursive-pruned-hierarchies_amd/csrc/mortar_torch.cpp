@@ -98,7 +98,15 @@ int run_mlp(const PackHandle *gu, const PackHandle *dn, const at::Tensor &x, int
     const int64_t d = (int64_t)gu->w->Cb * 16, f = (int64_t)gu->w->Rb * 8, dy = (int64_t)dn->w->Rb * 16;
     const uint16_t *xp = u16(x);
     at::Tensor xn;
-    if (n.on && !(gu->w->seg_cb >= gu->w->Cb && mortar_norm_fusable(gu->w->Cb))) {
+    const bool fused = !n.on || (gu->w->seg_cb >= gu->w->Cb && mortar_norm_fusable(gu->w->Cb));
+    at::Tensor h;
+    if (M <= DECODE_MAX_ROWS) h = new_bf16(x, {M, f});
+    if (!fused && M <= DECODE_MAX_ROWS && !gates) {
+        const int rc = mortar_norm_gateup_decode_bf16(gu->w, gu->sched2, xp, M, d, n.w, n.eps, u16m(h), f, st);
+        if (rc == MORTAR_OK) return mortar_spmm_bf16(dn->w, dn->sched1, u16(h), M, f, y, dy, st);
+        if (rc != MORTAR_NO_KERNEL) return rc;
+    }
+    if (!fused) {
         xn = new_bf16(x, {M, d});
         const int rc = mortar_rmsnorm_bf16(xp, M, (int32_t)d, d, n.w, n.eps, u16m(xn), d, st);
         if (rc) return rc;
@@ -106,10 +114,9 @@ int run_mlp(const PackHandle *gu, const PackHandle *dn, const at::Tensor &x, int
         n = Norm{};
     }
     if (M > DECODE_MAX_ROWS) {
-        const at::Tensor h = at::empty({mortar_mlp_hidden_bytes(M, (int32_t)f)}, x.options().dtype(at::kByte).requires_grad(false));
+        h = at::empty({mortar_mlp_hidden_bytes(M, (int32_t)f)}, x.options().dtype(at::kByte).requires_grad(false));
         return mortar_mlp_bf16(gu->w, gu->sched2, dn->w, dn->sched1, xp, M, d, n.on, n.w, n.eps, gates, ncl, h.data_ptr(), y, dy, 0, st);
     }
-    const at::Tensor h = new_bf16(x, {M, f});
     int rc = n.on ? mortar_norm_gateup_swiglu_bf16(gu->w, gu->sched2, xp, M, d, n.w, n.eps, u16m(h), f, gates, ncl, nullptr, nullptr, st)
                   : mortar_gateup_swiglu_bf16(gu->w, gu->sched2, xp, M, d, u16m(h), f, gates, ncl, nullptr, nullptr, st);
     if (rc == MORTAR_OK) rc = mortar_spmm_bf16(dn->w, dn->sched1, u16(h), M, f, y, dy, st);

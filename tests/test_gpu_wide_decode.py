@@ -1,7 +1,9 @@
-"""The stand-alone RMSNorm with its rows in registers: every width at which the registers change."""
+"""Decode calls of wide models: the RMSNorm inside gate_up beyond 2048 values, the stand-alone norm with its rows in registers."""
 import pytest
+import torch
 
-from mortar_amd import ops, synth
+import mortar_amd
+from mortar_amd import _lib, ops, synth
 from oracle import mortar_oracle as O
 from util import assert_close_bf16, to_dev, to_np
 
@@ -13,3 +15,29 @@ def test_rmsnorm_widths(dev, M, d):
     x = O.bf16_round(synth.synth_x(M, d, 90) * 3)
     w = O.bf16_round(1.0 + 0.1 * synth.synth_x(1, d, 91)[0])
     assert_close_bf16(to_np(ops.rmsnorm(to_dev(x, dev), to_dev(w, dev))), O.rmsnorm(x, w), "rmsnorm", ulps=2)
+
+
+# d_ff / 16 units: one or two per workgroup with the parts in chunks, four, eight (from 9 rows)
+@pytest.mark.parametrize("d,units", [(2512, 24), (2560, 300), (4096, 30), (4096, 560), (3072, 512)])
+@pytest.mark.parametrize("one_scale", [False, True])
+def test_wide_norm_has_the_bits_of_the_separate_one(dev, d, units, one_scale):
+    spec = synth.synth_mlp(d, 16 * units, 0.1, seed=d + units, zipf_s=1.2)
+    if one_scale:
+        for k in ("gate_up", "down"):
+            spec[k]["scales"][:] = spec[k]["scales"][0]
+    mlp = synth.mlp_module(spec, dev)
+    W = mlp.gate_up._cms.mortar_pack()
+    assert not ops.norm_fusable(W)
+    w = to_dev(O.bf16_round(1.0 + 0.1 * synth.synth_x(1, d, 3)[0]), dev)
+    for nw in (w, None):
+        call = mortar_amd.MortarDecodeMLP(mlp, norm_weight=nw)
+        for M in (1, 3, 4, 5, 8, 9, 16, 17, 40, 64):
+            x = to_dev(O.bf16_round(synth.synth_x(M, d, M) * 2.5), dev)
+            xn = ops.rmsnorm(x, nw, call.eps)
+            assert torch.equal(call(x).view(M, d), ops.mlp(xn, W, mlp.down._cms.mortar_pack())), (M, nw is None)
+            h = torch.full((M + 1, 16 * units), float("nan"), device=dev, dtype=torch.bfloat16)
+            rc = _lib.lib().mortar_norm_gateup_decode_bf16(W.ref, W.sched(2).data_ptr(), x.data_ptr(), M, d, nw.data_ptr() if nw is not None else None,
+                                                           call.eps, h.data_ptr(), 16 * units, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0 if M <= 16 else rc in (0, -100)
+            if rc == 0:
+                assert torch.equal(h[:M], ops.gateup_swiglu(xn, W)) and torch.isnan(h[M].float()).all()
