@@ -194,7 +194,7 @@ int dispatch_prefill(int kind, SpmmParams &p, hipStream_t st) {
 int dispatch(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
     // products over several K segments have small-tile forms beyond the decode sizes as well (the launcher returns -1
     // once they would need more than one round of workgroups)
-    if (p.M > MORTAR_SMALLM_MAX && p.nseg > 1) {
+    if ((p.M > MORTAR_SMALLM_MAX || mortar_smallm_pipe(kind, p)) && p.nseg > 1) {
         const u32x4_t *two_bit = p.codes_o;
         if (W->codes4_o) p.codes_o = reinterpret_cast<const u32x4_t *>(W->codes4_o);
         const int rc = mortar_pipe_launch(kind, !W->codes4_o ? CODE_2BIT : p.uscale != 0.f ? CODE_4BIT | CODE_UNIFORM : CODE_4BIT, p, st);

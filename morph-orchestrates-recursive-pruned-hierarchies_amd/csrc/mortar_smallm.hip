@@ -306,6 +306,15 @@ static int smallm_norm_wide(SpmmParams &p, hipStream_t st) {
     return w8 <= (partsplit_fits(16, 2, p) ? 256 : 512) ? launch_partsplit<8, CODE>(1, p, st) : -1;
 }
 
+// Plain products whose rows are too wide for an 8-token tile of all K, more rows than the 4-token tiles take (narrow_tiles): the two buffers of
+// mortar_pipe.hip over a chip of workgroups, where the K-segmented 16-token tiles with 8 waves that are left make few of them ([4096, 11008],
+// 33 to 64 rows, MLP with its gate_up: 36.2..37.8 -> 28.1..29.7 us at 25 %, 25.4..26.0 -> 22.0..24.4 at 12.5 %).  Where part-split tiles fit they
+// stay the better ones ([3072, 8192], 48 rows: 17.8 against 18.4, 14.5 against 16.9).
+bool mortar_smallm_pipe(int kind, const SpmmParams &p) {
+    return (kind == 0 || kind == 3) && p.M > 16 && p.M <= MORTAR_SMALLM_MAX && p.nseg > 1 && !p.hc_h && !fits(8, p.Cb) &&
+           (p.M + 3) / 4 * (int64_t)((p.n_units + 3) / 4) > 512 && pick_waves(-16, p, 1) == 2;
+}
+
 // The norm in front of a wide gate_up, up to 64 rows.  A launch of its own for it is a chain of round trips as long as half of gate_up; inside, the
 // rows and the pieces of the tile arrive while the first descriptors and weights do.  MLP with its norm, us (graph replay), own launch -> inside: d_model
 // 3072 at 1 / 8 / 16 rows 12.9 -> 10.3, 14.2 -> 11.8, 16.9 -> 14.3, d_model 4096 18.6 -> 15.5, 20.0 -> 16.9, 22.9 -> 19.3.

@@ -1,11 +1,13 @@
-"""Decode calls of wide models: the RMSNorm inside gate_up beyond 2048 values, the stand-alone norm with its rows in registers."""
+"""Decode calls of wide models: the RMSNorm inside gate_up beyond 2048 values, the stand-alone norm with its rows in registers, and `down`
+rows that fit no 8-token tile."""
+import numpy as np
 import pytest
 import torch
 
 import mortar_amd
 from mortar_amd import _lib, ops, synth
 from oracle import mortar_oracle as O
-from util import assert_close_bf16, to_dev, to_np
+from util import assert_close_bf16, oracle_spmm, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +43,21 @@ def test_wide_norm_has_the_bits_of_the_separate_one(dev, d, units, one_scale):
             assert rc == 0 if M <= 16 else rc in (0, -100)
             if rc == 0:
                 assert torch.equal(h[:M], ops.gateup_swiglu(xn, W)) and torch.isnan(h[M].float()).all()
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 49, 64])
+@pytest.mark.parametrize("masked", [False, True])
+def test_down_of_a_wide_model(dev, M, masked):
+    # (256 rows of blocks: from 33 rows on more 4-token tiles than are worth it)
+    m = synth.synth_matrix(4096, 16 * 620, 0.1, seed=M, zipf_s=1.2)
+    W = synth.to_pack(m, dev)
+    x = synth.synth_x(M, 9920, seed=M)
+    active = None
+    if masked:
+        on = np.random.default_rng(M).random((M, 155)) < 0.4
+        x = x * np.repeat(on, 64, axis=1)
+        active = torch.from_numpy(on.astype(np.uint8)).to(dev)
+    buf = torch.full((M + 1, 4096), float("nan"), device=dev, dtype=torch.bfloat16)
+    ops.spmm(to_dev(x, dev), W, out=buf[:M], **({"active": active} if masked else {}))
+    assert torch.isnan(buf[M].float()).all()
+    assert_close_bf16(to_np(buf[:M]), oracle_spmm(x, m), "down")
