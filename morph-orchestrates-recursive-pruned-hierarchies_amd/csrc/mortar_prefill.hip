@@ -136,8 +136,8 @@ SegShape segmented_shape(const SpmmParams &p) { return seg_shape(p, {4, 3, 2, 1}
 
 // gate_up: 1, 2 or 3 unit pairs per wave (four spill).  A unit pair takes about 6.7 us and staging the segments 5 us (d_model 3072 and
 // 4096).  With two units per wave throughout, 400 rows of d_model 4096 were 286 workgroups: 83 -> 70 us for the MLP; 150
-// rows 52 -> 44; d_model 3072 at 200 rows 40.9 -> 34.6, at 600 64 -> 52.5.
-SegShape gateup_shape(const SpmmParams &p) { return seg_shape(p, {2, 3, 1}, 3, 4, 0); }
+// rows 52 -> 44; d_model 3072 at 200 rows 40.9 -> 34.6, at 600 64 -> 52.5.  Runs with up to two: d_model 4096 at 1300 rows 164 -> 154.
+SegShape gateup_shape(const SpmmParams &p) { return seg_shape(p, {2, 3, 1}, 3, 4, 2); }
 
 template <bool MASKED, int CODE, bool TL = false>
 int launch_segmented_plain(SpmmParams &p, hipStream_t st) {

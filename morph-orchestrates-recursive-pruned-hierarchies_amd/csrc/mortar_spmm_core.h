@@ -229,14 +229,27 @@ __device__ __forceinline__ void mortar_load_batch(const SpmmView &p, MortarBatch
 // `b` holds the part's first batch, loaded by the caller (mortar_load_batch at g0) where it suits it.
 // FIRST_ONLY: only the batch in `b` (the part's first RES_GROUPS octets) is multiplied and no load is issued here, so
 // that a caller which keeps the next part's batch in flight gets a counted wait for `b` instead of a full one.
-template <int MSUB, int MT, bool ROUTED, int CODE = 0, bool FIRST_ONLY = false>
+// SW: the tile is in the order of mortar_stage_pairs.
+template <int MSUB, int MT, bool ROUTED, int CODE = 0, bool FIRST_ONLY = false, bool SW = false>
 __device__ __forceinline__ void mortar_row_part(const SpmmView &p, const uint4 *lx, MortarBatch b, int g0, int g1,
                                                 int nb, uint32_t xo_base, const uint32_t (&tk)[MSUB], int nsub, int n,
                                                 int bsel, int hsel, f32x4_t (&acc)[MSUB]) {
     const unsigned char *lb = reinterpret_cast<const unsigned char *>(lx);
+    // SW: `xo` is the LDS address itself (the tile is at 0, these kernels have no other LDS): with a base to be added the exclusive or becomes a
+    // three-operand instruction, which takes no DPP operand.
+    auto operand = [&](uint32_t xo, int ms) {
+        if constexpr (SW) {
+            typedef uint32_t v4 __attribute__((ext_vector_type(4)));
+            const v4 v = *(const __attribute__((address_space(3))) v4 *)(uintptr_t)(xo + ms * 1024u);
+            return make_uint4(v[0], v[1], v[2], v[3]);
+        } else {
+            return *reinterpret_cast<const uint4 *>(lb + xo + (ROUTED ? tk[ms] * 32u : ms * 512u));
+        }
+    };
     for (int gq = g0; gq < (FIRST_ONLY ? g0 + 1 : g1); gq += RES_GROUPS) {
         if (!FIRST_ONLY && gq != g0) mortar_load_batch<CODE>(p, b, gq, g1, n, bsel, hsel);
-        const uint32_t ccs = __umul24(b.ccv, (uint32_t)(MT * 32));   // byte offset of the block-column in the tile
+        // byte offset of the block-column in the tile
+        const uint32_t ccs = SW ? __umul24(b.ccv >> 1, (uint32_t)(MT * 64)) | (b.ccv & 1u) << 5 : __umul24(b.ccv, (uint32_t)(MT * 32));
         const int pairs = ((nb - (gq - g0) * 8) + 1) >> 1;      // block pairs left in the row from this batch on
         // Activation operands are fetched two pairs ahead of the MFMAs that use them.  The only branches are
         // per octet (a whole octet past the end of the part is skipped) and, for prefill tiles, per half octet;
@@ -246,9 +259,9 @@ __device__ __forceinline__ void mortar_row_part(const SpmmView &p, const uint4 *
         uint4 Bq[PD + 1][MSUB];
 #pragma unroll
         for (int d = 0; d < PD; ++d) {
-            const uint32_t xo = mortar_row_bcast(ccs, d) + xo_base;
+            const uint32_t xo = SW ? mortar_row_bcast(ccs, d) ^ xo_base : mortar_row_bcast(ccs, d) + xo_base;
 #pragma unroll
-            for (int ms = 0; ms < MSUB; ++ms) Bq[d][ms] = *reinterpret_cast<const uint4 *>(lb + xo + (ROUTED ? tk[ms] * 32u : ms * 512u));
+            for (int ms = 0; ms < MSUB; ++ms) Bq[d][ms] = operand(xo, ms);
         }
 #pragma unroll
         for (int k = 0; k < RES_GROUPS; ++k) {
@@ -260,10 +273,10 @@ __device__ __forceinline__ void mortar_row_part(const SpmmView &p, const uint4 *
                     const uint32_t nib = (CODE & CODE_4BIT) ? b.cw[k][t] : ((b.cw[k][t] << (2 * hsel)) & 0xCCCCCCCCu);
                     const u32x4_t A = (CODE & CODE_UNIFORM) ? mortar_nib4(nib, p.cscale) : mortar_scale4(nib, mortar_row_bcast(b.sdv, u));
                     if (u + PD < NP) {
-                        const uint32_t xo = mortar_row_bcast(ccs, u + PD) + xo_base;
+                        const uint32_t xo = SW ? mortar_row_bcast(ccs, u + PD) ^ xo_base : mortar_row_bcast(ccs, u + PD) + xo_base;
 #pragma unroll
                         for (int ms = 0; ms < MSUB; ++ms)
-                            Bq[(u + PD) % (PD + 1)][ms] = *reinterpret_cast<const uint4 *>(lb + xo + (ROUTED ? tk[ms] * 32u : ms * 512u));
+                            Bq[(u + PD) % (PD + 1)][ms] = operand(xo, ms);
                     }
 #pragma unroll
                     for (int ms = 0; ms < MSUB; ++ms) {
@@ -343,6 +356,32 @@ __device__ __forceinline__ void mortar_stage_tiled32(const SpmmView &p, uint4 *l
     const MORTAR_GLOBAL char *src = p.x + ((int64_t)mt * p.Cb + c0) * 1024 + lane * 16;
     const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lx;
     for (int c = wave; c < ncb; c += WAVES) mortar_load_to_lds(src + (int64_t)c * 1024, __builtin_amdgcn_readfirstlane(dst + c * 1024));
+    __builtin_amdgcn_s_waitcnt(0);
+}
+
+// Stages block-columns [c0, c0 + ncb) of rows m0 .. m0 + MT from row-major activations without registers, in an order that the asynchronous copy can
+// leave: [pair of block-columns][token][64 bytes], the four 16-byte units of a token at unit ^ mortar_unit_swz(token).  A wave instruction copies 16
+// rows x 64 bytes, four consecutive lanes 64 contiguous ones; an operand read (16 tokens x 2 units) still touches every bank once, and the offset of a
+// block-column meets the lane's by an exclusive or instead of a sum.  Rows past M repeat the last one, a missing second block-column of the last pair
+// the first: neither feeds a sum that is stored.
+template <int MT, int WAVES>
+__device__ __forceinline__ void mortar_stage_pairs(const SpmmView &p, uint4 *lx, int m0, int c0, int ncb, int tid) {
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, t = lane >> 2;
+    const uint32_t dst = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lx;
+    const int unit = (lane & 3) ^ mortar_unit_swz(t);
+    const MORTAR_GLOBAL char *src[MT / 16];
+#pragma unroll
+    for (int ms = 0; ms < MT / 16; ++ms) {
+        const int row = m0 + ms * 16 + t;
+        src[ms] = p.x + (int64_t)(row < p.M ? row : p.M - 1) * p.ldx * 2 + (int64_t)c0 * 32 + unit * 16;
+    }
+    const int np = (ncb + 1) >> 1;
+    for (int q = wave; q < np; q += WAVES) {
+        const int back = 2 * q + 1 < ncb ? 0 : (unit & 2) * 16;
+#pragma unroll
+        for (int ms = 0; ms < MT / 16; ++ms)
+            mortar_load_to_lds(src[ms] + q * 64 - back, __builtin_amdgcn_readfirstlane(dst + q * (MT * 64) + ms * 1024));
+    }
     __builtin_amdgcn_s_waitcnt(0);
 }
 
@@ -723,15 +762,22 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
 // The descriptors of the next segment are fetched before the barrier pair, so their latency hides behind the
 // staging.
 // ---------------------------------------------------------------------------------------------------------
-// Whether the kernel below has a form that walks runs (RUNS, SpmmParams::span): where the loop around the sums does not spill.  (gate_up with three units per wave:
-// 40 registers, 162 -> 221 us; four units per wave staged through registers: 12 registers, 36 -> 43 us.)
+// Row-major tiles of the kernel below are copied by mortar_stage_pairs (SW): the registers of the other staging held the waves up at every segment, and
+// beside four units the runs spilled (12 registers, 36 -> 43 us).  With it a wave's priority may fall as in the tile-ordered form.  us, staged through
+// registers -> this: [2048, 11264], 4096 rows 82.5 -> 79; one-scale, 600 rows 28.7 -> 27.5; MLP of d_model 3072 at 2000 rows 138 -> 130, of 4096 at 700
+// 98 -> 96.  Not gate_up with three units per wave, whose sums leave no register for it (26 spilled against 5).
 template <int MT, int NACC, bool MASKED, int UPW, bool TABLE, bool XT>
-constexpr bool mortar_seg_runs() { return MT >= 32 && !TABLE && NACC == 1 && !MASKED && (XT || UPW <= 3); }
+constexpr bool mortar_seg_pairs() { return MT == 32 && !MASKED && !XT && !TABLE && UPW * NACC < 6; }
+// Whether it has a form that walks runs (RUNS, SpmmParams::span): where the loop around the sums does not spill.  (gate_up with three units per wave:
+// 40 registers, 162 -> 221 us.)
+template <int MT, int NACC, bool MASKED, int UPW, bool TABLE, bool XT>
+constexpr bool mortar_seg_runs() { return MT >= 32 && !TABLE && !MASKED && UPW * NACC <= (NACC == 1 && !XT ? 3 : 4); }
 
 template <int MT, int NACC, bool MASKED, int WAVES, int UPW, bool TABLE, int CODE, bool TL = false, bool RUNS = false>
 __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const SpmmParams p0, const SpmmParams *table) {
     constexpr int MSUB = (MT + 15) / 16, NP = UPW * NACC;
     constexpr bool XT = TL && NACC == 1, YT = TL && NACC == 2;
+    constexpr bool SW = mortar_seg_pairs<MT, NACC, MASKED, UPW, TABLE, XT>();
     SpmmView p = mortar_view(TABLE ? mortar_table_entry(table, blockIdx.y) : p0);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint4 *lx = reinterpret_cast<uint4 *>(smem);
@@ -760,7 +806,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
     for (bool again = false;; again = true) {
         const int m0 = mt * MT, pos0 = slot0 * WAVES + wave;
         const int tid = RUNS ? mortar_opaque_tid(tid0) : tid0, lane = tid & 63, n = lane & 15, g = lane >> 4, bsel = g >> 1, hsel = g & 1;
-        const uint32_t lane_xo = (uint32_t)(hsel * 16 + n * 32);
+        const uint32_t lane_xo = SW ? (uint32_t)(n * 64 + (hsel ^ mortar_unit_swz(n)) * 16) : (uint32_t)(hsel * 16 + n * 32);
         int slots = left < UPW ? left : UPW;
         if (RUNS && tile_slots - slot0 < slots) slots = tile_slots - slot0;
         f32x4_t acc[UPW][NACC][MSUB];
@@ -809,7 +855,8 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
             MortarBatch bq;
             if (BATCH_AHEAD) first_batch(bq, 0);
             if (sg > 0 || (RUNS && again)) __syncthreads();
-            mortar_stage_tile<MT, WAVES, MASKED, XT>(p, lx, m0, c0, ncb, tid);
+            if constexpr (SW) mortar_stage_pairs<MT, WAVES>(p, lx, m0, c0, ncb, mortar_opaque_tid(tid0));
+            else mortar_stage_tile<MT, WAVES, MASKED, XT>(p, lx, m0, c0, ncb, tid);
             __syncthreads();
             if (!BATCH_AHEAD) {
 #pragma unroll
@@ -827,23 +874,23 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
             for (int q = 0; q < NP; ++q) {
                 // A wave lowers its priority with every part of the segment it has finished: the arbiter serves the oldest wave of
                 // a SIMD first, so without this the four waves finish a segment one after another (4.8 / 6.3 / 8.0 / 9.4 us measured)
-                // and the SIMD runs the end of it on one or two waves.  Tile-ordered form only: with the register-staged forms the
+                // and the SIMD runs the end of it on one or two waves.  Not the forms staged through registers, where the
                 // same priorities cost time (the staging of the next segment then starts from uneven waves).
-                if constexpr (XT) mortar_setprio(NP - 1 - q);
+                if constexpr (XT || SW) mortar_setprio(NP - 1 - q);
                 MortarBatch bn;
                 if (q + 1 < NP) first_batch(bn, q + 1);
                 const int nbq = g0[q] < g1[q] ? nb[q] : 0;
-                mortar_row_part<MSUB, MT, false, CODE, true>(p, lx, bq, g0[q], g1[q], nbq < FIRST ? nbq : FIRST, lane_xo, tk, MSUB,
+                mortar_row_part<MSUB, MT, false, CODE, true, SW>(p, lx, bq, g0[q], g1[q], nbq < FIRST ? nbq : FIRST, lane_xo, tk, MSUB,
                                                              n, bsel, hsel, acc[q / NACC][q % NACC]);
                 if (nbq > FIRST) {                                      // the rest of a long part
                     MortarBatch bt;
                     mortar_load_batch<CODE>(p, bt, g0[q] + RES_GROUPS, g1[q], n, bsel, hsel);
-                    mortar_row_part<MSUB, MT, false, CODE>(p, lx, bt, g0[q] + RES_GROUPS, g1[q], nbq - FIRST, lane_xo, tk, MSUB,
+                    mortar_row_part<MSUB, MT, false, CODE, false, SW>(p, lx, bt, g0[q] + RES_GROUPS, g1[q], nbq - FIRST, lane_xo, tk, MSUB,
                                                            n, bsel, hsel, acc[q / NACC][q % NACC]);
                 }
                 if (q + 1 < NP) bq = bn;
             }
-            if constexpr (XT) mortar_setprio(0);
+            if constexpr (XT || SW) mortar_setprio(0);
         }
 
         uint32_t tl[MSUB];
@@ -1137,8 +1184,8 @@ inline int64_t mortar_segmented_shape(SpmmParams &p, int layers) {
 template <int MT, int NACC, bool MASKED, int WAVES, int UPW, bool TABLE = false, int CODE = 0, bool TL = false>
 int mortar_launch_segmented(SpmmParams &p, const SpmmParams *table, int layers, hipStream_t st) {
     if (TABLE != (table != nullptr)) return mortar_fail(MORTAR_ERR_ARG, "spmm launch: parameter table mismatch");
-    const int smem = tile_bytes(MT, p.seg_cb);
-    if (smem > LDS_BUDGET + LDS_PAD * 16) return mortar_fail(MORTAR_ERR_LIMIT, "segment tile of %d bytes does not fit LDS", smem);
+    const int smem = tile_bytes(MT, (p.seg_cb + 1) & ~1);
+    if (tile_bytes(MT, p.seg_cb) > LDS_BUDGET + LDS_PAD * 16) return mortar_fail(MORTAR_ERR_LIMIT, "segment tile of %d bytes does not fit LDS", smem);
     static bool attr_done = false;
     if (TL != ((NACC == 1 ? p.x_tiled : p.y_tiled) != 0)) return mortar_fail(MORTAR_ERR_ARG, "spmm launch: activation layout mismatch");
     int rc;

@@ -58,3 +58,23 @@ def test_mlp_runs(dev, norm, gated):
     ref = O.swiglu_mlp(xo, spec["gate_up"], spec["down"], gates)["y"]
     out = _call(lambda y: ops.mlp(to_dev(x, dev), G, D, out=y, **kw), M, d, dev)
     assert_close_bf16(to_np(out[torch.from_numpy(rows).to(dev)]), ref, "mlp", ulps=8)
+
+
+@pytest.mark.parametrize("units,M", [(200, 1300), (688, 1300), (40, 97)])      # runs of one, of two units per wave, whole groups
+@pytest.mark.parametrize("one_scale", [False, True])
+def test_gateup_of_an_odd_width(dev, units, M, one_scale):
+    """K segments of an odd number of block-columns, copied in pairs; a partial last tile; the module's hidden activations in tile order."""
+    d = 16 * 161
+    spec = synth.synth_mlp(d, 16 * units, 0.1, seed=units, zipf_s=1.2)
+    if one_scale:
+        for k in ("gate_up", "down"):
+            spec[k]["scales"][:] = spec[k]["scales"][0]
+    G, D = synth.to_pack(spec["gate_up"], dev), synth.to_pack(spec["down"], dev)
+    x = synth.synth_x(M, d, seed=M)
+    rows = _sample(M)
+    idx = torch.from_numpy(rows).to(dev)
+    ref = O.swiglu_mlp(x[rows], spec["gate_up"], spec["down"])
+    h = _call(lambda y: ops.gateup_swiglu(to_dev(x, dev), G, out=y), M, 16 * units, dev)
+    assert_close_bf16(to_np(h[idx]), ref["h"], "h", ulps=8)
+    y = _call(lambda out: ops.mlp(to_dev(x, dev), G, D, out=out), M, d, dev)
+    assert_close_bf16(to_np(y[idx]), ref["y"], "mlp", ulps=8)
