@@ -765,9 +765,9 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
 // Row-major tiles of the kernel below are copied by mortar_stage_pairs (SW): the registers of the other staging held the waves up at every segment, and
 // beside four units the runs spilled (12 registers, 36 -> 43 us).  With it a wave's priority may fall as in the tile-ordered form.  us, staged through
 // registers -> this: [2048, 11264], 4096 rows 82.5 -> 79; one-scale, 600 rows 28.7 -> 27.5; MLP of d_model 3072 at 2000 rows 138 -> 130, of 4096 at 700
-// 98 -> 96.  Not gate_up with three units per wave, whose sums leave no register for it (26 spilled against 5).
+// 98 -> 96.
 template <int MT, int NACC, bool MASKED, int UPW, bool TABLE, bool XT>
-constexpr bool mortar_seg_pairs() { return MT == 32 && !MASKED && !XT && !TABLE && UPW * NACC < 6; }
+constexpr bool mortar_seg_pairs() { return MT == 32 && !MASKED && !XT && !TABLE; }
 // Whether it has a form that walks runs (RUNS, SpmmParams::span): where the loop around the sums does not spill.  (gate_up with three units per wave:
 // 40 registers, 162 -> 221 us.)
 template <int MT, int NACC, bool MASKED, int UPW, bool TABLE, bool XT>
@@ -845,9 +845,11 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
             // The first batch of every part is requested one part ahead (the first part's before the tile is staged), always
             // and in a fixed order (an empty part reads octet 0), and a part's first batch is multiplied without a load in
             // between: the wait for it then counts the loads issued since and never includes the newest ones.
-            // (Prefill tiles only: the decode tiles of this kernel run many waves per SIMD on few registers.)
+            // (Prefill tiles only: the decode tiles of this kernel run many waves per SIMD on few registers.  Nor gate_up with three units per wave, whose
+            // sums leave no room for a second batch: 26 registers spilled, 5 with the tile staged through registers, none like this; MLP of
+            // d_model 4096 at 1999 rows 224.4 -> 222.3 us.)
             constexpr int FIRST = 8 * RES_GROUPS;                      // blocks of a part's first batch
-            constexpr bool BATCH_AHEAD = MT >= 32;
+            constexpr bool BATCH_AHEAD = MT >= 32 && UPW * NACC < 6;
             auto first_batch = [&](MortarBatch &bb, int q) {
                 const bool any = g0[q] < g1[q];
                 mortar_load_batch<CODE>(p, bb, any ? g0[q] : 0, any ? g1[q] : 1, n, bsel, hsel);
@@ -864,7 +866,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
                     if (g0[q] < g1[q]) {
                         MortarBatch b;
                         mortar_load_batch<CODE>(p, b, g0[q], g1[q], n, bsel, hsel);
-                        mortar_row_part<MSUB, MT, false, CODE>(p, lx, b, g0[q], g1[q], nb[q], lane_xo, tk, MSUB, n, bsel, hsel,
+                        mortar_row_part<MSUB, MT, false, CODE, false, SW>(p, lx, b, g0[q], g1[q], nb[q], lane_xo, tk, MSUB, n, bsel, hsel,
                                                                acc[q / NACC][q % NACC]);
                     }
                 }
