@@ -847,7 +847,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
             // between: the wait for it then counts the loads issued since and never includes the newest ones.
             // (Prefill tiles only: the decode tiles of this kernel run many waves per SIMD on few registers.  Nor gate_up with three units per wave, whose
             // sums leave no room for a second batch: 26 registers spilled, 5 with the tile staged through registers, none like this; MLP of
-            // d_model 4096 at 1999 rows 224.4 -> 222.3 us.)
+            // d_model 4096 at 1999 rows 224.4 -> 222.3 us, with falling priorities as below, a step for two parts, 214.5; at 3000 rows 334 -> 325.)
             constexpr int FIRST = 8 * RES_GROUPS;                      // blocks of a part's first batch
             constexpr bool BATCH_AHEAD = MT >= 32 && UPW * NACC < 6;
             auto first_batch = [&](MortarBatch &bb, int q) {
@@ -863,6 +863,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
             if (!BATCH_AHEAD) {
 #pragma unroll
                 for (int q = 0; q < NP; ++q) {
+                    if constexpr (SW) mortar_setprio((NP - 1 - q) / 2);
                     if (g0[q] < g1[q]) {
                         MortarBatch b;
                         mortar_load_batch<CODE>(p, b, g0[q], g1[q], n, bsel, hsel);
@@ -870,6 +871,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const Spmm
                                                                acc[q / NACC][q % NACC]);
                     }
                 }
+                if constexpr (SW) mortar_setprio(0);
                 continue;
             }
 #pragma unroll
