@@ -113,8 +113,8 @@ __device__ __forceinline__ void val_multiply(const unsigned char *lb, const ValB
 // ones 24, a fill 21).  Bounded buffer stores drop the tokens past M and the rows past the end (`rows` of the RU exist).  No scalar
 // offset: behind a 16-byte store that has one the compiler may overwrite the data registers in the next instruction, and gfx950 then
 // stores the new values in the last lanes of a row.
-// NT: non-temporal, the values and the tiles stay in the L2 (16384 x 768 x 4096: 53 -> 46 us); not for pieces below 64 bytes, which the
-// L2 then passes on unmerged (three times as slow).
+// NT: non-temporal, the values and the tiles stay in the L2.  Only pieces that are whole (val_whole_lines): the parts of one that straddles
+// lines leave the L2 unmerged.
 template <int MT, int RU, bool NT>
 struct ValOut {
     static constexpr int TPI = RU == 4 ? 8 : 16;          // tokens per instruction
@@ -176,7 +176,7 @@ __device__ __forceinline__ int val_idx(const int32_t *p, int i) {
 // for.  Narrow K is bound by the results and the values together: 16384 x 768 x 4096 at 25 % (134 MB of results, a fill of which takes
 // 21 us) takes 50 us over rotating buffers, of which stage and store alone are 33, the values alone 21, the products alone 25 (before
 // the non-temporal 128-byte pieces: 59 us).  Wide K is bound by the values from the L2, once per 32 tokens (4096 x 2048 x 11264: 82 us).
-template <int MT, int RU>
+template <int MT, int RU, bool NT>
 __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const ValArgs a) {
     constexpr int MSUB = MT / 16;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -239,7 +239,7 @@ __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const V
 #pragma unroll
     for (int ms = 0; ms < MSUB; ++ms) acc[ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     int k = 0, j = u.p0, je = u.p1;                       // row of u that is being multiplied
-    const ValOut<MT, RU, true> out(a, m0, n, g);
+    const ValOut<MT, RU, NT> out(a, m0, n, g);
     // one batch; false when the wave's rows are done
     auto step = [&](const ValBatch &c, ValBatch &nx) {
         request(nx);
@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const V
 // 64 tokens from the L2) and the operand reads from LDS bound it.  16384 x 4096 x 768 at 25 %: 58 us over rotating buffers (62 before its
 // results left in 128-byte non-temporal pieces), of which the copies alone are 28, the values alone 28, the products alone 32.  Segments of 24 columns in three buffers took 6 % longer
 // (short parts leave a batch half empty), batches requested two ahead 18 % (registers, moves).
-template <int MT, int UPW>
+template <int MT, int UPW, bool NT>
 __global__ void __launch_bounds__((VAL_CW + VAL_LOADERS) * 64) values_segmented_kernel(const ValArgs a) {
     constexpr int MSUB = MT / 16;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -344,7 +344,7 @@ __global__ void __launch_bounds__((VAL_CW + VAL_LOADERS) * 64) values_segmented_
         __syncthreads();
     }
     constexpr int RU = UPW < 4 ? 2 : 4;
-    const ValOut<MT, RU, (UPW > 1)> out(a, m0, n, g);
+    const ValOut<MT, RU, NT> out(a, m0, n, g);
 #pragma unroll
     for (int k = 0; k < UPW; k += RU) {
         u32x2_t p[RU][MSUB];
@@ -390,30 +390,53 @@ int val_launch(K kern, bool &done, const ValArgs &a, int64_t grid, int threads, 
     return MORTAR_OK;
 }
 
+// Whether the pieces of `piece` bytes that a wave stores lie on lines, in every row of y: they may then be non-temporal.  us, plain -> non-temporal,
+// 16384 tokens x 4096 features of 768 at 12.5 / 25 %: 39.7 -> 36.3, 53 -> 48; in rows of 4112 values 46 -> 101, 56 -> 106; with an elementwise
+// kernel behind it that reads the result 83 -> 81, 97 -> 91, and 85 -> 130, 98 -> 136 for 4080 features.  16384 tokens x 768 features of 4096 58.9 -> 50.7
+// (66.4 -> 64.7 with the reader), in rows of 772 values 58.4 -> 56.6.  Results of a few MB gain as well (2048 tokens x 4096 features 12.6 -> 11.2, with the
+// reader 18.4 -> 18.1); of those between 30 and 70 MB some gain and some lose (8192 tokens x 2048 features of 768 19.8 -> 20.8, 30.3 -> 32.9).
+bool val_whole_lines(const ValArgs &a, int piece) {
+    return (reinterpret_cast<uintptr_t>(a.y) | (uintptr_t)(a.ldy * 2)) % (uintptr_t)piece == 0;
+}
+
+template <int MT, int RU, bool NT>
+int launch_resident_form(const ValArgs &a, int64_t grid, hipStream_t st) {
+    static bool done = false;
+    return val_launch(values_resident_kernel<MT, RU, NT>, done, a, grid, VAL_WAVES * 64, (a.Cb + 1) / 2 * (MT * 64) + 16, st);
+}
+
 template <int MT>
 int launch_resident(ValArgs &a, hipStream_t st) {
-    static bool done4 = false, done2 = false;
     const int tiles = (a.M + MT - 1) / MT, max_split = (a.Rb + VAL_WAVES - 1) / VAL_WAVES;
     int split = 256 / tiles;                 // about one workgroup per CU and round; every workgroup stages the whole tile
     split = split < 1 ? 1 : (split > max_split ? max_split : split);
     a.n_split = split;
     a.per = ((a.Rb + split - 1) / split + 3) & ~3;
-    const int smem = (a.Cb + 1) / 2 * (MT * 64) + 16;
+    const int64_t grid = (int64_t)tiles * split;
     // Four rows per unit while every wave has two such units, else two.  16384 x 768 x 4096 at 12.5 / 25 %: 37 / 51 us against 47 / 51 with
     // two rows, 8192 tokens 23 / 31 against 27 / 31; 4099 tokens (1.4 units of four per wave) 17.2 / 21.3 against 15.3 / 20.1, 300 tokens
-    // 7.0 / 8.8 against 5.7 / 6.7.
-    if (a.per >= 8 * VAL_WAVES) return val_launch(values_resident_kernel<MT, 4>, done4, a, (int64_t)tiles * split, VAL_WAVES * 64, smem, st);
-    return val_launch(values_resident_kernel<MT, 2>, done2, a, (int64_t)tiles * split, VAL_WAVES * 64, smem, st);
+    // 7.0 / 8.8 against 5.7 / 6.7.  (Few rows leave waves without a unit.  Half the workgroups instead: 24 to 128 rows, up to 1000 tokens, 5 to 40 % slower;
+    // one row at a time: 17 to 33 rows of 12 blocks 2 to 5 % faster, 64 and more 8 to 13 % slower.)
+    if (a.per >= 8 * VAL_WAVES) return val_whole_lines(a, 128) ? launch_resident_form<MT, 4, true>(a, grid, st) : launch_resident_form<MT, 4, false>(a, grid, st);
+    return val_whole_lines(a, 64) ? launch_resident_form<MT, 2, true>(a, grid, st) : launch_resident_form<MT, 2, false>(a, grid, st);
 }
 
-template <int MT, int UPW>
-int launch_segmented(ValArgs &a, hipStream_t st) {
+template <int MT, int UPW, bool NT>
+int launch_segmented_form(ValArgs &a, hipStream_t st) {
     static bool done = false;
     a.per = VAL_CW * UPW;
     a.n_split = (a.Rb + a.per - 1) / a.per;
     a.sub = MT == 64 ? 1 : 2;
-    return val_launch(values_segmented_kernel<MT, UPW>, done, a, (int64_t)((a.M + MT - 1) / MT) * a.n_split, (VAL_CW + VAL_LOADERS) * 64,
+    return val_launch(values_segmented_kernel<MT, UPW, NT>, done, a, (int64_t)((a.M + MT - 1) / MT) * a.n_split, (VAL_CW + VAL_LOADERS) * 64,
                       2 * (a.seg_cb * a.sub / 2 * (MT * 64)), st);
+}
+
+template <int MT, int UPW>
+int launch_segmented(ValArgs &a, hipStream_t st) {
+    if constexpr (UPW > 1) {                 // (one row's pieces are 32 bytes)
+        if (val_whole_lines(a, 64)) return launch_segmented_form<MT, UPW, true>(a, st);
+    }
+    return launch_segmented_form<MT, UPW, false>(a, st);
 }
 
 // A tile of all K: up to 156 block-columns (78 pairs) for 32 tokens, 78 for 64 (the row counter behind it is outside the tile's budget).

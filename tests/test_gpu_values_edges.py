@@ -44,6 +44,27 @@ def test_values_product_four_rows_at_a_time(dev, Rb, Cb, M, density):
     test_values_product_edges(dev, Rb, Cb, M, density)
 
 
+@pytest.mark.parametrize("Rb,Cb,M", [(34, 5, 130), (256, 3, 8200), (30, 80, 97), (128, 80, 8161),      # units of two and of four rows, 64- and 32-token tiles
+                                     (26, 200, 70), (50, 160, 4100), (12, 200, 16389)])               # K segments, one to four rows per wave
+@pytest.mark.parametrize("pad", [4, 32, 64])
+def test_values_product_has_the_same_bits_whatever_the_pitch(dev, Rb, Cb, M, pad):
+    """Rows of y that start on lines, on half lines and on neither (the stores differ), and a base off the lines."""
+    rng = np.random.default_rng(Rb)
+    mask = rng.random((Rb, Cb)) < 0.2
+    T = BcsrTopology(np.concatenate([[0], np.cumsum(mask.sum(1))]).astype(np.int32), np.nonzero(mask)[1].astype(np.int16), Rb * 16, Cb * 16, dev)
+    g = torch.Generator(device=dev).manual_seed(pad)
+    data = torch.randn(T.nnz, 16, 16, device=dev, generator=g).bfloat16()
+    x = torch.randn(M, Cb * 16, device=dev, generator=g).bfloat16()
+    want = ops.dds_values(x, data, T)
+    for base in (0, 4):
+        ld = Rb * 16 + pad
+        buf = torch.full((base + M * ld,), 7.0, device=dev, dtype=torch.bfloat16)
+        out = buf[base:].view(M, ld)
+        ops.dds_values(x, data, T, out=out[:, :Rb * 16])
+        assert torch.equal(out[:, :Rb * 16], want)
+        assert (out[:, Rb * 16:] == 7.0).all() and (buf[:base] == 7.0).all()
+
+
 @pytest.mark.parametrize("Rb,Cb", [(5, 3), (33, 170)])                 # all of K in one tile, K segments
 @pytest.mark.parametrize("ld,M", [(2 ** 23 + 8, 70), (2 ** 26, 19), (2 ** 30, 3)])      # 64 rows of y in 31 bits; 16 of them; one
 def test_values_product_into_rows_far_apart(dev, Rb, Cb, ld, M):
