@@ -413,11 +413,15 @@ int launch_resident(ValArgs &a, hipStream_t st) {
     a.n_split = split;
     a.per = ((a.Rb + split - 1) / split + 3) & ~3;
     const int64_t grid = (int64_t)tiles * split;
-    // Four rows per unit while every wave has two such units, else two.  16384 x 768 x 4096 at 12.5 / 25 %: 37 / 51 us against 47 / 51 with
+    // 64-token tiles: four rows per unit while every wave has two such units, else two.  16384 x 768 x 4096 at 12.5 / 25 %: 37 / 51 us against 47 / 51 with
     // two rows, 8192 tokens 23 / 31 against 27 / 31; 4099 tokens (1.4 units of four per wave) 17.2 / 21.3 against 15.3 / 20.1, 300 tokens
     // 7.0 / 8.8 against 5.7 / 6.7.  (Few rows leave waves without a unit.  Half the workgroups instead: 24 to 128 rows, up to 1000 tokens, 5 to 40 % slower;
     // one row at a time: 17 to 33 rows of 12 blocks 2 to 5 % faster, 64 and more 8 to 13 % slower.)
-    if (a.per >= 8 * VAL_WAVES) return val_whole_lines(a, 128) ? launch_resident_form<MT, 4, true>(a, grid, st) : launch_resident_form<MT, 4, false>(a, grid, st);
+    // 32-token tiles: always two.  Their units carry half the results and twice the values: [5632, 2048], 4096 tokens at 25 % 44.3 us against 46.4 with four
+    // rows, with a reader behind it 59.6 against 63; [5632, 1280] 31.9 against 34.2, 47.5 against 50; equal at [4096, 1280].
+    if constexpr (MT == 64) {
+        if (a.per >= 8 * VAL_WAVES) return val_whole_lines(a, 128) ? launch_resident_form<MT, 4, true>(a, grid, st) : launch_resident_form<MT, 4, false>(a, grid, st);
+    }
     return val_whole_lines(a, 64) ? launch_resident_form<MT, 2, true>(a, grid, st) : launch_resident_form<MT, 2, false>(a, grid, st);
 }
 

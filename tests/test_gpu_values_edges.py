@@ -38,13 +38,13 @@ def test_values_product_edges(dev, Rb, Cb, M, density):
         assert torch.equal(ops.transpose_blocks(data, src), data[src.long()].transpose(1, 2))
 
 
-@pytest.mark.parametrize("Rb,Cb,M", [(131, 5, 16400), (129, 80, 8161), (256, 3, 8137)])      # units of four rows: 64- and 32-token tiles, rows and tokens left over
+@pytest.mark.parametrize("Rb,Cb,M", [(131, 5, 16400), (129, 80, 8161), (256, 3, 8137)])      # units of four rows (64-token tiles), of two in the same range of 32-token ones; rows and tokens left over
 @pytest.mark.parametrize("density", [0.04, 0.5])
 def test_values_product_four_rows_at_a_time(dev, Rb, Cb, M, density):
     test_values_product_edges(dev, Rb, Cb, M, density)
 
 
-@pytest.mark.parametrize("Rb,Cb,M", [(34, 5, 130), (256, 3, 8200), (30, 80, 97), (128, 80, 8161),      # units of two and of four rows, 64- and 32-token tiles
+@pytest.mark.parametrize("Rb,Cb,M", [(34, 5, 130), (256, 3, 8200), (30, 80, 97), (128, 80, 8161),      # units of two and of four rows (64-token tiles), of two (32-token ones)
                                      (26, 200, 70), (50, 160, 4100), (12, 200, 16389)])               # K segments, one to four rows per wave
 @pytest.mark.parametrize("pad", [4, 32, 64])
 def test_values_product_has_the_same_bits_whatever_the_pitch(dev, Rb, Cb, M, pad):
