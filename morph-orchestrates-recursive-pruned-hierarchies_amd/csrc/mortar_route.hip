@@ -914,7 +914,7 @@ __global__ void __launch_bounds__(256) route_flags_kernel(const float *gates, in
 // the gate_up staging (rms_* in mortar_device.h): both give the same bits.
 // A call of few rows is a chain of latencies.  CU > 0: rows of at most 64 CU units stay in registers, everything requested at once; the loops
 // below are a round trip per 64 units, twice.  us (graph replay), the loops -> this: 16 rows of 2048 / 4096 / 8192 values 3.6 -> 2.7, 5.2 -> 3.4, 8.9 ->
-// 5.0; 16384 rows, which run at the rate of memory, 28 -> 21, 58 -> 41, 145 -> 100 (4096 rows of 2048 values: 6.5 -> 6.7).
+// 5.0; 16384 rows, which run at the rate of memory, 28 -> 21, 58 -> 41, 145 -> 100, 12000 rows of 512 6.5 -> 6.4.
 template <int CU>
 __global__ void __launch_bounds__(256) rmsnorm_rows_kernel(const uint16_t *x, int64_t M, int d, int64_t ldx,
                                                             const uint16_t *w, float eps, uint16_t *y, int64_t ldy) {
@@ -1179,16 +1179,18 @@ extern "C" int mortar_rmsnorm_bf16(const uint16_t *x, int64_t M, int32_t d, int6
     if (M <= 0 || d <= 0 || ldx < d || ldy < d) return mortar_fail(MORTAR_ERR_ARG, "rmsnorm: bad shape");
     const bool units = d % 8 == 0 && ldx % 8 == 0 && ldy % 8 == 0 &&
                        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
-    if (units)
-    {
+    if (units) {
         // few rows: a workgroup each
         const int rpw = M <= 1024 ? 1 : 4;
-        const auto kern = d <= 1024 ? rmsnorm_rows_kernel<2> : d <= 2048 ? rmsnorm_rows_kernel<4> : d <= 4096 ? rmsnorm_rows_kernel<8>
+        // The loops where they are still the faster form: calls of 12 to 17 MB, whose waves all fit the chip at once, of rows that fill their registers.
+        // us, loops against registers: 8192 rows of 1024 values 7.6 against 8.0, 4096 of 2048 8.1 against 8.4.  Beside the range: 3000 rows of 2048 6.7 against
+        // 6.5, 6000 10.8 against 9.5, 10000 of 1024 8.8 against 8.3; 1536 values, 4096 rows 6.5 either way; 1792 values, 5000 rows 9.1 against 8.7.
+        const bool loops = (d == 1024 || d == 2048) && M * d > (6 << 20) && M * d < (17 << 19);
+        const auto kern = loops ? rmsnorm_rows_kernel<0> : d <= 512 ? rmsnorm_rows_kernel<1> : d <= 1024 ? rmsnorm_rows_kernel<2> : d <= 2048 ? rmsnorm_rows_kernel<4> : d <= 4096 ? rmsnorm_rows_kernel<8>
                         : d <= 8192 ? rmsnorm_rows_kernel<16> : rmsnorm_rows_kernel<0>;
         hipLaunchKernelGGL(kern, dim3((unsigned)((M + rpw - 1) / rpw)), dim3(64 * rpw), 0, static_cast<hipStream_t>(stream),
                            x, M, d, ldx, w, eps, y, ldy);
-    }
-    else
+    } else
         hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)M), dim3(256), 0, static_cast<hipStream_t>(stream), x, M, d,
                            ldx, w, eps, y, ldy);
     return check_launch("rmsnorm");

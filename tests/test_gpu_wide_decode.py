@@ -19,6 +19,17 @@ def test_rmsnorm_widths(dev, M, d):
     assert_close_bf16(to_np(ops.rmsnorm(to_dev(x, dev), to_dev(w, dev))), O.rmsnorm(x, w), "rmsnorm", ulps=2)
 
 
+@pytest.mark.parametrize("M,d", [(1100, 512), (1030, 504), (4096, 2048), (6200, 1024), (8703, 1024), (4099, 1536), (4500, 2048), (4096, 2056)])
+@pytest.mark.parametrize("weight", [False, True])
+def test_rmsnorm_of_many_rows_has_the_bits_of_few(dev, M, d, weight):
+    """Calls of 12 to 17 MB run another form than smaller and larger ones, and calls of few rows."""
+    g = torch.Generator(device=dev).manual_seed(d)
+    x = (torch.randn(M, d, device=dev, generator=g) * 2).bfloat16()
+    w = torch.randn(d, device=dev, generator=g).bfloat16() if weight else None
+    want = torch.cat([ops.rmsnorm(c, w) for c in x.split(500)])
+    assert torch.equal(ops.rmsnorm(x, w), want)
+
+
 # d_ff / 16 units: one or two per workgroup with the parts in chunks, four, eight (from 9 rows)
 @pytest.mark.parametrize("d,units", [(2512, 24), (2560, 300), (4096, 30), (4096, 560), (3072, 512)])
 @pytest.mark.parametrize("one_scale", [False, True])
