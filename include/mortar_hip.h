@@ -222,7 +222,8 @@ int mortar_spmm_bf16_masked(const mortar_bcsr_t *W, const int32_t *sched, const 
  * (morph/inference/engine.py:996-1001, 1052-1060; morph/kernels/triton/fused_hyper_connection.py:927-970; wide carriers
  * hc_post_wide, morph/kernels/triton/fused_decode_step.py:1725-1739):
  *   out[t, i, :] = sum_j hres[t, i, j] * carrier[t, j, :] + hpost[t, i] * y[t, :] (+ term[t, :])
- * fp32 arithmetic in that order; y enters rounded to bf16 (what mortar_spmm_bf16 would have stored).
+ * fp32 arithmetic in that order; y enters rounded to bf16: what mortar_spmm_bf16 would have stored, except that calls of 17 rows
+ * and more on a matrix of one K segment add in another order here (small tiles instead of the prefill ones).
  *   carrier, out  [M, n_streams, Rb*16] contiguous, bf16 (carrier_f32 = 0; 8-byte aligned) or fp32 (1; 16-byte aligned);
  *                 1 <= n_streams <= 4;  hres fp32 [M, n, n], hpost fp32 [M, n];  term [M, Rb*16] of the carrier's type or NULL
  *   active / n_clusters  as mortar_spmm_bf16_masked (NULL: no input mask)

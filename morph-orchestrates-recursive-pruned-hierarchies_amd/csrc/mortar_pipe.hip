@@ -1,4 +1,5 @@
-// Calls of 65 to some hundred rows on a matrix of several K segments: 16-token tiles, the segments through two LDS buffers.
+// Calls of 65 to some hundred rows on a matrix of several K segments, and decode calls of wide `down` matrices (mortar_smallm_pipe), also with
+// the POST write: 16-token tiles, the segments through two LDS buffers.
 //
 // The K-segmented kernel stages a segment behind a barrier pair and its small tiles then wait for their first weight batch: with the few
 // workgroups that some hundred rows make, every segment paid both round trips (`down` of d_model 2048 at 200 rows: 11 us, of which the
@@ -137,9 +138,9 @@ __global__ void __launch_bounds__(PIPE_WAVES * 64) mortar_pipe_kernel(const Spmm
 #pragma unroll
             for (int w = 1; w < CS; ++w) s[a][0] += red[(wave + a * CS + w) * 64 + lane];
         }
-        mortar_store_tile<1, NACC, CODE, false>(p, unit, m0, tk, PIPE_MT, n, g, has_gates, s[0], s[NACC - 1]);
+        mortar_store_tile<1, NACC, CODE, NACC == 1>(p, unit, m0, tk, PIPE_MT, n, g, has_gates, s[0], s[NACC - 1]);
     } else if (unit >= 0) {
-        mortar_store_tile<1, NACC, CODE, false>(p, unit, m0, tk, PIPE_MT, n, g, has_gates, acc[0], acc[RW - 1]);
+        mortar_store_tile<1, NACC, CODE, NACC == 1>(p, unit, m0, tk, PIPE_MT, n, g, has_gates, acc[0], acc[RW - 1]);
     }
 }
 

@@ -186,6 +186,15 @@ int dispatch_prefill(int kind, SpmmParams &p, hipStream_t st) {
     }
 }
 
+// The two-buffer kernel of mortar_pipe.hip on the 4-bit stream where the matrix has one; -1 (nothing launched, p as it was) where it has no form.
+int try_pipe(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
+    const u32x4_t *two_bit = p.codes_o;
+    if (W->codes4_o) p.codes_o = reinterpret_cast<const u32x4_t *>(W->codes4_o);
+    const int rc = mortar_pipe_launch(kind, !W->codes4_o ? CODE_2BIT : p.uscale != 0.f ? CODE_4BIT | CODE_UNIFORM : CODE_4BIT, p, st);
+    if (rc < 0) p.codes_o = two_bit;
+    return rc;
+}
+
 // kind: 0 spmm, 1 gate_up + SwiGLU, 2 routed gate_up + SwiGLU, 3 spmm with an input mask.
 // Prefill-sized launches read the 4-bit code stream when the matrix carries one (cheaper unpack: one conversion
 // per register instead of shift + mask); decode-sized launches always stream the 2-bit codes (half the bytes).
@@ -195,11 +204,8 @@ int dispatch(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
     // products over several K segments have small-tile forms beyond the decode sizes as well (the launcher returns -1
     // once they would need more than one round of workgroups)
     if ((p.M > MORTAR_SMALLM_MAX || mortar_smallm_pipe(kind, p)) && p.nseg > 1) {
-        const u32x4_t *two_bit = p.codes_o;
-        if (W->codes4_o) p.codes_o = reinterpret_cast<const u32x4_t *>(W->codes4_o);
-        const int rc = mortar_pipe_launch(kind, !W->codes4_o ? CODE_2BIT : p.uscale != 0.f ? CODE_4BIT | CODE_UNIFORM : CODE_4BIT, p, st);
+        const int rc = try_pipe(kind, p, W, st);
         if (rc >= 0) return rc;
-        p.codes_o = two_bit;
     }
     if (p.M <= MORTAR_SMALLM_MAX || ((kind == 0 || kind == 1 || kind == 3) && p.nseg > 1)) {
         const int rc = mortar_smallm_launch(kind, p, nullptr, 1, st);
@@ -303,7 +309,8 @@ extern "C" int mortar_spmm_hc_post(const mortar_bcsr_t *W, const int32_t *sched,
         p.active = active; p.n_clusters = n_clusters; p.cluster_size = (W->Cb * 16) / n_clusters;
         kind = 3;
     }
-    rc = mortar_smallm_launch(kind, p, nullptr, 1, static_cast<hipStream_t>(stream));
+    rc = mortar_smallm_pipe(kind, p) ? try_pipe(kind, p, W, static_cast<hipStream_t>(stream)) : -1;      // as dispatch does: y has the bits of mortar_spmm_bf16
+    if (rc < 0) rc = mortar_smallm_launch(kind, p, nullptr, 1, static_cast<hipStream_t>(stream));
     if (rc < 0 && rc != MORTAR_ERR_HIP) return mortar_fail(MORTAR_ERR_LIMIT, "spmm_hc_post: shape has no small-tile kernel");
     return rc;
 }

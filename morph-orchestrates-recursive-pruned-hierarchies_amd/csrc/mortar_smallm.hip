@@ -311,7 +311,7 @@ static int smallm_norm_wide(SpmmParams &p, hipStream_t st) {
 // 33 to 64 rows, MLP with its gate_up: 36.2..37.8 -> 28.1..29.7 us at 25 %, 25.4..26.0 -> 22.0..24.4 at 12.5 %).  Where part-split tiles fit they
 // stay the better ones ([3072, 8192], 48 rows: 17.8 against 18.4, 14.5 against 16.9).
 bool mortar_smallm_pipe(int kind, const SpmmParams &p) {
-    return (kind == 0 || kind == 3) && p.M > 16 && p.M <= MORTAR_SMALLM_MAX && p.nseg > 1 && !p.hc_h && !fits(8, p.Cb) &&
+    return (kind == 0 || kind == 3) && p.M > 16 && p.M <= MORTAR_SMALLM_MAX && p.nseg > 1 && !fits(8, p.Cb) &&
            (p.M + 3) / 4 * (int64_t)((p.n_units + 3) / 4) > 512 && pick_waves(-16, p, 1) == 2;
 }
 

@@ -72,3 +72,29 @@ def test_down_of_a_wide_model(dev, M, masked):
     ops.spmm(to_dev(x, dev), W, out=buf[:M], **({"active": active} if masked else {}))
     assert torch.isnan(buf[M].float()).all()
     assert_close_bf16(to_np(buf[:M]), oracle_spmm(x, m), "down")
+
+
+# K beyond an 8-token tile of all of it: 4-token tiles and, from more of them than are worth it, the two-buffer kernel
+@pytest.mark.parametrize("Rb,M", [(256, 16), (256, 32), (256, 33), (256, 64), (320, 25), (520, 17)])
+@pytest.mark.parametrize("one_scale", [False, True])
+@pytest.mark.parametrize("masked", [False, True])
+def test_post_write_of_a_wide_down_has_the_bits_of_the_product(dev, Rb, M, one_scale, masked):
+    m = synth.synth_matrix(16 * Rb, 16 * 620, 0.05, seed=Rb + M, zipf_s=1.2)
+    if one_scale:
+        m["scales"][:] = m["scales"][0]
+    W = synth.to_pack(m, dev)
+    x = to_dev(synth.synth_x(M, 9920, seed=M), dev)
+    g = torch.Generator(device=dev).manual_seed(M)
+    kw = {"active": (torch.rand(M, 155, device=dev, generator=g) < 0.4).to(torch.uint8)} if masked else {}
+    y = ops.spmm(x, W, **kw).float()
+    for n, dt in ((1, torch.bfloat16), (4, torch.float32)):
+        h = torch.randn(M, n, 16 * Rb, device=dev, generator=g).to(dt)
+        one, zero = torch.ones(M, n, device=dev), torch.zeros(M, n, n, device=dev)
+        out = ops.spmm_hc_post(x, W, h, zero, one, **kw)
+        assert torch.equal(out.float(), y[:, None, :].expand(M, n, 16 * Rb))
+        res, post = torch.randn(M, n, n, device=dev, generator=g), torch.randn(M, n, device=dev, generator=g)
+        got = ops.spmm_hc_post(x, W, h, res, post, h[:, 0].contiguous(), **kw).double()
+        terms = (res.double()[..., None] * h.double()[:, None]).sum(2), post.double()[..., None] * y.double()[:, None], h.double()[:, :1]
+        size = (res.double().abs()[..., None] * h.double().abs()[:, None]).sum(2) + terms[1].abs() + terms[2].abs()
+        # six roundings to fp32 of sums no larger than `size`, and the one of the result
+        assert ((got - sum(terms)).abs() <= size * 6 * 2.0 ** -24 + got.abs() * (2.0 ** -8 if dt == torch.bfloat16 else 0.0)).all()
