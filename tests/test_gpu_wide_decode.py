@@ -79,13 +79,13 @@ def test_down_of_a_wide_model(dev, M, masked):
 @pytest.mark.parametrize("one_scale", [False, True])
 @pytest.mark.parametrize("masked", [False, True])
 def test_post_write_of_a_wide_down_has_the_bits_of_the_product(dev, Rb, M, one_scale, masked):
-    m = synth.synth_matrix(16 * Rb, 16 * 620, 0.05, seed=Rb + M, zipf_s=1.2)
+    m = synth.synth_matrix(16 * Rb, 16 * 688, 0.25, seed=Rb + M, zipf_s=1.2)      # rows long enough for another order of additions to show
     if one_scale:
         m["scales"][:] = m["scales"][0]
     W = synth.to_pack(m, dev)
-    x = to_dev(synth.synth_x(M, 9920, seed=M), dev)
+    x = to_dev(synth.synth_x(M, 11008, seed=M), dev)
     g = torch.Generator(device=dev).manual_seed(M)
-    kw = {"active": (torch.rand(M, 155, device=dev, generator=g) < 0.4).to(torch.uint8)} if masked else {}
+    kw = {"active": (torch.rand(M, 172, device=dev, generator=g) < 0.4).to(torch.uint8)} if masked else {}
     y = ops.spmm(x, W, **kw).float()
     for n, dt in ((1, torch.bfloat16), (4, torch.float32)):
         h = torch.randn(M, n, 16 * Rb, device=dev, generator=g).to(dt)
