@@ -69,8 +69,8 @@ __device__ __forceinline__ float bf16r(float f) { return __builtin_bit_cast(floa
 #define MORTAR_GLOBAL __attribute__((address_space(1)))
 
 // Asynchronous 16-byte-per-lane copy global -> LDS (lane l's bytes land at lds_base + 16 * l): no registers, no
-// address arithmetic beyond the source pointer.  The caller waits with s_waitcnt vmcnt(0) and a barrier before the
-// destination is read.  (One wait state separates the write of M0 from its use as the LDS base.)
+// address arithmetic beyond the source pointer.  The caller waits for the copies and at a barrier before the
+// destination is read: with s_waitcnt vmcnt(0), or with the number of vector loads that are certain to have been issued behind the last copy.  (One wait state separates the write of M0 from its use as the LDS base.)
 __device__ __forceinline__ void mortar_load_to_lds(const MORTAR_GLOBAL char *gsrc, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_base), "v"(gsrc) : "memory", "m0");
 }

@@ -64,7 +64,9 @@ struct ValBatch {
     u32x4_t A[4];
     int col;
 };
-constexpr int VAL_LOADS = 5;                          // load instructions of a batch
+// Load instructions of a batch.  values_resident_kernel counts on them: val_fetch issues every one of them, whatever the batch holds, and whoever makes
+// it leave one out lowers this (tests/test_isa_waits.py counts them in the compiled kernels).
+constexpr int VAL_LOADS = sizeof(ValBatch::A) / 16 + 1;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t val_rsrc(const void *base, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);
