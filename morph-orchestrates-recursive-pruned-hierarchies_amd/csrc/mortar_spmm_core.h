@@ -235,7 +235,7 @@ __device__ __forceinline__ void mortar_row_part(const SpmmView &p, const uint4 *
                                                 int nb, uint32_t xo_base, const uint32_t (&tk)[MSUB], int nsub, int n,
                                                 int bsel, int hsel, f32x4_t (&acc)[MSUB]) {
     const unsigned char *lb = reinterpret_cast<const unsigned char *>(lx);
-    // SW: `xo` is the LDS address itself (the tile is at 0, these kernels have no other LDS): with a base to be added the exclusive or becomes a
+    // SW: `xo` is the LDS address itself (the tile is at 0, mortar_allow_big_lds sees to it): with a base to be added the exclusive or becomes a
     // three-operand instruction, which takes no DPP operand.
     auto operand = [&](uint32_t xo, int ms) {
         if constexpr (SW) {
@@ -704,7 +704,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
             const int unit = __builtin_amdgcn_readfirstlane((int)d0[3]);
             int cnt = MT;
             uint32_t tk[MSUB];
-    #pragma unroll
+#pragma unroll
             for (int ms = 0; ms < MSUB; ++ms) tk[ms] = ms * 16 + n;
             bool skip = false;
             if (ROUTED) {
@@ -712,7 +712,7 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
                 const int64_t e = (int64_t)mt * p.n_clusters + cl;
                 cnt = __builtin_amdgcn_readfirstlane(p.tok_cnt[e]);
                 skip = cnt == 0;
-    #pragma unroll
+#pragma unroll
                 for (int ms = 0; ms < MSUB; ++ms) {
                     const int i = ms * 16 + n;
                     tk[ms] = i < cnt ? p.tok_list[e * MT + i] : 0;
@@ -720,14 +720,14 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
             }
             const int nsub = ROUTED ? (cnt + 15) >> 4 : MSUB;
             f32x4_t acc[NACC][MSUB];
-    #pragma unroll
+#pragma unroll
             for (int a = 0; a < NACC; ++a)
-    #pragma unroll
+#pragma unroll
                 for (int ms = 0; ms < MSUB; ++ms) acc[a][ms] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
             for (int sg = 0; sg < p.nseg; ++sg) {
                 const uint32_t xo_base = lane_xo + (uint32_t)(sg * p.seg_cb) * (uint32_t)(MT * 32);
-    #pragma unroll
+#pragma unroll
                 for (int a = 0; a < NACC; ++a) {
                     const bool last_part = sg + 1 == p.nseg && a + 1 == NACC;
                     if (last_part) npos = base + (int)__builtin_amdgcn_readfirstlane(drawn);
@@ -748,7 +748,8 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
 
             mortar_store_tile<MSUB, NACC, CODE, (MT <= 16 && NACC == 1 && !TABLE), YT>(p, unit, m0, tk, ROUTED ? cnt : MT, n, g, has_gates,
                                                                                        acc[0], acc[NACC - 1]);
-        }        left -= u_end - base;
+        }
+        left -= u_end - base;
         if (!RUNS || left <= 0) break;
         ++mt;
         base = 0;
@@ -1073,11 +1074,16 @@ __global__ void __launch_bounds__(PW * UW * 64) mortar_partsplit_kernel(const Sp
 // `layers` > 1 launches the table variant: `table` points at `layers` SpmmParams in device memory whose
 // n_mtiles / n_split fields were filled from the same shape as `p`.
 
+// Once per kernel.  A kernel that comes here has no LDS but the dynamic part, which then starts at address 0: the launch rules count on all of the
+// 160 KB, and mortar_row_part (SW) forms its operand addresses from 0.
 template <typename K>
 inline int mortar_allow_big_lds(K kern, bool &done) {
     if (!done) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        hipFuncAttributes a;
+        hipError_t e = hipFuncGetAttributes(&a, reinterpret_cast<const void *>(kern));
+        if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "hipFuncGetAttributes: %s", hipGetErrorString(e));
+        if (a.sharedSizeBytes != 0) return mortar_fail(MORTAR_ERR_LIMIT, "kernel with %zu bytes of static LDS beside its tile", a.sharedSizeBytes);
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return mortar_fail(MORTAR_ERR_HIP, "hipFuncSetAttribute: %s", hipGetErrorString(e));
         done = true;
     }
