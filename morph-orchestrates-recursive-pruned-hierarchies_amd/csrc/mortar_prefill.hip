@@ -96,12 +96,12 @@ struct SegShape { int upw, span; };
 
 // Fewer units per wave mean more workgroups per token tile (64 units per workgroup left 8 workgroups for 128 tokens), but every
 // workgroup stages the tile's segments again, and workgroups beyond the 256 CUs wait for a second round: the choice with the least
-// rounds x (staging + units).  In between, runs of equal length for 256 workgroups (up to run_upw units per wave, mortar_seg_runs):
-// the slowest one's units and stagings.  `down` of d_model 2048: 4500 rows (282 workgroups of four units per wave) 65 -> 52 us, 9000 112 ->
-// 101, 2500 (three units per wave, new with the runs) 33.5 -> 28; [2048, 11264] at 5000 rows 133 -> 104; 4096 and 8192 rows, whole
-// rounds as they were, unchanged.
-template <int N>
-SegShape seg_shape(const SpmmParams &p, const int (&upws)[N], int stage, int unit, int run_upw) {
+// rounds x (staging + units).  In between, runs of equal length for 256 workgroups: the slowest one's units and stagings, with RUN_UPW units
+// per wave (mortar_run_upw, 0: no runs; fewer would only add stagings).  `down` of d_model 2048: 4500 rows (282 workgroups of four units per
+// wave) 65 -> 52 us, 9000 112 -> 101, 2500 (three units per wave, new with the runs) 33.5 -> 28; [2048, 11264] at 5000 rows 133 -> 104; 4096 and
+// 8192 rows, whole rounds as they were, unchanged.
+template <int RUN_UPW, int N>
+SegShape seg_shape(const SpmmParams &p, const int (&upws)[N], int stage, int unit) {
     const int64_t tiles = (p.M + 31) / 32, rows = (p.n_units + SEG_WAVES - 1) / SEG_WAVES, all = tiles * rows;
     SegShape best{upws[0], 0};
     int64_t best_cost = INT64_MAX;
@@ -109,35 +109,31 @@ SegShape seg_shape(const SpmmParams &p, const int (&upws)[N], int stage, int uni
         const int64_t wgs = tiles * ((rows + upw - 1) / upw), cost = (wgs + 255) / 256 * (stage + unit * upw);
         if (cost < best_cost) { best = SegShape{upw, 0}; best_cost = cost; }
     }
-    if (all >= 0x7fffffff) return best;
-    const int64_t span = (all + 255) / 256;
-    for (int upw : upws) {
-        if (upw > run_upw) continue;
+    if constexpr (RUN_UPW > 0) {
+        if (all >= 0x7fffffff) return best;
+        const uint32_t span = (uint32_t)((all + 255) / 256), n = (uint32_t)rows;
+        auto groups_of = [](uint32_t len) { return (int64_t)((len + RUN_UPW - 1) / RUN_UPW); };
         int64_t groups = 0;                                           // of the workgroup that has most of them
-        for (int64_t w = 0; w < rows && w * span < all; ++w) {        // where the runs start repeats after at most `rows` of them
-            int64_t at = w * span % rows, left = span, n = 0;
-            while (left > 0) {
-                const int64_t len = rows - at < left ? rows - at : left;
-                n += (len + upw - 1) / upw;
-                left -= len;
-                at = 0;
-            }
-            groups = n > groups ? n : groups;
+        uint32_t at = 0;
+        for (uint32_t w = 0; w < n && (int64_t)w * span < all; ++w) { // where the runs start repeats after at most n of them
+            const uint32_t first = n - at < span ? n - at : span, rest = span - first;
+            const int64_t g = groups_of(first) + (int64_t)(rest / n) * groups_of(n) + groups_of(rest % n);
+            groups = g > groups ? g : groups;
+            at = (at + span % n) % n;
         }
-        const int64_t cost = unit * span + stage * groups;
-        if (cost * 21 < best_cost * 20) { best = SegShape{upw, (int)span}; best_cost = cost; }
+        if ((unit * (int64_t)span + stage * groups) * 21 < best_cost * 20) best = SegShape{RUN_UPW, (int)span};
     }
     return best;
 }
 
 // The plain product: staging weighs about three units.
 template <bool MASKED, bool TL>
-SegShape segmented_shape(const SpmmParams &p) { return seg_shape(p, {4, 3, 2, 1}, 3, 1, MASKED ? 0 : TL ? 4 : 3); }
+SegShape segmented_shape(const SpmmParams &p) { return seg_shape<mortar_run_upw<32, 1, MASKED, false, TL>()>(p, {4, 3, 2, 1}, 3, 1); }
 
 // gate_up: 1, 2 or 3 unit pairs per wave (four spill).  A unit pair takes about 6.7 us and staging the segments 5 us (d_model 3072 and
 // 4096).  With two units per wave throughout, 400 rows of d_model 4096 were 286 workgroups: 83 -> 70 us for the MLP; 150
-// rows 52 -> 44; d_model 3072 at 200 rows 40.9 -> 34.6, at 600 64 -> 52.5.  Runs with up to two: d_model 4096 at 1300 rows 164 -> 154.
-SegShape gateup_shape(const SpmmParams &p) { return seg_shape(p, {2, 3, 1}, 3, 4, 2); }
+// rows 52 -> 44; d_model 3072 at 200 rows 40.9 -> 34.6, at 600 64 -> 52.5.  Runs: d_model 4096 at 1300 rows 164 -> 154.
+SegShape gateup_shape(const SpmmParams &p) { return seg_shape<mortar_run_upw<32, 2, false, false, false>()>(p, {2, 3, 1}, 3, 4); }
 
 template <bool MASKED, int CODE, bool TL = false>
 int launch_segmented_plain(SpmmParams &p, hipStream_t st) {

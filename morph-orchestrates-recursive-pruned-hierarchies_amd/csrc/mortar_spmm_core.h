@@ -769,10 +769,12 @@ __global__ void __launch_bounds__(WAVES * 64) mortar_resident_kernel(const SpmmP
 // 98 -> 96.
 template <int MT, int NACC, bool MASKED, int UPW, bool TABLE, bool XT>
 constexpr bool mortar_seg_pairs() { return MT == 32 && !MASKED && !XT && !TABLE; }
-// Whether it has a form that walks runs (RUNS, SpmmParams::span): where the loop around the sums does not spill.  (gate_up with three units per wave:
-// 40 registers, 162 -> 221 us.)
-template <int MT, int NACC, bool MASKED, int UPW, bool TABLE, bool XT>
-constexpr bool mortar_seg_runs() { return MT >= 32 && !TABLE && !MASKED && UPW * NACC <= (NACC == 1 && !XT ? 3 : 4); }
+// Units per wave of the form that walks runs (RUNS, SpmmParams::span), 0: none.  Fewer than these only add stagings.  One more, us: gate_up of d_model 3072 and
+// 4096 with three spills 24 registers from tile-ordered per-block codes and with one scale (4096, 1700 rows 119 -> 149; MLP 207 -> 225, 3000 rows 346 -> 377)
+// and none row-major with a scale per block (1700 rows 136 -> 141, 1100 rows 87.5 against 91.5 without, 5000 371 -> 386).  The plain product with
+// four from row-major activations spills none and is as often slower as faster ([2048, 5632] 4500 rows 52.6 -> 54.3, 5000 53.6 -> 56.5, 6000 69.6 -> 63.7, 9000 107 -> 97).
+template <int MT, int NACC, bool MASKED, bool TABLE, bool XT>
+constexpr int mortar_run_upw() { return MT != 32 || TABLE || MASKED ? 0 : NACC == 2 ? 2 : XT ? 4 : 3; }
 
 template <int MT, int NACC, bool MASKED, int WAVES, int UPW, bool TABLE, int CODE, bool TL = false, bool RUNS = false>
 __global__ void __launch_bounds__(WAVES * 64) mortar_segmented_kernel(const SpmmParams p0, const SpmmParams *table) {
@@ -1202,7 +1204,7 @@ int mortar_launch_segmented(SpmmParams &p, const SpmmParams *table, int layers, 
     const int64_t grid = mortar_segmented_shape<MT, WAVES, UPW>(p, layers);
     if ((rc = mortar_launch_check(grid, layers))) return rc;
     if (p.span > 0) {
-        if constexpr (mortar_seg_runs<MT, NACC, MASKED, UPW, TABLE, TL && NACC == 1>()) {
+        if constexpr (UPW == mortar_run_upw<MT, NACC, MASKED, TABLE, TL && NACC == 1>()) {
             static bool runs_done = false;
             auto runs = mortar_segmented_kernel<MT, NACC, MASKED, WAVES, UPW, TABLE, CODE, TL, true>;
             if ((rc = mortar_allow_big_lds(runs, runs_done))) return rc;
