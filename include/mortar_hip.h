@@ -139,6 +139,12 @@ int mortar_transpose_topology_host(const int32_t *row_ptr, const int16_t *col, i
 /* Largest K segment (in block-columns) whose 32-token activation tile fits in LDS; a matrix with
  * Cb <= this runs the single-segment prefill kernel.  Use seg_cb = ceil(Cb / ceil(Cb / max)). */
 int mortar_prefill_max_seg_cb(void);
+/* Launch form that the prefill-sized kernels take for M rows (host only, nothing is launched; calls that the small tiles serve are not looked
+ * at).  kind 0: plain product of n_units block-rows, 1: gate_up of n_units gate/up pairs, 3: plain product with an input mask.  tiled: `down` of
+ * mortar_mlp_bf16 reading the hidden activations in tile order.  *upw_out: units per wave of a K-segmented launch, 0 for a tile of all K.
+ * *span_out: units (K-segmented: rows of one unit per wave) of the runs over all token tiles that the workgroups take, 0: whole groups of one tile. */
+int mortar_prefill_form_host(int32_t kind, int64_t M, int32_t n_units, int32_t Cb, int32_t seg_cb, int32_t tiled, int32_t *upw_out,
+                             int32_t *span_out);
 
 /* Largest K segment whose 4-token (rows <= 4) or 16-token (rows <= 16) tile fits in LDS.  A second stream of a matrix laid
  * out with segments that wide (same codes; fewer, longer row parts, so less padding to octets and fewer barrier pairs:

@@ -221,6 +221,29 @@ int dispatch(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
 
 }  // namespace
 
+extern "C" int mortar_prefill_form_host(int32_t kind, int64_t M, int32_t n_units, int32_t Cb, int32_t seg_cb, int32_t tiled, int32_t *upw_out,
+                                        int32_t *span_out) {
+    if ((kind != 0 && kind != 1 && kind != 3) || M <= 0 || M > (1 << 30) || n_units <= 0 || Cb <= 0 || seg_cb <= 0 || !upw_out || !span_out)
+        return mortar_fail(MORTAR_ERR_ARG, "prefill_form: bad argument");
+    SpmmParams p = SpmmParams{};
+    p.M = (int)M; p.n_units = n_units; p.Cb = Cb; p.seg_cb = seg_cb < Cb ? seg_cb : Cb;
+    p.nseg = (Cb + p.seg_cb - 1) / p.seg_cb;
+    if (p.nseg == 1 && kind != 3) {
+        const int mt = kind == 0 && tiled ? 32 : resident_mt(Cb);
+        if (mt == 0) return mortar_fail(MORTAR_ERR_LIMIT, "prefill_form: a row of %d block-columns fits no tile", Cb);
+        if (mt == 64) mortar_resident_shape<64, 16>(p, 1, true);
+        else mortar_resident_shape<32, 16>(p, 1, true);
+        *upw_out = 0;
+        *span_out = p.span;
+        return MORTAR_OK;
+    }
+    const SegShape f = kind == 1 ? gateup_shape(p) : kind == 3 ? segmented_shape<true, false>(p) : tiled ? segmented_shape<false, true>(p)
+                                                                                                         : segmented_shape<false, false>(p);
+    *upw_out = f.upw;
+    *span_out = f.span;
+    return MORTAR_OK;
+}
+
 extern "C" int mortar_prefill_max_seg_cb(void) { return (LDS_BUDGET - LDS_PAD * 16) / (32 * 32); }
 extern "C" int mortar_decode_max_seg_cb(int32_t rows) {
     return (LDS_BUDGET - LDS_PAD * 16) / ((rows <= 4 ? 4 : rows <= 16 ? 16 : 32) * 32);

@@ -12,6 +12,7 @@ import torch
 import mortar_amd
 from mortar_amd import _lib, pack as P, synth
 from oracle import mortar_oracle as O
+from util import prefill_form
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -48,6 +49,33 @@ def test_encode_round_trip_and_bit_layout():
         prod = (half.astype(np.float32) * np.float32(sign)).astype(np.float16).view(np.uint16)
         want = O.bf16_bits(scale) | (0x8000 if sign < 0 else 0)
         assert np.array_equal(prod, want)
+
+
+@pytest.mark.parametrize("kind,tiled,upws,run,stage,unit", [(0, False, (4, 3, 2, 1), 3, 3, 1), (0, True, (4, 3, 2, 1), 4, 3, 1), (3, False, (4, 3, 2, 1), 0, 3, 1),
+                                                            (1, False, (2, 3, 1), 2, 3, 4)])
+def test_form_of_a_k_segmented_prefill(kind, tiled, upws, run, stage, unit):
+    """The rule against a walk over every workgroup: rounds of whole groups, or runs for 256 workgroups where the slowest of them is 5 % faster."""
+    rng = np.random.default_rng(kind + 10 * tiled)
+    runs = 0
+    for _ in range(400):
+        M, n_units = int(rng.integers(1, 12000)), int(rng.integers(1, 1200))
+        tiles, rows = -(-M // 32), -(-n_units // 16)
+        cost, upw = min((-(-(tiles * -(-rows // u)) // 256) * (stage + unit * u), i, u) for i, u in enumerate(upws))[::2]
+        want = (upw, 0)
+        if run:
+            span = -(-(tiles * rows) // 256)
+            slowest = 0
+            for first in range(0, tiles * rows, span):
+                cuts = [first, *range((first // rows + 1) * rows, min(first + span, tiles * rows), rows), min(first + span, tiles * rows)]
+                if first + span > tiles * rows:
+                    continue                                   # the last run is shorter than the others
+                slowest = max(slowest, sum(-(-(b - a) // run) for a, b in zip(cuts, cuts[1:])))
+            if slowest and (unit * span + stage * slowest) * 21 < cost * 20:
+                want, runs = (run, span), runs + 1
+        got = prefill_form(kind, M, n_units, 200, tiled)
+        assert got == want, (M, n_units)
+    assert run == 0 or runs > 5
+    assert prefill_form(kind, 1 << 30, 1200, 200, tiled)[1] == 0        # more rows of units than 31 bits
 
 
 def test_uniform_scale_is_detected():

@@ -1,7 +1,10 @@
 """Shared helpers for the parity tests."""
+import ctypes as C
+
 import numpy as np
 import torch
 
+from mortar_amd import _lib
 from oracle import mortar_oracle as O
 
 
@@ -29,3 +32,10 @@ def assert_close_bf16(got: np.ndarray, ref: np.ndarray, what: str = "", ulps: fl
 
 def oracle_spmm(x, m):
     return O.bcsr_spmm(x, m["codes"], m["scales"], m["col_idx"], m["offsets"])
+
+
+def prefill_form(kind, M, n_units, Cb, tiled=False):
+    """(units per wave, 0 for a tile of all K; length of the runs, 0 for whole groups) of a prefill-sized launch: kind 0 plain, 1 gate_up, 3 masked."""
+    L, upw, span = _lib.lib(), C.c_int32(), C.c_int32()
+    _lib.check(L.mortar_prefill_form_host(kind, M, n_units, Cb, L.mortar_prefill_max_seg_cb(), int(tiled), C.byref(upw), C.byref(span)), "prefill_form")
+    return upw.value, span.value
