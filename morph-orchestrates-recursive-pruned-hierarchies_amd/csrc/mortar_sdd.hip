@@ -268,7 +268,9 @@ __global__ __launch_bounds__(256) void sdd_round_kernel(const float *acc, uint16
 // Workgroups of a plan with `nb` blocks per wavefront: per K segment, runs of consecutive block-rows holding at most
 // 16 * nb blocks of the segment and at most SDD_RMAX rows.  A run is staged from a multiple of four block-rows, so that a copied 128-byte
 // piece of a is a line and not parts of two (dW of 4096 x 768, 16384 tokens 70.5 -> 68.2 us, at density 0.5 and 8192 63.6 -> 61.8; 2048 x 5632,
-// 4096 tokens 66.4 -> 65.1).
+// 4096 tokens 66.4 -> 65.1) - unless the rows of a are no whole lines ([5328, 1600], 6000 tokens at 12.5 % 48.6 -> 51.5) or the rows staged in
+// addition make it many more runs: 53 for 51 of [8192, 1536], power-law rows of 12.5 %, 6000 tokens 70 -> 79, 68 for 66 of [11264, 2048] at 5 %, 2048 tokens
+// 36.6 -> 33.5; the line is one in 32.
 struct SddGroup { int row0, nrows, seg, blocks; std::vector<int32_t> j, o; };
 
 static bool sdd_nb_built(int nb) {
@@ -281,10 +283,11 @@ static void sdd_segments(int Cb, int &nseg, int &seg_cb) {
     seg_cb = ((Cb + nseg - 1) / nseg + 3) & ~3;                    // whole 128-byte lines
 }
 
-static void sdd_groups(const int32_t *row_ptr, const int16_t *col, int Rb, int Cb, int nb, bool fill,
-                       std::vector<SddGroup> &wgs, int &nseg, int &seg_cb) {
+static void sdd_groups_from(const int32_t *row_ptr, const int16_t *col, int Rb, int Cb, int nb, bool fill, bool lines,
+                            std::vector<SddGroup> &wgs, int &nseg, int &seg_cb) {
     const int G = SDD_WAVES * nb;
     sdd_segments(Cb, nseg, seg_cb);
+    wgs.clear();
     for (int sg = 0; sg < nseg; ++sg) {
         SddGroup cur{0, 0, sg, 0, {}, {}};
         int held = 0;
@@ -302,7 +305,7 @@ static void sdd_groups(const int32_t *row_ptr, const int16_t *col, int Rb, int C
             if (hi == lo) continue;
             const int slots = (hi - lo + 1) & ~1;              // pairs of slots share a block-row
             if (held && (held + slots > G || r - cur.row0 + 1 > SDD_RMAX)) flush();
-            if (!held) cur.row0 = r & ~3;                      // whole lines of a
+            if (!held) cur.row0 = lines ? r & ~3 : r;
             cur.nrows = r - cur.row0 + 1;
             cur.blocks += hi - lo;
             held += slots;
@@ -319,6 +322,18 @@ static void sdd_groups(const int32_t *row_ptr, const int16_t *col, int Rb, int C
         }
         flush();
     }
+}
+
+static void sdd_groups(const int32_t *row_ptr, const int16_t *col, int Rb, int Cb, int nb, bool fill,
+                       std::vector<SddGroup> &wgs, int &nseg, int &seg_cb) {
+    sdd_groups_from(row_ptr, col, Rb, Cb, nb, false, false, wgs, nseg, seg_cb);
+    const size_t fewest = wgs.size();
+    bool lines = Rb % 4 == 0;
+    if (lines) {
+        sdd_groups_from(row_ptr, col, Rb, Cb, nb, false, true, wgs, nseg, seg_cb);
+        lines = wgs.size() * 32 <= fewest * 33;
+    }
+    if (fill || (Rb % 4 == 0 && !lines)) sdd_groups_from(row_ptr, col, Rb, Cb, nb, fill, lines, wgs, nseg, seg_cb);
 }
 
 // Token ranges for M tokens over the n_wg workgroups of a plan with nb blocks per wavefront.  One workgroup runs per

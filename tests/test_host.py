@@ -464,6 +464,40 @@ def test_sdd_plan_partitions_the_blocks():
             assert np.array_equal(tile[ej[w] >= 0], col[js] - seg * seg_cb) and (col[js] // seg_cb == seg).all()
 
 
+@pytest.mark.parametrize("Rb,Cb,density,zipf,nb", [(512, 96, 0.125, 1.2, 10), (512, 96, 0.125, 1.2, 8), (333, 100, 0.125, None, 10), (704, 128, 0.25, None, 18),
+                                                   (128, 352, 0.25, None, 16), (704, 128, 0.05, 1.2, 8), (9, 44, 0.5, None, 8)])
+def test_sdd_plan_takes_whole_lines_where_they_are_free(Rb, Cb, density, zipf, nb):
+    """The workgroups of a plan start at a multiple of four block-rows (a 128-byte line of a), but only where the rows of a are whole lines
+    themselves and it takes hardly more workgroups than starting where the blocks do."""
+    m = synth.synth_matrix(16 * Rb, 16 * Cb, density, seed=5, zipf_s=zipf)
+    off, col = m["offsets"], m["col_idx"]
+    n = _lib.lib().mortar_sdd_plan_host(P._vp(off), P._vp(col), Rb, Cb, nb, None, 0)
+    plan = np.empty(n, np.int32)
+    assert _lib.lib().mortar_sdd_plan_host(P._vp(off), P._vp(col), Rb, Cb, nb, P._vp(plan), n) == n
+    n_wg, seg_cb, nseg = plan[:3]
+
+    def first_rows(step):
+        out = []
+        for sg in range(nseg):
+            held, row0 = 0, 0
+            for r in range(Rb):
+                c = col[off[r]:off[r + 1]]
+                slots = (int(((c >= sg * seg_cb) & (c < (sg + 1) * seg_cb)).sum()) + 1) & ~1
+                if not slots:
+                    continue
+                if held and (held + slots > 16 * nb or r - row0 + 1 > 32):
+                    held = 0
+                if not held:
+                    row0 = r - r % step
+                    out.append(row0)
+                held += slots
+        return out
+
+    fewest, lines = first_rows(1), first_rows(4)
+    want = lines if Rb % 4 == 0 and len(lines) * 32 <= len(fewest) * 33 else fewest
+    assert plan[4:4 + 4 * n_wg].reshape(n_wg, 4)[:, 0].tolist() == want
+
+
 def test_sdd_blocks_per_wave_is_a_built_size_and_fills_the_chip():
     """The chosen group size is one of the built kernels; at the headline shapes and 4096 tokens its plan has a count
     of token ranges that puts 200 to 256 workgroups on the 256 CUs (one per CU, one round)."""
