@@ -282,8 +282,8 @@ static int smallm_launch_code(int kind, SpmmParams &p, const SpmmParams *table, 
         if (w == 16) return launch_kind<4, 16, CODE>(kind, true, p, table, layers, st);
         return w == 8 ? launch_kind<4, 8, CODE>(kind, true, p, table, layers, st) : launch_kind<4, 2, CODE>(kind, true, p, table, layers, st);
     }
-    // one matrix whose rows are too wide for an 8-token tile of all K: K-segmented 16-token tiles with 8 waves, which
-    // stage a segment four times faster than 2-wave workgroups (4096 x 11008 at 5..64 rows: 13 against 20 us; 16 waves 15 us)
+    // one matrix whose rows are too wide for an 8-token tile of all K and which neither the narrow tiles nor the two buffers (mortar_smallm_pipe) take:
+    // K-segmented 16-token tiles with 8 waves, which stage a segment four times faster than 2-wave workgroups (4096 x 11008: 13 against 20 us; 16 waves 15 us)
     if (!table && !resident) return launch_kind<16, 8, CODE>(kind, resident, p, table, layers, st);
     if (w == 16) return launch_kind<16, 16, CODE>(kind, resident, p, table, layers, st);
     return w == 8 ? launch_kind<16, 8, CODE>(kind, resident, p, table, layers, st) : launch_kind<16, 2, CODE>(kind, resident, p, table, layers, st);
@@ -306,10 +306,11 @@ static int smallm_norm_wide(SpmmParams &p, hipStream_t st) {
     return w8 <= (partsplit_fits(16, 2, p) ? 256 : 512) ? launch_partsplit<8, CODE>(1, p, st) : -1;
 }
 
-// Plain products whose rows are too wide for an 8-token tile of all K, more rows than the 4-token tiles take (narrow_tiles): the two buffers of
-// mortar_pipe.hip over a chip of workgroups, where the K-segmented 16-token tiles with 8 waves that are left make few of them ([4096, 11008],
-// 33 to 64 rows, MLP with its gate_up: 36.2..37.8 -> 28.1..29.7 us at 25 %, 25.4..26.0 -> 22.0..24.4 at 12.5 %).  Where part-split tiles fit they
-// stay the better ones ([3072, 8192], 48 rows: 17.8 against 18.4, 14.5 against 16.9).
+// Plain products whose rows are too wide for an 8-token tile of all K, with more 4-token tiles than narrow_tiles takes: from 33 rows on 256 block-rows, 25 on
+// 320, 17 on 512.  The two buffers of mortar_pipe.hip over a chip of workgroups, where the K-segmented 16-token tiles with 8 waves that are left
+// make few of them.  us, these -> the two buffers, at 12.5 and 25 %: [4096, 11008], 33 rows 13.4 -> 10.4, 17.0 -> 10.8, 64 rows 13.5 -> 11.1, 17.3 -> 11.4;
+// [5120, 11008], 25 rows 13.4 -> 10.3, 17.1 -> 10.7; [8192, 13824], 17 rows 16.2 -> 12.0, 20.8 -> 13.0.  Where part-split tiles fit they stay the better ones
+// ([3072, 8192], 48 rows: 17.8 against 18.4, 14.5 against 16.9).
 bool mortar_smallm_pipe(int kind, const SpmmParams &p) {
     return (kind == 0 || kind == 3) && p.M > 16 && p.M <= MORTAR_SMALLM_MAX && p.nseg > 1 && !fits(8, p.Cb) &&
            (p.M + 3) / 4 * (int64_t)((p.n_units + 3) / 4) > 512 && pick_waves(-16, p, 1) == 2;

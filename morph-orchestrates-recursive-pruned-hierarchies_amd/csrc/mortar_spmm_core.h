@@ -1250,7 +1250,7 @@ int mortar_launch_partsplit(SpmmParams &p, hipStream_t st) {
 // 2 gate_up + SwiGLU routed, 3 spmm with an input mask.  Returns -1 when the shape has no small-M variant.
 __attribute__((visibility("hidden"))) int mortar_smallm_launch(int kind, SpmmParams &p, const SpmmParams *table,
                                                                int layers, hipStream_t st);
-// A decode call (up to 64 rows) that mortar_pipe_launch serves better.
+// A decode call (17 to 64 rows of a wide `down`) that mortar_pipe_launch serves better.
 __attribute__((visibility("hidden"))) bool mortar_smallm_pipe(int kind, const SpmmParams &p);
 // gate_up with p.norm == NORM_WIDE: the launch that mortar_smallm_launch makes for the same call without the norm, where that is a 4- or 8-token
 // tile of all K (the fused norm then gives the bits of the separate one), MORTAR_NO_KERNEL otherwise.
