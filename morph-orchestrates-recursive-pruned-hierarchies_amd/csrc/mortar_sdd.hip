@@ -283,25 +283,38 @@ static void sdd_segments(int Cb, int &nseg, int &seg_cb) {
     seg_cb = ((Cb + nseg - 1) / nseg + 3) & ~3;                    // whole 128-byte lines
 }
 
-static void sdd_groups_from(const int32_t *row_ptr, const int16_t *col, int Rb, int Cb, int nb, bool fill, bool lines,
-                            std::vector<SddGroup> &wgs, int &nseg, int &seg_cb) {
+// First block of every row in every K segment, [Rb][nseg + 1].
+struct SddRows { int nseg, seg_cb; std::vector<int32_t> at; };
+
+static SddRows sdd_rows(const int32_t *row_ptr, const int16_t *col, int Rb, int Cb) {
+    SddRows t;
+    sdd_segments(Cb, t.nseg, t.seg_cb);
+    t.at.resize((size_t)Rb * (t.nseg + 1));
+    for (int r = 0; r < Rb; ++r) {
+        int32_t *at = &t.at[(size_t)r * (t.nseg + 1)], j = row_ptr[r];
+        const int32_t e = row_ptr[r + 1];
+        for (int sg = 0; sg < t.nseg; ++sg) {
+            at[sg] = j;
+            while (j < e && col[j] < (sg + 1) * t.seg_cb) ++j;
+        }
+        at[t.nseg] = j;
+    }
+    return t;
+}
+
+static void sdd_groups_from(const SddRows &t, const int16_t *col, int Rb, int nb, bool fill, bool lines, std::vector<SddGroup> &wgs) {
     const int G = SDD_WAVES * nb;
-    sdd_segments(Cb, nseg, seg_cb);
     wgs.clear();
-    for (int sg = 0; sg < nseg; ++sg) {
+    for (int sg = 0; sg < t.nseg; ++sg) {
         SddGroup cur{0, 0, sg, 0, {}, {}};
         int held = 0;
         auto flush = [&]() {
-            if (held) wgs.push_back(cur);
+            if (held) wgs.push_back(std::move(cur));
             cur = SddGroup{0, 0, sg, 0, {}, {}};
             held = 0;
         };
         for (int r = 0; r < Rb; ++r) {
-            int lo = row_ptr[r];
-            const int e = row_ptr[r + 1];
-            while (lo < e && col[lo] < sg * seg_cb) ++lo;
-            int hi = lo;
-            while (hi < e && col[hi] < (sg + 1) * seg_cb) ++hi;
+            const int lo = t.at[(size_t)r * (t.nseg + 1) + sg], hi = t.at[(size_t)r * (t.nseg + 1) + sg + 1];
             if (hi == lo) continue;
             const int slots = (hi - lo + 1) & ~1;              // pairs of slots share a block-row
             if (held && (held + slots > G || r - cur.row0 + 1 > SDD_RMAX)) flush();
@@ -312,7 +325,7 @@ static void sdd_groups_from(const int32_t *row_ptr, const int16_t *col, int Rb, 
             if (!fill) continue;
             for (int j = lo; j < hi; ++j) {
                 cur.j.push_back(j);
-                const int cr = col[j] - sg * seg_cb;
+                const int cr = col[j] - sg * t.seg_cb;
                 cur.o.push_back(((r - cur.row0) << 20) | ((cr >> 2) * SDD_QS + (cr & 3) * 32));
             }
             if (slots > hi - lo) {
@@ -324,16 +337,17 @@ static void sdd_groups_from(const int32_t *row_ptr, const int16_t *col, int Rb, 
     }
 }
 
-static void sdd_groups(const int32_t *row_ptr, const int16_t *col, int Rb, int Cb, int nb, bool fill,
-                       std::vector<SddGroup> &wgs, int &nseg, int &seg_cb) {
-    sdd_groups_from(row_ptr, col, Rb, Cb, nb, false, false, wgs, nseg, seg_cb);
-    const size_t fewest = wgs.size();
-    bool lines = Rb % 4 == 0;
-    if (lines) {
-        sdd_groups_from(row_ptr, col, Rb, Cb, nb, false, true, wgs, nseg, seg_cb);
-        lines = wgs.size() * 32 <= fewest * 33;
+static void sdd_groups(const SddRows &t, const int16_t *col, int Rb, int nb, bool fill, std::vector<SddGroup> &wgs) {
+    sdd_groups_from(t, col, Rb, nb, false, false, wgs);
+    bool lines = false;
+    if (Rb % 4 == 0) {
+        const size_t fewest = wgs.size();
+        std::vector<SddGroup> whole;
+        sdd_groups_from(t, col, Rb, nb, false, true, whole);
+        lines = whole.size() * 32 <= fewest * 33;
+        if (lines) wgs = std::move(whole);
     }
-    if (fill || (Rb % 4 == 0 && !lines)) sdd_groups_from(row_ptr, col, Rb, Cb, nb, fill, lines, wgs, nseg, seg_cb);
+    if (fill) sdd_groups_from(t, col, Rb, nb, true, lines, wgs);
 }
 
 // Token ranges for M tokens over the n_wg workgroups of a plan with nb blocks per wavefront.  One workgroup runs per
@@ -371,13 +385,14 @@ extern "C" int32_t mortar_sdd_blocks_per_wave_host(const int32_t *row_ptr, const
     if (M < 0) return mortar_fail(MORTAR_ERR_ARG, "sdd_blocks_per_wave: M < 0");
     int best = SDD_NB_MAX;
     int64_t best_cost = INT64_MAX;
+    const SddRows t = sdd_rows(row_ptr, col, Rb, Cb);
     for (int nb : SDD_NB_SIZES) {
         std::vector<SddGroup> wgs;
-        int nseg, seg_cb, nsteps, sps, tsplit;
-        sdd_groups(row_ptr, col, Rb, Cb, nb, false, wgs, nseg, seg_cb);
+        int nsteps, sps, tsplit;
+        sdd_groups(t, col, Rb, nb, false, wgs);
         int64_t rows = 0;
         for (const SddGroup &g : wgs) rows += g.nrows;
-        const int tiles = seg_cb + (int)(rows / (int64_t)std::max<size_t>(1, wgs.size()));
+        const int tiles = t.seg_cb + (int)(rows / (int64_t)std::max<size_t>(1, wgs.size()));
         const int64_t cost = sdd_split((int32_t)wgs.size(), row_ptr[Rb], nb, M, tiles, nsteps, sps, tsplit);
         if (cost <= best_cost) { best_cost = cost; best = nb; }      // ties: the larger group (fewer staged bytes)
     }
@@ -397,8 +412,9 @@ extern "C" int64_t mortar_sdd_plan_host(const int32_t *row_ptr, const int16_t *c
         return mortar_fail(MORTAR_ERR_ARG, "sdd_plan: blocks_per_wave=%d is not a built size (8, 10, ... 22)", blocks_per_wave);
     const int SDD_G = SDD_WAVES * blocks_per_wave;
     std::vector<SddGroup> wgs;
-    int nseg, seg_cb;
-    sdd_groups(row_ptr, col, Rb, Cb, blocks_per_wave, true, wgs, nseg, seg_cb);
+    const SddRows t = sdd_rows(row_ptr, col, Rb, Cb);
+    const int nseg = t.nseg, seg_cb = t.seg_cb;
+    sdd_groups(t, col, Rb, blocks_per_wave, plan_out != nullptr, wgs);
     const int64_t n_wg = (int64_t)wgs.size();
     const int64_t tab = 4 + n_wg * 4 + n_wg * SDD_G * 2;          // word offset of the per-segment table
     const int64_t words = tab + n_wg;
