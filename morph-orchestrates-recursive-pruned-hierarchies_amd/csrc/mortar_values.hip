@@ -176,8 +176,8 @@ __device__ __forceinline__ int val_idx(const int32_t *p, int i) {
 // All of K in one tile.  The waves draw units of RU consecutive block-rows from a counter, so that rows of any length keep all of them
 // busy; a wave's batches form one stream across rows, requested two ahead of their products, the first two before the tile is waited
 // for.  Narrow K is bound by the results and the values together: 16384 x 768 x 4096 at 25 % (134 MB of results, a fill of which takes
-// 21 us) takes 50 us over rotating buffers, of which stage and store alone are 33, the values alone 21, the products alone 25 (before
-// the non-temporal 128-byte pieces: 59 us).  Wide K is bound by the values from the L2, once per 32 tokens (4096 x 2048 x 11264: 82 us).
+// 21 us) takes 52 us in a training step, 62 where several steps' buffers alternate and nothing of theirs is left in the last-level cache; stage and store
+// alone are 33, the values alone 21, the products alone 25 (before the non-temporal 128-byte pieces: 59 us where these leave 50).  Wide K is bound by the values from the L2, once per 32 tokens (4096 x 2048 x 11264: 82 us).
 template <int MT, int RU, bool NT>
 __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const ValArgs a) {
     constexpr int MSUB = MT / 16;
@@ -274,8 +274,9 @@ __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const V
 // Wider K: segments through two LDS buffers, one barrier each.  Four loader waves copy the next segment while twelve multiply the
 // current one: a wave's loads complete in order, so a wave that did both would wait for the copies (from beyond the L2) at its
 // next weights.  A consumer keeps the accumulators of its UPW block-rows in registers over the segments.  The values (once per
-// 64 tokens from the L2) and the operand reads from LDS bound it.  16384 x 4096 x 768 at 25 %: 58 us over rotating buffers (62 before its
-// results left in 128-byte non-temporal pieces), of which the copies alone are 28, the values alone 28, the products alone 32.  Segments of 24 columns in three buffers took 6 % longer
+// 64 tokens from the L2) and the operand reads from LDS bound it.  16384 x 4096 x 768 at 25 %: 54 us in a training step, 64
+// where several steps' buffers alternate (58 in a loop over its own, 62 before its results left in 128-byte non-temporal pieces); the copies alone are 28,
+// the values alone 28, the products alone 32.  Segments of 24 columns in three buffers took 6 % longer
 // (short parts leave a batch half empty), batches requested two ahead 18 % (registers, moves).
 template <int MT, int UPW, bool NT>
 __global__ void __launch_bounds__((VAL_CW + VAL_LOADERS) * 64) values_segmented_kernel(const ValArgs a) {
