@@ -41,7 +41,8 @@ __device__ __forceinline__ int val_enc(int c) { return (c >> 1) * (MT * 64) + (c
 
 // Copies block-columns [c0, c0 + ncb) of the tile at token m0 into `dst`, as loader `w` of NW.  Tokens past M repeat the last
 // one, a missing second column of the last pair repeats the first: both feed results that are never stored or never read.
-template <int MT, int NW>
+// PACED: at most four copies of a loader are in flight.
+template <int MT, int NW, bool PACED = false>
 __device__ __forceinline__ void val_stage(const ValArgs &a, unsigned char *dst, int m0, int c0, int ncb, int w, int lane) {
     constexpr int TG = MT / 16, PS = NW / TG;              // a loader keeps its 16 tokens and walks over the pairs
     static_assert(NW % TG == 0, "loaders x token groups");
@@ -53,6 +54,7 @@ __device__ __forceinline__ void val_stage(const ValArgs &a, unsigned char *dst, 
     uint32_t d = __builtin_amdgcn_readfirstlane(mortar_lds_addr(dst + (pr * MT + tg * 16) * 64));
     for (; 2 * pr + 1 < ncb; pr += PS) {
         mortar_load_to_lds(src, d);
+        if (PACED) asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
         src += PS * 64;
         d += PS * MT * 64;
     }
@@ -289,10 +291,14 @@ __global__ void __launch_bounds__((VAL_CW + VAL_LOADERS) * 64) values_segmented_
     const int seg = a.seg_cb * a.sub, nseg = (a.Cb + seg - 1) / seg;
     const int buf_bytes = seg / 2 * (MT * 64);
     if (wave >= VAL_CW) {
-        // segment sg is in its buffer at barrier sg; the other buffer was multiplied before that barrier
+        // Segment sg is in its buffer at barrier sg; the other buffer was multiplied before that barrier.  The first segment comes as fast as it can, nobody
+        // multiplies yet; copies of the others, all requested at once, stand in front of the values that the consumers wait for.  us, all at once -> four
+        // of a loader in flight: 16384 x 4096 x 1024 at 12.5 / 25 / 50 % 78.5 -> 73.0, 104 -> 98.7, 145 -> 139, 1024 x 4096 x 768 at 25 % 14.9 -> 14.4; three in flight leave
+        // calls of a few hundred tokens 2 % slower, two 10 %.
         for (int sg = 0; sg <= nseg; ++sg) {
             const int c0 = sg * seg, ncb = a.Cb - c0 < seg ? a.Cb - c0 : seg;
-            if (sg < nseg) val_stage<MT, VAL_LOADERS>(a, smem + (sg & 1) * buf_bytes, m0, c0, ncb, wave - VAL_CW, lane);
+            if (sg == 0) val_stage<MT, VAL_LOADERS>(a, smem, m0, c0, ncb, wave - VAL_CW, lane);
+            else if (sg < nseg) val_stage<MT, VAL_LOADERS, true>(a, smem + (sg & 1) * buf_bytes, m0, c0, ncb, wave - VAL_CW, lane);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
         }
