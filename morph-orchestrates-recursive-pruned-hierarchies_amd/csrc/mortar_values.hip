@@ -276,8 +276,8 @@ __global__ void __launch_bounds__(VAL_WAVES * 64) values_resident_kernel(const V
 // Wider K: segments through two LDS buffers, one barrier each.  Four loader waves copy the next segment while twelve multiply the
 // current one: a wave's loads complete in order, so a wave that did both would wait for the copies (from beyond the L2) at its
 // next weights.  A consumer keeps the accumulators of its UPW block-rows in registers over the segments.  The values (once per
-// 64 tokens from the L2) and the operand reads from LDS bound it.  16384 x 4096 x 768 at 25 %: 54 us in a training step, 64
-// where several steps' buffers alternate (58 in a loop over its own, 62 before its results left in 128-byte non-temporal pieces); the copies alone are 28,
+// 64 tokens from the L2) and the operand reads from LDS bound it.  16384 x 4096 x 768 at 25 %: 52 us in a training step, 61
+// where several steps' buffers alternate (62 in a loop over its own before its results left in 128-byte non-temporal pieces, 56 now); the copies alone are 28,
 // the values alone 28, the products alone 32.  Segments of 24 columns in three buffers took 6 % longer
 // (short parts leave a batch half empty), batches requested two ahead 18 % (registers, moves).
 template <int MT, int UPW, bool NT>
