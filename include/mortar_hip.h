@@ -140,7 +140,8 @@ int mortar_transpose_topology_host(const int32_t *row_ptr, const int16_t *col, i
  * Cb <= this runs the single-segment prefill kernel.  Use seg_cb = ceil(Cb / ceil(Cb / max)). */
 int mortar_prefill_max_seg_cb(void);
 /* Launch form that the prefill-sized kernels take for M rows (host only, nothing is launched; calls that the small tiles serve are not looked
- * at).  kind 0: plain product of n_units block-rows, 1: gate_up of n_units gate/up pairs, 3: plain product with an input mask.  tiled: `down` of
+ * at).  kind 0: plain product of n_units block-rows, 1: gate_up of n_units gate/up pairs, 2: the same with the
+ * RMSNorm in it (one K segment), 3: plain product with an input mask.  tiled: `down` of
  * mortar_mlp_bf16 reading the hidden activations in tile order.  *upw_out: units per wave of a K-segmented launch, 0 for a tile of all K.
  * *span_out: units (K-segmented: rows of one unit per wave) of the runs over all token tiles that the workgroups take, 0: whole groups of one tile. */
 int mortar_prefill_form_host(int32_t kind, int64_t M, int32_t n_units, int32_t Cb, int32_t seg_cb, int32_t tiled, int32_t *upw_out,

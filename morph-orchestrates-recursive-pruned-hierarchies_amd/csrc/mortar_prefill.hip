@@ -223,10 +223,10 @@ int dispatch(int kind, SpmmParams &p, const mortar_bcsr_t *W, hipStream_t st) {
 
 extern "C" int mortar_prefill_form_host(int32_t kind, int64_t M, int32_t n_units, int32_t Cb, int32_t seg_cb, int32_t tiled, int32_t *upw_out,
                                         int32_t *span_out) {
-    if ((kind != 0 && kind != 1 && kind != 3) || M <= 0 || M > (1 << 30) || n_units <= 0 || Cb <= 0 || seg_cb <= 0 || !upw_out || !span_out)
+    if (kind < 0 || kind > 3 || M <= 0 || M > (1 << 30) || n_units <= 0 || Cb <= 0 || seg_cb <= 0 || !upw_out || !span_out)
         return mortar_fail(MORTAR_ERR_ARG, "prefill_form: bad argument");
     SpmmParams p = SpmmParams{};
-    p.M = (int)M; p.n_units = n_units; p.Cb = Cb; p.seg_cb = seg_cb < Cb ? seg_cb : Cb;
+    p.M = (int)M; p.n_units = n_units; p.Cb = Cb; p.seg_cb = seg_cb < Cb ? seg_cb : Cb; p.norm = kind == 2;
     p.nseg = (Cb + p.seg_cb - 1) / p.seg_cb;
     if (p.nseg == 1 && kind != 3) {
         const int mt = kind == 0 && tiled ? 32 : resident_mt(Cb);
@@ -237,6 +237,7 @@ extern "C" int mortar_prefill_form_host(int32_t kind, int64_t M, int32_t n_units
         *span_out = p.span;
         return MORTAR_OK;
     }
+    if (kind == 2) return mortar_fail(MORTAR_ERR_LIMIT, "prefill_form: no norm inside a product over several K segments");
     const SegShape f = kind == 1 ? gateup_shape(p) : kind == 3 ? segmented_shape<true, false>(p) : tiled ? segmented_shape<false, true>(p)
                                                                                                          : segmented_shape<false, false>(p);
     *upw_out = f.upw;

@@ -1146,12 +1146,15 @@ inline int64_t mortar_resident_shape(SpmmParams &p, int layers, bool runs = fals
     // nearly empty round.  A workgroup costs its units and about twelve more, every further tile of a run (staged and multiplied by
     // itself) eighteen.  gate_up of d_model 2048: 4500 rows (141 workgroups of a whole tile each) 101 -> 72 us, 5000 101 -> 77, 6000
     // 102 -> 91, 9000 (282 tiles, two rounds) 211 -> 146, 3000 (188 half tiles) 55 -> 50; 2500 rows, where the rule keeps 237 workgroups
-    // of a third of a tile, 41.5 against 44; d_model 768, 9000 rows 35 -> 27.5, 5000 17.5 against 19.3.
+    // of a third of a tile, 41.5 against 44; d_model 768, 9000 rows 35 -> 27.5, 5000 17.5 against 19.3.  The norm makes every staging about seven units longer:
+    // d_model 1024 with it, 6000 rows, whole groups against runs 36 against 38.7, 5500 38.3 against 39.7, 2048 at 3300 61 against 62.5; 2048 at 3000 64.7 -> 63, 1536 at
+    // 3000 42.6 -> 41.7 (without it 1024 at 6000 32.6 -> 31, 2048 at 3000 58 -> 55).
     if (runs && layers == 1) {
         const int64_t all = (int64_t)p.n_mtiles * p.n_units, span = (all + 255) / 256;
         const int64_t rounds = ((int64_t)p.n_mtiles * split + 255) / 256, per = (p.n_units + split - 1) / split;
-        const int64_t cost = span + 12 + 18 * ((span + p.n_units - 2) / p.n_units);
-        if (all < 0x7fffffff && cost * 21 < rounds * (per + 12) * 20) return mortar_span_grid(p, all, (int)span);
+        const int norm = p.norm ? 7 : 0;
+        const int64_t cost = span + 12 + norm + (18 + norm) * ((span + p.n_units - 2) / p.n_units);
+        if (all < 0x7fffffff && cost * 21 < rounds * (per + 12 + norm) * 20) return mortar_span_grid(p, all, (int)span);
     }
     return mortar_grid_width(p, layers);
 }

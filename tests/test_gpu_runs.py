@@ -45,7 +45,7 @@ def test_spmm_runs(dev, Rb, Cb, M, one_scale, prefill_stream):
                                               (1280, 3200, 32 * 141 - 19, False, True), (768, 2048, 9000, False, False), (768, 2048, 9000, True, True),
                                               (16 * 161, 16 * 688, 1300, False, True)])
 def test_mlp_runs(dev, d, f, M, norm, gated):
-    upw, span = prefill_form(1, M, f // 16, d // 16)
+    upw, span = prefill_form(2 if norm else 1, M, f // 16, d // 16)
     assert span > 0 and upw == (2 if d > 2048 else 0)
     if d == 1280:
         assert prefill_form(0, M, d // 16, f // 16, tiled=True) == (4, 3)

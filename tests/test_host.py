@@ -78,6 +78,15 @@ def test_form_of_a_k_segmented_prefill(kind, tiled, upws, run, stage, unit):
     assert prefill_form(kind, 1 << 30, 1200, 200, tiled)[1] == 0        # more rows of units than 31 bits
 
 
+def test_form_of_a_prefill_with_all_of_k_in_a_tile():
+    """Runs where whole groups fill a round badly; the norm in the staging moves the line."""
+    for d, f, M, plain, normed in ((2048, 5632, 4500, 194, 194), (2048, 5632, 3000, 130, 130), (2048, 5632, 3300, 143, 0), (1024, 2816, 6000, 65, 0),
+                                   (1024, 2816, 9000, 97, 97), (1536, 4096, 3000, 94, 94), (2048, 5632, 4096, 0, 0), (768, 2048, 16384, 0, 0)):
+        assert prefill_form(1, M, f // 16, d // 16) == (0, plain) and prefill_form(2, M, f // 16, d // 16) == (0, normed), (d, M)
+    with pytest.raises(ValueError):
+        prefill_form(2, 5000, 512, 192)
+
+
 def test_uniform_scale_is_detected():
     codes = np.ones((5, 16, 16), np.int8)
     L = _lib.lib()

@@ -35,7 +35,8 @@ def oracle_spmm(x, m):
 
 
 def prefill_form(kind, M, n_units, Cb, tiled=False):
-    """(units per wave, 0 for a tile of all K; length of the runs, 0 for whole groups) of a prefill-sized launch: kind 0 plain, 1 gate_up, 3 masked."""
+    """(units per wave, 0 for a tile of all K; length of the runs, 0 for whole groups) of a prefill-sized launch: kind 0 plain, 1 gate_up, 2 gate_up
+    with the norm in it, 3 masked."""
     L, upw, span = _lib.lib(), C.c_int32(), C.c_int32()
     _lib.check(L.mortar_prefill_form_host(kind, M, n_units, Cb, L.mortar_prefill_max_seg_cb(), int(tiled), C.byref(upw), C.byref(span)), "prefill_form")
     return upw.value, span.value
