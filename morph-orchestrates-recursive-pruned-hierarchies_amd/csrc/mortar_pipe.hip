@@ -21,8 +21,9 @@ constexpr int PIPE_WAVES = 16, PIPE_MT = 16;
 constexpr int PIPE_KQ = 5;        // 16-byte pieces per lane of a segment's tile: 16 waves x 5 x 2 block-columns >= the widest segment (155)
 
 // NACC rows per unit (1 plain, 2 gate/up).  PW waves per unit: one wave takes all its rows, two or four take a row, or a run of a row's
-// octets, each.  MASKED: x is zero where the input mask is (plain products).
-template <int NACC, bool MASKED, int PW, int CODE>
+// octets, each.  MASKED: x is zero where the input mask is (plain products).  HC: the results go into the POST write (kernels of their own: its code in the
+// epilogue of the others cost them 0.05 to 0.15 us).
+template <int NACC, bool MASKED, int PW, int CODE, bool HC>
 __global__ void __launch_bounds__(PIPE_WAVES * 64) mortar_pipe_kernel(const SpmmParams p0) {
     constexpr int UW = PIPE_WAVES / PW, RW = PW == 1 ? NACC : 1, CS = PW == 1 ? 1 : PW / NACC;
     static_assert(PW == 1 || PW % NACC == 0, "a wave takes a unit, a row or a run of a row's octets");
@@ -138,18 +139,18 @@ __global__ void __launch_bounds__(PIPE_WAVES * 64) mortar_pipe_kernel(const Spmm
 #pragma unroll
             for (int w = 1; w < CS; ++w) s[a][0] += red[(wave + a * CS + w) * 64 + lane];
         }
-        mortar_store_tile<1, NACC, CODE, NACC == 1>(p, unit, m0, tk, PIPE_MT, n, g, has_gates, s[0], s[NACC - 1]);
+        mortar_store_tile<1, NACC, CODE, HC>(p, unit, m0, tk, PIPE_MT, n, g, has_gates, s[0], s[NACC - 1]);
     } else if (unit >= 0) {
-        mortar_store_tile<1, NACC, CODE, NACC == 1>(p, unit, m0, tk, PIPE_MT, n, g, has_gates, acc[0], acc[RW - 1]);
+        mortar_store_tile<1, NACC, CODE, HC>(p, unit, m0, tk, PIPE_MT, n, g, has_gates, acc[0], acc[RW - 1]);
     }
 }
 
-template <int NACC, bool MASKED, int PW, int CODE>
+template <int NACC, bool MASKED, int PW, int CODE, bool HC = false>
 int launch(SpmmParams &p, hipStream_t st) {
     const int smem = 2 * tile_bytes(PIPE_MT, p.seg_cb) > PIPE_WAVES * 1024 ? 2 * tile_bytes(PIPE_MT, p.seg_cb) : PIPE_WAVES * 1024;
     if (p.seg_cb > PIPE_KQ * PIPE_WAVES * 2 || smem > 160 * 1024) return mortar_fail(MORTAR_ERR_LIMIT, "segment of %d block-columns does not fit", p.seg_cb);
     static bool attr_done = false;
-    auto kern = mortar_pipe_kernel<NACC, MASKED, PW, CODE>;
+    auto kern = mortar_pipe_kernel<NACC, MASKED, PW, CODE, HC>;
     int rc = mortar_allow_big_lds(kern, attr_done);
     if (rc) return rc;
     p.n_mtiles = (p.M + PIPE_MT - 1) / PIPE_MT;
@@ -170,6 +171,10 @@ int launch(SpmmParams &p, hipStream_t st) {
 
 template <int NACC, bool MASKED, int CODE>
 int launch_waves(int pw, SpmmParams &p, hipStream_t st) {
+    if constexpr (NACC == 1) {
+        if (p.hc_h)
+            return pw == 4 ? launch<1, MASKED, 4, CODE, true>(p, st) : pw == 2 ? launch<1, MASKED, 2, CODE, true>(p, st) : launch<1, MASKED, 1, CODE, true>(p, st);
+    }
     return pw == 4 ? launch<NACC, MASKED, 4, CODE>(p, st) : pw == 2 ? launch<NACC, MASKED, 2, CODE>(p, st) : launch<NACC, MASKED, 1, CODE>(p, st);
 }
 
